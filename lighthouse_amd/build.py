@@ -19,7 +19,15 @@ LIB_DIR = ROOT / "lighthouse_amd" / "lib"
 LIB_PATH = LIB_DIR / "liblighthouse_hip.so"
 PROBE_LIB = LIB_DIR / "liblighthouse_probe.so"  # bench.py's MFMA-rate probe, not part of the product library
 
-HIP_SOURCES = ["runtime.hip", "gemm16.hip", "gemm32.hip", "gemm8.hip", "attention.hip", "rowwise.hip", "api.hip"]
+HIP_SOURCES = ["runtime.hip", "gemm16.hip", "gemm16_direct.hip", "gemm32.hip", "gemm8.hip", "gemm_small.hip", "attention.hip", "rowwise.hip", "api.hip"]
+
+# Sources compiled more than once, with different macros: {source: {suffix of the object: macros}}.
+INSTANCES = {
+    "gemm16_direct.hip": {
+        f"_{dt}_{tm}{tn}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", f"-DLH_GEMM16_TM={tm}", f"-DLH_GEMM16_TN={tn}"]
+        for dt in ("bf16", "f16") for tm, tn in ((4, 2), (4, 1), (2, 2), (2, 1), (0, 0))
+    },
+}
 
 HIPCC_FLAGS = [
     "-O3",
@@ -48,17 +56,19 @@ def build_hip(verbose: bool = False) -> Path:
     obj_dir.mkdir(parents=True, exist_ok=True)
     LIB_DIR.mkdir(parents=True, exist_ok=True)
 
-    def compile_one(src: str) -> str:
-        obj = obj_dir / (Path(src).stem + ".o")
-        cmd = [hipcc, *HIPCC_FLAGS, "-c", str(CSRC / src), "-o", str(obj)]
+    def compile_one(src: str, suffix: str = "", macros: tuple = ()) -> str:
+        obj = obj_dir / (Path(src).stem + suffix + ".o")
+        cmd = [hipcc, *HIPCC_FLAGS, *macros, "-c", str(CSRC / src), "-o", str(obj)]
         if verbose:
             print(" ".join(cmd), flush=True)
         _run(cmd)
         return str(obj)
 
-    with ThreadPoolExecutor(max_workers=min(8, len(HIP_SOURCES) + 1)) as pool:
+    jobs = [(src, suffix, macros) for src, many in INSTANCES.items() for suffix, macros in many.items()]
+    jobs += [(src, "", ()) for src in HIP_SOURCES if src not in INSTANCES]
+    with ThreadPoolExecutor(max_workers=8) as pool:
         probe = pool.submit(compile_one, "probe.hip")
-        objs = list(pool.map(compile_one, HIP_SOURCES))
+        objs = list(pool.map(lambda job: compile_one(*job), jobs))
         probe_obj = probe.result()
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", str(LIB_PATH)])
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", probe_obj, "-o", str(PROBE_LIB)])

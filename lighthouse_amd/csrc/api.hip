@@ -243,6 +243,10 @@ int lh_hip_gemm_fp8_ws(void* out, const void* a_q, const void* b_q, float scale_
   if (!(out_dtype == LH_BF16 || out_dtype == LH_F32))
     return fail(LH_ERR_UNSUPPORTED, "lh_hip_gemm_fp8_ws: out dtype %d must be bf16 or f32", out_dtype);
   if ((rc = workspace_checks("lh_hip_gemm_fp8_ws", workspace, workspace_bytes))) return rc;
+  const size_t need = lh_hip_gemm_fp8_workspace_bytes(M, N, K, lda, ldb, ldc, out_dtype);
+  LH_REQUIRE(need <= workspace_bytes,
+             "lh_hip_gemm_fp8_ws: workspace too small: this call needs %zu bytes of temporary memory, %zu were given", need,
+             workspace_bytes);
   Scratch ws;
   ws.base = workspace ? static_cast<char*>(workspace) : reinterpret_cast<char*>(uintptr_t(256));
   ws.bytes = workspace_bytes;

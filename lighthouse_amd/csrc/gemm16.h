@@ -1,0 +1,48 @@
+// Shared by the 16-bit GEMM sources: the matrix instructions and the launches of the direct-to-LDS kernels.
+#pragma once
+
+#include "gemm_common.h"
+
+namespace lh {
+
+template <int DT>
+struct Mfma16;
+template <>
+struct Mfma16<LH_BF16> {
+  __device__ static __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+  }
+  __device__ static __forceinline__ f32x4 mma16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+  }
+};
+template <>
+struct Mfma16<LH_F16> {
+  __device__ static __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+  }
+  __device__ static __forceinline__ f32x4 mma16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                  0);
+  }
+};
+
+// The direct kernels address a tile's operand panels with 32-bit byte offsets from the panel's
+// first element: 256 rows of A, K rows of B.
+static inline bool direct_offsets_fit(const GemmArgs& g) {
+  if (g.flags & LH_GEMM_TRANSPOSE_B) return g.lda < (1ll << 22) && g.ldb < (1ll << 22);  // 256 rows of B^T
+  return g.lda < (1ll << 22) && (int64_t)g.K * g.ldb < (1ll << 30);
+}
+
+// Launch of the direct-to-LDS kernel with a workgroup tile of (64 TM) x (128 TN) (gemm16_direct.hip; each
+// combination is an object of its own).
+template <int DT, int TM, int TN>
+int launch_direct(const GemmArgs& g, hipStream_t s);
+// The 128 x 128 tile on `g.splits` pieces of K, each with an f32 block of the output of its own.
+template <int DT>
+int launch_direct_splitk(const GemmArgs& g, hipStream_t s);
+
+}  // namespace lh

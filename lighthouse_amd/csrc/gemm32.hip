@@ -333,9 +333,29 @@ __global__ void __launch_bounds__(256) gemm32_generic(GemmArgs g) {
   }
 }
 
+// Time of an untransposed, aligned problem on the 64 x 64 tile kernels, in us, where few tiles make it
+// latency-bound (median 0.97 of the measured time on the problems of gemm_small.hip's fit, nine in ten between 0.88
+// and 1.04).
+static double direct32_us(const GemmArgs& g) {
+  const double x = (double)((g.M + 63) / 64) * ((g.N + 63) / 64) / num_cus();
+  return 3.6 + 0.0156 * g.K * (x <= 1.0 ? 1.0 : x <= 2.0 ? 2.0 : 1.1 * x);
+}
+
 int gemm32(const GemmArgs& g_in, hipStream_t s) {
   GemmArgs g = g_in;
   const uint32_t tile = g.flags & LH_GEMM_TILE_MASK;
+  if (tile == LH_GEMM_TILE_AUTO && !planning()) {
+    // Few tiles: the small-tile kernels, if they are the faster ones; against them stand the direct kernels plus the
+    // transposed or padded copies those would need.
+    const bool trans = g.flags & (LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
+    const bool fits = g.K % kBK32 == 0 && g.N % 4 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && g.ldc % 4 == 0 &&
+                      aligned16(g.a) && aligned16(g.b) && aligned16(g.out) && (!g.bias || aligned16(g.bias));
+    const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
+    const double other = direct32_us(g) + (!fits ? 14.0 + 6.0 * mb + 6e-6 * g.M * g.N : trans ? 4.0 + 3.2 * mb : 0.0);
+    int small;
+    const double us = gemm_small_choose(g, LH_F32, &small);
+    if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F32, small, s);
+  }
   if (tile == LH_GEMM_TILE_AUTO && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias))) {
     const int rc = untranspose_operands<4>(g, kBK32, 4, s);
     if (rc < 0) return rc;

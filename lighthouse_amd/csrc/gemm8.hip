@@ -908,12 +908,19 @@ static int skinny_partial_buffer(const GemmArgs& g, hipStream_t s, size_t need, 
   return LH_OK;
 }
 
+// Splits of the decode kernels' K: about one workgroup per CU, whole k-steps each (0: the M <= 16 kernel's A area
+// cannot hold the share of one workgroup).
+static int skinny_splits(int M, int N, int K) {
+  const int nblk = N / kSkinnyBN;
+  int splits = 1;
+  while ((nblk * splits < num_cus() || (M <= 16 && K / splits > kSkinnyMaxChunk)) && (K / kBK8) % (splits * 2) == 0) splits *= 2;
+  return M <= 16 && K / splits > kSkinnyMaxChunk ? 0 : splits;
+}
+
 template <int MT>
 static int launch_skinny_mt(const GemmArgs& g, hipStream_t s) {
-  // Split K until about one workgroup per CU streams B.
   const int nblk = g.N / kSkinnyBN;
-  int splits = 1;
-  while (nblk * splits < num_cus() && (g.K / kBK8) % (splits * 2) == 0) splits *= 2;
+  const int splits = skinny_splits(g.M, g.N, g.K);
   float* g_partial = nullptr;
   int rc = skinny_partial_buffer(g, s, (size_t)splits * 16 * MT * g.N * sizeof(float), &g_partial);
   if (rc) return rc;
@@ -934,7 +941,34 @@ static int launch_skinny_mt(const GemmArgs& g, hipStream_t s) {
   return check_launch("gemm8_skinny_reduce");
 }
 
+// Time of an aligned problem on the kernels below, in us, where few tiles make it latency-bound (median 1.09 of the
+// measured time on the problems of gemm_small.hip's fit, nine in ten between 0.83 and 1.30).
+static double tile8_us(const GemmArgs& g) {
+  if (g.M <= 128 && g.N % kSkinnyBN == 0) {
+    const int splits = skinny_splits(g.M, g.N, g.K);
+    const double share = splits ? (double)(g.N / kSkinnyBN) * splits / num_cus() : 0.0;  // of the CUs that stream B
+    if (splits) {
+      const double stream = (double)g.N * g.K / 5.6e6 / (share < 1.0 ? share : 1.0);
+      if (g.M <= 16) return 4.4 + stream;
+      return 5.0 + 0.0022 * g.K * (g.M <= 32 ? 1.0 : g.M <= 64 ? 1.3 : 1.9) + stream + 8e-6 * g.M * g.N;
+    }
+  }
+  const double x = (double)((g.M + 127) / 128) * ((g.N + 127) / 128) / num_cus();
+  return 4.6 + 0.0078 * g.K * (x > 1.0 ? x : 1.0) + (x > 1.0 ? 0.6 * (x - 1.0) : 0.0);
+}
+
 int gemm8(const GemmArgs& g, hipStream_t s) {
+  if (!planning()) {
+    // Few tiles: the small-tile kernels, if they are the faster ones; against them stand the kernels below plus the
+    // padded copies those would need.
+    const bool fits = g.K % kBK8 == 0 && g.N % 128 == 0 && g.lda % 16 == 0 && g.ldb % 4 == 0 && g.ldc % 4 == 0 &&
+                      aligned16(g.a) && aligned16(g.b) && aligned16(g.out);
+    const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
+    const double other = tile8_us(g) + (!fits ? 14.0 + 2.0 * mb + 4e-6 * g.M * g.N : 0.0);
+    int small;
+    const double us = gemm_small_choose(g, LH_F8E4M3, &small);
+    if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F8E4M3, small, s);
+  }
   const bool vec_ok = g.K % kBK8 == 0 && g.lda % 16 == 0 && g.ldb % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.a) &&
                       aligned16(g.b) && aligned16(g.out);
   if (!(vec_ok && g.N % 128 == 0) && (int64_t)g.M * g.N * g.K >= (1 << 22)) {
@@ -946,9 +980,8 @@ int gemm8(const GemmArgs& g, hipStream_t s) {
     // Split K so that about one workgroup per CU streams B (its ring alone keeps 96 KiB in
     // flight) and the A chunk fits its LDS area.
     const int nblk = g.N / kSkinnyBN;
-    int splits = 1;
-    while ((nblk * splits < num_cus() || g.K / splits > kSkinnyMaxChunk) && (g.K / kBK8) % (splits * 2) == 0) splits *= 2;
-    if (g.K / splits <= kSkinnyMaxChunk) {
+    const int splits = skinny_splits(g.M, g.N, g.K);
+    if (splits) {
       float* g_partial = nullptr;
       int prc = skinny_partial_buffer(g, s, (size_t)splits * 16 * g.N * sizeof(float), &g_partial);
       if (prc) return prc;

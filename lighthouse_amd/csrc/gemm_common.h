@@ -377,8 +377,62 @@ __device__ __forceinline__ void epilogue1(const GemmArgs& g, int m, int n, float
   else store_from_f32<DT>(g.out, off, x);
 }
 
+// Vectors of 4 output-side elements at element alignment (gfx9 global memory takes any alignment): the
+// outputs, biases and accumulator inputs of problems whose N or row stride is odd.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+
+// Epilogue for columns n .. n + 3 of row m, of which those below N exist.
+template <int DT>
+__device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, const f32x4& acc) {
+  if (n + 4 > g.N) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < g.N) epilogue1<DT>(g, m, n + e, acc[e]);
+    return;
+  }
+  float v[4] = {acc[0] * g.alpha, acc[1] * g.alpha, acc[2] * g.alpha, acc[3] * g.alpha};
+  const int64_t off = (int64_t)m * g.ldc + n;
+  auto load4 = [&](const void* p, int64_t at, int dt) -> f32x4 {
+    if (dt == LH_F32) return *reinterpret_cast<const f32x4_any*>(reinterpret_cast<const float*>(p) + at);
+    const u32x2 w = *reinterpret_cast<const u32x2_any*>(reinterpret_cast<const uint16_t*>(p) + at);
+    return f32x4{unpack_lo<DT>(w[0]), unpack_hi<DT>(w[0]), unpack_lo<DT>(w[1]), unpack_hi<DT>(w[1])};
+  };
+  if (g.flags & LH_GEMM_ACCUMULATE_C) {
+    const f32x4 c = load4(g.c, off, g.out_dt);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += c[e];
+  }
+  if (g.flags & LH_GEMM_HAS_BIAS) {
+    const f32x4 b = load4(g.bias, n, g.bias_dt);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += b[e];
+  }
+  if (g.flags & LH_GEMM_HAS_GELU) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
+  }
+  if (g.flags & LH_GEMM_HAS_RELU) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = relu_nan(v[e]);
+  }
+  if (g.out_dt == LH_F32)
+    *reinterpret_cast<f32x4_any*>(reinterpret_cast<float*>(g.out) + off) = f32x4{v[0], v[1], v[2], v[3]};
+  else if constexpr (DT != LH_F32)
+    *reinterpret_cast<u32x2_any*>(reinterpret_cast<uint16_t*>(g.out) + off) = u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+}
+
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s);
 int gemm32(const GemmArgs& g, hipStream_t s);
 int gemm8(const GemmArgs& g, hipStream_t s);
+// Kernels for problems with few output tiles (gemm_small.hip): the tile they would use (-1: none fits the
+// problem) with an estimate of its time in us, and the launch.  They need no temporary memory and take any
+// alignment; a workspace query (planning()) does not ask, so that its figure is an upper bound that does
+// not depend on which kernel is the faster one.
+double gemm_small_choose(const GemmArgs& g, int dtype, int* tile);
+// They are taken where their estimate is below the other kernels' by more than the two estimates' error: in a tie
+// the tile kernels stay, which add up k in one order whatever the tile.
+constexpr double kSmallMargin = 1.08;
+int gemm_small(const GemmArgs& g, int dtype, int tile, hipStream_t s);
 
 }  // namespace lh

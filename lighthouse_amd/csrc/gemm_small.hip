@@ -1,0 +1,421 @@
+// GEMM for problems with few output tiles, any operand layout and alignment: 16-bit, f32 and fp8 inputs
+// with the fused epilogue of the matmul payload (emit_mlp_layer,
+// lighthouse/ingress/mlir_gen/gpu_mlp_payload.py:110-156).
+//
+// What bounds a GEMM of a few dozen to a few hundred rows is not arithmetic but the chain of dependent
+// steps one workgroup walks: on the 128 x 128 tile kernel, M = 100, N = 2304, K = 768 is 18 workgroups that
+// each take 24 k-steps one after the other behind barriers (14 us).  Here a workgroup owns a small tile
+// (16 MT x 16 NT) and its NW waves share out the K dimension: wave w multiplies the k-steps w, w + NW, ...
+// on its own, without a barrier, with P steps of both operands requested ahead in registers; the NW
+// partial tiles are added through LDS once, in wave order.  A step is 64 bytes of k per row for every
+// element type (32 values of 16 bit, 64 of fp8, 16 of f32): a lane's operand is one 16-byte chunk.
+//
+//  * A k-contiguous operand (A stored [M, K], B stored [N, K]) is loaded straight into the MFMA's operand
+//    layout and never touches LDS.
+//  * An operand contiguous along M or N (A stored [K, M], B stored [K, N]) goes through a few KiB of LDS
+//    that belong to the wave alone and is read back with the transposing LDS reads.
+//
+// Global accesses are 16 bytes wide at element alignment (gfx9 global memory takes any alignment), so odd
+// leading dimensions and unaligned views need no padded copies; everything past K counts as zero.
+#include <cmath>
+#include <type_traits>
+
+#include "gemm_common.h"
+
+namespace lh {
+
+template <int ES>
+struct Chunk;  // 16 bytes at element alignment
+template <>
+struct Chunk<1> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(1))); typedef uint8_t elem; };
+template <>
+struct Chunk<2> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2))); typedef uint16_t elem; };
+template <>
+struct Chunk<4> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); typedef uint32_t elem; };
+
+typedef short small_s16x4 __attribute__((ext_vector_type(4)));
+typedef int small_i32x2 __attribute__((ext_vector_type(2)));
+
+// c += a b for one step: the lane's 16-byte chunks of a row of each operand (lane / 16 selects the chunk of
+// the step's four).  First operand = B fragment: a lane's result is 4 consecutive columns of one row.
+template <int DT>
+__device__ __forceinline__ f32x4 small_mma(u32x4 b, u32x4 a, f32x4 c) {
+  if constexpr (DT == LH_BF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
+  } else if constexpr (DT == LH_F16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
+  } else if constexpr (DT == LH_F8E4M3) {
+    typedef long l2 __attribute__((ext_vector_type(2)));
+    const l2 bl = __builtin_bit_cast(l2, b), al = __builtin_bit_cast(l2, a);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(bl[0], al[0], c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(bl[1], al[1], c, 0, 0, 0);
+  } else {
+    const f32x4 bf = __builtin_bit_cast(f32x4, b), af = __builtin_bit_cast(f32x4, a);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) c = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[t], af[t], c, 0, 0, 0);
+    return c;
+  }
+}
+
+template <int DT>
+constexpr int small_elem_bytes() { return DT == LH_F32 ? 4 : DT == LH_F8E4M3 ? 1 : 2; }
+
+// The chunk moved down by `n` elements (0 .. EPC, or more: nothing is left), zeros on top.
+template <int ES>
+__device__ __forceinline__ u32x4 small_shift_chunk(u32x4 c, int n) {
+  const int bytes = ES * n;
+  uint32_t d0 = c[0], d1 = c[1], d2 = c[2], d3 = c[3];
+  const bool by8 = bytes & 8, by4 = bytes & 4, all = bytes >= 16;
+  d0 = by8 ? d2 : d0;
+  d1 = by8 ? d3 : d1;
+  d2 = by8 ? 0u : d2;
+  d3 = by8 ? 0u : d3;
+  d0 = by4 ? d1 : d0;
+  d1 = by4 ? d2 : d1;
+  d2 = by4 ? d3 : d2;
+  d3 = by4 ? 0u : d3;
+  const int b = bytes & 3;
+  d0 = __builtin_amdgcn_alignbyte(d1, d0, b);
+  d1 = __builtin_amdgcn_alignbyte(d2, d1, b);
+  d2 = __builtin_amdgcn_alignbyte(d3, d2, b);
+  d3 = __builtin_amdgcn_alignbyte(0u, d3, b);
+  return u32x4{all ? 0u : d0, all ? 0u : d1, all ? 0u : d2, all ? 0u : d3};
+}
+
+// One operand panel of F fragments of 16 rows (A) or columns (B), k-contiguous (KC) or not.  Every load of
+// a step is one 16-byte access whatever the sizes: a chunk that would cross the end of its row is read
+// from the row's last EPC elements instead and moved down in registers (the contiguous dimension has at
+// least EPC elements), so the number of loads in flight is known at compile time and the waits stay exact.
+template <int DT, int F, bool KC>
+struct SmallPanel {
+  static constexpr int ES = small_elem_bytes<DT>(), EPC = 16 / ES, KSTEP = 64 / ES;
+  static constexpr int CPR = F * ES;             // !KC: 16-byte chunks per k row
+  static constexpr int RPL = 64 / CPR;           // !KC: k rows per load
+  static constexpr int RS = CPR * 16 + 16;       // !KC: bytes of a k row in LDS (one chunk of padding)
+  static constexpr int kLdsBytes = KC ? 0 : KSTEP * RS;
+  const uint8_t* base[KC ? F : 1];  // KC: the lane's chunk of its row in each fragment; !KC: of its first k row
+  int64_t ld_bytes;
+  int over = 0;              // !KC: elements by which the lane's chunk was moved back to stay inside the row
+  bool whole = true;         // !KC: (wave-uniform) no chunk of the panel was moved
+
+  // `p`: the operand as stored; `first`: the panel's first row / column; `count`: rows / columns of the
+  // matrix; `ld`: stored row stride.
+  __device__ __forceinline__ void place(const void* p, int first, int count, int64_t ld, int lane) {
+    ld_bytes = ld * ES;
+    const uint8_t* b = reinterpret_cast<const uint8_t*>(p);
+    if constexpr (KC) {
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        base[f] = b + (int64_t)min(first + 16 * f + (lane & 15), count - 1) * ld_bytes + (lane >> 4) * 16;
+    } else {
+      const int c = first + (lane % CPR) * EPC, cc = min(c, count - EPC);
+      over = c - cc;
+      whole = first + 16 * F <= count;
+      base[0] = b + (int64_t)(lane / CPR) * ld_bytes + (int64_t)cc * ES;
+    }
+  }
+  // Request the step at k0, all of it below K.
+  __device__ __forceinline__ void load(int k0, u32x4 (&r)[F]) const {
+    typedef typename Chunk<ES>::type C;
+    if constexpr (KC) {
+#pragma unroll
+      for (int f = 0; f < F; ++f) r[f] = *reinterpret_cast<const C*>(base[f] + (int64_t)k0 * ES);
+    } else {
+      const uint8_t* p = base[0] + (int64_t)k0 * ld_bytes;
+#pragma unroll
+      for (int f = 0; f < F; ++f) r[f] = *reinterpret_cast<const C*>(p + (int64_t)(f * RPL) * ld_bytes);
+    }
+  }
+  // Request the step at k0 that K ends in; `finish_tail` turns what lies past K into zeros.
+  __device__ __forceinline__ void load_tail(int k0, int K, int lane, u32x4 (&r)[F]) const {
+    typedef typename Chunk<ES>::type C;
+    if constexpr (KC) {
+      const int k = k0 + (lane >> 4) * EPC, back = max(k - (K - EPC), 0);
+#pragma unroll
+      for (int f = 0; f < F; ++f) r[f] = *reinterpret_cast<const C*>(base[f] + (int64_t)(k0 - back) * ES);
+    } else {
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        const int row = lane / CPR, k = min(k0 + f * RPL + row, K - 1) - row;
+        r[f] = *reinterpret_cast<const C*>(base[0] + (int64_t)k * ld_bytes);
+      }
+    }
+  }
+  __device__ __forceinline__ void finish_tail(int k0, int K, int lane, u32x4 (&r)[F]) const {
+    if constexpr (KC) {
+      const int k = k0 + (lane >> 4) * EPC, back = max(k - (K - EPC), 0);
+#pragma unroll
+      for (int f = 0; f < F; ++f) r[f] = small_shift_chunk<ES>(r[f], back);
+    } else {
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        if (k0 + f * RPL + lane / CPR >= K) r[f] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  // The step's fragments: the registers themselves (KC), or through the wave's LDS area.
+  template <bool WHOLE>
+  __device__ __forceinline__ void fragments(u32x4 (&r)[F], uint8_t* lds, int lane, u32x4 (&frag)[F]) const {
+    if constexpr (KC) {
+#pragma unroll
+      for (int f = 0; f < F; ++f) frag[f] = r[f];
+    } else {
+      const int l16 = lane & 15, g4 = lane >> 4;
+      if constexpr (!WHOLE) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) r[f] = small_shift_chunk<ES>(r[f], over);
+      }
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        *reinterpret_cast<u32x4*>(lds + (f * RPL + lane / CPR) * RS + (lane % CPR) * 16) = r[f];
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        if constexpr (ES == 2) {
+          // 16 lanes of group g4: k rows 8 g4 + l16 / 4 (+4), columns 16 f + 4 (l16 % 4) .. +4
+          uint8_t* p0 = lds + (8 * g4 + (l16 >> 2)) * RS + 32 * f + 8 * (l16 & 3);
+          const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                         (__attribute__((address_space(3))) small_s16x4*)p0));
+          const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                         (__attribute__((address_space(3))) small_s16x4*)(p0 + 4 * RS)));
+          frag[f] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        } else if constexpr (ES == 1) {
+          // k rows 16 g4 + l16 / 2 (+8), bytes 16 f + 8 (l16 % 2) .. +8
+          uint8_t* p0 = lds + (16 * g4 + (l16 >> 1)) * RS + 16 * f + 8 * (l16 & 1);
+          const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                                                         (__attribute__((address_space(3))) small_i32x2*)p0));
+          const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+                                                         (__attribute__((address_space(3))) small_i32x2*)(p0 + 8 * RS)));
+          frag[f] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            frag[f][t] = *reinterpret_cast<const uint32_t*>(lds + (4 * g4 + t) * RS + (16 * f + l16) * 4);
+        }
+      }
+    }
+  }
+};
+
+template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
+struct SmallCfg {
+  typedef SmallPanel<DT, MT, AKC> PA;
+  typedef SmallPanel<DT, NT, BKC> PB;
+  static constexpr int kWaveLds = PA::kLdsBytes + PB::kLdsBytes;
+  static constexpr int kSumBytes = NW * MT * NT * 1024;
+  static constexpr int kLdsBytes = kSumBytes > NW * kWaveLds ? kSumBytes : NW * kWaveLds;
+  // Steps requested ahead: what fits next to the accumulators in the registers of NW waves.
+  static constexpr int P = MT + NT <= 3 ? 3 : 2;
+};
+
+// The wave's share of the k-steps.
+template <typename Cfg, int DT, int MT, int NT, int NW, bool WHOLE>
+__device__ __forceinline__ void small_multiply(const typename Cfg::PA& pa, const typename Cfg::PB& pb, f32x4 (&acc)[MT][NT],
+                                               int K, int wave, int lane, uint8_t* lds_a, uint8_t* lds_b) {
+  constexpr int P = Cfg::P, KSTEP = Cfg::PA::KSTEP;
+  // Its list of steps: the one K ends in first (if it is not whole: the last wave's, whose share of the
+  // others is the smallest), then its contiguous share of the whole steps.
+  const int full = K / KSTEP;
+  const int begin = (full * wave + NW - 1) / NW;
+  const bool tail = K % KSTEP != 0 && wave == NW - 1;
+  const int mine = (tail ? 1 : 0) + (full * (wave + 1) + NW - 1) / NW - begin;
+  const int first = tail ? begin - 1 : begin;  // step i of the list is step first + i of K (the tail apart)
+  if (mine == 0) return;
+  u32x4 ra[P][MT], rb[P][NT];
+  auto consume = [&](u32x4 (&a)[MT], u32x4 (&b)[NT]) {
+    u32x4 fa[MT], fb[NT];
+    pb.template fragments<WHOLE>(b, lds_b, lane, fb);
+    pa.template fragments<WHOLE>(a, lds_a, lane, fa);
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) acc[j][i] = small_mma<DT>(fb[i], fa[j], acc[j][i]);
+  };
+  if (tail) {
+    pa.load_tail(full * KSTEP, K, lane, ra[0]);
+    pb.load_tail(full * KSTEP, K, lane, rb[0]);
+  } else {
+    pa.load(first * KSTEP, ra[0]);
+    pb.load(first * KSTEP, rb[0]);
+  }
+#pragma unroll
+  for (int p = 1; p < P; ++p)
+    if (p < mine) {
+      pa.load((first + p) * KSTEP, ra[p]);
+      pb.load((first + p) * KSTEP, rb[p]);
+    }
+  if (tail) {
+    pa.finish_tail(full * KSTEP, K, lane, ra[0]);
+    pb.finish_tail(full * KSTEP, K, lane, rb[0]);
+  }
+  // Steps i .. i + n - 1 of the list, the first P of them requested already: in straight-line code the
+  // number of loads in flight is known and a step waits for its own loads only.
+  int i = 0;
+  auto run = [&](auto count) {
+    constexpr int n = decltype(count)::value;
+#pragma unroll
+    for (int p = 0; p < n; ++p) {
+      consume(ra[p % P], rb[p % P]);
+      if (p + P < n) {
+        pa.load((first + i + P + p) * KSTEP, ra[p % P]);
+        pb.load((first + i + P + p) * KSTEP, rb[p % P]);
+      }
+    }
+  };
+#pragma unroll 1
+  for (; i + 2 * P <= mine; i += P) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      consume(ra[p], rb[p]);
+      pa.load((first + i + P + p) * KSTEP, ra[p]);
+      pb.load((first + i + P + p) * KSTEP, rb[p]);
+    }
+  }
+  const int left = mine - i;  // 1 .. 2 P - 1
+  if (left == 1) run(std::integral_constant<int, 1>{});
+  else if (left == 2) run(std::integral_constant<int, 2>{});
+  else if (left == 3) run(std::integral_constant<int, 3>{});
+  else if (P == 3 && left == 4) run(std::integral_constant<int, P == 3 ? 4 : 1>{});
+  else if (P == 3) run(std::integral_constant<int, P == 3 ? 5 : 1>{});
+}
+
+template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
+__global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
+  typedef SmallCfg<DT, MT, NT, NW, AKC, BKC> Cfg;
+  constexpr int EDT = DT == LH_F8E4M3 ? LH_BF16 : DT;  // the type a 16-bit output, bias or accumulator input has
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem_small[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // The workgroups of one XCD (ids congruent modulo 8) take a contiguous range of the tiles counted down
+  // the columns: a B panel is read by one XCD's L2 (two at the ends of a range), neighbouring panels
+  // share its cache lines.
+  const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
+  const int per_xcd = (tiles_m * tiles_n + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (tile >= tiles_m * tiles_n) return;
+  const int m0 = (tile % tiles_m) * 16 * MT, n0 = (tile / tiles_m) * 16 * NT;
+
+  typename Cfg::PA pa;
+  typename Cfg::PB pb;
+  pa.place(g.a, m0, g.M, g.lda, lane);
+  pb.place(g.b, n0, g.N, g.ldb, lane);
+  uint8_t* const lds_a = smem_small + wave * Cfg::kWaveLds;
+  uint8_t* const lds_b = lds_a + Cfg::PA::kLdsBytes;
+
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // (the panels that end inside the tile take a copy of the loop of their own: no branch inside a step)
+  if ((AKC || pa.whole) && (BKC || pb.whole)) small_multiply<Cfg, DT, MT, NT, NW, true>(pa, pb, acc, g.K, wave, lane, lds_a, lds_b);
+  else small_multiply<Cfg, DT, MT, NT, NW, false>(pa, pb, acc, g.K, wave, lane, lds_a, lds_b);
+
+  // Sum over the waves: fragment f = j NT + i of wave w is 1 KiB at (w MT NT + f) 1024, 16 bytes per lane.
+  f32x4* const sums = reinterpret_cast<f32x4*>(smem_small);
+  if constexpr (Cfg::kWaveLds > 0) __syncthreads();  // (the areas overlap)
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) sums[(wave * MT * NT + j * NT + i) * 64 + lane] = acc[j][i];
+  __syncthreads();
+#pragma unroll
+  for (int e0 = 0; e0 < MT * NT * 64; e0 += NW * 64) {
+    const int e = e0 + tid;
+    if (MT * NT * 64 % (NW * 64) != 0 && e >= MT * NT * 64) break;
+    f32x4 v = sums[e];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += sums[w * MT * NT * 64 + e];
+    const int f = e >> 6, l = e & 63;
+    const int m = m0 + 16 * (f / NT) + (l & 15), n = n0 + 16 * (f % NT) + 4 * (l >> 4);
+    if (m < g.M && n < g.N) epilogue4_any<EDT>(g, m, n, v);
+  }
+}
+
+template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
+static int launch_small_layout(const GemmArgs& g, hipStream_t s) {
+  typedef SmallCfg<DT, MT, NT, NW, AKC, BKC> Cfg;
+  auto kern = gemm_small_kernel<DT, MT, NT, NW, AKC, BKC>;
+  static bool configured = false;
+  if (Cfg::kLdsBytes > 64 * 1024 && !configured && !planning()) {
+    LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     Cfg::kLdsBytes));
+    configured = true;
+  }
+  const int tiles = ((g.M + 16 * MT - 1) / (16 * MT)) * ((g.N + 16 * NT - 1) / (16 * NT));
+  LH_LAUNCH(kern, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(NW * 64), Cfg::kLdsBytes, s, g);
+  return check_launch("gemm_small");
+}
+
+template <int DT, int MT, int NT, int NW>
+static int launch_small(const GemmArgs& g, hipStream_t s) {
+  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
+  if (ta) return tb ? launch_small_layout<DT, MT, NT, NW, false, true>(g, s) : launch_small_layout<DT, MT, NT, NW, false, false>(g, s);
+  return tb ? launch_small_layout<DT, MT, NT, NW, true, true>(g, s) : launch_small_layout<DT, MT, NT, NW, true, false>(g, s);
+}
+
+// ---- choice of tile ---------------------------------------------------------------------------
+// Time of a launch, in us: kSmallFixed + r (b + c steps), r = workgroups per compute unit (at least 1), steps =
+// 64-byte steps of K.  What a step costs is the operand bytes the CU pulls from its L2 (about 20 bytes per
+// clock whatever the depth of the prefetch), so a larger tile costs less per result and more per workgroup:
+// the cheapest tile is about the largest that still gives every CU one.  b and c are least squares over 400
+// problems per type (M 1 .. 3000, N and K 16 .. 8192, both log-uniform); choosing by them is within 4 % of the
+// best tile on average.  Not for more than 4 workgroups per CU, where tiles whose waves share their operands win.
+struct SmallTile {
+  int mt, nt;
+  float b[3], c[3];  // 16-bit, f32, fp8
+};
+constexpr SmallTile kSmallTiles[] = {
+    {1, 1, {1.10f, 1.33f, 1.22f}, {0.0468f, 0.0392f, 0.0665f}},  // 16 waves
+    {1, 2, {0.74f, 0.93f, 0.80f}, {0.0586f, 0.0606f, 0.0700f}},  // 8 waves
+    {1, 4, {1.02f, 1.23f, 1.03f}, {0.0791f, 0.1047f, 0.0749f}},  // 8 waves
+    {2, 2, {0.93f, 1.16f, 1.00f}, {0.0720f, 0.0938f, 0.0829f}},  // 8 waves
+    {2, 4, {1.42f, 1.47f, 1.36f}, {0.1024f, 0.1819f, 0.0995f}},  // 4 waves
+    {4, 4, {2.40f, 2.90f, 2.40f}, {0.1200f, 0.3020f, 0.1200f}},  // 8 waves, whose sums fill a CU's LDS: whole rounds
+};
+constexpr float kSmallFixed = 2.0f;
+
+double gemm_small_choose(const GemmArgs& g, int dtype, int* tile) {
+  const int es = (int)dtype_size(dtype), epc = 16 / es, type = dtype == LH_F32 ? 1 : es == 1 ? 2 : 0;
+  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
+  *tile = -1;
+  // (every chunk load reads one whole chunk of a row; 32-bit step and tile counts)
+  if ((ta ? g.M : g.K) < epc || (tb ? g.K : g.N) < epc || g.K >= 1 << 24 || (int64_t)g.M * g.N >= 1ll << 36) return 0.0;
+  const int steps = (g.K + 64 / es - 1) / (64 / es);
+  const double stream = 1e-6 * es * ((double)g.M * g.K + (double)g.K * g.N) / 3.6;  // (each operand from memory once)
+  double best = 0.0;
+  for (int i = 0; i < (int)(sizeof(kSmallTiles) / sizeof(kSmallTiles[0])); ++i) {
+    const SmallTile& t = kSmallTiles[i];
+    const int64_t tiles = (int64_t)((g.M + 16 * t.mt - 1) / (16 * t.mt)) * ((g.N + 16 * t.nt - 1) / (16 * t.nt));
+    double r = tiles > num_cus() ? (double)tiles / num_cus() : 1.0;
+    if (t.mt * t.nt == 16) r = ceil(r);
+    const double us = kSmallFixed + fmax(r * (t.b[type] + t.c[type] * steps), stream);
+    if (r <= 4.0 && (*tile < 0 || us < best)) {
+      best = us;
+      *tile = i;
+    }
+  }
+  return best;
+}
+
+template <int DT>
+static int gemm_small_dispatch(const GemmArgs& g, int tile, hipStream_t s) {
+  switch (tile) {
+    case 0: return launch_small<DT, 1, 1, 16>(g, s);
+    case 1: return launch_small<DT, 1, 2, 8>(g, s);
+    case 2: return launch_small<DT, 1, 4, 8>(g, s);
+    case 3: return launch_small<DT, 2, 2, 8>(g, s);
+    case 4: return launch_small<DT, 2, 4, 4>(g, s);
+    default: return launch_small<DT, 4, 4, 8>(g, s);
+  }
+}
+
+int gemm_small(const GemmArgs& g, int dtype, int tile, hipStream_t s) {
+  switch (dtype) {
+    case LH_F32: return gemm_small_dispatch<LH_F32>(g, tile, s);
+    case LH_BF16: return gemm_small_dispatch<LH_BF16>(g, tile, s);
+    case LH_F16: return gemm_small_dispatch<LH_F16>(g, tile, s);
+    default: return gemm_small_dispatch<LH_F8E4M3>(g, tile, s);
+  }
+}
+
+}  // namespace lh

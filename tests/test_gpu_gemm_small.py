@@ -1,0 +1,55 @@
+"""The small-tile GEMM kernels: tile and K edges, every layout, unaligned views, each element type."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32, "fp8": torch.float8_e4m3fn}
+
+
+def _matrix(rows, cols, dtype, seed, pad):
+    """Integers -3 .. 3 as a column range of a wider matrix whose other columns hold NaN: a kernel that counts
+    anything outside the operand shows it."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    v = torch.randint(-3, 4, (rows, cols), device="cuda", generator=g).float()
+    buf = torch.full((rows, cols + 2 * pad), float("nan"), device="cuda").to(DTYPES[dtype])
+    buf[:, pad:pad + cols] = v.to(DTYPES[dtype])
+    return buf[:, pad:pad + cols], v
+
+
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("shape", [(16, 16, 16),       # one tile, less than a k-step of 16-bit values
+                                   (17, 65, 64),       # one past a tile in both directions
+                                   (33, 31, 63),       # K one short of a step
+                                   (100, 129, 65),     # ... and one past it
+                                   (1, 1000, 513), (250, 33, 1100), (64, 2050, 97),
+                                   (300, 300, 777)])   # the larger tiles
+def test_small_tiles(shape, dtype, layout, pad):
+    """Integer operands: the f32 sum is exact in any order, so the result has one right bit pattern."""
+    from lighthouse_amd import ops
+
+    M, N, K = shape
+    if dtype == "fp8" and layout != "nn":
+        pytest.skip("the fp8 entry point has no transposed form")
+    ta, tb = layout[0] == "t", layout[1] == "t"
+    a, av = _matrix(K if ta else M, M if ta else K, dtype, 1, pad)
+    b, bv = _matrix(N if tb else K, K if tb else N, dtype, 2, pad)
+    want = (av.T if ta else av).double() @ (bv.T if tb else bv).double()
+    out = torch.full((M, N + 2), 7.0, device="cuda")
+    view = out[:, :N]
+    if dtype == "fp8":
+        ops.gemm_fp8(a, b, 0.5, 2.0, out=view)
+        assert torch.equal(view.double(), want)
+    else:
+        bias = torch.arange(N, device="cuda").float() % 5 - 2
+        ops.gemm(a, b, bias, out=view, relu=True, transpose_a=ta, transpose_b=tb)
+        assert torch.equal(view.double(), torch.relu(want + bias.double()))
+        ops.gemm(a, b, out=view, accumulate_c=True, transpose_a=ta, transpose_b=tb)
+        assert torch.equal(view.double(), torch.relu(want + bias.double()) + want)
+        if dtype != "f32":  # 16-bit output: one rounding of the exact sum
+            got = ops.gemm(a, b, transpose_a=ta, transpose_b=tb)
+            assert torch.equal(got, want.to(DTYPES[dtype]))
+    assert bool((out[:, N:] == 7.0).all())
