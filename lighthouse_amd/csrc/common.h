@@ -64,6 +64,16 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x8 __attribute__((ext_vector_type(8)));
 
+// 16 bytes at the alignment of their elements of ES bytes (gfx9 global memory takes any alignment).
+template <int ES>
+struct Chunk;
+template <>
+struct Chunk<1> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(1))); };
+template <>
+struct Chunk<2> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2))); };
+template <>
+struct Chunk<4> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); };
+
 // ---- scalar conversions (device) ----------------------------------------------
 // float -> bfloat16 bits, round to nearest even, quiet NaN (arith.truncf semantics).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
@@ -163,8 +173,18 @@ hipStream_t default_stream();
 int transpose_matrix(void* out, const void* in, int R, int C, int64_t ld_in, int64_t ld_out, int elem_bytes,
                      hipStream_t s);
 // dst (rows_dst x cols_dst) = src (rows_src x cols_src) padded with zeros or cut; any alignment.
-int pad_copy_matrix(void* dst, int64_t ld_dst, int rows_dst, int cols_dst, const void* src, int64_t ld_src, int rows_src,
-                    int cols_src, int elem_bytes, hipStream_t s);
+struct PadCopy {
+  void* dst;
+  const void* src;
+  int64_t ld_dst, ld_src;
+  int rows_dst, cols_dst, rows_src, cols_src;
+};
+int pad_copy_matrices(const PadCopy* copies, int n, int elem_bytes, hipStream_t s);  // n <= 2, one launch
+inline int pad_copy_matrix(void* dst, int64_t ld_dst, int rows_dst, int cols_dst, const void* src, int64_t ld_src,
+                           int rows_src, int cols_src, int elem_bytes, hipStream_t s) {
+  const PadCopy c = {dst, src, ld_dst, ld_src, rows_dst, cols_dst, rows_src, cols_src};
+  return pad_copy_matrices(&c, 1, elem_bytes, s);
+}
 
 // ---- temporary device memory of a call ------------------------------------------------------
 // Kernels that need memory beyond their operands (transposed or zero-padded operand copies, the

@@ -379,13 +379,13 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (g.flags & LH_GEMM_SPLITK_MASK) <= LH_GEMM_SPLITK_NONE &&
       !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones.  Against them stand the direct kernels, plus
-    // the transposed copy of A (K x M read and written, a launch of its own) or the padded copies of operands
-    // (and of the result) that the direct kernels cannot take as they are.
+    // the transposed copy of A (K x M read and written, a launch of its own) or the padded copies of operands that
+    // the direct kernels cannot take as they are.
     const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
-    const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0) && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.ldc % 8 == 0 &&
-                      aligned16(g.a) && aligned16(g.b) && aligned16(g.out) && (!g.bias || aligned16(g.bias));
+    const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0) && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) &&
+                      aligned16(g.b);
     const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
-    const double other = direct_us(g) + (!fits ? 14.0 + 4.0 * mb + 4e-6 * g.M * g.N : ta ? 3.5 + 1.6e-6 * g.M * g.K : 0.0);
+    const double other = direct_us(g) + (!fits ? 4.0 + 1.3 * mb : ta ? 3.5 + 1.6e-6 * g.M * g.K : 0.0);
     int tile;
     const double us = gemm_small_choose(g, DT, &tile);
     if (tile >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, DT, tile, s);
@@ -393,8 +393,10 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;
-  if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && g.ldc % 8 == 0 && aligned16(g.out) &&
-      (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias))) {
+  // What the direct kernels used to ask of the output side; a size query still does, so that its figure stays,
+  // and so do requests.
+  const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
+  if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (vec_c || !planning())) {
     if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
     const int rc = untranspose_operands<2>(g, kBK, 8, s);
     if (b_in_place) g.flags |= LH_GEMM_TRANSPOSE_B;
@@ -402,42 +404,40 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   }
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A;
   const bool tb = (g.flags & LH_GEMM_TRANSPOSE_B) && !b_in_place;  // a transposed B the direct kernels cannot take
-  const bool vec_ok = !ta && g.K % kBK == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.ldc % 4 == 0 &&
-                      aligned16(g.a) && aligned16(g.b) && aligned16(g.out) &&
-                      (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
+  const bool operands_ok = !ta && g.K % kBK == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) && aligned16(g.b);
+  const bool direct = operands_ok && (b_in_place || (!tb && (g.N % 8 == 0 || g.b_padded))) && (vec_c || !planning());
   const uint32_t tile = g.flags & LH_GEMM_TILE_MASK;
   const uint32_t splitk = g.flags & LH_GEMM_SPLITK_MASK;
   const bool cut_requested = splitk > LH_GEMM_SPLITK_NONE;
-  if (tile == LH_GEMM_TILE_AUTO && !cut_requested && !(vec_ok && !tb && g.ldc % 8 == 0 && g.N % 8 == 0) &&
-      (int64_t)g.M * g.N * g.K >= (1 << 22)) {
+  if (tile == LH_GEMM_TILE_AUTO && !cut_requested && !direct && (int64_t)g.M * g.N * g.K >= (1 << 22)) {
     // not a shape for the direct kernels as it stands: run it on padded copies of the operands
-    const int rc = gemm_padded<2>(g, kBK, 8, s, [&](const GemmArgs& p) { return gemm16_dispatch<DT>(p, s); });
+    const int rc = gemm_padded<2, false>(g, kBK, 8, s, [&](const GemmArgs& p) { return gemm16_dispatch<DT>(p, s); });
     if (rc <= 0) return rc;
   }
   if (tile != LH_GEMM_TILE_AUTO) {
     static const int bm[4] = {256, 256, 128, 128}, bn[4] = {256, 128, 256, 128};
     const int v = (int)(tile >> 8) - 1;
-    LH_REQUIRE(vec_ok && !tb && g.ldc % 8 == 0 && g.M % bm[v] == 0 && g.N % bn[v] == 0 && direct_offsets_fit(g),
+    LH_REQUIRE(direct && vec_c && g.M % bm[v] == 0 && g.N % bn[v] == 0 && direct_offsets_fit(g),
                "gemm: the requested %d x %d tile needs an untransposed A, M %% %d == 0, N %% %d == 0, "
                "K %% 64 == 0 and 16-byte aligned rows, also of a transposed B (M=%d N=%d K=%d)",
                bm[v], bn[v], bm[v], bn[v], g.M, g.N, g.K);
   }
   if (cut_requested)
-    LH_REQUIRE(vec_ok && !tb && g.ldc % 8 == 0 && g.N % 8 == 0 && direct_offsets_fit(g),
+    LH_REQUIRE(direct && vec_c && direct_offsets_fit(g),
                "gemm: a split-K request needs an untransposed A, K %% 64 == 0, N %% 8 == 0 and 16-byte aligned rows, "
                "also of a transposed B (M=%d N=%d K=%d)", g.M, g.N, g.K);
-  if (vec_ok) {
-    if (!tb && g.ldc % 8 == 0 && g.N % 8 == 0 && direct_offsets_fit(g)) {
-      if (tile == LH_GEMM_TILE_AUTO) {
-        const int rc = gemm16_splitk<DT>(g, splitk, s);
-        if (rc <= 0) return rc;
-      }
-      const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g.M, g.N, g.K, g.out_dt == LH_F32 || (g.flags & LH_GEMM_ACCUMULATE_C) != 0);
-      if (v == 0) return launch_direct<DT, 4, 2>(g, s);
-      if (v == 1) return launch_direct<DT, 4, 1>(g, s);
-      if (v == 2) return launch_direct<DT, 2, 2>(g, s);
-      if (v == 3) return launch_direct<DT, 2, 1>(g, s);
+  if (direct && direct_offsets_fit(g)) {
+    if (tile == LH_GEMM_TILE_AUTO && vec_c) {
+      const int rc = gemm16_splitk<DT>(g, splitk, s);
+      if (rc <= 0) return rc;
     }
+    const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g.M, g.N, g.K, g.out_dt == LH_F32 || (g.flags & LH_GEMM_ACCUMULATE_C) != 0);
+    if (v == 0) return launch_direct<DT, 4, 2>(g, s);
+    if (v == 1) return launch_direct<DT, 4, 1>(g, s);
+    if (v == 2) return launch_direct<DT, 2, 2>(g, s);
+    if (v == 3) return launch_direct<DT, 2, 1>(g, s);
+  }
+  if (operands_ok && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias))) {
     const int cus = num_cus();
     const bool big = g.M % 256 == 0 && g.N % 256 == 0 && (int64_t)(g.M / 256) * (g.N / 256) >= cus;
     if (big) {

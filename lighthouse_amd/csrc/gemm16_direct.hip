@@ -232,9 +232,10 @@ __device__ __forceinline__ void direct_step_pair(const DirectCtx<TM, TN>& c, f32
 }
 
 // Source pointers of tile `id` (its position in the XCD-grouped order) and the tile's origin.
-// EDGE: M and N need not be multiples of the tile (N still a multiple of 8, K of 64): loads of
-// rows / column chunks past the end are redirected to the last valid row / chunk (their products
-// land in accumulators that are never stored) and the epilogue skips what lies outside the matrix.
+// EDGE: M and N need not be multiples of the tile (K still of 64; an n-contiguous B has rows of a multiple of
+// 8 columns, padded if N is none): loads of rows / column chunks past the end are redirected to the last valid
+// row / chunk (their products land in accumulators that are never stored).  The epilogue skips what lies
+// outside the matrix and takes any alignment of output, bias and accumulator input.
 template <int TM, int TN, bool EDGE, bool BT = false>
 __device__ __forceinline__ void direct_place(const GemmArgs& g, int id, DirectCtx<TM, TN>& c, int& m0, int& n0) {
   using Cfg = DirectCfg<TM, TN>;
@@ -282,7 +283,7 @@ __device__ __forceinline__ void direct_place(const GemmArgs& g, int id, DirectCt
     for (int i = 0; i < TN; ++i) {
       const int bk = (8 * i + c.wave) * Cfg::kBRowsPerLoad + lane / Cfg::kBChunks;
       const int bc = (lane % Cfg::kBChunks) ^ (4 * (bk & 3)) ^ (2 * ((bk >> 3) & 1));
-      const int bcol = EDGE ? min(bc * 8, g.N - 8 - n0) : bc * 8;  // column within the panel
+      const int bcol = EDGE ? min(bc * 8, (g.N + 7) / 8 * 8 - 8 - n0) : bc * 8;  // column within the panel
       c.b_src[i] = (bk * ldb + bcol) * 2;
     }
   }
@@ -347,7 +348,18 @@ __device__ __forceinline__ void direct_load_bias(const GemmArgs& g, int n_base, 
 #pragma unroll
   for (int i = 0; i < 2 * TN; ++i) {
     const int n = n_base + 16 * i;
-    bias[i] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(g.bias) + (EDGE ? min(n, g.N - 4) : n));
+    const uint16_t* b = reinterpret_cast<const uint16_t*>(g.bias);
+    if constexpr (EDGE) {
+      if (n + 4 <= g.N) {
+        bias[i] = *reinterpret_cast<const u32x2_any*>(b + n);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (n + e < g.N) bias[i][e >> 1] |= (uint32_t)b[n + e] << (16 * (e & 1));
+      }
+    } else {
+      bias[i] = *reinterpret_cast<const u32x2*>(b + n);
+    }
   }
 }
 
@@ -460,7 +472,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
         if constexpr (!E::kAny && !E::kBias) return f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         const int n = n_base + 16 * i;
         return (g.bias_dt == LH_F32)
-                   ? bias4<DT>(g, EDGE ? min(n, g.N - 4) : n)  // the bias row ends at N
+                   ? bias4<DT, EDGE>(g, n)
                    : f32x4{unpack_lo<DT>(bias[i][0]), unpack_hi<DT>(bias[i][0]), unpack_lo<DT>(bias[i][1]),
                            unpack_hi<DT>(bias[i][1])};
       };
@@ -481,9 +493,12 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
         for (int t = 0; t < JB * 32 / rows_per_pass; ++t) {
           const int row = rows_per_pass * t + lane / chunks, ch = lane % chunks;
           u32x4 w = *reinterpret_cast<const u32x4*>(cw + row * RB + ((ch ^ ((row >> 1) & (chunks - 1))) << 4));
-          const int m = m0 + wm0 + 32 * j0 + row;
-          if (!EDGE || (m < g.M && n0 + wn0 + ch * 8 < g.N))
-            *reinterpret_cast<u32x4*>(outp + (int64_t)m * g.ldc + n0 + wn0 + ch * 8) = w;
+          const int m = m0 + wm0 + 32 * j0 + row, n = n0 + wn0 + ch * 8;
+          if constexpr (EDGE) {
+            if (m < g.M && n < g.N) store8_any(outp + (int64_t)m * g.ldc + n, w, g.N - n);
+          } else {
+            *reinterpret_cast<u32x4*>(outp + (int64_t)m * g.ldc + n) = w;
+          }
         }
       }
     });
@@ -515,8 +530,10 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
       // tile instead of eight.  The larger tiles have no registers for that.
       constexpr bool kPreloadC = TM * TN == 2 && has_c;
       constexpr int NPASS = 32 / rows_per_pass;
-      auto load_c = [&](int64_t off) -> f32x4 {
-        if constexpr (out32) {
+      auto load_c = [&](int64_t off, int n) -> f32x4 {
+        if constexpr (EDGE) {
+          return load4_any<out32 ? LH_F32 : DT>(g.c, off, g.N - n);
+        } else if constexpr (out32) {
           return *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(g.c) + off);
         } else {
           const u32x2 cc = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(g.c) + off);
@@ -534,7 +551,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
               const int n = n0 + wn0 + 16 * NI * ib + 4 * ch;
               const int m = m0 + wm0 + 32 * j32 + rows_per_pass * t + row0;
               f32x4 c4 = {0.0f, 0.0f, 0.0f, 0.0f};
-              if (!EDGE || (n < g.N && m < g.M)) c4 = load_c((int64_t)m * g.ldc + n);
+              if (!EDGE || (n < g.N && m < g.M)) c4 = load_c((int64_t)m * g.ldc + n, n);
               cin[(ib * TM + j32) * NPASS + t] = c4;
             }
       }
@@ -543,7 +560,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
         const int n = n0 + wn0 + 16 * NI * ib + 4 * ch;  // the lane's 4 output columns
         const bool n_ok = !EDGE || n < g.N;
         f32x4 b4 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (epi_has_bias<E>(g)) b4 = bias4<DT>(g, EDGE ? min(n, g.N - 4) : n);
+        if (epi_has_bias<E>(g)) b4 = bias4<DT, EDGE>(g, n);
 #pragma unroll
         for (int j32 = 0; j32 < TM; ++j32) {
 #pragma unroll
@@ -566,7 +583,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
             if constexpr (has_c) {
               f32x4 c4;
               if constexpr (kPreloadC) c4 = cin[(ib * TM + j32) * NPASS + t];
-              else c4 = load_c(off);
+              else c4 = load_c(off, n);
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[e] += c4[e];
             }
@@ -587,7 +604,9 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[e] += b4[e];
             }
-            if constexpr (out32)
+            if constexpr (EDGE)
+              store4_any<out32 ? LH_F32 : DT>(g.out, off, v, g.N - n);
+            else if constexpr (out32)
               *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off) = v;
             else
               *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(g.out) + off) =
@@ -740,7 +759,9 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
 template <int DT, int TM, int TN>
 int launch_direct(const GemmArgs& g, hipStream_t s) {
   using Cfg = DirectCfg<TM, TN>;
-  const bool whole = g.M % Cfg::BM == 0 && g.N % Cfg::BN == 0;
+  const bool whole = g.M % Cfg::BM == 0 && g.N % Cfg::BN == 0 && g.ldc % 8 == 0 && aligned16(g.out) &&
+                     (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias)) &&
+                     (!(g.flags & LH_GEMM_ACCUMULATE_C) || aligned16(g.c));
   if (g.flags & LH_GEMM_TRANSPOSE_B)
     return whole ? launch_direct_edge<DT, TM, TN, false, true>(g, s) : launch_direct_edge<DT, TM, TN, true, true>(g, s);
   return whole ? launch_direct_edge<DT, TM, TN, false>(g, s) : launch_direct_edge<DT, TM, TN, true>(g, s);

@@ -120,9 +120,10 @@ __device__ __forceinline__ void direct32_wait_barrier() {
 }
 
 // Source pointers of tile `id` (row-major over the tile grid) and the tile's origin.  EDGE: M and
-// N need not be multiples of the tile (N still a multiple of 4): loads of rows / column chunks
-// past the end are redirected to the last valid row / chunk (their products land in accumulators
-// that are never stored) and the epilogue skips what lies outside the matrix.
+// N need not be multiples of the tile (the rows of B hold a multiple of 4 columns, padded if N is none): loads of
+// rows / column chunks past the end are redirected to the last valid row / chunk (their products land in
+// accumulators that are never stored); the epilogue skips what lies outside the matrix and takes any
+// alignment of output, bias and accumulator input.
 template <bool EDGE, int TM, int TN, int NW>
 __device__ __forceinline__ void direct32_place(const GemmArgs& g, int id, Direct32Ctx<TM, TN, NW>& c, int& m0, int& n0) {
   using C = Direct32Ctx<TM, TN, NW>;
@@ -151,7 +152,7 @@ __device__ __forceinline__ void direct32_place(const GemmArgs& g, int id, Direct
     constexpr int chunks = 16 * TN;
     const int k = (C::NW * i + c.wave) * (64 / chunks) + lane / chunks;
     const int gc = (lane % chunks) ^ (8 * ((k >> 2) & 1));
-    c.b_src[i] = (k * ldb + (EDGE ? min(gc * 4, g.N - 4 - n0) : gc * 4)) * 4;
+    c.b_src[i] = (k * ldb + (EDGE ? min(gc * 4, (g.N + 3) / 4 * 4 - 4 - n0) : gc * 4)) * 4;
   }
 }
 
@@ -252,9 +253,14 @@ __global__ void __launch_bounds__(NW * 64) gemm32_direct(GemmArgs g) {
       for (int j = 0; j < WTM; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          if (!EDGE || (m_base + 32 * j < g.M && n_base + 32 * i + 8 * q < g.N))
+          if constexpr (EDGE) {
+            if (m_base + 32 * j < g.M && n_base + 32 * i + 8 * q < g.N)
+              epilogue4_any<LH_F32>(g, m_base + 32 * j, n_base + 32 * i + 8 * q,
+                                    f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]});
+          } else {
             epilogue4<LH_F32>(g, m_base + 32 * j, n_base + 32 * i + 8 * q, acc[i][j][4 * q], acc[i][j][4 * q + 1],
                               acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+          }
     if (!more) break;
     t = tn;
   }
@@ -278,7 +284,9 @@ static int launch_direct32_edge(const GemmArgs& g, hipStream_t s) {
 
 template <int TM, int TN, int NS, int NW = 4>
 static int launch_direct32(const GemmArgs& g, hipStream_t s) {
-  if (g.M % (64 * TM) == 0 && g.N % (64 * TN) == 0) return launch_direct32_edge<TM, TN, NS, NW, false>(g, s);
+  if (g.M % (64 * TM) == 0 && g.N % (64 * TN) == 0 && g.ldc % 4 == 0 && aligned16(g.out) &&
+      (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias)) && (!(g.flags & LH_GEMM_ACCUMULATE_C) || aligned16(g.c)))
+    return launch_direct32_edge<TM, TN, NS, NW, false>(g, s);
   return launch_direct32_edge<TM, TN, NS, NW, true>(g, s);
 }
 
@@ -348,24 +356,24 @@ int gemm32(const GemmArgs& g_in, hipStream_t s) {
     // Few tiles: the small-tile kernels, if they are the faster ones; against them stand the direct kernels plus the
     // transposed or padded copies those would need.
     const bool trans = g.flags & (LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
-    const bool fits = g.K % kBK32 == 0 && g.N % 4 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && g.ldc % 4 == 0 &&
-                      aligned16(g.a) && aligned16(g.b) && aligned16(g.out) && (!g.bias || aligned16(g.bias));
+    const bool fits = g.K % kBK32 == 0 && g.N % 4 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && aligned16(g.a) && aligned16(g.b);
     const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
-    const double other = direct32_us(g) + (!fits ? 14.0 + 6.0 * mb + 6e-6 * g.M * g.N : trans ? 4.0 + 3.2 * mb : 0.0);
+    const double other = direct32_us(g) + (!fits ? 4.0 + 2.5 * mb : trans ? 4.0 + 3.2 * mb : 0.0);
     int small;
     const double us = gemm_small_choose(g, LH_F32, &small);
     if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F32, small, s);
   }
-  if (tile == LH_GEMM_TILE_AUTO && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias))) {
+  // What the fast kernels used to ask of the output side; a size query still does, so that its figure stays.
+  const bool vec_c = g.N % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
+  if (tile == LH_GEMM_TILE_AUTO && (vec_c || !planning())) {
     const int rc = untranspose_operands<4>(g, kBK32, 4, s);
     if (rc < 0) return rc;
   }
   const bool trans = g.flags & (LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
-  const bool vec_ok = !trans && g.K % kBK32 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && g.ldc % 4 == 0 &&
-                      aligned16(g.a) && aligned16(g.b) && aligned16(g.out) &&
-                      (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
+  const bool direct = !trans && g.K % kBK32 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && (g.N % 4 == 0 || g.b_padded) &&
+                      aligned16(g.a) && aligned16(g.b) && (vec_c || !planning());
   if (tile != LH_GEMM_TILE_AUTO) {
-    LH_REQUIRE(vec_ok && g.N % 4 == 0 && direct32_offsets_fit(g),
+    LH_REQUIRE(direct && vec_c && direct32_offsets_fit(g),
                "gemm: a tile request on f32 inputs needs untransposed operands, K %% 32 == 0, N %% 4 == 0 and 16-byte "
                "aligned rows (M=%d N=%d K=%d)", g.M, g.N, g.K);
     if (tile == LH_GEMM_TILE_128x128) return launch_direct32<2, 2, 4, 8>(g, s);
@@ -373,12 +381,12 @@ int gemm32(const GemmArgs& g_in, hipStream_t s) {
     if ((int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) <= 512) return launch_direct32<1, 1, 8>(g, s);
     return launch_direct32<1, 1, 3>(g, s);
   }
-  if (!(vec_ok && g.N % 4 == 0) && (int64_t)g.M * g.N * g.K >= (1 << 22)) {
+  if (!direct && (int64_t)g.M * g.N * g.K >= (1 << 22)) {
     // not a shape for the direct kernels as it stands: run it on padded copies of the operands
-    const int rc = gemm_padded<4>(g, kBK32, 4, s, [&](const GemmArgs& p) { return gemm32(p, s); });
+    const int rc = gemm_padded<4, false>(g, kBK32, 4, s, [&](const GemmArgs& p) { return gemm32(p, s); });
     if (rc <= 0) return rc;
   }
-  if (vec_ok && g.N % 4 == 0 && direct32_offsets_fit(g)) {
+  if (direct && direct32_offsets_fit(g)) {
     // Tiles are counted with edge tiles in full (M, N need not be multiples of a tile).
     const int cus = num_cus();
     const int64_t t128 = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);

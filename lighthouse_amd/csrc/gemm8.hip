@@ -973,7 +973,7 @@ int gemm8(const GemmArgs& g, hipStream_t s) {
                       aligned16(g.b) && aligned16(g.out);
   if (!(vec_ok && g.N % 128 == 0) && (int64_t)g.M * g.N * g.K >= (1 << 22)) {
     // K that is no multiple of the k-step, N of no tile, unaligned rows: zero-padded copies (code 0 is +0)
-    const int rc = gemm_padded<1>(g, kBK8, 128, s, [&](const GemmArgs& p) { return gemm8(p, s); });
+    const int rc = gemm_padded<1, true>(g, kBK8, 128, s, [&](const GemmArgs& p) { return gemm8(p, s); });
     if (rc <= 0) return rc;
   }
   if (vec_ok && g.M <= 16 && g.N % kSkinnyBN == 0 && g.ldb % 16 == 0) {

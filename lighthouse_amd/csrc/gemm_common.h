@@ -25,6 +25,8 @@ struct GemmArgs {
   // 16-bit direct kernel, 128 x 128 tile: main loop with one barrier per 64 k (set by the launcher
   // when more than one workgroup falls on a compute unit).
   int one_barrier = 0;
+  // B is a copy whose rows hold whole 16-byte chunks past column N (zeros): N need not be a multiple of them.
+  bool b_padded = false;
 };
 
 // Epilogue for 4 consecutive columns of one row.
@@ -76,11 +78,58 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& g, int m, int n, float
   }
 }
 
-// Bias of 4 consecutive columns as f32 (zeros without a bias).
+// Vectors of 4 output-side elements at element alignment (gfx9 global memory takes any alignment): the
+// outputs, biases and accumulator inputs of problems whose N or row stride is odd.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
+
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+// 4 elements at p[at], of which the first `left` exist (zeros for the others), as f32.
 template <int DT>
+__device__ __forceinline__ f32x4 load4_any(const void* p, int64_t at, int left) {
+  f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (left >= 4) {
+    if constexpr (DT == LH_F32) return *reinterpret_cast<const f32x4_any*>(reinterpret_cast<const float*>(p) + at);
+    const u32x2 w = *reinterpret_cast<const u32x2_any*>(reinterpret_cast<const uint16_t*>(p) + at);
+    return f32x4{unpack_lo<DT>(w[0]), unpack_hi<DT>(w[0]), unpack_lo<DT>(w[1]), unpack_hi<DT>(w[1])};
+  }
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+    if (e < left) v[e] = load_as_f32<DT>(p, at + e);
+  return v;
+}
+// ... and stored.
+template <int DT>
+__device__ __forceinline__ void store4_any(void* p, int64_t at, const f32x4& v, int left) {
+  if (left >= 4) {
+    if constexpr (DT == LH_F32)
+      *reinterpret_cast<f32x4_any*>(reinterpret_cast<float*>(p) + at) = v;
+    else
+      *reinterpret_cast<u32x2_any*>(reinterpret_cast<uint16_t*>(p) + at) = u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+    if (e < left) store_from_f32<DT>(p, at + e, v[e]);
+}
+// 8 packed 16-bit values, of which the first `left` are stored.
+__device__ __forceinline__ void store8_any(uint16_t* p, const u32x4& w, int left) {
+  if (left >= 8) {
+    *reinterpret_cast<u32x4_any*>(p) = w;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 7; ++e)
+    if (e < left) p[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+}
+
+// Bias of 4 consecutive columns as f32 (zeros without a bias).  ANY: any alignment, zeros from column N on.
+template <int DT, bool ANY = false>
 __device__ __forceinline__ f32x4 bias4(const GemmArgs& g, int n) {
   f32x4 r = {0.0f, 0.0f, 0.0f, 0.0f};
   if (g.flags & LH_GEMM_HAS_BIAS) {
+    if constexpr (ANY) return g.bias_dt == LH_F32 ? load4_any<LH_F32>(g.bias, n, g.N - n) : load4_any<DT>(g.bias, n, g.N - n);
     if (g.bias_dt == LH_F32) {
       r = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(g.bias) + n);
     } else {
@@ -254,13 +303,14 @@ inline int untranspose_operands(GemmArgs& g, int k_multiple, int n_multiple, hip
   return 0;
 }
 
-// A problem whose K or N the direct kernels cannot take (K not a multiple of the k-step, N not a
-// multiple of the vector width, or rows that are not 16-byte aligned) runs on them all the same:
-// A and B are copied into temporary matrices padded with zeros, the kernel writes a padded
-// result, and that is copied back (bf16 4096 x 4100 x 4096: 2012 -> about 200 us; the generic
-// kernel it replaces reads element by element).  `run` launches the padded problem.  Returns 1
-// when nothing needs padding, a negative status on failure.
-template <int ELEM_BYTES, typename Run>
+// A problem whose K the direct kernels cannot take (no multiple of the k-step), or whose operand rows are not
+// 16-byte aligned, runs on them all the same: A and B are copied into temporary matrices padded with zeros,
+// both in one launch.  The kernels write any N, row stride and alignment themselves, except those of fp8
+// (PAD_C), which write a padded result that is copied back.  `run` launches the padded problem.  Returns 1
+// when nothing needs padding, a negative status on failure.  (bf16 4096 x 4100 x 4096: 2012 us on the
+// bounds-checked kernel, 224 with every operand padded; M = 8192, N = 50257, K = 768 with f32 output: the copy of
+// the 1.6 GB result back alone took 1751 us.)
+template <int ELEM_BYTES, bool PAD_C, typename Run>
 inline int gemm_padded(const GemmArgs& g, int k_multiple, int n_multiple, hipStream_t s, Run run) {
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
   const int out_bytes = g.out_dt == LH_F32 ? 4 : 2, bias_bytes = g.bias_dt == LH_F32 ? 4 : 2;
@@ -270,61 +320,64 @@ inline int gemm_padded(const GemmArgs& g, int k_multiple, int n_multiple, hipStr
   // (a transposed operand is copied in any case: the copy is where it gets untransposed)
   const bool pad_a = ta || Kp != g.K || g.lda % (16 / ELEM_BYTES) != 0 || !aligned16(g.a);
   const bool pad_b = tb || Kp != g.K || Np != g.N || g.ldb % (16 / ELEM_BYTES) != 0 || !aligned16(g.b);
-  const bool pad_c = Np != g.N || g.ldc % n_multiple != 0 || !aligned16(g.out) || (acc && !aligned16(g.c));
-  const bool pad_bias = has_bias && (Np != g.N || !aligned16(g.bias));
-  if (!(pad_a || pad_b || pad_c || pad_bias)) return 1;
+  const bool odd_c = Np != g.N || g.ldc % n_multiple != 0 || !aligned16(g.out) || (acc && !aligned16(g.c));
+  const bool odd_bias = has_bias && (Np != g.N || !aligned16(g.bias));
+  if (!(pad_a || pad_b || odd_c || odd_bias)) return 1;
   auto round256 = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t a_bytes = pad_a ? round256((size_t)g.M * Kp * ELEM_BYTES) : 0;
   const size_t b_bytes = pad_b ? round256((size_t)Kp * Np * ELEM_BYTES) : 0;
-  const size_t c_bytes = pad_c ? round256((size_t)g.M * Np * out_bytes) : 0;
-  const size_t bias_bytes_total = pad_bias ? round256((size_t)Np * bias_bytes) : 0;
-  void* taken = nullptr;
-  if (int rc = scratch_take(g.ws, s, kScratchPad, a_bytes + b_bytes + c_bytes + bias_bytes_total, "gemm (padded operands)",
-                            &taken))
-    return rc;
-  char* buf = static_cast<char*>(taken);
+  size_t bytes = a_bytes + b_bytes;
+  // (a workspace query counts a padded result and bias whichever kernel will run)
+  if ((PAD_C || planning()) && odd_c) bytes += round256((size_t)g.M * Np * out_bytes);
+  if (planning() && odd_bias) bytes += round256((size_t)Np * bias_bytes);
   GemmArgs p = g;
   p.K = Kp;
-  p.N = Np;
-  if (pad_a) {
-    if (ta) {  // stored [K, M]: zeros first (the padding), then the transposed matrix on top
-      if (Kp != g.K)
-        if (int rc = pad_copy_matrix(buf, Kp, g.M, Kp, g.a, g.lda, 0, 0, ELEM_BYTES, s)) return rc;
-      if (int rc = transpose_matrix(buf, g.a, g.K, g.M, g.lda, Kp, ELEM_BYTES, s)) return rc;
-    } else if (int rc = pad_copy_matrix(buf, Kp, g.M, Kp, g.a, g.lda, g.M, g.K, ELEM_BYTES, s)) {
-      return rc;
+  if (bytes > 0) {
+    void* taken = nullptr;
+    if (int rc = scratch_take(g.ws, s, kScratchPad, bytes, "gemm (padded operands)", &taken)) return rc;
+    char* buf = static_cast<char*>(taken);
+    PadCopy copies[2];
+    int ncopies = 0;
+    if (pad_a) {
+      if (ta) {  // stored [K, M]: zeros first (the padding), then the transposed matrix on top
+        if (Kp != g.K)
+          if (int rc = pad_copy_matrix(buf, Kp, g.M, Kp, g.a, g.lda, 0, 0, ELEM_BYTES, s)) return rc;
+        if (int rc = transpose_matrix(buf, g.a, g.K, g.M, g.lda, Kp, ELEM_BYTES, s)) return rc;
+      } else {
+        copies[ncopies++] = PadCopy{buf, g.a, Kp, g.lda, g.M, Kp, g.M, g.K};
+      }
+      p.a = buf;
+      p.lda = Kp;
     }
-    p.a = buf;
-    p.lda = Kp;
-  }
-  if (pad_b) {
-    char* bp = buf + a_bytes;
-    if (tb) {  // stored [N, K]
-      if (Kp != g.K || Np != g.N)
-        if (int rc = pad_copy_matrix(bp, Np, Kp, Np, g.b, g.ldb, 0, 0, ELEM_BYTES, s)) return rc;
-      if (int rc = transpose_matrix(bp, g.b, g.N, g.K, g.ldb, Np, ELEM_BYTES, s)) return rc;
-    } else if (int rc = pad_copy_matrix(bp, Np, Kp, Np, g.b, g.ldb, g.K, g.N, ELEM_BYTES, s)) {
-      return rc;
+    if (pad_b) {
+      char* bp = buf + a_bytes;
+      if (tb) {  // stored [N, K]
+        if (Kp != g.K || Np != g.N)
+          if (int rc = pad_copy_matrix(bp, Np, Kp, Np, g.b, g.ldb, 0, 0, ELEM_BYTES, s)) return rc;
+        if (int rc = transpose_matrix(bp, g.b, g.N, g.K, g.ldb, Np, ELEM_BYTES, s)) return rc;
+      } else {
+        copies[ncopies++] = PadCopy{bp, g.b, Np, g.ldb, Kp, Np, g.K, g.N};
+      }
+      p.b = bp;
+      p.ldb = Np;
+      p.b_padded = true;
     }
-    p.b = bp;
-    p.ldb = Np;
-  }
-  p.flags &= ~(uint32_t)(LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
-  if (pad_c) {
-    char* cp = buf + a_bytes + b_bytes;
-    if (acc)
-      if (int rc = pad_copy_matrix(cp, Np, g.M, Np, g.c, g.ldc, g.M, g.N, out_bytes, s)) return rc;
-    p.out = cp;
-    p.c = cp;
-    p.ldc = Np;
-  }
-  if (pad_bias) {
-    char* bp = buf + a_bytes + b_bytes + c_bytes;
-    if (int rc = pad_copy_matrix(bp, Np, 1, Np, g.bias, g.N, 1, g.N, bias_bytes, s)) return rc;
-    p.bias = bp;
+    if (ncopies)
+      if (int rc = pad_copy_matrices(copies, ncopies, ELEM_BYTES, s)) return rc;
+    p.flags &= ~(uint32_t)(LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
+    static_assert(!PAD_C || ELEM_BYTES == 1, "fp8 products have neither a bias nor an accumulator input");
+    if (PAD_C || planning()) {
+      p.N = Np;
+      if (odd_c) {
+        p.out = buf + a_bytes + b_bytes;
+        p.c = p.out;
+        p.ldc = Np;
+      }
+      if (odd_bias) p.bias = buf;  // (planning: any aligned address)
+    }
   }
   if (int rc = run(p)) return rc;
-  if (pad_c) return pad_copy_matrix(g.out, g.ldc, g.M, g.N, p.out, Np, g.M, g.N, out_bytes, s);
+  if (PAD_C && odd_c) return pad_copy_matrix(g.out, g.ldc, g.M, g.N, p.out, Np, g.M, g.N, out_bytes, s);
   return LH_OK;
 }
 
@@ -377,34 +430,19 @@ __device__ __forceinline__ void epilogue1(const GemmArgs& g, int m, int n, float
   else store_from_f32<DT>(g.out, off, x);
 }
 
-// Vectors of 4 output-side elements at element alignment (gfx9 global memory takes any alignment): the
-// outputs, biases and accumulator inputs of problems whose N or row stride is odd.
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
-
-// Epilogue for columns n .. n + 3 of row m, of which those below N exist.
+// epilogue4 for columns n .. n + 3 of row m, of which those below N exist; any alignment.
 template <int DT>
 __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, const f32x4& acc) {
-  if (n + 4 > g.N) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (n + e < g.N) epilogue1<DT>(g, m, n + e, acc[e]);
-    return;
-  }
   float v[4] = {acc[0] * g.alpha, acc[1] * g.alpha, acc[2] * g.alpha, acc[3] * g.alpha};
   const int64_t off = (int64_t)m * g.ldc + n;
-  auto load4 = [&](const void* p, int64_t at, int dt) -> f32x4 {
-    if (dt == LH_F32) return *reinterpret_cast<const f32x4_any*>(reinterpret_cast<const float*>(p) + at);
-    const u32x2 w = *reinterpret_cast<const u32x2_any*>(reinterpret_cast<const uint16_t*>(p) + at);
-    return f32x4{unpack_lo<DT>(w[0]), unpack_hi<DT>(w[0]), unpack_lo<DT>(w[1]), unpack_hi<DT>(w[1])};
-  };
+  const int left = g.N - n;
   if (g.flags & LH_GEMM_ACCUMULATE_C) {
-    const f32x4 c = load4(g.c, off, g.out_dt);
+    const f32x4 c = g.out_dt == LH_F32 ? load4_any<LH_F32>(g.c, off, left) : load4_any<DT>(g.c, off, left);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += c[e];
   }
   if (g.flags & LH_GEMM_HAS_BIAS) {
-    const f32x4 b = load4(g.bias, n, g.bias_dt);
+    const f32x4 b = bias4<DT, true>(g, n);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += b[e];
   }
@@ -416,10 +454,9 @@ __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, c
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = relu_nan(v[e]);
   }
-  if (g.out_dt == LH_F32)
-    *reinterpret_cast<f32x4_any*>(reinterpret_cast<float*>(g.out) + off) = f32x4{v[0], v[1], v[2], v[3]};
-  else if constexpr (DT != LH_F32)
-    *reinterpret_cast<u32x2_any*>(reinterpret_cast<uint16_t*>(g.out) + off) = u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+  const f32x4 o = {v[0], v[1], v[2], v[3]};
+  if (g.out_dt == LH_F32) store4_any<LH_F32>(g.out, off, o, left);
+  else store4_any<DT>(g.out, off, o, left);
 }
 
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s);

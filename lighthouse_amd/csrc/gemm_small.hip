@@ -24,15 +24,6 @@
 
 namespace lh {
 
-template <int ES>
-struct Chunk;  // 16 bytes at element alignment
-template <>
-struct Chunk<1> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(1))); typedef uint8_t elem; };
-template <>
-struct Chunk<2> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(2))); typedef uint16_t elem; };
-template <>
-struct Chunk<4> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4))); typedef uint32_t elem; };
-
 typedef short small_s16x4 __attribute__((ext_vector_type(4)));
 typedef int small_i32x2 __attribute__((ext_vector_type(2)));
 

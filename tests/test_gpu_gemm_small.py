@@ -19,8 +19,7 @@ def _matrix(rows, cols, dtype, seed, pad):
 
 
 @pytest.mark.parametrize("pad", [0, 1])
-@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
-@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("dtype,layout", [(d, l) for d in ("bf16", "f16", "f32") for l in ("nn", "nt", "tn", "tt")] + [("fp8", "nn")])
 @pytest.mark.parametrize("shape", [(16, 16, 16),       # one tile, less than a k-step of 16-bit values
                                    (17, 65, 64),       # one past a tile in both directions
                                    (33, 31, 63),       # K one short of a step
@@ -32,8 +31,6 @@ def test_small_tiles(shape, dtype, layout, pad):
     from lighthouse_amd import ops
 
     M, N, K = shape
-    if dtype == "fp8" and layout != "nn":
-        pytest.skip("the fp8 entry point has no transposed form")
     ta, tb = layout[0] == "t", layout[1] == "t"
     a, av = _matrix(K if ta else M, M if ta else K, dtype, 1, pad)
     b, bv = _matrix(N if tb else K, K if tb else N, dtype, 2, pad)
@@ -53,3 +50,29 @@ def test_small_tiles(shape, dtype, layout, pad):
             got = ops.gemm(a, b, transpose_a=ta, transpose_b=tb)
             assert torch.equal(got, want.to(DTYPES[dtype]))
     assert bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("shape,offset", [((2100, 2051, 64), 0),    # N odd: 128- and 256-wide tiles that end inside a row
+                                          ((2304, 2304, 128), 1),   # whole tiles, rows that start 2 (4) bytes off
+                                          ((600, 8190, 96), 3)])
+def test_tile_kernels_write_any_alignment(shape, offset, dtype):
+    """Problems too large for the small tiles whose result, bias and accumulator input are not 16-byte aligned:
+    the tile kernels write them in place, and nothing beside them."""
+    from lighthouse_amd import ops
+
+    M, N, K = shape
+    a, av = _matrix(M, K, dtype, 3, 0)
+    b, bv = _matrix(K, N, dtype, 4, 0)
+    want = av.double() @ bv.double()
+    for out_dtype in {DTYPES[dtype], torch.float32}:
+        buf = torch.full((M, N + 5), 7.0, device="cuda", dtype=out_dtype)
+        view = buf[:, offset:offset + N]
+        bias = (torch.arange(N + 1, device="cuda").float() % 5 - 2).to(out_dtype)[1:]
+        ops.gemm(a, b, bias, out=view)
+        assert torch.equal(view, (want + bias.double()).to(out_dtype))
+        view.copy_(view.clamp(-8, 8).round())
+        before = view.double().clone()
+        ops.gemm(a, b, out=view, accumulate_c=True)
+        assert torch.equal(view, (want + before).to(out_dtype))
+        assert bool((buf[:, :offset] == 7.0).all()) and bool((buf[:, offset + N:] == 7.0).all())
