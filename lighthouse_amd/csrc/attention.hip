@@ -19,39 +19,9 @@
 // layout produces.
 #include <type_traits>
 
-#include "common.h"
+#include "attention.h"
 
 namespace lh {
-
-struct AttnArgs {
-  void* out;
-  const void* q;
-  const void* k;
-  const void* v;
-  int Z, H, T;
-  lh_strides3 so, sq, sk, sv;
-  float scale_log2e;  // scale * log2(e)
-  float scale;
-  int causal;
-  int cus;  // compute units of the device (causal launch order)
-  int request = 0;  // LH_ATTN_ROWS_* | LH_ATTN_STAGES_* bits of the call (0: the library chooses)
-  bool scale_f32 = false;  // LH_ATTN_SCALE_F32: Q stays as stored and the scores are scaled in f32
-  int d = 0;        // head dimension of the call (the padded kernels mask the columns from d on)
-  // Key range split between workgroups (few query blocks, long sequences): `kv_groups` workgroups
-  // per query block each take a contiguous share of its key tiles and leave (unnormalised output,
-  // offset, row sum) in `part`; attention16_merge combines them.  1: one workgroup per query block.
-  int kv_groups = 1;
-  float* part = nullptr;
-  // Causal launches of up to a third more query blocks than fit the CUs at once (32 rows per wave,
-  // three workgroups per CU): the grid is `chain` = 3 x CUs workgroups, all resident, and the first
-  // third of them take a second query block each (see attention16_kernel).  0: one block per workgroup.
-  int chain = 0;
-  // 64 rows per wave, two workgroups per CU: of every 8 key tiles, the number for which the younger
-  // workgroup's waves hold the higher priority (0: the two take turns tile by tile).
-  int pair_bias = 0;
-  bool allow_grid_split = true;  // the caller lets the launch take temporary memory for it
-  Scratch* ws = nullptr;         // where that memory comes from: a caller workspace, or (nullptr) the stream's pool
-};
 
 template <int DT>
 __device__ __forceinline__ f32x16 mfma16(u32x4 a, u32x4 b, f32x16 c) {
@@ -835,6 +805,11 @@ static int attention16_launch(const AttnArgs& a, hipStream_t s) {
       }
     }
     if (best_groups > 1) return attention16_launch_split<DT, 2>(a, best_groups, s);
+  }
+  // Few query rows in all: small workgroups whose waves share out the keys (the rule stands there); they scale the
+  // scores in f32 whether asked to or not.
+  if (!a.request) {
+    if (const int tiles = attention_small_tiles(a)) return attention_small(a, DT, tiles, s);
   }
   // Unasked, the split pays where at most one 256-row workgroup falls on a CU but more than half
   // the CUs get one: a lone group of four waves leaves each SIMD with a single wave, and splitting the
