@@ -438,13 +438,16 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
     if (v == 3) return launch_direct<DT, 2, 1>(g, s);
   }
   if (operands_ok && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias))) {
+    // (B as it is stored, also where the direct kernels would have read a transposed one in place but a row stride
+    // is too large for their 32-bit offsets)
+    const bool b_kc = g.flags & LH_GEMM_TRANSPOSE_B;
     const int cus = num_cus();
     const bool big = g.M % 256 == 0 && g.N % 256 == 0 && (int64_t)(g.M / 256) * (g.N / 256) >= cus;
     if (big) {
-      return tb ? launch_fast<DT, 256, 256, 2, 4, true>(g, s) : launch_fast<DT, 256, 256, 2, 4, false>(g, s);
+      return b_kc ? launch_fast<DT, 256, 256, 2, 4, true>(g, s) : launch_fast<DT, 256, 256, 2, 4, false>(g, s);
     }
     if (g.M % 128 == 0 && g.N % 128 == 0) {
-      return tb ? launch_fast<DT, 128, 128, 2, 2, true>(g, s) : launch_fast<DT, 128, 128, 2, 2, false>(g, s);
+      return b_kc ? launch_fast<DT, 128, 128, 2, 2, true>(g, s) : launch_fast<DT, 128, 128, 2, 2, false>(g, s);
     }
   }
   dim3 grid((g.N + 63) / 64, (g.M + 63) / 64);

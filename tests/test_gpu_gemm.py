@@ -751,6 +751,23 @@ def test_gemm_transposed_b_in_place(shape, dtype, elt):
         assert torch.equal(ops.gemm(da, dbt, transpose_b=True, out_dtype=torch.float32, split_k=4), out)
 
 
+@pytest.mark.parametrize("strided", ["a", "b"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gemm_transposed_b_with_a_huge_row_stride(dtype, strided):
+    """Rows 2^22 elements apart, more than the direct kernels' 32-bit offsets reach, next to a B stored [N, K] that they
+    would otherwise read in place: the kernels that take over read it as it is stored.  Integer operands, exact result."""
+    from lighthouse_amd import ops
+
+    M, N, K, ld = (256, 4096, 64, 1 << 22) if strided == "a" else (4096, 256, 64, 1 << 22)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = (torch.randint(-3, 4, (rows, K), device="cuda", generator=g).to(dtype) for rows in (M, N))
+    want = a.double() @ b.double().T.contiguous()
+    wide = torch.empty(256 * ld, device="cuda", dtype=dtype).view(256, ld)[:, :K]
+    wide.copy_(a if strided == "a" else b)
+    got = ops.gemm(wide if strided == "a" else a, wide if strided == "b" else b, transpose_b=True, out_dtype=torch.float32)
+    assert torch.equal(got.double(), want)
+
+
 def test_gemm_fp8_with_caller_workspace():
     from lighthouse_amd import ops
 
