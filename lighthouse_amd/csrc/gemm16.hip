@@ -393,10 +393,12 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;
-  // What the direct kernels used to ask of the output side; a size query still does, so that its figure stays,
-  // and so do requests.
+  // An output side of whole 16-byte chunks: what requests ask for.  Without it a small problem takes no temporary
+  // memory, here and in a size query alike, so that it never needs a workspace (it has fewer flops than the copy of an
+  // operand is worth).
   const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
-  if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (vec_c || !planning())) {
+  const bool may_copy = vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22);
+  if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && may_copy) {
     if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
     const int rc = untranspose_operands<2>(g, kBK, 8, s);
     if (b_in_place) g.flags |= LH_GEMM_TRANSPOSE_B;
@@ -405,7 +407,7 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A;
   const bool tb = (g.flags & LH_GEMM_TRANSPOSE_B) && !b_in_place;  // a transposed B the direct kernels cannot take
   const bool operands_ok = !ta && g.K % kBK == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) && aligned16(g.b);
-  const bool direct = operands_ok && (b_in_place || (!tb && (g.N % 8 == 0 || g.b_padded))) && (vec_c || !planning());
+  const bool direct = operands_ok && (b_in_place || (!tb && (g.N % 8 == 0 || g.b_padded)));
   const uint32_t tile = g.flags & LH_GEMM_TILE_MASK;
   const uint32_t splitk = g.flags & LH_GEMM_SPLITK_MASK;
   const bool cut_requested = splitk > LH_GEMM_SPLITK_NONE;

@@ -363,15 +363,15 @@ int gemm32(const GemmArgs& g_in, hipStream_t s) {
     const double us = gemm_small_choose(g, LH_F32, &small);
     if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F32, small, s);
   }
-  // What the fast kernels used to ask of the output side; a size query still does, so that its figure stays.
+  // (as in gemm16_dispatch: without aligned chunks on the output side a small problem takes no temporary memory)
   const bool vec_c = g.N % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
-  if (tile == LH_GEMM_TILE_AUTO && (vec_c || !planning())) {
+  if (tile == LH_GEMM_TILE_AUTO && (vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22))) {
     const int rc = untranspose_operands<4>(g, kBK32, 4, s);
     if (rc < 0) return rc;
   }
   const bool trans = g.flags & (LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
   const bool direct = !trans && g.K % kBK32 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && (g.N % 4 == 0 || g.b_padded) &&
-                      aligned16(g.a) && aligned16(g.b) && (vec_c || !planning());
+                      aligned16(g.a) && aligned16(g.b);
   if (tile != LH_GEMM_TILE_AUTO) {
     LH_REQUIRE(direct && vec_c && direct32_offsets_fit(g),
                "gemm: a tile request on f32 inputs needs untransposed operands, K %% 32 == 0, N %% 4 == 0 and 16-byte "

@@ -717,6 +717,30 @@ def test_gemm_with_caller_workspace(case):
             ops.gemm(a, b, bias, relu=True, transpose_a=ta, transpose_b=tb, workspace=ws[:0], out=sentinel)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("M,N,K,ta", [(1, 64, 64, True), (4, 64, 64, True), (7, 72, 128, True),   # below the smallest tile
+                                      (3, 64, 64, True), (2, 8, 8192, True), (4, 64, 8192, False),
+                                      (512, 256, 512, True)])                                     # worth the copy of A
+def test_gemm_workspace_query_with_an_unaligned_result(dtype, M, N, K, ta):
+    """A result whose rows start anywhere: the call runs on exactly the workspace that the query gives for it, and small
+    problems on none.  Integer operands, exact result."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(4)
+    a = torch.zeros((K if ta else M, ((M if ta else K) + 7) // 8 * 8), device="cuda", dtype=dtype)[:, :M if ta else K]
+    a.copy_(torch.randint(-2, 3, a.shape, device="cuda", generator=g))
+    b = torch.randint(-2, 3, (K, N), device="cuda", generator=g).to(dtype)
+    want = (a.T if ta else a).double() @ b.double()
+    for ld, offset in ((N + 1, 0), (N + 8, 1)):
+        out = torch.full((M, ld), 7.0, device="cuda")
+        view = out[:, offset:offset + N]
+        need = ops.gemm_workspace_bytes(M, N, K, dtype, torch.float32, transpose_a=ta, operands=(view, a, b, None))
+        assert (need == 0) == (M * N * K < 1 << 22)
+        ops.gemm(a, b, out=view, transpose_a=ta, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+        assert torch.equal(view.double(), want)
+        assert bool((out[:, :offset] == 7.0).all()) and bool((out[:, offset + N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("dtype,elt", [(torch.bfloat16, "bf16"), (torch.float16, "f16")])
 @pytest.mark.parametrize("shape", [(4096, 4096, 1024), (8192, 768, 768), (2048, 2304, 768), (512, 1024, 4096), (16, 4096, 8192),
                                    (200, 136, 192), (1000, 520, 320), (64, 8192, 2048)])
