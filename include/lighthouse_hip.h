@@ -154,7 +154,8 @@ int lh_hip_gemm(void* out, const void* a, const void* b, const void* bias, int64
 /*
  * lh_hip_gemm with its temporary memory in a caller workspace of at least
  * lh_hip_gemm_workspace_bytes(...) bytes (0 for most problems; the query assumes 16-byte aligned
- * operands).  No allocation happens inside the call; a workspace that is too small fails with
+ * operands and still counts a copy of a result whose N or row stride is no multiple of 16 bytes, which no
+ * kernel makes any more; lh_hip_gemm_workspace_bytes_for gives what the call takes).  No allocation happens inside the call; a workspace that is too small fails with
  * LH_ERR_INVALID.  Same role as the workspace of lh_hip_nanogpt_block for callers that manage
  * device memory themselves (GPUMemoryManager, lighthouse/execution/memory_manager.py:97-151).
  */

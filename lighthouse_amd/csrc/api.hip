@@ -95,6 +95,8 @@ static int gemm_dtype_checks(const char* who, int32_t ab_dtype, int32_t out_dtyp
   return LH_OK;
 }
 
+static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
 static int workspace_checks(const char* who, const void* workspace, size_t workspace_bytes) {
   LH_REQUIRE(workspace != nullptr || workspace_bytes == 0, "%s: null workspace of %zu bytes", who, workspace_bytes);
   LH_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, "%s: workspace must be 256-byte aligned", who);
@@ -153,7 +155,14 @@ size_t lh_hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda,
   void* const fake = reinterpret_cast<void*>(uintptr_t(1) << 20);
   if (gemm_common_checks("lh_hip_gemm_workspace_bytes", fake, fake, fake, fake, M, N, K, lda, ldb, ldc, flags)) return 0;
   if (gemm_dtype_checks("lh_hip_gemm_workspace_bytes", ab_dtype, out_dtype)) return 0;
-  return gemm_need(M, N, K, lda, ldb, ldc, ab_dtype, out_dtype, out_dtype, flags);
+  const size_t need = gemm_need(M, N, K, lda, ldb, ldc, ab_dtype, out_dtype, out_dtype, flags);
+  // Results are written in place whatever their rows; a result (and bias) copied into rows of whole 16-byte chunks is in
+  // this figure all the same, as it always has been: callers that lay out their memory by it keep their layout.
+  const int64_t chunk = 16 / (int64_t)dtype_size(ab_dtype), rows_of = (N + chunk - 1) / chunk * chunk;
+  const bool requested = flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK);
+  if (requested || (double)M * N * K < (1 << 22) || (rows_of == N && ldc % chunk == 0)) return need;
+  return need + align256((size_t)M * rows_of * dtype_size(out_dtype)) +
+         ((flags & LH_GEMM_HAS_BIAS) && rows_of != N ? align256((size_t)rows_of * dtype_size(out_dtype)) : 0);
 }
 
 size_t lh_hip_gemm_workspace_bytes_for(const void* out, const void* a, const void* b, const void* bias, int64_t M,
@@ -255,7 +264,6 @@ int lh_hip_gemm_fp8_ws(void* out, const void* a_q, const void* b_q, float scale_
 }
 
 // ---- nanoGPT block -------------------------------------------------------------------------
-static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 struct BlockConfig {
   bool causal;

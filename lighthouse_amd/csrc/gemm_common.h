@@ -313,23 +313,20 @@ inline int untranspose_operands(GemmArgs& g, int k_multiple, int n_multiple, hip
 template <int ELEM_BYTES, bool PAD_C, typename Run>
 inline int gemm_padded(const GemmArgs& g, int k_multiple, int n_multiple, hipStream_t s, Run run) {
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
-  const int out_bytes = g.out_dt == LH_F32 ? 4 : 2, bias_bytes = g.bias_dt == LH_F32 ? 4 : 2;
+  const int out_bytes = g.out_dt == LH_F32 ? 4 : 2;
   const int Kp = (g.K + k_multiple - 1) / k_multiple * k_multiple;
   const int Np = (g.N + n_multiple - 1) / n_multiple * n_multiple;
-  const bool has_bias = g.flags & LH_GEMM_HAS_BIAS, acc = g.flags & LH_GEMM_ACCUMULATE_C;
+  const bool acc = g.flags & LH_GEMM_ACCUMULATE_C;
   // (a transposed operand is copied in any case: the copy is where it gets untransposed)
   const bool pad_a = ta || Kp != g.K || g.lda % (16 / ELEM_BYTES) != 0 || !aligned16(g.a);
   const bool pad_b = tb || Kp != g.K || Np != g.N || g.ldb % (16 / ELEM_BYTES) != 0 || !aligned16(g.b);
   const bool odd_c = Np != g.N || g.ldc % n_multiple != 0 || !aligned16(g.out) || (acc && !aligned16(g.c));
-  const bool odd_bias = has_bias && (Np != g.N || !aligned16(g.bias));
-  if (!(pad_a || pad_b || odd_c || odd_bias)) return 1;
+  if (!(pad_a || pad_b || (PAD_C && odd_c))) return 1;
   auto round256 = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t a_bytes = pad_a ? round256((size_t)g.M * Kp * ELEM_BYTES) : 0;
   const size_t b_bytes = pad_b ? round256((size_t)Kp * Np * ELEM_BYTES) : 0;
   size_t bytes = a_bytes + b_bytes;
-  // (a workspace query counts a padded result and bias whichever kernel will run)
-  if ((PAD_C || planning()) && odd_c) bytes += round256((size_t)g.M * Np * out_bytes);
-  if (planning() && odd_bias) bytes += round256((size_t)Np * bias_bytes);
+  if (PAD_C && odd_c) bytes += round256((size_t)g.M * Np * out_bytes);
   GemmArgs p = g;
   p.K = Kp;
   if (bytes > 0) {
@@ -366,14 +363,13 @@ inline int gemm_padded(const GemmArgs& g, int k_multiple, int n_multiple, hipStr
       if (int rc = pad_copy_matrices(copies, ncopies, ELEM_BYTES, s)) return rc;
     p.flags &= ~(uint32_t)(LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
     static_assert(!PAD_C || ELEM_BYTES == 1, "fp8 products have neither a bias nor an accumulator input");
-    if (PAD_C || planning()) {
+    if (PAD_C) {
       p.N = Np;
       if (odd_c) {
         p.out = buf + a_bytes + b_bytes;
         p.c = p.out;
         p.ldc = Np;
       }
-      if (odd_bias) p.bias = buf;  // (planning: any aligned address)
     }
   }
   if (int rc = run(p)) return rc;

@@ -226,6 +226,20 @@ def test_workspace_queries_run_without_a_gpu():
     assert lib.lh_hip_nanogpt_block_workspace_bytes(1, 256, 256, _lib.F64, None) == 0  # unsupported type
 
 
+def test_workspace_queries_count_no_copy_of_a_result():
+    """Results are written in place at any N and row stride: a call needs room for operand copies only."""
+    lib = _lib.load()
+    fake = 1 << 20
+    query = lib.lh_hip_gemm_workspace_bytes_for
+    assert query(fake, fake, fake, None, 4096, 4100, 4096, 4096, 4100, 4100, _lib.BF16, _lib.BF16, 0) == 4096 * 4104 * 2
+    assert query(fake + 2, fake, fake, None, 4096, 4096, 4096, 4096, 4096, 4099, _lib.BF16, _lib.BF16, 0) == 0
+    assert query(fake, fake, fake, fake + 4, 1000, 1001, 1024, 1024, 1004, 1001, _lib.F32, _lib.F32,
+                 _lib.GEMM_HAS_BIAS) == 1024 * 1004 * 4
+    # a vocabulary whose rows are not aligned: the forward needs an aligned copy of lm_w, not of 1.6 GB of logits
+    forward = lambda vocab: lib.lh_hip_nanogpt_forward_workspace_bytes(8, 1024, 768, vocab, _lib.BF16, None)  # noqa: E731
+    assert forward(50257) - forward(50264) == 768 * 50264 * 2
+
+
 def test_gpt_fused_payload_signature():
     """The argument list of build_gpt_fused_payload, examples/xegpu/nanoGPT_payload.py:333-351."""
     T, C, hidden, vocab, L = 256, 256, 1024, 256, 2
