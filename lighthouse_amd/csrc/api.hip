@@ -87,6 +87,15 @@ static int gemm8_run(void* out, const void* a_q, const void* b_q, float scale_a,
   return gemm8(g, s);
 }
 
+// ... and of gemm8_run; again only the alignment of the pointers matters.
+static size_t gemm8_need(void* out, const void* a_q, const void* b_q, int64_t M, int64_t N, int64_t K, int64_t lda,
+                         int64_t ldb, int64_t ldc, int32_t out_dtype) {
+  PlanningScope plan;
+  Scratch ws;
+  const int rc = gemm8_run(out, a_q, b_q, 1.0f, 1.0f, M, N, K, lda, ldb, ldc, out_dtype, nullptr, &ws);
+  return rc ? 0 : ws.need;
+}
+
 static int gemm_dtype_checks(const char* who, int32_t ab_dtype, int32_t out_dtype) {
   if (!(ab_dtype == LH_F32 || ab_dtype == LH_BF16 || ab_dtype == LH_F16))
     return fail(LH_ERR_UNSUPPORTED, "%s: unsupported A/B dtype %d", who, ab_dtype);
@@ -238,10 +247,7 @@ size_t lh_hip_gemm_fp8_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t 
   void* const fake = reinterpret_cast<void*>(uintptr_t(1) << 20);
   if (gemm_common_checks("lh_hip_gemm_fp8_workspace_bytes", fake, fake, fake, nullptr, M, N, K, lda, ldb, ldc, 0)) return 0;
   if (!(out_dtype == LH_BF16 || out_dtype == LH_F32)) return 0;
-  PlanningScope plan;
-  Scratch ws;
-  const int rc = gemm8_run(fake, fake, fake, 1.0f, 1.0f, M, N, K, lda, ldb, ldc, out_dtype, nullptr, &ws);
-  return rc ? 0 : ws.need;
+  return gemm8_need(fake, fake, fake, M, N, K, lda, ldb, ldc, out_dtype);
 }
 
 int lh_hip_gemm_fp8_ws(void* out, const void* a_q, const void* b_q, float scale_a, float scale_b, int64_t M, int64_t N,
@@ -252,7 +258,8 @@ int lh_hip_gemm_fp8_ws(void* out, const void* a_q, const void* b_q, float scale_
   if (!(out_dtype == LH_BF16 || out_dtype == LH_F32))
     return fail(LH_ERR_UNSUPPORTED, "lh_hip_gemm_fp8_ws: out dtype %d must be bf16 or f32", out_dtype);
   if ((rc = workspace_checks("lh_hip_gemm_fp8_ws", workspace, workspace_bytes))) return rc;
-  const size_t need = lh_hip_gemm_fp8_workspace_bytes(M, N, K, lda, ldb, ldc, out_dtype);
+  // (the need of THESE operands: the query, which assumes aligned ones, may say more, for kernels that they do not run)
+  const size_t need = gemm8_need(out, a_q, b_q, M, N, K, lda, ldb, ldc, out_dtype);
   LH_REQUIRE(need <= workspace_bytes,
              "lh_hip_gemm_fp8_ws: workspace too small: this call needs %zu bytes of temporary memory, %zu were given", need,
              workspace_bytes);

@@ -809,6 +809,21 @@ def test_gemm_fp8_with_caller_workspace():
                 ops.gemm_fp8(aq, bq, 0.5, 0.25, workspace=ws[: need // 2])
 
 
+def test_gemm_fp8_unaligned_operands_need_no_workspace():
+    """A small product of codes that start at an odd address runs without temporary memory, although the same product of
+    aligned codes is cut along K into blocks: an empty workspace is enough."""
+    from lighthouse_amd import ops
+
+    M, N, K = 1, 512, 4096
+    assert ops.gemm_fp8_workspace_bytes(M, N, K) > 0
+    g = torch.Generator(device="cuda").manual_seed(6)
+    codes = torch.randint(-3, 4, (M * K + 1,), device="cuda", generator=g).to(torch.float8_e4m3fn)
+    a = codes[1:].view(M, K)
+    b = torch.randint(-3, 4, (K, N), device="cuda", generator=g).to(torch.float8_e4m3fn)
+    out = ops.gemm_fp8(a, b, 1.0, 1.0, out_dtype=torch.float32, workspace=torch.empty(0, dtype=torch.uint8, device="cuda"))
+    assert torch.equal(out.double(), a.double() @ b.double())
+
+
 def test_split_k_gemms_on_two_streams():
     """Two streams run decode-shaped GEMMs of different shapes (both cut along K, so both use f32
     partial blocks) at the same time, many times over: each stream has its own temporaries, so
