@@ -433,7 +433,10 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
 // against bank conflicts), and leave as full row segments of 16 bytes per lane.  `ring` and
 // `stage` are separate restrict parameters so that the staging traffic does not wait for the
 // asynchronous ring writes.
-template <int DT, int TM, int TN, bool EDGE, bool HAS_NEXT, bool BT = false>
+// BLOCKS (a launch cut along K): the accumulators go out as they are, f32, to rows of whole aligned 16-byte chunks.
+// None of the epilogue variants is in that code: with the element-aligned accesses of an edge tile they took the
+// 128 x 128 tile to 136 registers, where two workgroups no longer fit a CU (M = 16, N = K = 8192 bf16: 34 -> 40 us).
+template <int DT, int TM, int TN, bool EDGE, bool HAS_NEXT, bool BT = false, bool BLOCKS = false>
 __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx<TM, TN>& next, int nk,
                                               uint8_t* __restrict__ ring, uint8_t* __restrict__ stage,
                                               const f32x4 (&acc)[2 * TN][2 * TM], const u32x2 (&bias)[2 * TN], int m0,
@@ -446,7 +449,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
   const int lane = lane_now();
   const int l16 = lane & 15, g4 = lane >> 4;
   const int n_base = n0 + wn0 + 4 * g4;
-  if (g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C)) {
+  if (!BLOCKS && g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C)) {
     // The bias values (loaded by the main loop, whose last wait covered them) are pinned down here:
     // a wait for them placed after the ring loads below would wait for those loads as well.
 #pragma unroll
@@ -604,7 +607,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[e] += b4[e];
             }
-            if constexpr (EDGE)
+            if constexpr (EDGE && !BLOCKS)
               store4_any<out32 ? LH_F32 : DT>(g.out, off, v, g.N - n);
             else if constexpr (out32)
               *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off) = v;
@@ -615,13 +618,17 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
         }
       }
     };
-    const bool out32 = g.out_dt == LH_F32;
-    const bool has_c = (g.flags & LH_GEMM_ACCUMULATE_C) != 0;
-    epi_dispatch_linear(g, [&](auto variant) {
-      if (out32 && has_c) body(variant, std::true_type{}, std::true_type{});
-      else if (out32) body(variant, std::true_type{}, std::false_type{});
-      else body(variant, std::false_type{}, std::true_type{});  // a 16-bit output comes here only with an accumulator input
-    });
+    if constexpr (BLOCKS) {
+      body(EpiFixed<false, false, 0>{}, std::true_type{}, std::false_type{});
+    } else {
+      const bool out32 = g.out_dt == LH_F32;
+      const bool has_c = (g.flags & LH_GEMM_ACCUMULATE_C) != 0;
+      epi_dispatch_linear(g, [&](auto variant) {
+        if (out32 && has_c) body(variant, std::true_type{}, std::true_type{});
+        else if (out32) body(variant, std::true_type{}, std::false_type{});
+        else body(variant, std::false_type{}, std::true_type{});  // a 16-bit output comes here only with an accumulator input
+      });
+    }
   }
 }
 
@@ -693,7 +700,7 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
   }
   direct_prologue<TM, TN, BT>(c, nk, smem_d);
   // Without EDGE every lane issues all stores of a staged epilogue.
-  const bool staged = g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
+  const bool staged = !SPLITK && g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
   const bool counted_stores = !EDGE && staged;
   bool first = true;
   for (;;) {
@@ -716,9 +723,9 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
     if (more) {
       const int idn = select(tn, g_nxt);
       direct_place<TM, TN, EDGE, BT>(SPLITK ? g_nxt : g, xcd_remap(idn, tiles1), cn, m1, n1);
-      direct_finish<DT, TM, TN, EDGE, true, BT>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
+      direct_finish<DT, TM, TN, EDGE, true, BT, SPLITK>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
     } else {
-      direct_finish<DT, TM, TN, EDGE, false, BT>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
+      direct_finish<DT, TM, TN, EDGE, false, BT, SPLITK>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
     }
     if (!more) break;
     if constexpr (SPLITK) g_cur = g_nxt;
