@@ -165,8 +165,8 @@ size_t lh_hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda,
   if (gemm_common_checks("lh_hip_gemm_workspace_bytes", fake, fake, fake, fake, M, N, K, lda, ldb, ldc, flags)) return 0;
   if (gemm_dtype_checks("lh_hip_gemm_workspace_bytes", ab_dtype, out_dtype)) return 0;
   const size_t need = gemm_need(M, N, K, lda, ldb, ldc, ab_dtype, out_dtype, out_dtype, flags);
-  // Results are written in place whatever their rows; a result (and bias) copied into rows of whole 16-byte chunks is in
-  // this figure all the same, as it always has been: callers that lay out their memory by it keep their layout.
+  // Results are written in place whatever their rows; a copy of a result (and bias) in rows of whole 16-byte chunks stays
+  // in this figure all the same, an upper bound that memory may have been laid out by.
   const int64_t chunk = 16 / (int64_t)dtype_size(ab_dtype), rows_of = (N + chunk - 1) / chunk * chunk;
   const bool requested = flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK);
   if (requested || (double)M * N * K < (1 << 22) || (rows_of == N && ldc % chunk == 0)) return need;

@@ -289,14 +289,18 @@ static int direct_variant(int M, int N, int K, bool slow_epilogue) {
   return best;
 }
 
-// Sum of the split-K blocks (f32, [splits][M][N]) and the problem's own epilogue, 4 columns per thread.
+// Columns of a row of the split-K blocks: whole 16-byte chunks.
+__host__ __device__ static inline int splitk_row(int N) { return (N + 3) / 4 * 4; }
+
+// Sum of the split-K blocks (f32, [splits][M][splitk_row(N)]) and the problem's own epilogue, 4 columns per thread; any
+// alignment of output, bias and accumulator input.
 template <int DT>
 __global__ void __launch_bounds__(256) gemm16_splitk_reduce(GemmArgs g, const float* partial, int splits) {
+  const int row = splitk_row(g.N);
   const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (idx >= (int64_t)g.M * g.N) return;
-  const int m = (int)(idx / g.N), n = (int)(idx % g.N);
-  const f32x4 v = splitk_sum4(partial + (int64_t)m * g.N + n, (int64_t)g.M * g.N, splits, blockDim.x == 64);
-  epilogue4<DT>(g, m, n, v[0], v[1], v[2], v[3]);
+  if (idx >= (int64_t)g.M * row) return;
+  const int m = (int)(idx / row), n = (int)(idx % row);
+  epilogue4_any<DT>(g, m, n, splitk_sum4(partial + idx, (int64_t)g.M * row, splits, blockDim.x == 64));
 }
 
 // Cuts along K for the library's own choice: decode shapes, so few 128 x 128 tiles that most CUs would idle, and
@@ -327,9 +331,8 @@ static int splitk_count(int M, int N, int K) {
 
 // Time of an untransposed, aligned problem on the direct kernels, in us, where few tiles make it latency-bound
 // (what the small-tile kernels are weighed against; median 0.97 of the measured time on the problems of
-// gemm_small.hip's fit, nine in ten between 0.86 and 1.14).
-static double direct_us(const GemmArgs& g) {
-  const int sp = splitk_count(g.M, g.N, g.K);
+// gemm_small.hip's fit, nine in ten between 0.86 and 1.14).  `sp`: the cuts along K that it will run with.
+static double direct_us(const GemmArgs& g, int sp) {
   const double x = (double)sp * ((g.M + 127) / 128) * ((g.N + 127) / 128) / num_cus();
   const double per_cu = x <= 1.0 ? 1.0 : 1.0 + 0.55 * (x - 1.0);
   return 3.6 + 0.0072 * g.K / sp * per_cu + (x > 1.0 ? 0.6 * (x - 1.0) : 0.0) +
@@ -353,7 +356,7 @@ static int gemm16_splitk(const GemmArgs& g, uint32_t request, hipStream_t s) {
     if (splits == 1) return 1;
   }
   void* taken = nullptr;
-  if (int rc = scratch_take(g.ws, s, kScratchSplitK, (size_t)splits * g.M * g.N * sizeof(float), "gemm (split K)", &taken))
+  if (int rc = scratch_take(g.ws, s, kScratchSplitK, (size_t)splits * g.M * splitk_row(g.N) * sizeof(float), "gemm (split K)", &taken))
     return rc;
   float* partial = static_cast<float*>(taken);
   GemmArgs p = g;
@@ -361,13 +364,13 @@ static int gemm16_splitk(const GemmArgs& g, uint32_t request, hipStream_t s) {
   p.splits = splits;
   p.out = partial;
   p.c = partial;
-  p.ldc = g.N;
+  p.ldc = splitk_row(g.N);
   p.out_dt = LH_F32;
   p.bias = nullptr;
   p.flags = g.flags & LH_GEMM_TRANSPOSE_B;
   p.one_barrier = 0;  // B is streamed from memory here: the deeper look-ahead wins (M = 16, N = K = 8192: 26.7 against 27.4 us)
   if (int rc = launch_direct_splitk<DT>(p, s)) return rc;
-  const int64_t groups = (int64_t)g.M * g.N / 4;
+  const int64_t groups = (int64_t)g.M * splitk_row(g.N) / 4;
   const int rb = reduce_block(groups);
   LH_LAUNCH(gemm16_splitk_reduce<DT>, dim3((unsigned)((groups + rb - 1) / rb)), dim3(rb), 0, s, g, partial, splits);
   return check_launch("gemm16_splitk_reduce");
@@ -376,6 +379,11 @@ static int gemm16_splitk(const GemmArgs& g, uint32_t request, hipStream_t s) {
 template <int DT>
 static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   GemmArgs g = g_in;
+  // An output side of whole 16-byte chunks: what requests ask for.  Without it a small problem takes no temporary
+  // memory, here and in a size query alike, so that it never needs a workspace (it has fewer flops than the copy of an
+  // operand is worth).
+  const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
+  const bool may_copy = vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22);
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (g.flags & LH_GEMM_SPLITK_MASK) <= LH_GEMM_SPLITK_NONE &&
       !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones.  Against them stand the direct kernels, plus
@@ -385,7 +393,9 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
     const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0) && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) &&
                       aligned16(g.b);
     const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
-    const double other = direct_us(g) + (!fits ? 4.0 + 1.3 * mb : ta ? 3.5 + 1.6e-6 * g.M * g.K : 0.0);
+    // (a padded copy has whole k-steps)
+    const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) : 1;
+    const double other = direct_us(g, cuts) + (!fits ? 4.0 + 1.3 * mb : ta ? 3.5 + 1.6e-6 * g.M * g.K : 0.0);
     int tile;
     const double us = gemm_small_choose(g, DT, &tile);
     if (tile >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, DT, tile, s);
@@ -393,11 +403,6 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;
-  // An output side of whole 16-byte chunks: what requests ask for.  Without it a small problem takes no temporary
-  // memory, here and in a size query alike, so that it never needs a workspace (it has fewer flops than the copy of an
-  // operand is worth).
-  const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
-  const bool may_copy = vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22);
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && may_copy) {
     if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
     const int rc = untranspose_operands<2>(g, kBK, 8, s);
@@ -429,7 +434,7 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
                "gemm: a split-K request needs an untransposed A, K %% 64 == 0, N %% 8 == 0 and 16-byte aligned rows, "
                "also of a transposed B (M=%d N=%d K=%d)", g.M, g.N, g.K);
   if (direct && direct_offsets_fit(g)) {
-    if (tile == LH_GEMM_TILE_AUTO && vec_c) {
+    if (tile == LH_GEMM_TILE_AUTO && may_copy) {
       const int rc = gemm16_splitk<DT>(g, splitk, s);
       if (rc <= 0) return rc;
     }

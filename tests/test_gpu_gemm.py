@@ -606,6 +606,41 @@ def test_gemm_16bit_split_k(shape, elt, epi):
         assert_close(_host(out), ref, rtol, f"{elt} gemm {shape} {epi} (split K)")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,layout,copies", [
+    (128, 1001, 8192, "nt", 0),                           # odd N, B read in place
+    (16, 1003, 4096, "nn", 4096 * 1008 * 2),              # odd N, B copied into aligned rows
+    (130, 1024, 4096, "nn", 0), (256, 1024, 4096, "nn", 0),  # rows that start anywhere; edge and whole tiles
+    (256, 1024, 4096, "tn", 256 * 4096 * 2)])
+def test_gemm_split_k_with_an_unaligned_result(M, N, K, layout, copies, dtype):
+    """A product cut along K whose result, bias and accumulator input have rows that start anywhere: the blocks are sums in
+    aligned rows, the second kernel writes the result in place and nothing beside it.  Integer operands, exact sums."""
+    from lighthouse_amd import ops
+
+    ta, tb = layout[0] == "t", layout[1] == "t"
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = torch.randint(-3, 4, (M, K), device="cuda", generator=g).to(dtype)
+    b = torch.randint(-3, 4, (K, N), device="cuda", generator=g).to(dtype)
+    want = a.double() @ b.double()
+    a, b = (a.T.contiguous() if ta else a), (b.T.contiguous() if tb else b)
+    for out_dtype in (dtype, torch.float32):
+        buf = torch.full((M, N + 5), 7.0, device="cuda", dtype=out_dtype)
+        view = buf[:, 1:1 + N]
+        bias = (torch.arange(N + 1, device="cuda").float() % 5 - 2).to(out_dtype)[1:]
+        need = ops.gemm_workspace_bytes(M, N, K, dtype, out_dtype, bias=True, relu=True, transpose_a=ta, transpose_b=tb,
+                                        operands=(view, a, b, bias))
+        blocks = need - copies  # 2, 4 or 8 of them
+        assert blocks in [c * M * ((N + 3) // 4 * 4) * 4 for c in (2, 4, 8)]
+        ops.gemm(a, b, bias, out=view, relu=True, transpose_a=ta, transpose_b=tb,
+                 workspace=torch.empty((need + 255) // 256 * 256, dtype=torch.uint8, device="cuda"))
+        assert torch.equal(view, torch.relu(want + bias.double()).to(out_dtype))
+        view.copy_(view.clamp(-8, 8).round())
+        before = view.double().clone()
+        ops.gemm(a, b, out=view, accumulate_c=True, transpose_a=ta, transpose_b=tb)
+        assert torch.equal(view, (want + before).to(out_dtype))
+        assert bool((buf[:, :1] == 7.0).all()) and bool((buf[:, 1 + N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("elt", ["bf16", "f32"])
 @pytest.mark.parametrize("ta,tb", [(True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("shape", [(300, 521, 200), (512, 1000, 1000)])
