@@ -390,8 +390,9 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
     // the transposed copy of A (K x M read and written, a launch of its own) or the padded copies of operands that
     // the direct kernels cannot take as they are.
     const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
-    const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0) && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) &&
-                      aligned16(g.b);
+    // (padded copies that are there already cost nothing more)
+    const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0 || g.b_padded) && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
+                      aligned16(g.a) && aligned16(g.b);
     const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
     // (a padded copy has whole k-steps)
     const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) : 1;

@@ -356,7 +356,9 @@ int gemm32(const GemmArgs& g_in, hipStream_t s) {
     // Few tiles: the small-tile kernels, if they are the faster ones; against them stand the direct kernels plus the
     // transposed or padded copies those would need.
     const bool trans = g.flags & (LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
-    const bool fits = g.K % kBK32 == 0 && g.N % 4 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && aligned16(g.a) && aligned16(g.b);
+    // (padded copies that are there already cost nothing more)
+    const bool fits = g.K % kBK32 == 0 && (g.N % 4 == 0 || g.b_padded) && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
+                      aligned16(g.a) && aligned16(g.b);
     const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
     const double other = direct32_us(g) + (!fits ? 4.0 + 2.5 * mb : trans ? 4.0 + 3.2 * mb : 0.0);
     int small;

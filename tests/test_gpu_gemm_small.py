@@ -76,3 +76,19 @@ def test_tile_kernels_write_any_alignment(shape, offset, dtype):
         ops.gemm(a, b, out=view, accumulate_c=True)
         assert torch.equal(view, (want + before).to(out_dtype))
         assert bool((buf[:, :offset] == 7.0).all()) and bool((buf[:, offset + N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype,M,N,K", [("bf16", 457, 5401, 901), ("f16", 457, 5401, 901), ("f32", 345, 5237, 166)])
+def test_a_problem_copied_for_the_tile_kernels_runs_on_them(dtype, M, N, K):
+    """Here the tile kernels plus padded copies of both operands beat the small tiles on the operands as they are, by
+    little: once the copies are made the tile kernels run.  They add up k in one order whatever the tile, the
+    small tiles in another, so the f32 sums have the bits of the same product on operands that need no copy."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(7)
+    a = torch.randn(M, K, device="cuda", generator=g).to(DTYPES[dtype])
+    b = torch.randn(K, N, device="cuda", generator=g).to(DTYPES[dtype])
+    a0, b0 = torch.zeros(M, (K + 63) // 64 * 64, device="cuda", dtype=a.dtype), torch.zeros((K + 63) // 64 * 64, N + 7, device="cuda", dtype=a.dtype)
+    a0[:, :K], b0[:K, :N] = a, b
+    want = ops.gemm(a0, b0, out_dtype=torch.float32)[:, :N]
+    assert torch.equal(ops.gemm(a, b, out_dtype=torch.float32), want)
