@@ -143,14 +143,10 @@ struct SmallPanel {
         if (k0 + f * RPL + lane / CPR >= K) r[f] = u32x4{0u, 0u, 0u, 0u};
     }
   }
-  // The step's fragments: the registers themselves (KC), or through the wave's LDS area.
+  // The step's chunks go into the wave's LDS area (!KC) ...
   template <bool WHOLE>
-  __device__ __forceinline__ void fragments(u32x4 (&r)[F], uint8_t* lds, int lane, u32x4 (&frag)[F]) const {
-    if constexpr (KC) {
-#pragma unroll
-      for (int f = 0; f < F; ++f) frag[f] = r[f];
-    } else {
-      const int l16 = lane & 15, g4 = lane >> 4;
+  __device__ __forceinline__ void stage(u32x4 (&r)[F], uint8_t* lds, int lane) const {
+    if constexpr (!KC) {
       if constexpr (!WHOLE) {
 #pragma unroll
         for (int f = 0; f < F; ++f) r[f] = small_shift_chunk<ES>(r[f], over);
@@ -158,6 +154,15 @@ struct SmallPanel {
 #pragma unroll
       for (int f = 0; f < F; ++f)
         *reinterpret_cast<u32x4*>(lds + (f * RPL + lane / CPR) * RS + (lane % CPR) * 16) = r[f];
+    }
+  }
+  // ... where its fragments come from; KC: the registers themselves.
+  __device__ __forceinline__ void fragments(const u32x4 (&r)[F], uint8_t* lds, int lane, u32x4 (&frag)[F]) const {
+    if constexpr (KC) {
+#pragma unroll
+      for (int f = 0; f < F; ++f) frag[f] = r[f];
+    } else {
+      const int l16 = lane & 15, g4 = lane >> 4;
 #pragma unroll
       for (int f = 0; f < F; ++f) {
         if constexpr (ES == 2) {
@@ -195,6 +200,7 @@ struct SmallCfg {
   static constexpr int kLdsBytes = kSumBytes > NW * kWaveLds ? kSumBytes : NW * kWaveLds;
   // Steps requested ahead: what fits next to the accumulators in the registers of NW waves.
   static constexpr int P = MT + NT <= 3 ? 3 : 2;
+  static constexpr bool kTight = MT * NT == 16 && !AKC && !BKC && PA::ES == 2;  // (all 256 registers that 8 waves have)
 };
 
 // The wave's share of the k-steps.
@@ -213,12 +219,17 @@ __device__ __forceinline__ void small_multiply(const typename Cfg::PA& pa, const
   u32x4 ra[P][MT], rb[P][NT];
   auto consume = [&](u32x4 (&a)[MT], u32x4 (&b)[NT]) {
     u32x4 fa[MT], fb[NT];
-    pb.template fragments<WHOLE>(b, lds_b, lane, fb);
-    pa.template fragments<WHOLE>(a, lds_a, lane, fa);
+    pb.template stage<WHOLE>(b, lds_b, lane);
+    if constexpr (Cfg::kTight) pa.template stage<WHOLE>(a, lds_a, lane);
+    pb.fragments(b, lds_b, lane, fb);
+    if constexpr (!Cfg::kTight) pa.template stage<WHOLE>(a, lds_a, lane);
+    pa.fragments(a, lds_a, lane, fa);
 #pragma unroll
     for (int j = 0; j < MT; ++j)
 #pragma unroll
       for (int i = 0; i < NT; ++i) acc[j][i] = small_mma<DT>(fb[i], fa[j], acc[j][i]);
+    // (a step on its own: with the next one's reads and shifts pulled into it this kernel spills registers)
+    if constexpr (Cfg::kTight && !WHOLE) __builtin_amdgcn_sched_barrier(0);
   };
   if (tail) {
     pa.load_tail(full * KSTEP, K, lane, ra[0]);

@@ -41,3 +41,10 @@ def test_two_128x128_gemm_workgroups_fit_a_compute_unit(kernels):
     tiles = {n: k["vgpr_count"] for n, k in kernels.items() if re.search(r"gemm16_directILi[12]ELi2ELi1E", n)}
     assert len(tiles) == 16  # bf16 / f16, whole / edge tiles, whole / cut K, B [K, N] / [N, K]
     assert {n: v for n, v in tiles.items() if v > 128} == {}
+
+
+def test_only_wide_element_access_attention_uses_scratch(kernels):
+    """A kernel that touches scratch memory at all costs microseconds more per dispatch.  The attention kernels that load
+    element by element at the widths 224 (f32) and 256 are the ones that do."""
+    scratch = {n for n, k in kernels.items() if k["private_segment_fixed_size"] > 0}
+    assert {n for n in scratch if not re.search(r"attention16_anyd_kernelILi[12]ELi8ELi2E|attention32_anyd_kernelILi[78]ELi2E", n)} == set()
