@@ -350,9 +350,13 @@ static int launch_small_layout(const GemmArgs& g, hipStream_t s) {
 
 template <int DT, int MT, int NT, int NW>
 static int launch_small(const GemmArgs& g, hipStream_t s) {
-  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
-  if (ta) return tb ? launch_small_layout<DT, MT, NT, NW, false, true>(g, s) : launch_small_layout<DT, MT, NT, NW, false, false>(g, s);
-  return tb ? launch_small_layout<DT, MT, NT, NW, true, true>(g, s) : launch_small_layout<DT, MT, NT, NW, true, false>(g, s);
+  if constexpr (DT == LH_F8E4M3) {  // (fp8 products take no transposed operands)
+    return launch_small_layout<DT, MT, NT, NW, true, false>(g, s);
+  } else {
+    const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
+    if (ta) return tb ? launch_small_layout<DT, MT, NT, NW, false, true>(g, s) : launch_small_layout<DT, MT, NT, NW, false, false>(g, s);
+    return tb ? launch_small_layout<DT, MT, NT, NW, true, true>(g, s) : launch_small_layout<DT, MT, NT, NW, true, false>(g, s);
+  }
 }
 
 // ---- choice of tile ---------------------------------------------------------------------------

@@ -48,3 +48,10 @@ def test_only_wide_element_access_attention_uses_scratch(kernels):
     element by element at the widths 224 (f32) and 256 are the ones that do."""
     scratch = {n for n, k in kernels.items() if k["private_segment_fixed_size"] > 0}
     assert {n for n in scratch if not re.search(r"attention16_anyd_kernelILi[12]ELi8ELi2E|attention32_anyd_kernelILi[78]ELi2E", n)} == set()
+
+
+def test_small_tile_gemms_are_built_for_the_layouts_that_exist(kernels):
+    """Six tiles; four layouts of a 16-bit or f32 product, one of an fp8 product, whose operands are never transposed."""
+    small = [re.search(r"gemm_small_kernelILi(\d)E", n) for n in kernels]
+    of_type = [int(m.group(1)) for m in small if m]
+    assert {t: of_type.count(t) for t in set(of_type)} == {_lib.F32: 24, _lib.BF16: 24, _lib.F16: 24, _lib.F8E4M3: 6}
