@@ -69,8 +69,16 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, int lane_byte
                                       uint8_t* lds_wave_base) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)lds_wave_base, 16, lane_bytes, scalar_bytes, 0, 0);
 }
-// A resource over [base, base + 4 GiB): raw (unstructured) addressing, offsets in bytes.
+// A resource over [base, base + 4 GiB): raw (unstructured) addressing, offsets in bytes.  The kernels cut along K (the
+// object without a tile) say that the base is uniform: the compiler keeps the panel addresses of their edge tiles, which come
+// out of the divisions that select a piece of K, in vector registers and wrote a loop over the lanes' resources around every
+// load (M = 1, N = 5376, K = 4736 bf16: 24.0 us without such loops, 28.4 with them).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t panel_resource(const void* base) {
+#if LH_GEMM16_TM == 0
+  const uint64_t address = reinterpret_cast<uint64_t>(base);
+  base = reinterpret_cast<const void*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(address >> 32)) << 32 |
+                                       (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)address));
+#endif
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xffffffff, 0x00020000);
 }
 template <int TM, int TN>

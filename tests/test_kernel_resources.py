@@ -1,5 +1,5 @@
-"""What the compiler gave the kernels of the built library: registers where a launch counts on two workgroups per compute
-unit.  Read from the metadata notes of the library's own code objects."""
+"""What the compiler made of the kernels of the built library: registers where a launch counts on two workgroups per compute
+unit, scratch memory, loads.  Read from the library's own code objects, their metadata notes and their instructions."""
 
 import re
 import struct
@@ -10,15 +10,16 @@ import pytest
 from lighthouse_amd import _lib
 
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
-    """{mangled name: {metadata key: value}} of every kernel in the library."""
+    """{mangled name: {metadata key: value, "object": path of its code object}} of every kernel in the library."""
     _lib.load()
     blob = _lib.library_path().read_bytes()
-    obj = tmp_path_factory.mktemp("code") / "object"
+    folder = tmp_path_factory.mktemp("code")
     found, at = {}, blob.find(MAGIC)
     while at >= 0:
         pos = at + len(MAGIC) + 8
@@ -26,11 +27,13 @@ def kernels(tmp_path_factory):
             offset, size, length = struct.unpack_from("<QQQ", blob, pos)
             target, pos = blob[pos + 24:pos + 24 + length], pos + 24 + length
             if size and b"gfx950" in target:
+                obj = folder / f"object{at + offset}"
                 obj.write_bytes(blob[at + offset:at + offset + size])
                 notes = subprocess.run([READELF, "--notes", str(obj)], capture_output=True, text=True, check=True).stdout
                 for kernel in re.split(r"\n +- \.agpr_count", notes)[1:]:
                     name = re.search(r"\.name: +(\S+)", kernel).group(1)
                     found[name] = {k: int(v) for k, v in re.findall(r"\.(\w+): +(\d+)", kernel)}
+                    found[name]["object"] = obj
         at = blob.find(MAGIC, at + 1)
     assert len(found) > 100
     return found
@@ -55,3 +58,15 @@ def test_small_tile_gemms_are_built_for_the_layouts_that_exist(kernels):
     small = [re.search(r"gemm_small_kernelILi(\d)E", n) for n in kernels]
     of_type = [int(m.group(1)) for m in small if m]
     assert {t: of_type.count(t) for t in set(of_type)} == {_lib.F32: 24, _lib.BF16: 24, _lib.F16: 24, _lib.F8E4M3: 6}
+
+
+def test_cut_gemms_load_without_loops_over_resources(kernels):
+    """The panels of a workgroup are the same for its lanes: a load whose resource the compiler holds in vector registers sits
+    in a loop over the lanes' resources (exec is narrowed right before it), which the kernels cut along K once had in
+    their main loop."""
+    cut = {n: k["object"] for n, k in kernels.items() if re.search(r"gemm16_directILi[12]ELi2ELi1ELb[01]ELb1E", n)}
+    assert len(cut) == 8
+    for obj in set(cut.values()):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", str(obj)], capture_output=True, text=True, check=True).stdout
+        assert "buffer_load_dwordx4" in text and " lds" in text
+        assert not re.search(r"s_and_saveexec_b64[^\n]*\n(?:\s+s_nop[^\n]*\n)*\s+buffer_load_dwordx4[^\n]* lds", text)
