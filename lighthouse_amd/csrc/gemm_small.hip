@@ -379,6 +379,11 @@ constexpr SmallTile kSmallTiles[] = {
     {4, 4, {2.40f, 2.90f, 2.40f}, {0.1200f, 0.3020f, 0.1200f}},  // 8 waves, whose sums fill a CU's LDS: whole rounds
 };
 constexpr float kSmallFixed = 2.0f;
+// What a step costs more per 16 rows of a k-contiguous operand whose rows do not start at multiples of 4 bytes, in us: its
+// chunks go through the L1 at a fraction of the rate (multiples of 4 bytes cost nothing measurable, and an operand that is
+// not k-contiguous little).  178 x 1576 x 7168 bf16 with both operands k-contiguous, one element off: 136 us, 46 on copies
+// for the tile kernels, where the estimate said 22.  Fitted on 1000 such problems on every tile.
+constexpr float kSmallSplit[3] = {0.045f, 0.0f, 0.058f};
 
 double gemm_small_choose(const GemmArgs& g, int dtype, int* tile) {
   const int es = (int)dtype_size(dtype), epc = 16 / es, type = dtype == LH_F32 ? 1 : es == 1 ? 2 : 0;
@@ -387,6 +392,10 @@ double gemm_small_choose(const GemmArgs& g, int dtype, int* tile) {
   // (every chunk load reads one whole chunk of a row; 32-bit step and tile counts)
   if ((ta ? g.M : g.K) < epc || (tb ? g.K : g.N) < epc || g.K >= 1 << 24 || (int64_t)g.M * g.N >= 1ll << 36) return 0.0;
   const int steps = (g.K + 64 / es - 1) / (64 / es);
+  auto split_cost = [&](const void* p, int64_t ld, bool k_contiguous) {
+    return k_contiguous && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(ld * es)) & 3) ? kSmallSplit[type] : 0.0f;
+  };
+  const float split_a = split_cost(g.a, g.lda, !ta), split_b = split_cost(g.b, g.ldb, tb);
   const double stream = 1e-6 * es * ((double)g.M * g.K + (double)g.K * g.N) / 3.6;  // (each operand from memory once)
   double best = 0.0;
   for (int i = 0; i < (int)(sizeof(kSmallTiles) / sizeof(kSmallTiles[0])); ++i) {
@@ -394,7 +403,8 @@ double gemm_small_choose(const GemmArgs& g, int dtype, int* tile) {
     const int64_t tiles = (int64_t)((g.M + 16 * t.mt - 1) / (16 * t.mt)) * ((g.N + 16 * t.nt - 1) / (16 * t.nt));
     double r = tiles > num_cus() ? (double)tiles / num_cus() : 1.0;
     if (t.mt * t.nt == 16) r = ceil(r);
-    const double us = kSmallFixed + fmax(r * (t.b[type] + t.c[type] * steps), stream);
+    const double step = t.c[type] + fmin(t.mt, g.M / 16.0) * split_a + fmin(t.nt, g.N / 16.0) * split_b;
+    const double us = kSmallFixed + fmax(r * (t.b[type] + step * steps), stream);
     if (r <= 4.0 && (*tile < 0 || us < best)) {
       best = us;
       *tile = i;

@@ -92,3 +92,18 @@ def test_a_problem_copied_for_the_tile_kernels_runs_on_them(dtype, M, N, K):
     a0[:, :K], b0[:K, :N] = a, b
     want = ops.gemm(a0, b0, out_dtype=torch.float32)[:, :N]
     assert torch.equal(ops.gemm(a, b, out_dtype=torch.float32), want)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_rows_that_split_dwords_are_priced(dtype):
+    """k-contiguous operands whose rows start at odd elements go through the L1 at a fraction of the rate: this product runs
+    on copies for the tile kernels (same bits as a requested tile on aligned operands), not on the small tiles."""
+    from lighthouse_amd import ops
+
+    M, N, K = 1408, 1024, 2368
+    g = torch.Generator(device="cuda").manual_seed(8)
+    a, b = (torch.randn(rows, K, device="cuda", generator=g).to(DTYPES[dtype]) for rows in (M, N))
+    odd_a, odd_b = torch.empty(M, K + 1, device="cuda", dtype=a.dtype)[:, 1:], torch.empty(N, K + 1, device="cuda", dtype=a.dtype)[:, 1:]
+    odd_a.copy_(a), odd_b.copy_(b)
+    want = ops.gemm(a, b, transpose_b=True, out_dtype=torch.float32, tile=(128, 128))
+    assert torch.equal(ops.gemm(odd_a, odd_b, transpose_b=True, out_dtype=torch.float32), want)
