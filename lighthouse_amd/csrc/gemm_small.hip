@@ -361,11 +361,12 @@ static int launch_small(const GemmArgs& g, hipStream_t s) {
 
 // ---- choice of tile ---------------------------------------------------------------------------
 // Time of a launch, in us: kSmallFixed + r (b + c steps), r = workgroups per compute unit (at least 1), steps =
-// 64-byte steps of K.  What a step costs is the operand bytes the CU pulls from its L2 (about 20 bytes per
+// 64-byte steps of K.  From 8 steps on the last round of workgroups counts for more than its share, from 24 on 0.7 of what it
+// lacks of a whole one: 672 x 512 x 3072 bf16, 1.3 workgroups per CU, takes 20 us where 1.3 alone would say 12.  What a step costs is the operand bytes the CU pulls from its L2 (about 20 bytes per
 // clock whatever the depth of the prefetch), so a larger tile costs less per result and more per workgroup:
 // the cheapest tile is about the largest that still gives every CU one.  b and c are least squares over 400
-// problems per type (M 1 .. 3000, N and K 16 .. 8192, both log-uniform); choosing by them is within 4 % of the
-// best tile on average.  Not for more than 4 workgroups per CU, where tiles whose waves share their operands win.
+// problems per type (M 1 .. 3000, N and K 16 .. 8192, both log-uniform); choosing by them is within 2.5 % of the
+// best tile, or of the other kernels where those are faster, on average.  Not for more than 4 workgroups per CU, where tiles whose waves share their operands win.
 struct SmallTile {
   int mt, nt;
   float b[3], c[3];  // 16-bit, f32, fp8
@@ -402,7 +403,7 @@ double gemm_small_choose(const GemmArgs& g, int dtype, int* tile) {
     const SmallTile& t = kSmallTiles[i];
     const int64_t tiles = (int64_t)((g.M + 16 * t.mt - 1) / (16 * t.mt)) * ((g.N + 16 * t.nt - 1) / (16 * t.nt));
     double r = tiles > num_cus() ? (double)tiles / num_cus() : 1.0;
-    if (t.mt * t.nt == 16) r = ceil(r);
+    r += (t.mt * t.nt == 16 ? 1.0 : 0.7 * fmin(fmax((steps - 8) / 16.0, 0.0), 1.0)) * (ceil(r) - r);
     const double step = t.c[type] + fmin(t.mt, g.M / 16.0) * split_a + fmin(t.nt, g.N / 16.0) * split_b;
     const double us = kSmallFixed + fmax(r * (t.b[type] + step * steps), stream);
     if (r <= 4.0 && (*tile < 0 || us < best)) {

@@ -107,3 +107,15 @@ def test_rows_that_split_dwords_are_priced(dtype):
     odd_a.copy_(a), odd_b.copy_(b)
     want = ops.gemm(a, b, transpose_b=True, out_dtype=torch.float32, tile=(128, 128))
     assert torch.equal(ops.gemm(odd_a, odd_b, transpose_b=True, out_dtype=torch.float32), want)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_a_second_round_of_small_tiles_is_priced(dtype):
+    """1.3 workgroups of small tiles per compute unit take nearly as long as 2: cut along K the tile kernel is faster."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a = torch.randn(672, 3072, device="cuda", generator=g).to(DTYPES[dtype])
+    b = torch.randn(3072, 512, device="cuda", generator=g).to(DTYPES[dtype])
+    want = ops.gemm(a, b, out_dtype=torch.float32, split_k=4)
+    assert torch.equal(ops.gemm(a, b, out_dtype=torch.float32), want)
