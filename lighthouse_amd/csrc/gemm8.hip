@@ -964,7 +964,8 @@ int gemm8(const GemmArgs& g, hipStream_t s) {
     const bool fits = g.K % kBK8 == 0 && g.N % 128 == 0 && g.lda % 16 == 0 && g.ldb % 4 == 0 && g.ldc % 4 == 0 &&
                       aligned16(g.a) && aligned16(g.b) && aligned16(g.out);
     const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
-    const double other = tile8_us(g) + (!fits ? 14.0 + 2.0 * mb + 4e-6 * g.M * g.N : 0.0);
+    // (copies of the operands in one launch, one of the result: fitted on 285 problems of gemm_small.hip's ranges)
+    const double other = tile8_us(g) + (!fits ? 5.3 + 0.24 * mb + 2.2e-6 * g.M * g.N : 0.0);
     int small;
     const double us = gemm_small_choose(g, LH_F8E4M3, &small);
     if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F8E4M3, small, s);
