@@ -384,26 +384,23 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // operand is worth).
   const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
   const bool may_copy = vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22);
+  // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
+  // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
+  const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (g.flags & LH_GEMM_SPLITK_MASK) <= LH_GEMM_SPLITK_NONE &&
       !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones.  Against them stand the direct kernels, plus
-    // the transposed copy of A (K x M read and written, a launch of its own) or the padded copies of operands that
-    // the direct kernels cannot take as they are.
-    const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
-    // (padded copies that are there already cost nothing more)
+    // the transposed or padded copies of operands that the direct kernels cannot take as they are.
+    const bool tb = g.flags & LH_GEMM_TRANSPOSE_B;
     const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0 || g.b_padded) && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
                       aligned16(g.a) && aligned16(g.b);
-    const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
     // (a padded copy has whole k-steps)
     const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) : 1;
-    const double other = direct_us(g, cuts) + (!fits ? 4.0 + 1.3 * mb : ta ? 3.5 + 1.6e-6 * g.M * g.K : 0.0);
+    const double other = direct_us(g, cuts) + operand_copies_us<2>(g, kBK, 8, b_in_place, 0.65);
     int tile;
     const double us = gemm_small_choose(g, DT, &tile);
     if (tile >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, DT, tile, s);
   }
-  // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
-  // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
-  const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && may_copy) {
     if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
     const int rc = untranspose_operands<2>(g, kBK, 8, s);

@@ -355,12 +355,9 @@ int gemm32(const GemmArgs& g_in, hipStream_t s) {
   if (tile == LH_GEMM_TILE_AUTO && !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones; against them stand the direct kernels plus the
     // transposed or padded copies those would need.
-    const bool trans = g.flags & (LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B);
-    // (padded copies that are there already cost nothing more)
     const bool fits = g.K % kBK32 == 0 && (g.N % 4 == 0 || g.b_padded) && g.lda % 4 == 0 && g.ldb % 4 == 0 &&
                       aligned16(g.a) && aligned16(g.b);
-    const double mb = 1e-6 * ((double)g.M * g.K + (double)g.K * g.N);
-    const double other = direct32_us(g) + (!fits ? 4.0 + 2.5 * mb : trans ? 4.0 + 3.2 * mb : 0.0);
+    const double other = direct32_us(g) + operand_copies_us<4>(g, kBK32, 4, false, 0.45);
     int small;
     const double us = gemm_small_choose(g, LH_F32, &small);
     if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F32, small, s);

@@ -303,6 +303,22 @@ inline int untranspose_operands(GemmArgs& g, int k_multiple, int n_multiple, hip
   return 0;
 }
 
+// Time of the copies that the direct kernels need in front of them, in us (0: none): what untranspose_operands and gemm_padded
+// will launch, at 3.5 us a launch and `us_per_mb` per MB of operand copied or zeroed.
+template <int ELEM_BYTES>
+inline double operand_copies_us(const GemmArgs& g, int k_multiple, int n_multiple, bool b_in_place, double us_per_mb) {
+  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
+  const bool odd_k = g.K % k_multiple != 0, odd_n = g.N % n_multiple != 0 && !g.b_padded;
+  auto odd_rows = [](const void* p, int64_t ld) { return ld % (16 / ELEM_BYTES) != 0 || !aligned16(p); };
+  const bool a = ta || odd_k || odd_rows(g.a, g.lda);
+  const bool a_padded = a && (!ta || odd_k || odd_n);  // (by gemm_padded, which then copies a B that could stay, too)
+  const bool b = tb ? !b_in_place || a_padded : odd_k || odd_n || odd_rows(g.b, g.ldb);
+  const double mb_a = a ? 1e-6 * ELEM_BYTES * g.M * g.K : 0.0, mb_b = b ? 1e-6 * ELEM_BYTES * g.K * g.N : 0.0;
+  const bool fill_a = a && ta && odd_k, fill_b = b && tb && (odd_k || odd_n);  // zeros below a transposed copy
+  const int launches = (a && ta) + (b && tb) + fill_a + fill_b + ((a && !ta) || (b && !tb));
+  return 3.5 * launches + us_per_mb * (mb_a * (1 + fill_a) + mb_b * (1 + fill_b));
+}
+
 // A problem whose K the direct kernels cannot take (no multiple of the k-step), or whose operand rows are not
 // 16-byte aligned, runs on them all the same: A and B are copied into temporary matrices padded with zeros,
 // both in one launch.  The kernels write any N, row stride and alignment themselves, except those of fp8

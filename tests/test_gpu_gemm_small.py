@@ -135,3 +135,17 @@ def test_fp8_operand_copies_are_priced_as_they_are_made():
     odd_a.copy_(a)
     want = ops.gemm_fp8(a, b, 0.5, 2.0, out_dtype=torch.float32)[:, :N]
     assert torch.equal(ops.gemm_fp8(odd_a, b[:, :N].contiguous(), 0.5, 2.0, out_dtype=torch.float32), want)
+
+
+def test_only_the_operands_that_are_copied_are_priced():
+    """A few rows of an odd stride next to an aligned B: copying the rows costs little, and the product cut along K is faster than
+    small tiles on rows that split dwords.  The sums have the bits of the requested cut on aligned operands."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(11)
+    a = torch.randn(16, 6144, device="cuda", generator=g).to(torch.bfloat16)
+    b = torch.randn(6144, 2048, device="cuda", generator=g).to(torch.bfloat16)
+    odd = torch.empty(16, 6145, device="cuda", dtype=a.dtype)[:, 1:]
+    odd.copy_(a)
+    want = ops.gemm(a, b, out_dtype=torch.float32, split_k=8)
+    assert torch.equal(ops.gemm(odd, b, out_dtype=torch.float32), want)
