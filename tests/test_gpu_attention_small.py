@@ -41,3 +41,31 @@ def test_small_attention(Z, H, T, gain, dtype, eps, causal):
     q_rounding = eps * largest if T == 1500 and not causal else 0.0
     bound = (2 * eps + 2.0**-20 * largest + 2 * q_rounding) * (p @ v.double().abs().contiguous()) + 2.0**-24 * T
     assert bool(((out[:, :, :T].double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("scale_in_f32", [False, True])
+@pytest.mark.parametrize("stages", [3, 4])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype,eps", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-11)])
+@pytest.mark.parametrize("Z,H,T", [(2, 3, 1000), (1, 2, 200), (1, 1, 300), (1, 2, 65), (2, 3, 512)])
+def test_large_kernels_on_request(Z, H, T, dtype, eps, causal, stages, scale_in_f32):
+    """Few query rows on the 128-row kernels, which these shapes run only on request: lengths that end inside a key
+    tile, Q scaled and rounded or the scores scaled in f32."""
+    from lighthouse_amd import ops
+
+    q, k, v = (_view(Z, H, T, dtype, seed) for seed in (4, 5, 6))
+    out = torch.full((Z, H, T + 9, 64), 7.0, device="cuda", dtype=dtype)
+    ops.attention(q, k, v, causal=causal, out=out[:, :, :T], rows_per_wave=32, stages=stages, scale_in_f32=scale_in_f32)
+    assert bool((out[:, :, T:] == 7.0).all())
+    s = q.double() @ k.double().transpose(-1, -2).contiguous() * 0.125
+    size = q.double().abs() @ k.double().abs().transpose(-1, -2).contiguous() * 0.125
+    if causal:
+        mask = torch.ones(T, T, dtype=torch.bool, device="cuda").triu(1)
+        s, size = s.masked_fill(mask, -float("inf")), size.masked_fill(mask, 0.0)
+    p = s.softmax(-1)
+    want = p @ v.double().contiguous()
+    # P and the result are rounded once, by eps at most (f16: P may also lose 2^-25 where it is subnormal).  A score is off
+    # by 2^-20 of the sum of its terms' sizes (f32) plus, where the scaled Q is rounded, eps of it; P by e^(2 off) - 1.
+    off = float(size.max()) * (2.0**-20 + (0.0 if scale_in_f32 else eps))
+    bound = (2 * eps + 2.7183**(2 * off) - 1) * (p @ v.double().abs().contiguous()) + 2.0**-24 * T
+    assert bool(((out[:, :, :T].double() - want).abs() <= bound).all())

@@ -149,3 +149,32 @@ def test_only_the_operands_that_are_copied_are_priced():
     odd.copy_(a)
     want = ops.gemm(a, b, out_dtype=torch.float32, split_k=8)
     assert torch.equal(ops.gemm(odd, b, out_dtype=torch.float32), want)
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shape,offset", [((2100, 2051, 64), 0), ((2304, 2304, 128), 1),
+                                          ((2100, 2050, 4096), 3)])  # a long K
+def test_tile_kernels_write_any_alignment_in_every_layout(shape, offset, dtype, layout):
+    """Transposed operands too, with bias and activation, on exactly the workspace that the query gives."""
+    from lighthouse_amd import ops
+
+    M, N, K = shape
+    ta, tb = layout[0] == "t", layout[1] == "t"
+    a, av = _matrix(M, K, dtype, 5, 0)
+    b, bv = _matrix(K, N, dtype, 6, 0)
+    a, b = (a.T.contiguous() if ta else a), (b.T.contiguous() if tb else b)
+    want = av.double() @ bv.double()
+    for out_dtype in {DTYPES[dtype], torch.float32}:
+        buf = torch.full((M, N + 5), 7.0, device="cuda", dtype=out_dtype)
+        view = buf[:, offset:offset + N]
+        bias = (torch.arange(N + 1, device="cuda").float() % 5 - 2).to(out_dtype)[1:]
+        options = {"transpose_a": ta, "transpose_b": tb}
+        need = ops.gemm_workspace_bytes(M, N, K, DTYPES[dtype], out_dtype, bias=True, relu=True, operands=(view, a, b, bias), **options)
+        workspace = torch.empty((need + 255) // 256 * 256, dtype=torch.uint8, device="cuda")
+        ops.gemm(a, b, bias, out=view, relu=True, workspace=workspace, **options)
+        assert torch.equal(view, torch.relu(want + bias.double()).to(out_dtype))
+        ops.gemm(a, b, bias, out=view, gelu=True, **options)  # the bits of the same product into aligned rows
+        wide = torch.empty((M, (N + 7) // 8 * 8), device="cuda", dtype=out_dtype)[:, :N]
+        assert torch.equal(view, ops.gemm(a, b, bias, out=wide, gelu=True, **options))
+        assert bool((buf[:, :offset] == 7.0).all()) and bool((buf[:, offset + N:] == 7.0).all())
