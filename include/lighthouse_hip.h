@@ -242,12 +242,12 @@ int lh_hip_gemm_fp8_ws(void* out, const void* a_q, const void* b_q, float scale_
  * LH_ATTN_KSPLIT_2 gives a workgroup of the 64-row kernel two groups of four waves that walk the two
  * halves of the key range side by side and are combined at the end (LH_ATTN_KSPLIT_1: never).
  * 0 lets the library choose by shape.  A request that does not apply fails with LH_ERR_INVALID.
- * LH_ATTN_SCALE_F32 selects where the softmax scale is applied: by default Q is multiplied by
- * scale * log2(e) once and rounded to the element type again (one rounding more than the reference,
- * inside every tolerance of the payload); with this bit Q stays as stored and every score is scaled in
- * f32, as ReplaceWithFusedAttentionOp does (replace_with_fused_attention.py:386), at one more
- * vector instruction per score (about 7 % of the time at [4,16,2048,64]).  The f32 kernel always
- * scales in f32. */
+ * LH_ATTN_SCALE_F32 selects where the softmax scale is applied.  With this bit Q stays as stored and
+ * every score is scaled in f32, as ReplaceWithFusedAttentionOp does (replace_with_fused_attention.py:386).
+ * Without it the library chooses by shape: most problems multiply Q by scale * log2(e) once and round it
+ * to the element type again (one rounding more than the reference, inside every tolerance of the payload),
+ * which saves a vector instruction per score (about 7 % of the time at [4,16,2048,64]); problems with few
+ * query rows (about one small workgroup per compute unit) scale in f32, like the f32 kernel always does. */
 #define LH_ATTN_CAUSAL 0x1
 #define LH_ATTN_ROWS_MASK 0x300
 #define LH_ATTN_ROWS_32 0x100

@@ -5,7 +5,7 @@
 // What bounds a GEMM of a few dozen to a few hundred rows is not arithmetic but the chain of dependent
 // steps one workgroup walks: on the 128 x 128 tile kernel, M = 100, N = 2304, K = 768 is 18 workgroups that
 // each take 24 k-steps one after the other behind barriers (14 us).  Here a workgroup owns a small tile
-// (16 MT x 16 NT) and its NW waves share out the K dimension: wave w multiplies the k-steps w, w + NW, ...
+// (16 MT x 16 NT) and its NW waves share out the K dimension: a wave multiplies a contiguous share of the k-steps
 // on its own, without a barrier, with P steps of both operands requested ahead in registers; the NW
 // partial tiles are added through LDS once, in wave order.  A step is 64 bytes of k per row for every
 // element type (32 values of 16 bit, 64 of fp8, 16 of f32): a lane's operand is one 16-byte chunk.
@@ -16,7 +16,8 @@
 //    that belong to the wave alone and is read back with the transposing LDS reads.
 //
 // Global accesses are 16 bytes wide at element alignment (gfx9 global memory takes any alignment), so odd
-// leading dimensions and unaligned views need no padded copies; everything past K counts as zero.
+// leading dimensions and unaligned views need no padded copies; everything past K counts as zero.  Rows that split
+// dwords are slow all the same (kSmallSplit below).
 #include <cmath>
 #include <type_traits>
 

@@ -254,8 +254,9 @@ def attention(q, k, v, *, causal=False, scale=None, out=None, rows_per_wave=None
     `workspace` (uint8, see attention_workspace_bytes) makes the call take its temporary memory
     from there instead of the library's pool (lh_hip_attention_ws).
     `scale_in_f32` (16-bit tensors, head dimension 64): Q stays as stored and every score is scaled
-    in f32, the reference's rounding points exactly (LH_ATTN_SCALE_F32; about 7 % slower), instead
-    of Q multiplied by the scale once and rounded to the element type again."""
+    in f32, the reference's rounding points exactly (LH_ATTN_SCALE_F32; about 7 % slower). Without it
+    most problems multiply Q by the scale once and round it to the element type again; those with few
+    query rows scale in f32 all the same."""
     if q.dim() != 4 or q.shape != k.shape or q.shape != v.shape:
         raise ValueError("attention expects Q, K, V of equal 4-D shape [Z,H,T,d]")
     _require(q.dtype in _FLOATS and k.dtype == q.dtype and v.dtype == q.dtype,
