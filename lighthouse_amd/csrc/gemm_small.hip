@@ -18,7 +18,6 @@
 // Global accesses are 16 bytes wide at element alignment (gfx9 global memory takes any alignment), so odd
 // leading dimensions and unaligned views need no padded copies; everything past K counts as zero.  Rows that split
 // dwords are slow all the same (kSmallSplit below).
-#include <cmath>
 #include <type_traits>
 
 #include "gemm_common.h"
@@ -399,15 +398,24 @@ double gemm_small_choose(const GemmArgs& g, int dtype, int* tile) {
   };
   const float split_a = split_cost(g.a, g.lda, !ta), split_b = split_cost(g.b, g.ldb, tb);
   const double stream = 1e-6 * es * ((double)g.M * g.K + (double)g.K * g.N) / 3.6;  // (each operand from memory once)
+  // (this runs in front of every launch: shifts for divisions, no library calls; 0.1 us of host time were measurable)
+  const int cus = num_cus(), m16 = (g.M + 15) >> 4, n16 = (g.N + 15) >> 4;
+  const double rows_a = g.M / 16.0, rows_b = g.N / 16.0;
+  const double rest = steps <= 8 ? 0.0 : steps >= 24 ? 0.7 : 0.7 / 16.0 * (steps - 8);
   double best = 0.0;
   for (int i = 0; i < (int)(sizeof(kSmallTiles) / sizeof(kSmallTiles[0])); ++i) {
     const SmallTile& t = kSmallTiles[i];
-    const int64_t tiles = (int64_t)((g.M + 16 * t.mt - 1) / (16 * t.mt)) * ((g.N + 16 * t.nt - 1) / (16 * t.nt));
-    double r = tiles > num_cus() ? (double)tiles / num_cus() : 1.0;
-    r += (t.mt * t.nt == 16 ? 1.0 : 0.7 * fmin(fmax((steps - 8) / 16.0, 0.0), 1.0)) * (ceil(r) - r);
-    const double step = t.c[type] + fmin(t.mt, g.M / 16.0) * split_a + fmin(t.nt, g.N / 16.0) * split_b;
-    const double us = kSmallFixed + fmax(r * (t.b[type] + step * steps), stream);
-    if (r <= 4.0 && (*tile < 0 || us < best)) {
+    const int64_t tiles = (int64_t)((m16 + t.mt - 1) >> __builtin_ctz(t.mt)) * ((n16 + t.nt - 1) >> __builtin_ctz(t.nt));
+    if (tiles > 4 * (int64_t)cus) continue;
+    double r = 1.0;
+    if (tiles > cus) {
+      const double rounds = tiles <= 2 * cus ? 2.0 : tiles <= 3 * cus ? 3.0 : 4.0;
+      r = (double)tiles / cus;
+      r += (t.mt * t.nt == 16 ? 1.0 : rest) * (rounds - r);
+    }
+    const double step = t.c[type] + (t.mt < rows_a ? t.mt : rows_a) * split_a + (t.nt < rows_b ? t.nt : rows_b) * split_b;
+    const double busy = r * (t.b[type] + step * steps), us = kSmallFixed + (busy > stream ? busy : stream);
+    if (*tile < 0 || us < best) {
       best = us;
       *tile = i;
     }
