@@ -379,11 +379,13 @@ static int gemm16_splitk(const GemmArgs& g, uint32_t request, hipStream_t s) {
 template <int DT>
 static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   GemmArgs g = g_in;
-  // An output side of whole 16-byte chunks: what requests ask for.  Without it a small problem takes no temporary
-  // memory, here and in a size query alike, so that it never needs a workspace (it has fewer flops than the copy of an
-  // operand is worth).
+  // An output side of whole 16-byte chunks: what requests ask for.  Without it a small problem takes no memory of a caller's
+  // workspace, here and in a size query alike, so that it never needs one.  The library's own pool it may use where the
+  // untransposed operands then fit the direct kernels, or K is long: a transposed A of fewer rows than the small tiles take,
+  // 1 x 768 x 3200 bf16, runs 34 us on a copy and 260 on the bounds-checked kernel, which gains from one as well (B unaligned,
+  // 1 x 896 x 2560: 221 -> 171; at K = 128 it loses 2 of 14).
   const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
-  const bool may_copy = vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22);
+  const bool may_copy = vec_c || (!g.ws && (g.K >= 512 || rows_fit_untransposed<2>(g))) || (int64_t)g.M * g.N * g.K >= (1 << 22);
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;

@@ -362,9 +362,9 @@ int gemm32(const GemmArgs& g_in, hipStream_t s) {
     const double us = gemm_small_choose(g, LH_F32, &small);
     if (small >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, LH_F32, small, s);
   }
-  // (as in gemm16_dispatch: without aligned chunks on the output side a small problem takes no temporary memory)
+  // (as in gemm16_dispatch: without aligned chunks on the output side a small problem takes no memory of a workspace)
   const bool vec_c = g.N % 4 == 0 && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
-  if (tile == LH_GEMM_TILE_AUTO && (vec_c || (int64_t)g.M * g.N * g.K >= (1 << 22))) {
+  if (tile == LH_GEMM_TILE_AUTO && (vec_c || (!g.ws && (g.K >= 512 || rows_fit_untransposed<4>(g))) || (int64_t)g.M * g.N * g.K >= (1 << 22))) {
     const int rc = untranspose_operands<4>(g, kBK32, 4, s);
     if (rc < 0) return rc;
   }

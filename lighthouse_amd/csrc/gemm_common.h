@@ -303,6 +303,13 @@ inline int untranspose_operands(GemmArgs& g, int k_multiple, int n_multiple, hip
   return 0;
 }
 
+// Every operand that is not transposed (and so copied into rows that are) has rows of aligned 16-byte chunks.
+template <int ELEM_BYTES>
+inline bool rows_fit_untransposed(const GemmArgs& g) {
+  auto fit = [](const void* p, int64_t ld) { return ld % (16 / ELEM_BYTES) == 0 && aligned16(p); };
+  return ((g.flags & LH_GEMM_TRANSPOSE_A) || fit(g.a, g.lda)) && ((g.flags & LH_GEMM_TRANSPOSE_B) || fit(g.b, g.ldb));
+}
+
 // Time of the copies that the direct kernels need in front of them, in us (0: none): what untranspose_operands and gemm_padded
 // will launch, at 3.5 us a launch and `us_per_mb` per MB of operand copied or zeroed.
 template <int ELEM_BYTES>

@@ -776,6 +776,22 @@ def test_gemm_workspace_query_with_an_unaligned_result(dtype, M, N, K, ta):
         assert bool((out[:, :offset] == 7.0).all()) and bool((out[:, offset + N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("dtype,M,N,K", [(torch.bfloat16, 1, 768, 3200), (torch.float16, 2, 536, 1792), (torch.float32, 3, 48, 7552)])
+def test_gemm_few_rows_of_a_transposed_a_with_an_unaligned_result(dtype, M, N, K):
+    """Fewer rows than the small tiles take: with the library's own temporary memory A is copied for the tile kernels whatever
+    the alignment of the result, whose sums have the bits of the same product into aligned rows."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(12)
+    a = torch.randn(K, M, device="cuda", generator=g).to(dtype)
+    b = torch.randn(K, N, device="cuda", generator=g).to(dtype)
+    want = ops.gemm(a, b, transpose_a=True, out_dtype=torch.float32)
+    out = torch.full((M, N + 9), 7.0, device="cuda")
+    ops.gemm(a, b, out=out[:, 1:1 + N], transpose_a=True)
+    assert torch.equal(out[:, 1:1 + N], want)
+    assert bool((out[:, :1] == 7.0).all()) and bool((out[:, 1 + N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("dtype,elt", [(torch.bfloat16, "bf16"), (torch.float16, "f16")])
 @pytest.mark.parametrize("shape", [(4096, 4096, 1024), (8192, 768, 768), (2048, 2304, 768), (512, 1024, 4096), (16, 4096, 8192),
                                    (200, 136, 192), (1000, 520, 320), (64, 8192, 2048)])
