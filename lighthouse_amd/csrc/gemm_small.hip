@@ -361,12 +361,14 @@ static int launch_small(const GemmArgs& g, hipStream_t s) {
 
 // ---- choice of tile ---------------------------------------------------------------------------
 // Time of a launch, in us: kSmallFixed + r (b + c steps), r = workgroups per compute unit (at least 1), steps =
-// 64-byte steps of K.  From 8 steps on the last round of workgroups counts for more than its share, from 24 on 0.7 of what it
-// lacks of a whole one: 672 x 512 x 3072 bf16, 1.3 workgroups per CU, takes 20 us where 1.3 alone would say 12.  What a step costs is the operand bytes the CU pulls from its L2 (about 20 bytes per
+// 64-byte steps of K.  From 8 steps on the last round of workgroups counts for more than its share, from 24 on 0.7 of
+// what it lacks of a whole one: 672 x 512 x 3072 bf16, 1.3 workgroups per CU, takes 20 us where 1.3 alone would say 12.
+// What a step costs is the operand bytes the CU pulls from its L2 (about 20 bytes per
 // clock whatever the depth of the prefetch), so a larger tile costs less per result and more per workgroup:
 // the cheapest tile is about the largest that still gives every CU one.  b and c are least squares over 400
 // problems per type (M 1 .. 3000, N and K 16 .. 8192, both log-uniform); choosing by them is within 2.5 % of the
-// best tile, or of the other kernels where those are faster, on average.  Not for more than 4 workgroups per CU, where tiles whose waves share their operands win.
+// best tile, or of the other kernels where those are faster, on average.  Not for more than 4 workgroups per CU,
+// where tiles whose waves share their operands win.
 struct SmallTile {
   int mt, nt;
   float b[3], c[3];  // 16-bit, f32, fp8
