@@ -244,46 +244,40 @@ static int launch_fast(const GemmArgs& g, hipStream_t s) {
 }
 
 // Tile choice for the direct kernels: 0 = 256 x 256, 1 = 256 x 128, 2 = 128 x 256, 3 = 128 x 128.
-// Cost model: rounds of resident workgroups times the tile area (edge tiles count in full) times a
-// measured cost per flop relative to the 256 x 256 tile (256 x 128 1.19, 128 x 256 1.17; 128 x 128
-// 1.19 with two workgroups on a CU, 1.05 of it for short K, 1.30 alone).  A last round that does
-// not fill the CUs costs less than a full one: the persistent workgroups are not in step, so the
-// extra tiles run while others still finish, and fewer busy CUs hold a higher clock.  Measured at
-// M = 8192, K = 3072 and 4096: a fraction r of a round of the large tiles costs 0.6 + 0.4 r^2 of a
-// round (also when it is the only one), of the 128 x 128 tile (two workgroups per CU) 0.12 + 0.88 r.
-// The 128 x 128 tile runs two workgroups per CU, which share the CU's rate: a round is 2 CUs' worth
-// of tiles at twice a tile's cost, except when no CU gets a second tile.  For short K a tile's
-// prologue and epilogue weigh as much as its main loop, and the 128 x 128 tile, whose two
-// co-resident workgroups cover each other's, costs little more per flop than the large ones.
-// On 84 shapes (M 2048 ... 8192, N 768 ... 4096, K 768 ... 4096) the choice is within 1.3 % of the best
-// explicit tile.  `slow_epilogue`:
-// an accumulator input or an f32 output is staged block by block, which the tiles with a 256 side
-// pay more for (M = 8192, N = 768, K = 3072 + residual: 49.1 / 49.6 us against 46.6 us for 128 x 128;
-// without the residual 42.6 / 43.3 against 43.0).
-static int direct_variant(int M, int N, int K, bool slow_epilogue) {
-  static const int bm[4] = {256, 256, 128, 128}, bn[4] = {256, 128, 256, 128};
+// Time of a launch, in us and apart from what all four share: rounds of resident workgroups (edge tiles count in full)
+// times a tile's a + b K, where a is what its output costs and b K the main loop.  The 128 x 128 tile has two workgroups
+// on a CU; alone on it (no CU gets a second one) a workgroup's loop takes 0.6 of the pair's and its output 0.7.  A last
+// round that does not fill the CUs costs less than a full one: the persistent workgroups are not in step, so the
+// extra tiles run while others still finish, and fewer busy CUs hold a higher clock.  Of a round, a fraction r costs
+// part + (1 - part) r^2 (the 128 x 128 tile: r).  Least squares over 1870 problems on each of the four tiles (M 128 ... 8192,
+// N 512 ... 50256, K 256 ... 4096); what is chosen is within 0.9 % of the best tile on average, 1.24 x at worst (the rule
+// before it, which priced a tile by its flops, 2.4 to 5.0 %, 1.67 x).
+struct DirectTile {
+  int bm, bn;
+  double b, part;
+  double a[4];  // 16-bit result; f32 in rows of whole 64-byte pieces; other f32; accumulator input
+};
+static int direct_variant(const GemmArgs& g) {
+  static constexpr DirectTile tiles[4] = {
+      {256, 256, 0.0244, 0.69, {6.5, 9.6, 12.9, 20.5}},
+      {256, 128, 0.0141, 0.72, {4.4, 6.4, 7.5, 11.3}},
+      {128, 256, 0.0138, 0.77, {4.1, 5.9, 7.4, 10.9}},
+      {128, 128, 0.0136, 0.47, {4.1, 6.4, 6.8, 9.6}},
+  };
+  const int out = (g.flags & LH_GEMM_ACCUMULATE_C) ? 3 : g.out_dt != LH_F32 ? 0 : rows_of_pieces(g) ? 1 : 2;
   const int cus = num_cus();
-  const double big = slow_epilogue ? 1.08 : 1.0;
-  int best = -1;
-  double best_cost = 0.0;
+  int best = 0;
+  double best_us = 0.0;
   for (int v = 0; v < 4; ++v) {
-    const int64_t tiles = (int64_t)((M + bm[v] - 1) / bm[v]) * ((N + bn[v] - 1) / bn[v]);
-    double cost;
-    if (v < 3) {
-      const double per_flop = v == 0 ? 1.0 : v == 1 ? 1.19 : 1.17;
-      const double r = (double)(tiles % cus) / cus;
-      const double rounds = (double)(tiles / cus) + (r > 0.0 ? 0.6 + 0.4 * r * r : 0.0);
-      cost = rounds * bm[v] * bn[v] * per_flop * big;
-    } else if (tiles <= cus) {
-      cost = 128.0 * 128.0 * (K <= 1536 ? 1.08 : 1.30);
-    } else {
-      const double r = (double)(tiles % (2 * cus)) / (2 * cus);
-      const double rounds = (double)(tiles / (2 * cus)) + (r > 0.0 ? 0.12 + 0.88 * r : 0.0);
-      cost = rounds * 2.0 * 128.0 * 128.0 * (K <= 1536 ? 1.05 : 1.19);
-    }
-    if (best < 0 || cost < best_cost) {
+    const DirectTile& t = tiles[v];
+    const int64_t n = (int64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
+    const int slots = v < 3 ? cus : 2 * cus;
+    const double r = (double)(n % slots) / slots;
+    const double rounds = (double)(n / slots) + (r > 0.0 ? t.part + (1.0 - t.part) * (v < 3 ? r * r : r) : 0.0);
+    const double us = v == 3 && n <= cus ? 0.7 * t.a[out] + 0.0082 * g.K : rounds * (t.a[out] + t.b * g.K);
+    if (v == 0 || us < best_us) {
       best = v;
-      best_cost = cost;
+      best_us = us;
     }
   }
   return best;
@@ -438,7 +432,7 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
       const int rc = gemm16_splitk<DT>(g, splitk, s);
       if (rc <= 0) return rc;
     }
-    const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g.M, g.N, g.K, g.out_dt == LH_F32 || (g.flags & LH_GEMM_ACCUMULATE_C) != 0);
+    const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g);
     if (v == 0) return launch_direct<DT, 4, 2>(g, s);
     if (v == 1) return launch_direct<DT, 4, 1>(g, s);
     if (v == 2) return launch_direct<DT, 2, 2>(g, s);

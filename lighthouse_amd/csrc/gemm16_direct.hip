@@ -434,6 +434,124 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
   }
 }
 
+// f32 results in rows that do not start at multiples of 64 bytes (a language-model head over 50257 words), without an
+// accumulator input.  A store that covers part of a 64-byte piece of memory costs far more than its share (the pieces
+// are read and merged on the way out), and a row segment per wave leaves two such pieces in every 128 bytes.  Here the
+// four waves side by side put 16 rows of their columns next to each other in `stage`, a wave then writes whole rows of
+// the tile: the pieces that lie inside the row in 16-byte stores past the caches, the up to 15 elements in front of
+// the first and behind the last such piece one by one through the L2, where the neighbouring tile's may still join them.
+// M = 8192, N = 50257, K = 768 bf16, 256 x 256 tile: 1338 us with a segment per wave, 680 with whole rows.
+template <int DT, int TM, int TN>
+__device__ __forceinline__ void direct_finish_rows(const GemmArgs& g, int wave, uint8_t* __restrict__ stage,
+                                                   const f32x4 (&acc)[2 * TN][2 * TM], int m0, int n0, int wm0, int wn0) {
+  using Cfg = DirectCfg<TM, TN>;
+  constexpr int BN = Cfg::BN, RB = BN * 4;            // bytes of a staged row, 32 of them
+  static_assert(32 * RB == Cfg::kStageBytes, "16 rows of each half of the tile's rows");
+  constexpr int RPS = 2 / TN, NS = 4 / RPS;           // rows per 64-lane store of 16 bytes; stores per wave
+  const int lane = lane_now();
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int len = min(BN, g.N - n0);
+  // Staged row r in turn j: row (r / 16) WTM + 16 j + r % 16 of the tile.  16 rows are a multiple of 64 bytes, so where
+  // the pieces of a row start does not depend on j and all addresses below move by `turn` from one j to the next.
+  const int64_t turn = 16 * g.ldc;
+  auto tile_row = [](int r) { return (r >> 4) * Cfg::WTM + (r & 15); };
+  // 16-byte chunk k of staged row r, swapped with one of 8 by the row against bank conflicts
+  auto at = [](int r, int k) { return r * RB + ((k ^ (r & 7)) << 4); };
+  struct Row {
+    float* p;    // the row's first element in the tile
+    int head;    // elements in front of the first piece
+    int pieces;  // whole pieces
+  };
+  auto row_of = [&](int r) -> Row {
+    float* const p = reinterpret_cast<float*>(g.out) + (int64_t)(m0 + tile_row(r)) * g.ldc + n0;
+    const int head = (int)(-(reinterpret_cast<uintptr_t>(p) >> 2) & 15);
+    return Row{p, head, max(len - head, 0) >> 4};
+  };
+  // Whole pieces: the lane stores elements head + 4 c .. +4 of its row, the end of one chunk and the start of the next.
+  float* wide[NS];
+  int wide_row[NS], wide_lds[NS];
+  bool wide_ok[NS], by1[NS], by2[NS];
+#pragma unroll
+  for (int t = 0; t < NS; ++t) {
+    const int r = 4 * wave + RPS * t + (RPS == 2 ? lane >> 5 : 0), c = RPS == 2 ? lane & 31 : lane;
+    const Row row = row_of(r);
+    wide[t] = row.p + row.head + 4 * c;
+    wide_row[t] = m0 + tile_row(r);
+    wide_ok[t] = c < 4 * row.pieces;
+    wide_lds[t] = at(r, min((row.head >> 2) + c, RB / 16 - 1));
+    by1[t] = row.head & 1;
+    by2[t] = row.head & 2;
+  }
+  // The elements in front and behind: lanes 0 .. 15 and 16 .. 31 of a row's 32.
+  float* edge[2];
+  int edge_row[2], edge_lds[2];
+  bool edge_ok[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int r = 4 * wave + 2 * t + (lane >> 5), c = lane & 15;
+    const Row row = row_of(r);
+    const bool tail = lane & 16;
+    const int d = tail ? row.head + 16 * row.pieces + c : c;
+    edge[t] = row.p + d;
+    edge_row[t] = m0 + tile_row(r);
+    edge_ok[t] = d < (tail ? len : min(row.head, len));
+    edge_lds[t] = at(r, min(d, BN - 1) >> 2) + 4 * (d & 3);
+  }
+  epi_dispatch_linear(g, [&](auto variant) {
+    using E = decltype(variant);
+    f32x4 b4[2 * TN];
+    int put[2 * TN];
+#pragma unroll
+    for (int i = 0; i < 2 * TN; ++i) {
+      b4[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (epi_has_bias<E>(g)) b4[i] = bias4<DT, true>(g, n0 + wn0 + 16 * i + 4 * g4);
+      put[i] = at((wm0 ? 16 : 0) + l16, (wn0 >> 2) + 4 * i + g4);
+    }
+#pragma unroll
+    for (int j = 0; j < 2 * TM; ++j) {
+#pragma unroll
+      for (int i = 0; i < 2 * TN; ++i) {
+        float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        epi_apply4<E>(g, b4[i], v);
+        *reinterpret_cast<f32x4*>(stage + put[i]) = f32x4{v[0], v[1], v[2], v[3]};
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      u32x4 own[NS];
+      uint32_t one[2];
+#pragma unroll
+      for (int t = 0; t < NS; ++t) own[t] = *reinterpret_cast<const u32x4*>(stage + wide_lds[t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) one[t] = *reinterpret_cast<const uint32_t*>(stage + edge_lds[t]);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        // (every lane takes part: the next chunk comes from the next lane; the last lane of a row needs none)
+        uint32_t w[7], u[6];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = own[t][e];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) w[4 + e] = __builtin_amdgcn_update_dpp(0, own[t][e], 0x130, 0xf, 0xf, false);
+#pragma unroll
+        for (int e = 0; e < 6; ++e) {
+          const uint32_t a = w[e], b = w[e + 1];
+          u[e] = by1[t] ? b : a;
+        }
+        u32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t a = u[e], b = u[e + 2];
+          v[e] = by2[t] ? b : a;
+        }
+        if (wide_ok[t] && wide_row[t] + 16 * j < g.M)
+          __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(wide[t] + j * turn));
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        if (edge_ok[t] && edge_row[t] + 16 * j < g.M) reinterpret_cast<uint32_t*>(edge[t] + j * turn)[0] = one[t];
+    }
+  });
+}
+
 // End of a tile: once every wave has left the rings, the first loads of the workgroup's NEXT tile
 // are issued into them (their latency and the cold start of the pipeline hide behind this tile's
 // stores), then the accumulators are written out.  16-bit outputs are staged through `stage`, an
@@ -508,7 +626,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
           if constexpr (EDGE) {
             if (m < g.M && n < g.N) store8_any(outp + (int64_t)m * g.ldc + n, w, g.N - n);
           } else {
-            *reinterpret_cast<u32x4*>(outp + (int64_t)m * g.ldc + n) = w;
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(outp + (int64_t)m * g.ldc + n));
           }
         }
       }
@@ -517,6 +635,12 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
   }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (HAS_NEXT) direct_prologue<TM, TN, BT>(next, nk, ring);
+  if constexpr (EDGE && !BLOCKS) {
+    if (g.out_dt == LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C) && !rows_of_pieces(g)) {
+      direct_finish_rows<DT, TM, TN>(g, next.wave, stage, acc, m0, n0, wm0, wn0);
+      return;
+    }
+  }
   {
     // f32 output (with or without an accumulator input), or a 16-bit output with an accumulator
     // input: the scaled f32 accumulators of a block of 32 rows x 16 NI columns go through the wave's
@@ -615,13 +739,16 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[e] += b4[e];
             }
+            // (the blocks of a launch cut along K are read again at once)
             if constexpr (EDGE && !BLOCKS)
-              store4_any<out32 ? LH_F32 : DT>(g.out, off, v, g.N - n);
-            else if constexpr (out32)
+              store4_any<out32 ? LH_F32 : DT, out32 && !has_c>(g.out, off, v, g.N - n);
+            else if constexpr (out32 && BLOCKS)
               *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off) = v;
+            else if constexpr (out32)
+              __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off));
             else
-              *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(g.out) + off) =
-                  u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+              __builtin_nontemporal_store(u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])},
+                                          reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(g.out) + off));
           }
         }
       }
@@ -672,6 +799,9 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
   constexpr int WN = 4;
   const int wm0 = (wave / WN) * Cfg::WTM, wn0 = (wave % WN) * Cfg::WTN;
   const int l16 = lane & 15, g4 = lane >> 4;
+
+  if (g.late_units && (int)blockIdx.x >= g.late_from)
+    for (int i = 0; i < g.late_units; ++i) __builtin_amdgcn_s_sleep(16);  // 16 x 64 clocks
 
   DirectCtx<TM, TN> c;
   c.wave = wave;
@@ -767,6 +897,17 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
   const int resident = num_cus() * (2 * lds <= 160 * 1024 ? 2 : 1);
   GemmArgs ga = g;
   ga.one_barrier = ntiles > num_cus();
+  // 256 x 256 tiles, one workgroup per CU: workgroups in step store their tiles in step, and the main loops in between leave
+  // the memory idle.  So some start half a tile late: those that have a tile fewer than the others where that is up to half
+  // of them (they have the time), half of them where all have as many and those are enough.  M = 8192, N = 50432, K = 768
+  // bf16: 559 -> 540 us, with f32 results 633 -> 605.
+  if (TM * TN == 8) {
+    const int rest = ntiles % resident, rounds = ntiles / resident;
+    if (rounds >= 1 && (rest || rounds >= 8)) {
+      ga.late_from = rest > resident / 2 ? rest : resident / 2;
+      ga.late_units = 2 + (g.K < 8192 ? g.K : 8192) / 40;
+    }
+  }
   LH_LAUNCH(kern, dim3(ntiles < resident ? ntiles : resident), dim3(512), lds, s, ga);
   return check_launch("gemm16_direct");
 }

@@ -27,6 +27,9 @@ struct GemmArgs {
   int one_barrier = 0;
   // B is a copy whose rows hold whole 16-byte chunks past column N (zeros): N need not be a multiple of them.
   bool b_padded = false;
+  // 16-bit direct kernel: workgroups from `late_from` on start `late_units` x 1024 clocks after the others (set by the
+  // launcher; 0: none).
+  int late_from = 0, late_units = 0;
 };
 
 // Epilogue for 4 consecutive columns of one row.
@@ -99,24 +102,30 @@ __device__ __forceinline__ f32x4 load4_any(const void* p, int64_t at, int left) 
     if (e < left) v[e] = load_as_f32<DT>(p, at + e);
   return v;
 }
-// ... and stored.
-template <int DT>
+// ... and stored (STREAM: whole vectors past the caches).
+template <int DT, bool STREAM = false>
 __device__ __forceinline__ void store4_any(void* p, int64_t at, const f32x4& v, int left) {
   if (left >= 4) {
-    if constexpr (DT == LH_F32)
-      *reinterpret_cast<f32x4_any*>(reinterpret_cast<float*>(p) + at) = v;
-    else
-      *reinterpret_cast<u32x2_any*>(reinterpret_cast<uint16_t*>(p) + at) = u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+    if constexpr (DT == LH_F32) {
+      f32x4_any* const d = reinterpret_cast<f32x4_any*>(reinterpret_cast<float*>(p) + at);
+      if constexpr (STREAM) __builtin_nontemporal_store(f32x4_any(v), d);
+      else *d = v;
+    } else {
+      u32x2_any* const d = reinterpret_cast<u32x2_any*>(reinterpret_cast<uint16_t*>(p) + at);
+      const u32x2 w = {pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+      if constexpr (STREAM) __builtin_nontemporal_store(u32x2_any(w), d);
+      else *d = w;
+    }
     return;
   }
 #pragma unroll
   for (int e = 0; e < 3; ++e)
     if (e < left) store_from_f32<DT>(p, at + e, v[e]);
 }
-// 8 packed 16-bit values, of which the first `left` are stored.
+// 8 packed 16-bit values, of which the first `left` are stored, past the caches if all are.
 __device__ __forceinline__ void store8_any(uint16_t* p, const u32x4& w, int left) {
   if (left >= 8) {
-    *reinterpret_cast<u32x4_any*>(p) = w;
+    __builtin_nontemporal_store(u32x4_any(w), reinterpret_cast<u32x4_any*>(p));
     return;
   }
 #pragma unroll

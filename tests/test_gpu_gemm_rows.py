@@ -1,0 +1,49 @@
+"""f32 results of the tile GEMM kernels in rows that do not start at multiples of 64 bytes, and launches whose workgroups
+start late."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16}
+
+
+@pytest.mark.parametrize("dtype,transpose_b", [("bf16", False), ("bf16", True), ("f16", False)])
+@pytest.mark.parametrize("M,N,K,pad,offset", [(129, 9001, 64, 0, 0),      # 128 x 128 tiles, the last of 41 columns
+                                              (300, 16641, 64, 0, 0),     # ... and of one column, fewer than stand in front of a piece
+                                              (2050, 3000, 128, 4, 0),    # rows 16 bytes past a piece, each by 16 more
+                                              (1024, 8192, 64, 1, 3),     # whole tiles, every phase of a row
+                                              (513, 8197, 192, 8, 7),
+                                              (4096, 9216, 64, 5, 1),     # several rounds of the large tiles
+                                              (4100, 8450, 64, 0, 0)])
+def test_rows_between_pieces(M, N, K, pad, offset, dtype, transpose_b):
+    """Integer operands: the f32 sum is exact in any order, so every element has one right bit pattern."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator().manual_seed(M + N)
+    draw = lambda *shape: torch.randint(-3, 4, shape, generator=g).float()
+    a, b, bias = draw(M, K), draw(N, K) if transpose_b else draw(K, N), draw(N)
+    want = (a @ (b.T if transpose_b else b)).cuda()
+    a, b = a.cuda().to(DTYPES[dtype]), b.cuda().to(DTYPES[dtype])
+    buf = torch.full((offset + M * (N + pad),), 7.0, device="cuda")
+    rows = buf[offset:].view(M, N + pad)
+    out = rows[:, :N]
+    for extra in ({}, {"relu": True}):
+        want_now = torch.relu(want + bias.cuda()) if extra else want
+        out.fill_(float("nan"))
+        ops.gemm(a, b, bias.cuda() if extra else None, out=out, transpose_b=transpose_b, **extra)
+        assert torch.equal(out, want_now)
+        assert bool((rows[:, N:] == 7.0).all()) and bool((buf[:offset] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N", [(2048, 33280),    # 1040 tiles of 256 x 256: four rounds and 16 tiles, half the workgroups start late
+                                 (2048, 45056),    # 5.5 rounds: those that have a tile fewer do
+                                 (2048, 65536)])   # eight whole rounds: half of them do
+def test_workgroups_that_start_late(M, N):
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(N)
+    a, b = (torch.randint(-3, 4, s, device="cuda", generator=g).float() for s in ((M, 64), (64, N)))
+    got = ops.gemm(a.bfloat16(), b.bfloat16())
+    assert torch.equal(got, (a @ b).bfloat16())
