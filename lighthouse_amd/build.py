@@ -19,7 +19,7 @@ LIB_DIR = ROOT / "lighthouse_amd" / "lib"
 LIB_PATH = LIB_DIR / "liblighthouse_hip.so"
 PROBE_LIB = LIB_DIR / "liblighthouse_probe.so"  # bench.py's MFMA-rate probe, not part of the product library
 
-HIP_SOURCES = ["runtime.hip", "gemm16.hip", "gemm16_direct.hip", "gemm32.hip", "gemm8.hip", "gemm_small.hip", "attention.hip", "attention_small.hip", "rowwise.hip", "api.hip"]
+HIP_SOURCES = ["runtime.hip", "gemm16.hip", "gemm16_direct.hip", "gemm32.hip", "gemm8.hip", "gemm_small.hip", "gemm_small_norm.hip", "attention.hip", "attention_small.hip", "rowwise.hip", "api.hip"]
 
 # Sources compiled more than once, with different macros: {source: {suffix of the object: macros}}.
 INSTANCES = {

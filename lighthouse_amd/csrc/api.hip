@@ -344,22 +344,39 @@ int lh_hip_nanogpt_block(float* y, const float* x, const lh_nanogpt_block_params
   ws.bytes = workspace_bytes - (size_t)(w - reinterpret_cast<char*>(workspace));
   auto bias_flag = [](const void* b) -> uint32_t { return b ? LH_GEMM_HAS_BIAS : 0u; };
   int rc;
-  // ln1 = LN(x), rounded to the matmul input type.
-  if ((rc = layer_norm(ln, x, p->ln1_g, p->ln1_b, rows, C, eps, LH_F32, dtype, false, s))) return rc;
-  if (p->w_qkv) {
-    // qkv = ln1 Wqkv + bqkv
-    if ((rc = gemm_run(qkv, nullptr, ln, p->w_qkv, p->b_qkv, rows, 3 * C, C, C, 3 * C, 3 * C, dtype, dtype, bdt,
-                       bias_flag(p->b_qkv), s, &ws)))
-      return rc;
-  } else {
-    // q, k, v = ln1 Wq, ln1 Wk, ln1 Wv into the three column blocks of the same buffer
-    const void* wsep[3] = {p->w_q, p->w_k, p->w_v};
+  // out = act(LN(xs) W_i + bias_i), the `groups` products side by side in rows of groups * N: one launch where that is the
+  // faster way, else the LayerNorm, rounded to the matmul input type, and the products.
+  auto normed_products = [&](void* out, const float* xs, const float* gamma, const float* beta, int groups, const void* const* wi,
+                             const void* const* bi, int64_t N, uint32_t act) -> int {
+    NormedGemm n;
+    GemmArgs& g = n.g;
+    g.out = out; g.c = nullptr; g.a = xs; g.b = wi[0]; g.bias = bi[0];
+    g.M = (int)rows; g.N = (int)N; g.K = (int)C;
+    g.lda = C; g.ldb = N; g.ldc = groups * N;
+    g.flags = bias_flag(bi[0]) | act; g.out_dt = dtype; g.bias_dt = bdt; g.alpha = 1.0f;
+    n.gamma = gamma; n.beta = beta; n.eps = eps; n.inv_n = (float)(1.0 / (double)C);
     for (int i = 0; i < 3; ++i) {
-      const void* bi = p->b_qkv ? static_cast<const char*>(p->b_qkv) + (size_t)i * C * eb : nullptr;
-      if ((rc = gemm_run(static_cast<char*>(qkv) + (size_t)i * C * e, nullptr, ln, wsep[i], bi, rows, C, C, C, C, 3 * C,
-                         dtype, dtype, bdt, bias_flag(bi), s, &ws)))
-        return rc;
+      n.b[i] = wi[i < groups ? i : 0];
+      n.bias[i] = bi[i < groups ? i : 0];
     }
+    n.groups = groups;
+    const int tile = gemm_normed_choose(n, dtype);
+    if (tile >= 0) return gemm_normed(n, dtype, tile, s);
+    if (int e = layer_norm(ln, xs, gamma, beta, rows, C, eps, LH_F32, dtype, false, s)) return e;
+    for (int i = 0; i < groups; ++i)
+      if (int e2 = gemm_run(static_cast<char*>(out) + (size_t)i * N * e, nullptr, ln, wi[i], bi[i], rows, N, C, C, N, groups * N, dtype,
+                            dtype, bdt, bias_flag(bi[i]) | act, s, &ws))
+        return e2;
+    return LH_OK;
+  };
+  // q, k, v = LN(x) Wq, LN(x) Wk, LN(x) Wv (+ biases) into the three column blocks of one buffer
+  if (p->w_qkv) {
+    if ((rc = normed_products(qkv, x, p->ln1_g, p->ln1_b, 1, &p->w_qkv, &p->b_qkv, 3 * C, 0))) return rc;
+  } else {
+    const void* const wsep[3] = {p->w_q, p->w_k, p->w_v};
+    const void* bsep[3];
+    for (int i = 0; i < 3; ++i) bsep[i] = p->b_qkv ? static_cast<const char*>(p->b_qkv) + (size_t)i * C * eb : nullptr;
+    if ((rc = normed_products(qkv, x, p->ln1_g, p->ln1_b, 3, wsep, bsep, C, 0))) return rc;
   }
   // Attention on (B, H, T, hs) strided views of the (B*T, 3C) projection buffer.
   {
@@ -375,12 +392,9 @@ int lh_hip_nanogpt_block(float* y, const float* x, const lh_nanogpt_block_params
   if ((rc = gemm_run(a, x, att, p->w_o, p->b_o, rows, C, C, C, C, C, dtype, LH_F32, bdt,
                      bias_flag(p->b_o) | LH_GEMM_ACCUMULATE_C, s, &ws)))
     return rc;
-  // ln2 = LN(a)
-  if ((rc = layer_norm(ln, a, p->ln2_g, p->ln2_b, rows, C, eps, LH_F32, dtype, false, s))) return rc;
-  // h = act(ln2 W1 + b1)
-  const uint32_t act = cfg.activation == LH_ACT_RELU ? LH_GEMM_HAS_RELU : LH_GEMM_HAS_GELU;
-  if ((rc = gemm_run(hid, nullptr, ln, p->w_fc, p->b_fc, rows, hidden, C, C, hidden, hidden, dtype, dtype, bdt,
-                     bias_flag(p->b_fc) | act, s, &ws)))
+  // h = act(LN(a) W1 + b1)
+  if ((rc = normed_products(hid, a, p->ln2_g, p->ln2_b, 1, &p->w_fc, &p->b_fc, hidden,
+                            cfg.activation == LH_ACT_RELU ? LH_GEMM_HAS_RELU : LH_GEMM_HAS_GELU)))
     return rc;
   // y = a + h W2 + b2
   return gemm_run(y, a, hid, p->w_proj, p->b_proj, rows, C, hidden, hidden, C, C, dtype, LH_F32, bdt,

@@ -456,6 +456,12 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   return check_launch("gemm16_generic");
 }
 
+double gemm16_us(const GemmArgs& g, int ab_dtype) {
+  int tile;
+  const double direct = direct_us(g, 1), small = gemm_small_choose(g, ab_dtype, &tile);
+  return tile >= 0 && small * kSmallMargin < direct ? small * kSmallMargin : direct;
+}
+
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s) {
   if (ab_dtype == LH_BF16) return gemm16_dispatch<LH_BF16>(g, s);
   return gemm16_dispatch<LH_F16>(g, s);

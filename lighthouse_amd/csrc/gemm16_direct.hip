@@ -800,8 +800,18 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
   const int wm0 = (wave / WN) * Cfg::WTM, wn0 = (wave % WN) * Cfg::WTN;
   const int l16 = lane & 15, g4 = lane >> 4;
 
-  if (g.late_units && (int)blockIdx.x >= g.late_from)
-    for (int i = 0; i < g.late_units; ++i) __builtin_amdgcn_s_sleep(16);  // 16 x 64 clocks
+  // 256 x 256 tiles, one workgroup per CU: workgroups in step store their tiles in step, and the main loops in between leave
+  // the memory idle.  So some start half a tile late: those that have a tile fewer than the others where that is up to half
+  // of them (they have the time), half of them where all have as many and those are enough.  M = 8192, N = 50432, K = 768
+  // bf16: 559 -> 540 us, with f32 results 633 -> 605.
+  if constexpr (TM * TN == 8) {
+    const int grid = (int)gridDim.x;
+    if (ntiles > grid) {
+      const int rest = ntiles % grid;
+      if ((rest || ntiles >= 8 * grid) && (int)blockIdx.x >= max(rest, grid / 2))
+        for (int i = min(g.K, 8192) / 40 + 2; i > 0; --i) __builtin_amdgcn_s_sleep(16);  // 16 x 64 clocks
+    }
+  }
 
   DirectCtx<TM, TN> c;
   c.wave = wave;
@@ -897,17 +907,6 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
   const int resident = num_cus() * (2 * lds <= 160 * 1024 ? 2 : 1);
   GemmArgs ga = g;
   ga.one_barrier = ntiles > num_cus();
-  // 256 x 256 tiles, one workgroup per CU: workgroups in step store their tiles in step, and the main loops in between leave
-  // the memory idle.  So some start half a tile late: those that have a tile fewer than the others where that is up to half
-  // of them (they have the time), half of them where all have as many and those are enough.  M = 8192, N = 50432, K = 768
-  // bf16: 559 -> 540 us, with f32 results 633 -> 605.
-  if (TM * TN == 8) {
-    const int rest = ntiles % resident, rounds = ntiles / resident;
-    if (rounds >= 1 && (rest || rounds >= 8)) {
-      ga.late_from = rest > resident / 2 ? rest : resident / 2;
-      ga.late_units = 2 + (g.K < 8192 ? g.K : 8192) / 40;
-    }
-  }
   LH_LAUNCH(kern, dim3(ntiles < resident ? ntiles : resident), dim3(512), lds, s, ga);
   return check_launch("gemm16_direct");
 }

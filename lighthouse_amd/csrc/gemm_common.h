@@ -27,9 +27,6 @@ struct GemmArgs {
   int one_barrier = 0;
   // B is a copy whose rows hold whole 16-byte chunks past column N (zeros): N need not be a multiple of them.
   bool b_padded = false;
-  // 16-bit direct kernel: workgroups from `late_from` on start `late_units` x 1024 clocks after the others (set by the
-  // launcher; 0: none).
-  int late_from = 0, late_units = 0;
 };
 
 // Epilogue for 4 consecutive columns of one row.
@@ -488,6 +485,8 @@ __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, c
 }
 
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s);
+// Estimated time of a 16-bit product with few tiles, untransposed and aligned, not cut along K, in us.
+double gemm16_us(const GemmArgs& g, int ab_dtype);
 int gemm32(const GemmArgs& g, hipStream_t s);
 int gemm8(const GemmArgs& g, hipStream_t s);
 // Kernels for problems with few output tiles (gemm_small.hip): the tile they would use (-1: none fits the
@@ -499,5 +498,18 @@ double gemm_small_choose(const GemmArgs& g, int dtype, int* tile);
 // the tile kernels stay, which add up k in one order whatever the tile.
 constexpr double kSmallMargin = 1.08;
 int gemm_small(const GemmArgs& g, int dtype, int tile, hipStream_t s);
+
+// LayerNorm of x and up to three products of its result, side by side in the output, in one launch (gemm_small_norm.hip).
+struct NormedGemm {
+  GemmArgs g;  // a: x, f32; N: columns of one product; b and bias unused
+  const float *gamma, *beta;
+  float eps, inv_n;
+  const void* b[3];
+  const void* bias[3];
+  int groups;
+};
+// The tile it would run on; -1: the LayerNorm and the products on their own are the faster way, or it does not take them.
+int gemm_normed_choose(const NormedGemm& n, int dtype);
+int gemm_normed(const NormedGemm& n, int dtype, int tile, hipStream_t s);
 
 }  // namespace lh

@@ -18,178 +18,9 @@
 // Global accesses are 16 bytes wide at element alignment (gfx9 global memory takes any alignment), so odd
 // leading dimensions and unaligned views need no padded copies; everything past K counts as zero.  Rows that split
 // dwords are slow all the same (kSmallSplit below).
-#include <type_traits>
-
-#include "gemm_common.h"
+#include "gemm_small.h"
 
 namespace lh {
-
-typedef short small_s16x4 __attribute__((ext_vector_type(4)));
-typedef int small_i32x2 __attribute__((ext_vector_type(2)));
-
-// c += a b for one step: the lane's 16-byte chunks of a row of each operand (lane / 16 selects the chunk of
-// the step's four).  First operand = B fragment: a lane's result is 4 consecutive columns of one row.
-template <int DT>
-__device__ __forceinline__ f32x4 small_mma(u32x4 b, u32x4 a, f32x4 c) {
-  if constexpr (DT == LH_BF16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b), __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
-  } else if constexpr (DT == LH_F16) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, b), __builtin_bit_cast(f16x8, a), c, 0, 0, 0);
-  } else if constexpr (DT == LH_F8E4M3) {
-    typedef long l2 __attribute__((ext_vector_type(2)));
-    const l2 bl = __builtin_bit_cast(l2, b), al = __builtin_bit_cast(l2, a);
-    c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(bl[0], al[0], c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(bl[1], al[1], c, 0, 0, 0);
-  } else {
-    const f32x4 bf = __builtin_bit_cast(f32x4, b), af = __builtin_bit_cast(f32x4, a);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) c = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[t], af[t], c, 0, 0, 0);
-    return c;
-  }
-}
-
-template <int DT>
-constexpr int small_elem_bytes() { return DT == LH_F32 ? 4 : DT == LH_F8E4M3 ? 1 : 2; }
-
-// The chunk moved down by `n` elements (0 .. EPC, or more: nothing is left), zeros on top.
-template <int ES>
-__device__ __forceinline__ u32x4 small_shift_chunk(u32x4 c, int n) {
-  const int bytes = ES * n;
-  uint32_t d0 = c[0], d1 = c[1], d2 = c[2], d3 = c[3];
-  const bool by8 = bytes & 8, by4 = bytes & 4, all = bytes >= 16;
-  d0 = by8 ? d2 : d0;
-  d1 = by8 ? d3 : d1;
-  d2 = by8 ? 0u : d2;
-  d3 = by8 ? 0u : d3;
-  d0 = by4 ? d1 : d0;
-  d1 = by4 ? d2 : d1;
-  d2 = by4 ? d3 : d2;
-  d3 = by4 ? 0u : d3;
-  const int b = bytes & 3;
-  d0 = __builtin_amdgcn_alignbyte(d1, d0, b);
-  d1 = __builtin_amdgcn_alignbyte(d2, d1, b);
-  d2 = __builtin_amdgcn_alignbyte(d3, d2, b);
-  d3 = __builtin_amdgcn_alignbyte(0u, d3, b);
-  return u32x4{all ? 0u : d0, all ? 0u : d1, all ? 0u : d2, all ? 0u : d3};
-}
-
-// One operand panel of F fragments of 16 rows (A) or columns (B), k-contiguous (KC) or not.  Every load of
-// a step is one 16-byte access whatever the sizes: a chunk that would cross the end of its row is read
-// from the row's last EPC elements instead and moved down in registers (the contiguous dimension has at
-// least EPC elements), so the number of loads in flight is known at compile time and the waits stay exact.
-template <int DT, int F, bool KC>
-struct SmallPanel {
-  static constexpr int ES = small_elem_bytes<DT>(), EPC = 16 / ES, KSTEP = 64 / ES;
-  static constexpr int CPR = F * ES;             // !KC: 16-byte chunks per k row
-  static constexpr int RPL = 64 / CPR;           // !KC: k rows per load
-  static constexpr int RS = CPR * 16 + 16;       // !KC: bytes of a k row in LDS (one chunk of padding)
-  static constexpr int kLdsBytes = KC ? 0 : KSTEP * RS;
-  const uint8_t* base[KC ? F : 1];  // KC: the lane's chunk of its row in each fragment; !KC: of its first k row
-  int64_t ld_bytes;
-  int over = 0;              // !KC: elements by which the lane's chunk was moved back to stay inside the row
-  bool whole = true;         // !KC: (wave-uniform) no chunk of the panel was moved
-
-  // `p`: the operand as stored; `first`: the panel's first row / column; `count`: rows / columns of the
-  // matrix; `ld`: stored row stride.
-  __device__ __forceinline__ void place(const void* p, int first, int count, int64_t ld, int lane) {
-    ld_bytes = ld * ES;
-    const uint8_t* b = reinterpret_cast<const uint8_t*>(p);
-    if constexpr (KC) {
-#pragma unroll
-      for (int f = 0; f < F; ++f)
-        base[f] = b + (int64_t)min(first + 16 * f + (lane & 15), count - 1) * ld_bytes + (lane >> 4) * 16;
-    } else {
-      const int c = first + (lane % CPR) * EPC, cc = min(c, count - EPC);
-      over = c - cc;
-      whole = first + 16 * F <= count;
-      base[0] = b + (int64_t)(lane / CPR) * ld_bytes + (int64_t)cc * ES;
-    }
-  }
-  // Request the step at k0, all of it below K.
-  __device__ __forceinline__ void load(int k0, u32x4 (&r)[F]) const {
-    typedef typename Chunk<ES>::type C;
-    if constexpr (KC) {
-#pragma unroll
-      for (int f = 0; f < F; ++f) r[f] = *reinterpret_cast<const C*>(base[f] + (int64_t)k0 * ES);
-    } else {
-      const uint8_t* p = base[0] + (int64_t)k0 * ld_bytes;
-#pragma unroll
-      for (int f = 0; f < F; ++f) r[f] = *reinterpret_cast<const C*>(p + (int64_t)(f * RPL) * ld_bytes);
-    }
-  }
-  // Request the step at k0 that K ends in; `finish_tail` turns what lies past K into zeros.
-  __device__ __forceinline__ void load_tail(int k0, int K, int lane, u32x4 (&r)[F]) const {
-    typedef typename Chunk<ES>::type C;
-    if constexpr (KC) {
-      const int k = k0 + (lane >> 4) * EPC, back = max(k - (K - EPC), 0);
-#pragma unroll
-      for (int f = 0; f < F; ++f) r[f] = *reinterpret_cast<const C*>(base[f] + (int64_t)(k0 - back) * ES);
-    } else {
-#pragma unroll
-      for (int f = 0; f < F; ++f) {
-        const int row = lane / CPR, k = min(k0 + f * RPL + row, K - 1) - row;
-        r[f] = *reinterpret_cast<const C*>(base[0] + (int64_t)k * ld_bytes);
-      }
-    }
-  }
-  __device__ __forceinline__ void finish_tail(int k0, int K, int lane, u32x4 (&r)[F]) const {
-    if constexpr (KC) {
-      const int k = k0 + (lane >> 4) * EPC, back = max(k - (K - EPC), 0);
-#pragma unroll
-      for (int f = 0; f < F; ++f) r[f] = small_shift_chunk<ES>(r[f], back);
-    } else {
-#pragma unroll
-      for (int f = 0; f < F; ++f)
-        if (k0 + f * RPL + lane / CPR >= K) r[f] = u32x4{0u, 0u, 0u, 0u};
-    }
-  }
-  // The step's chunks go into the wave's LDS area (!KC) ...
-  template <bool WHOLE>
-  __device__ __forceinline__ void stage(u32x4 (&r)[F], uint8_t* lds, int lane) const {
-    if constexpr (!KC) {
-      if constexpr (!WHOLE) {
-#pragma unroll
-        for (int f = 0; f < F; ++f) r[f] = small_shift_chunk<ES>(r[f], over);
-      }
-#pragma unroll
-      for (int f = 0; f < F; ++f)
-        *reinterpret_cast<u32x4*>(lds + (f * RPL + lane / CPR) * RS + (lane % CPR) * 16) = r[f];
-    }
-  }
-  // ... where its fragments come from; KC: the registers themselves.
-  __device__ __forceinline__ void fragments(const u32x4 (&r)[F], uint8_t* lds, int lane, u32x4 (&frag)[F]) const {
-    if constexpr (KC) {
-#pragma unroll
-      for (int f = 0; f < F; ++f) frag[f] = r[f];
-    } else {
-      const int l16 = lane & 15, g4 = lane >> 4;
-#pragma unroll
-      for (int f = 0; f < F; ++f) {
-        if constexpr (ES == 2) {
-          // 16 lanes of group g4: k rows 8 g4 + l16 / 4 (+4), columns 16 f + 4 (l16 % 4) .. +4
-          uint8_t* p0 = lds + (8 * g4 + (l16 >> 2)) * RS + 32 * f + 8 * (l16 & 3);
-          const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                                         (__attribute__((address_space(3))) small_s16x4*)p0));
-          const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                                         (__attribute__((address_space(3))) small_s16x4*)(p0 + 4 * RS)));
-          frag[f] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-        } else if constexpr (ES == 1) {
-          // k rows 16 g4 + l16 / 2 (+8), bytes 16 f + 8 (l16 % 2) .. +8
-          uint8_t* p0 = lds + (16 * g4 + (l16 >> 1)) * RS + 16 * f + 8 * (l16 & 1);
-          const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                                                         (__attribute__((address_space(3))) small_i32x2*)p0));
-          const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                                                         (__attribute__((address_space(3))) small_i32x2*)(p0 + 8 * RS)));
-          frag[f] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-        } else {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            frag[f][t] = *reinterpret_cast<const uint32_t*>(lds + (4 * g4 + t) * RS + (16 * f + l16) * 4);
-        }
-      }
-    }
-  }
-};
 
 template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
 struct SmallCfg {
@@ -312,25 +143,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
   if ((AKC || pa.whole) && (BKC || pb.whole)) small_multiply<Cfg, DT, MT, NT, NW, true>(pa, pb, acc, g.K, wave, lane, lds_a, lds_b);
   else small_multiply<Cfg, DT, MT, NT, NW, false>(pa, pb, acc, g.K, wave, lane, lds_a, lds_b);
 
-  // Sum over the waves: fragment f = j NT + i of wave w is 1 KiB at (w MT NT + f) 1024, 16 bytes per lane.
-  f32x4* const sums = reinterpret_cast<f32x4*>(smem_small);
   if constexpr (Cfg::kWaveLds > 0) __syncthreads();  // (the areas overlap)
-#pragma unroll
-  for (int j = 0; j < MT; ++j)
-#pragma unroll
-    for (int i = 0; i < NT; ++i) sums[(wave * MT * NT + j * NT + i) * 64 + lane] = acc[j][i];
-  __syncthreads();
-#pragma unroll
-  for (int e0 = 0; e0 < MT * NT * 64; e0 += NW * 64) {
-    const int e = e0 + tid;
-    if (MT * NT * 64 % (NW * 64) != 0 && e >= MT * NT * 64) break;
-    f32x4 v = sums[e];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) v += sums[w * MT * NT * 64 + e];
-    const int f = e >> 6, l = e & 63;
-    const int m = m0 + 16 * (f / NT) + (l & 15), n = n0 + 16 * (f % NT) + 4 * (l >> 4);
-    if (m < g.M && n < g.N) epilogue4_any<EDT>(g, m, n, v);
-  }
+  small_sum_and_store<EDT, MT, NT, NW>(g, acc, smem_small, m0, n0, tid);
 }
 
 template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
