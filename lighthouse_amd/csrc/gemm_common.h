@@ -455,21 +455,20 @@ __device__ __forceinline__ void epilogue1(const GemmArgs& g, int m, int n, float
   else store_from_f32<DT>(g.out, off, x);
 }
 
-// epilogue4 for columns n .. n + 3 of row m, of which those below N exist; any alignment.
+// epilogue4 for columns n .. n + 3 of row m, of which those below N exist; any alignment.  The bias and accumulator input of the
+// call are in `bias` and `c`.
 template <int DT>
-__device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, const f32x4& acc) {
+__device__ __forceinline__ void epilogue4_loaded(const GemmArgs& g, int m, int n, const f32x4& acc, const f32x4& bias, const f32x4& c) {
   float v[4] = {acc[0] * g.alpha, acc[1] * g.alpha, acc[2] * g.alpha, acc[3] * g.alpha};
   const int64_t off = (int64_t)m * g.ldc + n;
   const int left = g.N - n;
   if (g.flags & LH_GEMM_ACCUMULATE_C) {
-    const f32x4 c = g.out_dt == LH_F32 ? load4_any<LH_F32>(g.c, off, left) : load4_any<DT>(g.c, off, left);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += c[e];
   }
   if (g.flags & LH_GEMM_HAS_BIAS) {
-    const f32x4 b = bias4<DT, true>(g, n);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += b[e];
+    for (int e = 0; e < 4; ++e) v[e] += bias[e];
   }
   if (g.flags & LH_GEMM_HAS_GELU) {
 #pragma unroll
@@ -482,6 +481,18 @@ __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, c
   const f32x4 o = {v[0], v[1], v[2], v[3]};
   if (g.out_dt == LH_F32) store4_any<LH_F32>(g.out, off, o, left);
   else store4_any<DT>(g.out, off, o, left);
+}
+// ... loaded here.
+template <int DT>
+__device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, const f32x4& acc) {
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 bias = zero, c = zero;
+  if (g.flags & LH_GEMM_ACCUMULATE_C) {
+    const int64_t off = (int64_t)m * g.ldc + n;
+    c = g.out_dt == LH_F32 ? load4_any<LH_F32>(g.c, off, g.N - n) : load4_any<DT>(g.c, off, g.N - n);
+  }
+  if (g.flags & LH_GEMM_HAS_BIAS) bias = bias4<DT, true>(g, n);
+  epilogue4_loaded<DT>(g, m, n, acc, bias, c);
 }
 
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s);

@@ -175,30 +175,83 @@ struct SmallPanel {
   }
 };
 
-// Sum of the waves' partial tiles through LDS, in wave order, and the epilogue of the tile at (m0, n0).  EDT: the type a
-// 16-bit output, bias or accumulator input has.
-template <int EDT, int MT, int NT, int NW>
-__device__ __forceinline__ void small_sum_and_store(const GemmArgs& g, const f32x4 (&acc)[MT][NT], uint8_t* lds, int m0, int n0,
-                                                    int tid) {
-  // Fragment f = j NT + i of wave w is 1 KiB at (w MT NT + f) 1024, 16 bytes per lane.
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  f32x4* const sums = reinterpret_cast<f32x4*>(lds);
-#pragma unroll
-  for (int j = 0; j < MT; ++j)
-#pragma unroll
-    for (int i = 0; i < NT; ++i) sums[(wave * MT * NT + j * NT + i) * 64 + lane] = acc[j][i];
-  __syncthreads();
-#pragma unroll
-  for (int e0 = 0; e0 < MT * NT * 64; e0 += NW * 64) {
-    const int e = e0 + tid;
-    if (MT * NT * 64 % (NW * 64) != 0 && e >= MT * NT * 64) break;
-    f32x4 v = sums[e];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) v += sums[w * MT * NT * 64 + e];
-    const int f = e >> 6, l = e & 63;
-    const int m = m0 + 16 * (f / NT) + (l & 15), n = n0 + 16 * (f % NT) + 4 * (l >> 4);
-    if (m < g.M && n < g.N) epilogue4_any<EDT>(g, m, n, v);
+// Four consecutive elements of a row as they are in memory, f32 when asked for.  Held unconverted and loaded without a
+// branch, so that nothing waits for the load in between.
+template <int EDT>
+struct SmallRaw4 {
+  u32x4 w;
+  // Columns n .. n + 3 of the row of N >= 4 at p[at]; four that would cross the end of the row are its last four.
+  __device__ __forceinline__ void load(const void* p, bool f32, int64_t at, int n, int N) {
+    const int64_t i = at + min(n, N - 4);
+    if constexpr (EDT == LH_F32) {
+      w = *reinterpret_cast<const Chunk<4>::type*>(reinterpret_cast<const uint32_t*>(p) + i);
+    } else {
+      const uint16_t* q = reinterpret_cast<const uint16_t*>(p) + (f32 ? 2 * i : i);
+      const u32x2 lo = *reinterpret_cast<const u32x2_any*>(q), hi = *reinterpret_cast<const u32x2_any*>(q + (f32 ? 4 : 0));
+      w = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
   }
-}
+  // ... as f32, those past the end undefined; `whole` (uniform): no lane's cross it.
+  __device__ __forceinline__ f32x4 get(bool f32, int n, int N, bool whole) const {
+    f32x4 v = __builtin_bit_cast(f32x4, w);
+    if constexpr (EDT != LH_F32)
+      if (!f32) v = f32x4{unpack_lo<EDT>(w[0]), unpack_hi<EDT>(w[0]), unpack_lo<EDT>(w[1]), unpack_hi<EDT>(w[1])};
+    if (!whole) {
+      const int over = n - min(n, N - 4);
+      v = over == 1 ? f32x4{v[1], v[2], v[3], 0.0f} : over == 2 ? f32x4{v[2], v[3], 0.0f, 0.0f} : over == 3 ? f32x4{v[3], 0.0f, 0.0f, 0.0f} : v;
+    }
+    return v;
+  }
+};
+
+// The elements of the tile at (m0, n0) that a thread finishes: their bias and accumulator input.  Requested in front of the
+// main loop: at its end each would be a trip to memory of its own (M = 100, N = 768, K = 768 bf16 with an f32 residual: 0.9 us
+// from the sums to the stores' end).
+template <int EDT, int MT, int NT, int NW>
+struct SmallEpilogue {
+  static constexpr int IT = (MT * NT + NW - 1) / NW;
+  SmallRaw4<EDT> bias[IT], c[IT];
+  // Fragment f = it NW + wave of the tile: the lane's row and columns.
+  static __device__ __forceinline__ void at(int m0, int n0, int f, int lane, int& m, int& n) {
+    m = m0 + 16 * (f / NT) + (lane & 15);
+    n = n0 + 16 * (f % NT) + 4 * (lane >> 4);
+  }
+  __device__ __forceinline__ void load(const GemmArgs& g, int m0, int n0, int wave, int lane) {
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int f = it * NW + wave;
+      if (MT * NT % NW != 0 && f >= MT * NT) break;
+      int m, n;
+      at(m0, n0, f, lane, m, n);
+      if (g.flags & LH_GEMM_HAS_BIAS) bias[it].load(g.bias, g.bias_dt == LH_F32, 0, n, g.N);
+      if (g.flags & LH_GEMM_ACCUMULATE_C) c[it].load(g.c, g.out_dt == LH_F32, (int64_t)min(m, g.M - 1) * g.ldc, n, g.N);
+    }
+  }
+  // The waves' partial tiles are added through LDS, in wave order, and finished; `loaded` (uniform): with what `load` has brought.
+  __device__ __forceinline__ void sum_and_store(bool loaded, const GemmArgs& g, const f32x4 (&acc)[MT][NT], uint8_t* lds, int m0, int n0,
+                                                int wave, int lane) const {
+    // Fragment f = j NT + i of wave w is 1 KiB at (w MT NT + f) 1024, 16 bytes per lane.
+    f32x4* const sums = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) sums[(wave * MT * NT + j * NT + i) * 64 + lane] = acc[j][i];
+    __syncthreads();
+    const bool whole = n0 + 16 * NT <= g.N;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int f = it * NW + wave;
+      if (MT * NT % NW != 0 && f >= MT * NT) break;
+      f32x4 v = sums[f * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) v += sums[(w * MT * NT + f) * 64 + lane];
+      int m, n;
+      at(m0, n0, f, lane, m, n);
+      if (m >= g.M || n >= g.N) continue;
+      if (loaded) epilogue4_loaded<EDT>(g, m, n, v, bias[it].get(g.bias_dt == LH_F32, n, g.N, whole), c[it].get(g.out_dt == LH_F32, n, g.N, whole));
+      else epilogue4_any<EDT>(g, m, n, v);
+    }
+  }
+};
 
 }  // namespace lh

@@ -31,6 +31,7 @@ struct SmallCfg {
   static constexpr int kLdsBytes = kSumBytes > NW * kWaveLds ? kSumBytes : NW * kWaveLds;
   // Steps requested ahead: what fits next to the accumulators in the registers of NW waves.
   static constexpr int P = MT + NT <= 3 ? 3 : 2;
+  static constexpr bool kLoadEpilogue = MT * NT < 16;  // (the largest tile has no registers to hold it)
   static constexpr bool kTight = MT * NT == 16 && !AKC && !BKC && PA::ES == 2;  // (all 256 registers that 8 waves have)
 };
 
@@ -126,6 +127,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
   if (tile >= tiles_m * tiles_n) return;
   const int m0 = (tile % tiles_m) * 16 * MT, n0 = (tile / tiles_m) * 16 * NT;
 
+  SmallEpilogue<EDT, MT, NT, NW> epilogue;
+  const bool loaded = Cfg::kLoadEpilogue && g.N >= 4;
+  if (loaded) epilogue.load(g, m0, n0, wave, lane);
   typename Cfg::PA pa;
   typename Cfg::PB pb;
   pa.place(g.a, m0, g.M, g.lda, lane);
@@ -144,7 +148,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
   else small_multiply<Cfg, DT, MT, NT, NW, false>(pa, pb, acc, g.K, wave, lane, lds_a, lds_b);
 
   if constexpr (Cfg::kWaveLds > 0) __syncthreads();  // (the areas overlap)
-  small_sum_and_store<EDT, MT, NT, NW>(g, acc, smem_small, m0, n0, tid);
+  epilogue.sum_and_store(loaded, g, acc, smem_small, m0, n0, wave, lane);
 }
 
 template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>

@@ -6,20 +6,16 @@
 // With few rows each of the block's launches is a chain of latencies of a few us.  Here every workgroup of the
 // small-tile GEMM (gemm_small.hip) normalises the 16 MT rows of its tile itself: its waves request the weights of their
 // whole share of K first, normalise a few rows each while those are on their way (a wave holds its rows in registers,
-// the arithmetic is layer_norm_vec's) and leave them in LDS, from where every wave reads its operand.  The rows are
+// the arithmetic is layer_norm_vec's but for the order of the sums) and leave them in LDS, from where every wave reads its operand.  The rows are
 // normalised again by every workgroup beside this one: L2 traffic and a few hundred instructions, against a launch
 // and a trip of the result through memory.  Up to three weight matrices side by side (separate q, k and v) are one launch.
 #include "gemm_small.h"
 
 namespace lh {
 
-// Sum over the wave's 64 lanes, in every lane; the pairs of a butterfly from distance 32 down, without its trips through
-// LDS.  (From distance 8 on a rotation within 16 lanes brings a lane that holds what its partner holds.)
-__device__ __forceinline__ float norm_wave_sum(float v) {
+// Sum over 32 lanes, in each of them: the other half's 16 lanes, then rotations within 16 lanes.
+__device__ __forceinline__ float norm_half_sum(float v) {
   float a = v, b = v;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-  v = a + b;
-  a = v, b = v;
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
   v = a + b;
   auto rotated = [](float x, auto n) {
@@ -31,27 +27,24 @@ __device__ __forceinline__ float norm_wave_sum(float v) {
   return v + rotated(v, std::integral_constant<int, 1>{});
 }
 
-// V: K <= 256 V.
+// K = 128 V.  Half a wave holds a row (4 V elements per lane).
 template <int DT, int MT, int NT, int NW, int V>
 struct NormCfg {
   typedef SmallPanel<DT, NT, false> PB;
-  static constexpr int ES = PB::ES, KSTEP = PB::KSTEP;
-  static constexpr int kSteps = (256 * V / KSTEP + NW - 1) / NW;  // k-steps of a wave, at most
-  static constexpr int P = kSteps < 4 ? kSteps : 4;               // ... of which so many are requested up front
+  static constexpr int ES = PB::ES, KSTEP = PB::KSTEP, K = 128 * V;
+  static constexpr int P = (K / KSTEP + NW - 1) / NW;             // k-steps of a wave, at most; all are requested up front
+  static constexpr int kRowBytes = K * ES + 16;                   // of a normalised row in LDS (one chunk of padding)
+  static constexpr int kWorkBytes = 16 * MT * kRowBytes + NW * PB::kLdsBytes;
   static constexpr int kSumBytes = NW * MT * NT * 1024;
-  static int row_bytes(int K) { return K * ES + 16; }             // of a normalised row in LDS (one chunk of padding)
-  static int lds_bytes(int K) {
-    const int work = 16 * MT * row_bytes(K) + NW * PB::kLdsBytes;
-    return work > kSumBytes ? work : kSumBytes;
-  }
+  static constexpr int kLdsBytes = kWorkBytes > kSumBytes ? kWorkBytes : kSumBytes;
 };
 
 template <int DT, int MT, int NT, int NW, int V>
 __global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
   typedef NormCfg<DT, MT, NT, NW, V> Cfg;
-  constexpr int KSTEP = Cfg::KSTEP, P = Cfg::P, ES = Cfg::ES;
-  constexpr int R = 16 * MT / NW;  // rows a wave normalises
-  static_assert(R >= 1 && R * NW == 16 * MT, "whole rows per wave");
+  constexpr int K = Cfg::K, KSTEP = Cfg::KSTEP, P = Cfg::P, ES = Cfg::ES;
+  constexpr int R = 8 * MT / NW;  // pairs of rows a wave normalises
+  static_assert(R >= 1 && R * NW == 8 * MT, "whole pairs of rows per wave");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_norm[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -63,60 +56,62 @@ __global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
   if (tile >= tiles) return;
   const int panel = tile / tiles_m, group = panel / tiles_n;
   const int m0 = (tile % tiles_m) * 16 * MT, n0 = (panel % tiles_n) * 16 * NT;
-  const int row_bytes = g.K * ES + 16;
+  // (the group's columns of the output, and its bias)
+  g.out = reinterpret_cast<uint8_t*>(g.out) + (int64_t)group * g.N * ES;
+  g.bias = group == 0 ? n.bias[0] : group == 1 ? n.bias[1] : n.bias[2];
   uint8_t* const rows = smem_norm;
-  uint8_t* const lds_b = smem_norm + 16 * MT * row_bytes + wave * Cfg::PB::kLdsBytes;
+  uint8_t* const lds_b = smem_norm + 16 * MT * Cfg::kRowBytes + wave * Cfg::PB::kLdsBytes;
 
-  // The wave's rows of x, gamma and beta, then its steps of the weights: requested in this order, waited for in this order.
+  // The wave's rows of x, gamma and beta, then its steps of the weights and what the epilogue needs: requested in this order,
+  // waited for in this order.
+  const int l32 = lane & 31, row0 = wave * 2 * R + (lane >> 5);
   f32x4 x[R][V], gamma[V], beta[V];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const float* p = reinterpret_cast<const float*>(g.a) + (int64_t)min(m0 + wave * R + r, g.M - 1) * g.lda;
+    const float* p = reinterpret_cast<const float*>(g.a) + (int64_t)min(m0 + row0 + 2 * r, g.M - 1) * g.lda + 4 * l32;
 #pragma unroll
-    for (int i = 0; i < V; ++i) x[r][i] = *reinterpret_cast<const f32x4*>(p + min((i * 64 + lane) * 4, g.K - 4));
+    for (int i = 0; i < V; ++i) x[r][i] = *reinterpret_cast<const f32x4*>(p + 128 * i);
   }
 #pragma unroll
   for (int i = 0; i < V; ++i) {
-    gamma[i] = *reinterpret_cast<const f32x4*>(n.gamma + min((i * 64 + lane) * 4, g.K - 4));
-    beta[i] = *reinterpret_cast<const f32x4*>(n.beta + min((i * 64 + lane) * 4, g.K - 4));
+    gamma[i] = *reinterpret_cast<const f32x4*>(n.gamma + 128 * i + 4 * l32);
+    beta[i] = *reinterpret_cast<const f32x4*>(n.beta + 128 * i + 4 * l32);
   }
+  asm volatile("" ::: "memory");  // (the weights, which come from further away, behind them)
   typename Cfg::PB pb;
   pb.place(group == 0 ? n.b[0] : group == 1 ? n.b[1] : n.b[2], n0, g.N, g.ldb, lane);
-  const int full = g.K / KSTEP, begin = full * wave / NW, mine = full * (wave + 1) / NW - begin;
+  constexpr int full = K / KSTEP;
+  const int begin = full * wave / NW, mine = full * (wave + 1) / NW - begin;
   u32x4 rb[P][NT];
 #pragma unroll
   for (int p = 0; p < P; ++p) pb.load(min(begin + p, full - 1) * KSTEP, rb[p]);
+  asm volatile("" ::: "memory");
+  SmallEpilogue<DT, MT, NT, NW> epilogue;
+  epilogue.load(g, m0, n0, wave, lane);
 
-  // LayerNorm of the rows
+  // LayerNorm of the rows, two at a time
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     float s = 0.0f;
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      if ((i * 64 + lane) * 4 >= g.K) x[r][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      s += (x[r][i][0] + x[r][i][1]) + (x[r][i][2] + x[r][i][3]);
-    }
-    const float mean = norm_wave_sum(s) * n.inv_n;
+    for (int i = 0; i < V; ++i) s += (x[r][i][0] + x[r][i][1]) + (x[r][i][2] + x[r][i][3]);
+    const float mean = norm_half_sum(s) * n.inv_n;
     float q = 0.0f;
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      const bool in = (i * 64 + lane) * 4 < g.K;
+    for (int i = 0; i < V; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float c = x[r][i][e] - mean;
-        q = in ? q + c * c : q;
+        x[r][i][e] -= mean;
+        q += x[r][i][e] * x[r][i][e];
       }
-    }
-    const float inv_std = rsqrtf(norm_wave_sum(q) * n.inv_n + n.eps);
-    uint8_t* const row = rows + (wave * R + r) * row_bytes;
+    const float inv_std = rsqrtf(norm_half_sum(q) * n.inv_n + n.eps);
+    uint8_t* const row = rows + (row0 + 2 * r) * Cfg::kRowBytes + 4 * ES * l32;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      const int col = (i * 64 + lane) * 4;
-      if (col >= g.K) continue;
       f32x4 o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = (x[r][i][e] - mean) * inv_std * gamma[i][e] + beta[i][e];
-      *reinterpret_cast<u32x2*>(row + 2 * col) = u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
+      for (int e = 0; e < 4; ++e) o[e] = x[r][i][e] * inv_std * gamma[i][e] + beta[i][e];
+      *reinterpret_cast<u32x2*>(row + 128 * ES * i) = u32x2{pack2<DT>(o[0], o[1]), pack2<DT>(o[2], o[3])};
     }
   }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -126,33 +121,24 @@ __global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
   for (int j = 0; j < MT; ++j)
 #pragma unroll
     for (int i = 0; i < NT; ++i) acc[j][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const uint8_t* const frag_row = rows + (lane & 15) * row_bytes + (lane >> 4) * 16;
+  const uint8_t* const frag_row = rows + (lane & 15) * Cfg::kRowBytes + (lane >> 4) * 16 + begin * 64;
   const bool whole = pb.whole;
-#pragma unroll 1
-  for (int i0 = 0; i0 < mine; i0 += P) {
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-      if (i0 + p >= mine) break;
-      u32x4 fa[MT], fb[NT];
-      if (whole) pb.template stage<true>(rb[p], lds_b, lane);
-      else pb.template stage<false>(rb[p], lds_b, lane);
+  for (int p = 0; p < P; ++p) {
+    if (p >= mine) break;
+    u32x4 fa[MT], fb[NT];
+    if (whole) pb.template stage<true>(rb[p], lds_b, lane);
+    else pb.template stage<false>(rb[p], lds_b, lane);
 #pragma unroll
-      for (int j = 0; j < MT; ++j)
-        fa[j] = *reinterpret_cast<const u32x4*>(frag_row + 16 * j * row_bytes + (begin + i0 + p) * 64);
-      pb.fragments(rb[p], lds_b, lane, fb);
+    for (int j = 0; j < MT; ++j) fa[j] = *reinterpret_cast<const u32x4*>(frag_row + 16 * j * Cfg::kRowBytes + p * 64);
+    pb.fragments(rb[p], lds_b, lane, fb);
 #pragma unroll
-      for (int j = 0; j < MT; ++j)
+    for (int j = 0; j < MT; ++j)
 #pragma unroll
-        for (int i = 0; i < NT; ++i) acc[j][i] = small_mma<DT>(fb[i], fa[j], acc[j][i]);
-      if (Cfg::kSteps > P && i0 + p + P < mine) pb.load((begin + i0 + p + P) * KSTEP, rb[p]);
-    }
+      for (int i = 0; i < NT; ++i) acc[j][i] = small_mma<DT>(fb[i], fa[j], acc[j][i]);
   }
-
-  // (the group's columns of the output, and its bias)
-  g.out = reinterpret_cast<uint8_t*>(g.out) + (int64_t)group * g.N * (g.out_dt == LH_F32 ? 4 : 2);
-  g.bias = group == 0 ? n.bias[0] : group == 1 ? n.bias[1] : n.bias[2];
   __syncthreads();  // (the areas overlap)
-  small_sum_and_store<DT, MT, NT, NW>(g, acc, smem_norm, m0, n0, tid);
+  epilogue.sum_and_store(true, g, acc, smem_norm, m0, n0, wave, lane);
 }
 
 template <int DT, int MT, int NT, int NW, int V>
@@ -160,42 +146,46 @@ static int launch_normed_rows(const NormedGemm& n, hipStream_t s) {
   typedef NormCfg<DT, MT, NT, NW, V> Cfg;
   auto kern = gemm_normed_kernel<DT, MT, NT, NW, V>;
   static bool configured = false;
-  if (!configured && !planning()) {
+  if (Cfg::kLdsBytes > 64 * 1024 && !configured && !planning()) {
     LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     Cfg::lds_bytes(256 * V)));
+                                     Cfg::kLdsBytes));
     configured = true;
   }
   const int tiles = ((n.g.M + 16 * MT - 1) / (16 * MT)) * ((n.g.N + 16 * NT - 1) / (16 * NT)) * n.groups;
-  LH_LAUNCH(kern, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(NW * 64), Cfg::lds_bytes(n.g.K), s, n);
+  LH_LAUNCH(kern, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(NW * 64), Cfg::kLdsBytes, s, n);
   return check_launch("gemm_normed");
 }
 
 template <int DT, int MT, int NT, int NW>
 static int launch_normed(const NormedGemm& n, hipStream_t s) {
-  switch ((n.g.K + 255) / 256) {
+  switch (n.g.K / 128) {
     case 1: return launch_normed_rows<DT, MT, NT, NW, 1>(n, s);
     case 2: return launch_normed_rows<DT, MT, NT, NW, 2>(n, s);
     case 3: return launch_normed_rows<DT, MT, NT, NW, 3>(n, s);
-    default: return launch_normed_rows<DT, MT, NT, NW, 4>(n, s);
+    case 4: return launch_normed_rows<DT, MT, NT, NW, 4>(n, s);
+    case 5: return launch_normed_rows<DT, MT, NT, NW, 5>(n, s);
+    case 6: return launch_normed_rows<DT, MT, NT, NW, 6>(n, s);
+    case 7: return launch_normed_rows<DT, MT, NT, NW, 7>(n, s);
+    default: return launch_normed_rows<DT, MT, NT, NW, 8>(n, s);
   }
 }
 
 // ---- choice of tile ---------------------------------------------------------------------------
 // Time of the launch, in us: fixed + r (b + c K), r = workgroups per compute unit (at least 1; a last round that is not whole
-// counts for 0.6 of what it lacks).  Least squares over 140 problems (M 16 .. 1000, K 256 .. 1024, N 3 K and 4 K; 6 to 7 % rms); 16 x 16 and
-// 32 x 32 tiles were never the fastest by more than 0.3 us.  What stands against it: 4.5 us for the LayerNorm's launch and its
-// gap, and each product at 1.2 times gemm16_us (which was fitted on operands that stayed in the caches) plus 1.5 for
-// every launch after the first.  Choosing so is within 1.3 % of the faster way on average; M = 100, K = 768, N = 2304 bf16:
-// 3.6 + 5.8 us and a gap against 7.8 us, M = 400: 4.3 + 9.0 against 15.5, and the LayerNorm stays on its own.
+// counts for 0.6 of what it lacks).  Least squares over 140 problems (M 16 .. 1000, K 256 .. 1024, N 3 K and 4 K; 5 to 7 % rms); 16 x 16 and
+// 32 x 32 tiles were never the fastest by more than 0.3 us.  What stands against it: 5.25 us for the LayerNorm's launch and its
+// gap, and each product at 1.4 times gemm16_us (which was fitted on operands that stayed in the caches) plus 1.5 for
+// every launch after the first.  Choosing so is within 0.4 % of the faster way on average (1.13 x at worst); M = 100, K = 768,
+// N = 2304 bf16: 3.1 + 5.6 us and a gap against 7.3 us, M = 400: 3.9 + 9.3 against 14.3, and the LayerNorm stays on its own.
 struct NormedTile {
   int mt, nt;
   double fixed, b, c;
 };
-constexpr NormedTile kNormedTiles[] = {{1, 2, 3.45, 0.138, 0.0031}, {1, 4, 3.39, 0.151, 0.0047}, {2, 4, 2.87, 1.20, 0.0067}};
+constexpr NormedTile kNormedTiles[] = {{1, 2, 3.05, -0.11, 0.0040}, {1, 4, 2.99, -0.02, 0.0055}, {2, 4, 2.50, 0.89, 0.0066}};
 
 int gemm_normed_choose(const NormedGemm& n, int dtype) {
   const GemmArgs& g = n.g;
-  if (dtype == LH_F32 || g.K % 64 != 0 || g.K > 1024 || g.N < 8 || g.lda % 4 != 0 || !aligned16(g.a) || !aligned16(n.gamma) ||
+  if (dtype == LH_F32 || g.K % 128 != 0 || g.K > 1024 || g.N < 8 || g.lda % 4 != 0 || !aligned16(g.a) || !aligned16(n.gamma) ||
       !aligned16(n.beta) || (int64_t)g.M * g.N >= 1ll << 36)
     return -1;
   const int cus = num_cus();
@@ -220,7 +210,7 @@ int gemm_normed_choose(const NormedGemm& n, int dtype) {
   GemmArgs one = g;
   one.a = n.b[0];  // (for its alignment, which the LayerNorm's own output has as well)
   one.lda = g.K;
-  const double apart = 4.5 + 1.2 * n.groups * gemm16_us(one, dtype) + 1.5 * (n.groups - 1);
+  const double apart = 5.25 + 1.4 * n.groups * gemm16_us(one, dtype) + 1.5 * (n.groups - 1);
   return best < apart ? tile : -1;
 }
 
