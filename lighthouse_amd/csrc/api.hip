@@ -316,19 +316,13 @@ size_t lh_hip_nanogpt_block_workspace_bytes(int64_t B, int64_t T, int64_t C, int
          block_gemm_need(B * T, C, cfg.hidden, dtype, cfg.bias_dtype);
 }
 
-int lh_hip_nanogpt_block(float* y, const float* x, const lh_nanogpt_block_params* p, int64_t B, int64_t T, int64_t C,
-                         int64_t n_head, float eps, int32_t dtype, const lh_nanogpt_block_opts* opts, void* workspace,
-                         size_t workspace_bytes, void* stream) {
-  LH_REQUIRE(y && x && p && workspace, "lh_hip_nanogpt_block: null pointer");
-  BlockConfig cfg;
-  if (int rc = block_config("lh_hip_nanogpt_block", opts, C, dtype, &cfg)) return rc;
+// The block's launches; `workspace` is large enough (a size query is not free: the forward asks once for all its blocks).
+static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p, int64_t B, int64_t T, int64_t C, int64_t n_head,
+                     float eps, int32_t dtype, const BlockConfig& cfg, void* workspace, size_t workspace_bytes, void* stream) {
   LH_REQUIRE(B > 0 && T > 0 && C > 0 && n_head > 0 && C % n_head == 0, "lh_hip_nanogpt_block: bad shape");
   LH_REQUIRE(p->ln1_g && p->ln1_b && p->ln2_g && p->ln2_b && p->w_o && p->w_fc && p->w_proj,
              "lh_hip_nanogpt_block: null parameter");
   LH_REQUIRE(p->w_qkv || (p->w_q && p->w_k && p->w_v), "lh_hip_nanogpt_block: w_qkv or all of w_q, w_k, w_v must be set");
-  LH_REQUIRE(workspace_bytes >= lh_hip_nanogpt_block_workspace_bytes(B, T, C, dtype, opts),
-             "lh_hip_nanogpt_block: workspace too small (%zu bytes)", workspace_bytes);
-  LH_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, "lh_hip_nanogpt_block: workspace must be 256-byte aligned");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const size_t e = dtype_size(dtype), eb = dtype_size(cfg.bias_dtype);
   const int64_t rows = B * T, hs = C / n_head, hidden = cfg.hidden;
@@ -401,6 +395,19 @@ int lh_hip_nanogpt_block(float* y, const float* x, const lh_nanogpt_block_params
                   bias_flag(p->b_proj) | LH_GEMM_ACCUMULATE_C, s, &ws);
 }
 
+int lh_hip_nanogpt_block(float* y, const float* x, const lh_nanogpt_block_params* p, int64_t B, int64_t T, int64_t C,
+                         int64_t n_head, float eps, int32_t dtype, const lh_nanogpt_block_opts* opts, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+  LH_REQUIRE(y && x && p && workspace, "lh_hip_nanogpt_block: null pointer");
+  BlockConfig cfg;
+  if (int rc = block_config("lh_hip_nanogpt_block", opts, C, dtype, &cfg)) return rc;
+  LH_REQUIRE(B > 0 && T > 0 && C > 0, "lh_hip_nanogpt_block: bad shape");
+  LH_REQUIRE(workspace_bytes >= lh_hip_nanogpt_block_workspace_bytes(B, T, C, dtype, opts),
+             "lh_hip_nanogpt_block: workspace too small (%zu bytes)", workspace_bytes);
+  LH_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, "lh_hip_nanogpt_block: workspace must be 256-byte aligned");
+  return block_run(y, x, p, B, T, C, n_head, eps, dtype, cfg, workspace, workspace_bytes, stream);
+}
+
 static size_t forward_head_need(int64_t rows, int64_t C, int64_t vocab, int32_t dtype, int bias_dt) {
   return align256(gemm_need(rows, vocab, C, C, vocab, vocab, dtype, LH_F32, bias_dt, LH_GEMM_HAS_BIAS));
 }
@@ -425,19 +432,20 @@ int lh_hip_nanogpt_forward(float* logits, const float* x, const lh_nanogpt_block
   BlockConfig cfg;
   if (int rc = block_config("lh_hip_nanogpt_forward", opts, C, dtype, &cfg)) return rc;
   LH_REQUIRE(B > 0 && T > 0 && C > 0 && vocab > 0, "lh_hip_nanogpt_forward: bad shape");
-  LH_REQUIRE(workspace_bytes >= lh_hip_nanogpt_forward_workspace_bytes(B, T, C, vocab, dtype, opts),
+  const size_t block_ws = lh_hip_nanogpt_block_workspace_bytes(B, T, C, dtype, opts);
+  const size_t head_ws = forward_head_need(B * T, C, vocab, dtype, cfg.bias_dtype);
+  LH_REQUIRE(workspace_bytes >= block_ws + 2 * align256((size_t)B * T * C * 4) + head_ws,
              "lh_hip_nanogpt_forward: workspace too small (%zu bytes)", workspace_bytes);
   LH_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255u) == 0, "lh_hip_nanogpt_forward: workspace must be 256-byte aligned");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int64_t rows = B * T;
-  const size_t block_ws = lh_hip_nanogpt_block_workspace_bytes(B, T, C, dtype, opts);
   char* w = reinterpret_cast<char*>(workspace);
   float* h[2] = {reinterpret_cast<float*>(w + block_ws),
                  reinterpret_cast<float*>(w + block_ws + align256((size_t)rows * C * 4))};
   const float* cur = x;
   for (int64_t l = 0; l < n_layer; ++l) {
     float* nxt = h[l & 1];
-    int rc = lh_hip_nanogpt_block(nxt, cur, &blocks[l], B, T, C, n_head, eps, dtype, opts, workspace, block_ws, stream);
+    int rc = block_run(nxt, cur, &blocks[l], B, T, C, n_head, eps, dtype, cfg, workspace, block_ws, stream);
     if (rc) return rc;
     cur = nxt;
   }

@@ -63,21 +63,28 @@ def _rows_aligned16(*tensors) -> bool:
 
 
 def _is_matrix(t, rows, cols, what: str) -> None:
-    _require(t.dim() == 2 and tuple(t.shape) == (rows, cols), f"{what} must have shape [{rows}, {cols}], got {tuple(t.shape)}")
-    _require(t.stride(1) == 1 or cols == 1, f"{what}: innermost stride must be 1")
-    _require(t.stride(0) >= cols or rows == 1, f"{what}: rows overlap (stride {t.stride(0)} < {cols} columns)")
+    if t.shape != (rows, cols):
+        raise ValueError(f"{what} must have shape [{rows}, {cols}], got {tuple(t.shape)}")
+    if t.stride(1) != 1 and cols != 1:
+        raise ValueError(f"{what}: innermost stride must be 1")
+    if t.stride(0) < cols and rows != 1:
+        raise ValueError(f"{what}: rows overlap (stride {t.stride(0)} < {cols} columns)")
 
 
 def _is_vector(t, n, dtype, what: str) -> None:
-    _require(t.dim() == 1 and t.shape[0] == n, f"{what} must have shape [{n}], got {tuple(t.shape)}")
-    _require(t.dtype == dtype, f"{what} must be {dtype}, got {t.dtype}")
-    _require(t.stride(0) == 1 or n == 1, f"{what} must be contiguous")
+    if t.shape != (n,):
+        raise ValueError(f"{what} must have shape [{n}], got {tuple(t.shape)}")
+    if t.dtype != dtype:
+        raise ValueError(f"{what} must be {dtype}, got {t.dtype}")
+    if t.stride(0) != 1 and n != 1:
+        raise ValueError(f"{what} must be contiguous")
 
 
 def _same_dense(out, x, what: str) -> None:
-    _require(tuple(out.shape) == tuple(x.shape) and out.dtype == x.dtype,
-             f"{what}: out must have the shape and dtype of the input ({tuple(x.shape)}, {x.dtype})")
-    _require(x.is_contiguous() and out.is_contiguous(), f"{what} expects contiguous tensors")
+    if out.shape != x.shape or out.dtype != x.dtype:
+        raise ValueError(f"{what}: out must have the shape and dtype of the input ({tuple(x.shape)}, {x.dtype})")
+    if not x.is_contiguous() or not out.is_contiguous():
+        raise ValueError(f"{what} expects contiguous tensors")
 
 
 def device_info() -> dict:
@@ -104,13 +111,14 @@ def gemm(a, b, bias=None, *, out=None, out_dtype=None, relu=False, gelu=False, a
         raise ValueError("gemm expects 2-D tensors")
     if a.stride(1) != 1 or b.stride(1) != 1:
         raise ValueError("innermost stride must be 1")
-    _require(a.dtype in _FLOATS, f"unsupported A/B dtype {a.dtype}")
+    if a.dtype not in _FLOATS:
+        raise ValueError(f"unsupported A/B dtype {a.dtype}")
     if a.dtype != b.dtype:
         raise ValueError("A and B must have the same dtype")
     M, K = (a.shape[1], a.shape[0]) if transpose_a else a.shape
     N = b.shape[0] if transpose_b else b.shape[1]
-    _require((b.shape[1] if transpose_b else b.shape[0]) == K,
-             f"B has {b.shape[1] if transpose_b else b.shape[0]} rows of K, A has {K}")
+    if not ((b.shape[1] if transpose_b else b.shape[0]) == K):
+        raise ValueError(f"B has {b.shape[1] if transpose_b else b.shape[0]} rows of K, A has {K}")
     _require(a.stride(0) >= a.shape[1] and b.stride(0) >= b.shape[1], "rows of A or B overlap")
     if out is None:
         if accumulate_c:
@@ -212,7 +220,8 @@ def gemm_fp8(a_q, b_q, scale_a: float, scale_b: float, *, out=None, out_dtype=to
              "gemm_fp8 expects float8_e4m3fn operands")
     M, K = a_q.shape
     N = b_q.shape[1]
-    _require(b_q.shape[0] == K, f"B has {b_q.shape[0]} rows, A has {K} columns")
+    if not (b_q.shape[0] == K):
+        raise ValueError(f"B has {b_q.shape[0]} rows, A has {K} columns")
     _require(a_q.stride(1) == 1 and b_q.stride(1) == 1, "innermost stride must be 1")
     _require(a_q.stride(0) >= K and b_q.stride(0) >= N, "rows of A or B overlap")
     if out is None:
@@ -275,10 +284,9 @@ def attention(q, k, v, *, causal=False, scale=None, out=None, rows_per_wave=None
             rows_per_wave, stages, kv_split = db.lookup_attention("bf16" if q.dtype == torch.bfloat16 else "f16", Z * H, T, d, causal)
             if (rows_per_wave or stages or kv_split) and not _rows_aligned16(q, k, v, out):
                 rows_per_wave = stages = kv_split = None
-    _require((rows_per_wave or 0) in _lib.ATTN_ROWS and (stages or 0) in _lib.ATTN_STAGES
-             and (kv_split or 0) in _lib.ATTN_KSPLIT,
-             f"rows_per_wave must be one of {sorted(_lib.ATTN_ROWS)[1:]}, stages one of {sorted(_lib.ATTN_STAGES)[1:]}, "
-             f"kv_split one of {sorted(_lib.ATTN_KSPLIT)[1:]}")
+    if not ((rows_per_wave or 0) in _lib.ATTN_ROWS and (stages or 0) in _lib.ATTN_STAGES and (kv_split or 0) in _lib.ATTN_KSPLIT):
+        raise ValueError(f"rows_per_wave must be one of {sorted(_lib.ATTN_ROWS)[1:]}, stages one of {sorted(_lib.ATTN_STAGES)[1:]}, "
+                         f"kv_split one of {sorted(_lib.ATTN_KSPLIT)[1:]}")
     word = ((_lib.ATTN_CAUSAL if causal else 0) | _lib.ATTN_ROWS[rows_per_wave or 0] | _lib.ATTN_STAGES[stages or 0]
             | _lib.ATTN_KSPLIT[kv_split or 0] | (_lib.ATTN_SCALE_F32 if scale_in_f32 else 0))
     if workspace is not None:
@@ -320,7 +328,8 @@ def layer_norm(x, gamma, beta, eps=1e-5, *, out=None, out_dtype=None):
         raise ValueError("gamma and beta must be float32")
     _is_vector(gamma, N, torch.float32, "gamma")
     _is_vector(beta, N, torch.float32, "beta")
-    _require(tuple(out.shape) == (M, N), f"out must have shape [{M}, {N}]")
+    if not (tuple(out.shape) == (M, N)):
+        raise ValueError(f"out must have shape [{M}, {N}]")
     if not x.is_contiguous() or not out.is_contiguous():
         raise ValueError("layer_norm expects contiguous tensors")
     _need_cuda(x, gamma, beta, out)
@@ -387,42 +396,48 @@ BLOCK_PARAM_NAMES = ("ln1_g", "ln1_b", "w_qkv", "b_qkv", "w_o", "b_o", "ln2_g", 
 
 def _block_opts(dtype, causal, activation, bias_dtype, hidden):
     acts = {"gelu_tanh": _lib.ACT_GELU_TANH, "relu": _lib.ACT_RELU}
-    _require(activation in acts, f"activation must be one of {sorted(acts)}")
+    if activation not in acts:
+        raise ValueError(f"activation must be one of {sorted(acts)}")
     return _lib.NanoGPTBlockOpts(1 if causal else 0, acts[activation], lh_dtype(bias_dtype or dtype), int(hidden))
 
 
 def _block_params(params: dict, C: int, n_head: int):
     """Validate one block's parameter tensors and pack their pointers.  Returns (struct, dtype,
-    bias dtype or None, hidden)."""
-    _require(C % n_head == 0, f"C={C} is not a multiple of n_head={n_head}")
-    fused = params.get("w_qkv") is not None
-    if not fused:
-        _require(all(params.get(k) is not None for k in ("w_q", "w_k", "w_v")),
-                 "the block needs w_qkv or all of w_q, w_k, w_v")
-    dtype = (params["w_qkv"] if fused else params["w_q"]).dtype
-    _require(dtype in _FLOATS, f"unsupported weight dtype {dtype}")
+    bias dtype or None, hidden).  (Runs for every block of every call: a block of few rows takes the device about 25 us,
+    so messages are put together only to be raised.)"""
+    if C % n_head != 0:
+        raise ValueError(f"C={C} is not a multiple of n_head={n_head}")
+    get = params.get
+    w = {name: get(name) for name in ("w_qkv", "w_q", "w_k", "w_v", "w_o", "w_fc", "w_proj")}
+    fused = w["w_qkv"] is not None
+    if not fused and (w["w_q"] is None or w["w_k"] is None or w["w_v"] is None):
+        raise ValueError("the block needs w_qkv or all of w_q, w_k, w_v")
+    dtype = (w["w_qkv"] if fused else w["w_q"]).dtype
+    if dtype not in _FLOATS:
+        raise ValueError(f"unsupported weight dtype {dtype}")
     hidden = params["w_fc"].shape[1] if params["w_fc"].dim() == 2 else -1
-    want = {"w_qkv": (C, 3 * C), "w_q": (C, C), "w_k": (C, C), "w_v": (C, C), "w_o": (C, C), "w_fc": (C, hidden),
-            "w_proj": (hidden, C)}
-    for name, shape in want.items():
-        t = params.get(name)
+    for name, shape in (("w_qkv", (C, 3 * C)), ("w_q", (C, C)), ("w_k", (C, C)), ("w_v", (C, C)), ("w_o", (C, C)),
+                        ("w_fc", (C, hidden)), ("w_proj", (hidden, C))):
+        t = w[name]
         if t is None:
-            _require(name in ("w_qkv", "w_q", "w_k", "w_v"), f"missing block parameter {name}")
+            if name in ("w_o", "w_fc", "w_proj"):
+                raise ValueError(f"missing block parameter {name}")
             continue
-        _require(tuple(t.shape) == shape and t.dtype == dtype and t.is_contiguous(),
-                 f"{name} must be a contiguous {dtype} tensor of shape {shape}, got {tuple(t.shape)} {t.dtype}")
+        if t.shape != shape or t.dtype != dtype or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous {dtype} tensor of shape {shape}, got {tuple(t.shape)} {t.dtype}")
     for name in ("ln1_g", "ln1_b", "ln2_g", "ln2_b"):
         _is_vector(params[name], C, torch.float32, name)
     bias_dtype = None
     for name, n in (("b_qkv", 3 * C), ("b_o", C), ("b_fc", hidden), ("b_proj", C)):
-        t = params.get(name)
+        t = get(name)
         if t is None:
             continue
         bias_dtype = bias_dtype or t.dtype
-        _require(t.dtype in (dtype, torch.float32), f"{name} must be float32 or have the weight dtype")
+        if t.dtype != dtype and t.dtype != torch.float32:
+            raise ValueError(f"{name} must be float32 or have the weight dtype")
         _is_vector(t, n, bias_dtype, name)
-    ptr = lambda n: params[n].data_ptr() if params.get(n) is not None else None  # noqa: E731
-    return _lib.NanoGPTBlockParams(*[ptr(n) for n in BLOCK_PARAM_NAMES]), dtype, bias_dtype, hidden
+    pointers = [None if get(name) is None else params[name].data_ptr() for name in BLOCK_PARAM_NAMES]
+    return _lib.NanoGPTBlockParams(*pointers), dtype, bias_dtype, hidden
 
 
 def nanogpt_block_workspace_bytes(B, T, C, dtype, *, causal=True, activation="gelu_tanh", bias_dtype=None,
@@ -434,8 +449,8 @@ def nanogpt_block_workspace_bytes(B, T, C, dtype, *, causal=True, activation="ge
 def _workspace(workspace, need, device):
     if workspace is None:
         return torch.empty(need, dtype=torch.uint8, device=device)
-    _require(workspace.dtype == torch.uint8 and workspace.dim() == 1 and workspace.is_contiguous()
-             and workspace.numel() >= need, f"workspace must be a contiguous uint8 vector of at least {need} bytes")
+    if not (workspace.dtype == torch.uint8 and workspace.dim() == 1 and workspace.is_contiguous() and workspace.numel() >= need):
+        raise ValueError(f"workspace must be a contiguous uint8 vector of at least {need} bytes")
     return workspace
 
 
@@ -469,7 +484,8 @@ def nanogpt_forward(x, layers: list, lnf_g, lnf_b, lm_w, lm_b, n_head: int, *, e
     their bias dtype. Returns float32 logits [B,T,vocab]."""
     _require(x.dim() == 3 and x.dtype == torch.float32 and x.is_contiguous(), "x must be a contiguous float32 [B,T,C] tensor")
     B, T, C = x.shape
-    _require(lm_w.dim() == 2 and lm_w.shape[0] == C and lm_w.is_contiguous(), f"lm_w must be a contiguous [{C}, vocab] matrix")
+    if not (lm_w.dim() == 2 and lm_w.shape[0] == C and lm_w.is_contiguous()):
+        raise ValueError(f"lm_w must be a contiguous [{C}, vocab] matrix")
     vocab = lm_w.shape[1]
     dtype = lm_w.dtype
     packed = [_block_params(p, C, n_head) for p in layers]
@@ -485,8 +501,8 @@ def nanogpt_forward(x, layers: list, lnf_g, lnf_b, lm_w, lm_b, n_head: int, *, e
         _is_vector(lm_b, vocab, bias_dtype, "lm_b")
     if out is None:
         out = torch.empty((B, T, vocab), dtype=torch.float32, device=x.device)
-    _require(tuple(out.shape) == (B, T, vocab) and out.dtype == torch.float32 and out.is_contiguous(),
-             f"out must be a contiguous float32 [{B}, {T}, {vocab}] tensor")
+    if not (tuple(out.shape) == (B, T, vocab) and out.dtype == torch.float32 and out.is_contiguous()):
+        raise ValueError(f"out must be a contiguous float32 [{B}, {T}, {vocab}] tensor")
     o = _block_opts(dtype, causal, activation, bias_dtype, hidden)
     _need_cuda(x, out, workspace, lnf_g, lnf_b, lm_w, lm_b, *[t for p in layers for t in p.values() if t is not None])
     need = int(_lib.load().lh_hip_nanogpt_forward_workspace_bytes(B, T, C, vocab, lh_dtype(dtype), ctypes.byref(o)))
