@@ -37,9 +37,9 @@ static inline bool direct_offsets_fit(const GemmArgs& g) {
   return g.lda < (1ll << 22) && (int64_t)g.K * g.ldb < (1ll << 30);
 }
 
-// Every row of an f32 result starts at a multiple of 64 bytes.
+// Every row of the result starts at a multiple of 64 bytes: stores of whole row segments cover whole 64-byte pieces of memory.
 __host__ __device__ static inline bool rows_of_pieces(const GemmArgs& g) {
-  return ((reinterpret_cast<uintptr_t>(g.out) | (uintptr_t)(g.ldc * 4)) & 63) == 0;
+  return ((reinterpret_cast<uintptr_t>(g.out) | (uintptr_t)(g.ldc * (g.out_dt == LH_F32 ? 4 : 2))) & 63) == 0;
 }
 
 // Launch of the direct-to-LDS kernel with a workgroup tile of (64 TM) x (128 TN) (gemm16_direct.hip; each

@@ -252,12 +252,13 @@ static int launch_fast(const GemmArgs& g, hipStream_t s) {
 // part + (1 - part) r^2 (the 128 x 128 tile: r).  Least squares over 1870 problems on each of the four tiles (M 128 ... 8192,
 // N 512 ... 50256, K 256 ... 4096); what is chosen is within 0.9 % of the best tile on average, 1.24 x at worst (the rule
 // before it, which priced a tile by its flops, 2.4 to 5.0 %, 1.67 x).
+// `whole_k`: K is a multiple of 64; else the 256 x 256 tile is left out.  `time`: the estimate.
 struct DirectTile {
   int bm, bn;
   double b, part;
   double a[4];  // 16-bit result; f32 in rows of whole 64-byte pieces; other f32; accumulator input
 };
-static int direct_variant(const GemmArgs& g) {
+static int direct_variant(const GemmArgs& g, bool whole_k, double* time) {
   static constexpr DirectTile tiles[4] = {
       {256, 256, 0.0244, 0.69, {6.5, 9.6, 12.9, 20.5}},
       {256, 128, 0.0141, 0.72, {4.4, 6.4, 7.5, 11.3}},
@@ -266,20 +267,21 @@ static int direct_variant(const GemmArgs& g) {
   };
   const int out = (g.flags & LH_GEMM_ACCUMULATE_C) ? 3 : g.out_dt != LH_F32 ? 0 : rows_of_pieces(g) ? 1 : 2;
   const int cus = num_cus();
-  int best = 0;
+  int best = -1;
   double best_us = 0.0;
-  for (int v = 0; v < 4; ++v) {
+  for (int v = whole_k ? 0 : 1; v < 4; ++v) {
     const DirectTile& t = tiles[v];
     const int64_t n = (int64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
     const int slots = v < 3 ? cus : 2 * cus;
     const double r = (double)(n % slots) / slots;
     const double rounds = (double)(n / slots) + (r > 0.0 ? t.part + (1.0 - t.part) * (v < 3 ? r * r : r) : 0.0);
     const double us = v == 3 && n <= cus ? 0.7 * t.a[out] + 0.0082 * g.K : rounds * (t.a[out] + t.b * g.K);
-    if (v == 0 || us < best_us) {
+    if (best < 0 || us < best_us) {
       best = v;
       best_us = us;
     }
   }
+  *time = best_us;
   return best;
 }
 
@@ -314,7 +316,7 @@ static int splitk_count(int M, int N, int K) {
   const double block_mb = (double)M * N * sizeof(float) * 1e-6;
   while (splits < 8) {
     const int to = splits * 2;
-    if (tiles * to > 2 * cus || (K / to) % kBK != 0 || K / to < 512) break;
+    if (tiles * to > 2 * cus || K % (to * kBK) != 0 || K / to < 512) break;
     const double saved = (double)(K / splits - K / to) / 32 * 0.225 * (tiles * to > cus ? 0.5 : 1.0);
     const double added = (splits == 1 ? to * block_mb * 0.62 + 2.5 : (to - splits) * block_mb * 0.62);
     if (saved <= added) break;
@@ -331,6 +333,30 @@ static double direct_us(const GemmArgs& g, int sp) {
   const double per_cu = x <= 1.0 ? 1.0 : 1.0 + 0.55 * (x - 1.0);
   return 3.6 + 0.0072 * g.K / sp * per_cu + (x > 1.0 ? 0.6 * (x - 1.0) : 0.0) +
          (sp > 1 ? 3.2 + 1.2e-6 * sp * g.M * g.N : 0.0);
+}
+
+// What K has to be a multiple of for the operands to stay as they are: 8, or the 64 of a whole step where copies that make
+// it one pay:
+//  * a long K and tiles for less than half the CUs, which stream the operands at a fraction of the rate at which all of them
+//    copy them, and where K may be cut (5 x 2032 x 5480 with a transposed A: 31 us on copies, 56 as it is);
+//  * the 256 x 256 tile, which has no registers for the end of K; with more than two tiles per CU rows that do not start on
+//    128-byte lines cost a tile 1.4 times its time besides (2555 x 5480 x 3000: 103 us on copies and the 256 x 256 tile, 127 on
+//    smaller tiles as it is; 1000 x 4096 x 1000, one tile per CU: 23 and 14).
+static int direct_k_multiple(const GemmArgs& g) {
+  if (g.K % kBK == 0 || (g.flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK)) || !direct_offsets_fit(g)) return kBK;
+  const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const int cus = num_cus();
+  if (tiles * 2 <= cus && g.K >= 2048) return kBK;
+  GemmArgs p = g;
+  p.K = (g.K + kBK - 1) / kBK * kBK;
+  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A;
+  const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % 8 == 0;
+  const double copies = operand_copies_us<2>(g, kBK, 8, false, 0.65) - operand_copies_us<2>(g, 8, 8, b_in_place, 0.65);
+  double as_is, whole;
+  direct_variant(p, false, &as_is);
+  direct_variant(p, true, &whole);
+  if (tiles > 2 * cus && (ta ? g.K : g.lda) % 64 != 0) as_is *= 1.4;
+  return whole + copies <= as_is ? kBK : 8;
 }
 
 // Decode shapes: so few 128 x 128 tiles that most CUs would idle, and a K long enough to cut.
@@ -380,51 +406,54 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // 1 x 896 x 2560: 221 -> 171; at K = 128 it loses 2 of 14).
   const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
   const bool may_copy = vec_c || (!g.ws && (g.K >= 512 || rows_fit_untransposed<2>(g))) || (int64_t)g.M * g.N * g.K >= (1 << 22);
+  // (a size query counts the copies of whole steps, the upper bound it always was; calls take no more)
+  const int kmul = planning() ? kBK : direct_k_multiple(g);
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
-  const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kBK == 0;
+  const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kmul == 0;
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (g.flags & LH_GEMM_SPLITK_MASK) <= LH_GEMM_SPLITK_NONE &&
       !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones.  Against them stand the direct kernels, plus
     // the transposed or padded copies of operands that the direct kernels cannot take as they are.
     const bool tb = g.flags & LH_GEMM_TRANSPOSE_B;
-    const bool fits = g.K % kBK == 0 && (tb || g.N % 8 == 0 || g.b_padded) && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
+    const bool fits = g.K % kmul == 0 && (tb || g.N % 8 == 0 || g.b_padded) && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
                       aligned16(g.a) && aligned16(g.b);
-    // (a padded copy has whole k-steps)
-    const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) : 1;
-    const double other = direct_us(g, cuts) + operand_copies_us<2>(g, kBK, 8, b_in_place, 0.65);
+    // (a copy has whole k-steps where kmul says so)
+    const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kmul - 1) / kmul * kmul) : 1;
+    const double other = direct_us(g, cuts) + operand_copies_us<2>(g, kmul, 8, b_in_place, 0.65);
     int tile;
     const double us = gemm_small_choose(g, DT, &tile);
     if (tile >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, DT, tile, s);
   }
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && may_copy) {
     if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
-    const int rc = untranspose_operands<2>(g, kBK, 8, s);
+    const int rc = untranspose_operands<2>(g, kmul, 8, s);
     if (b_in_place) g.flags |= LH_GEMM_TRANSPOSE_B;
     if (rc < 0) return rc;
   }
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A;
   const bool tb = (g.flags & LH_GEMM_TRANSPOSE_B) && !b_in_place;  // a transposed B the direct kernels cannot take
-  const bool operands_ok = !ta && g.K % kBK == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) && aligned16(g.b);
-  const bool direct = operands_ok && (b_in_place || (!tb && (g.N % 8 == 0 || g.b_padded)));
+  const bool rows_ok = !ta && g.K % kmul == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.a) && aligned16(g.b);
+  const bool operands_ok = rows_ok && g.K % kBK == 0;
+  const bool direct = rows_ok && (b_in_place || (!tb && (g.N % 8 == 0 || g.b_padded)));
   const uint32_t tile = g.flags & LH_GEMM_TILE_MASK;
   const uint32_t splitk = g.flags & LH_GEMM_SPLITK_MASK;
   const bool cut_requested = splitk > LH_GEMM_SPLITK_NONE;
   if (tile == LH_GEMM_TILE_AUTO && !cut_requested && !direct && (int64_t)g.M * g.N * g.K >= (1 << 22)) {
     // not a shape for the direct kernels as it stands: run it on padded copies of the operands
-    const int rc = gemm_padded<2, false>(g, kBK, 8, s, [&](const GemmArgs& p) { return gemm16_dispatch<DT>(p, s); });
+    const int rc = gemm_padded<2, false>(g, kmul, 8, s, [&](const GemmArgs& p) { return gemm16_dispatch<DT>(p, s); });
     if (rc <= 0) return rc;
   }
   if (tile != LH_GEMM_TILE_AUTO) {
     static const int bm[4] = {256, 256, 128, 128}, bn[4] = {256, 128, 256, 128};
     const int v = (int)(tile >> 8) - 1;
-    LH_REQUIRE(direct && vec_c && g.M % bm[v] == 0 && g.N % bn[v] == 0 && direct_offsets_fit(g),
+    LH_REQUIRE(direct && g.K % kBK == 0 && vec_c && g.M % bm[v] == 0 && g.N % bn[v] == 0 && direct_offsets_fit(g),
                "gemm: the requested %d x %d tile needs an untransposed A, M %% %d == 0, N %% %d == 0, "
                "K %% 64 == 0 and 16-byte aligned rows, also of a transposed B (M=%d N=%d K=%d)",
                bm[v], bn[v], bm[v], bn[v], g.M, g.N, g.K);
   }
   if (cut_requested)
-    LH_REQUIRE(direct && vec_c && direct_offsets_fit(g),
+    LH_REQUIRE(direct && g.K % kBK == 0 && vec_c && direct_offsets_fit(g),
                "gemm: a split-K request needs an untransposed A, K %% 64 == 0, N %% 8 == 0 and 16-byte aligned rows, "
                "also of a transposed B (M=%d N=%d K=%d)", g.M, g.N, g.K);
   if (direct && direct_offsets_fit(g)) {
@@ -432,7 +461,8 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
       const int rc = gemm16_splitk<DT>(g, splitk, s);
       if (rc <= 0) return rc;
     }
-    const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g);
+    double us;
+    const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g, g.K % kBK == 0, &us);
     if (v == 0) return launch_direct<DT, 4, 2>(g, s);
     if (v == 1) return launch_direct<DT, 4, 1>(g, s);
     if (v == 2) return launch_direct<DT, 2, 2>(g, s);

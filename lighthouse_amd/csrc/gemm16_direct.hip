@@ -69,17 +69,19 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, int lane_byte
                                       uint8_t* lds_wave_base) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t*)lds_wave_base, 16, lane_bytes, scalar_bytes, 0, 0);
 }
-// A resource over [base, base + 4 GiB): raw (unstructured) addressing, offsets in bytes.  The kernels cut along K (the
+// A resource over [base, base + 2 GiB): raw (unstructured) addressing, offsets in bytes; a load at kOutside or beyond
+// touches no memory and leaves zeros in LDS.  The kernels cut along K (the
 // object without a tile) say that the base is uniform: the compiler keeps the panel addresses of their edge tiles, which come
 // out of the divisions that select a piece of K, in vector registers and wrote a loop over the lanes' resources around every
 // load (M = 1, N = 5376, K = 4736 bf16: 24.0 us without such loops, 28.4 with them).
+constexpr uint32_t kOutside = 0x80000000u;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t panel_resource(const void* base) {
 #if LH_GEMM16_TM == 0
   const uint64_t address = reinterpret_cast<uint64_t>(base);
   base = reinterpret_cast<const void*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(address >> 32)) << 32 |
                                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)address));
 #endif
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xffffffff, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, kOutside, 0x00020000);
 }
 template <int TM, int TN>
 struct DirectCtx {
@@ -93,6 +95,7 @@ struct DirectCtx {
   // swizzle term (row / 2) % 8 does not change with 16 rows).
   int a_rd[2];
   int wave, b_off, b_chunk, b_swz;
+  int k_end;                  // (TAIL) K: loads past it bring zeros
   // B stored transposed ([N, K], k contiguous): its panel is laid out, loaded and read like A's
   int bt_src[2 * TN];         // lane's byte offset in the B^T panel for load i at k = 0
   int bt_rd[2];               // like a_rd, for row wn0 + lane % 16 of a B^T stage
@@ -106,22 +109,50 @@ struct DirectFrags {
   u32x4 b[2 * TN];
 };
 
-// A stage `sa` (k = 64 sa .. +64): TM loads per lane.
-template <int TM, int TN>
+// The lane's 16-byte chunk of a 128-byte row of a k-contiguous stage lies past the end of K (of which `left` remain at the
+// start of the stage): the chunk is (lane % 8) ^ ((row / 2) % 8) of row 8 (8 i + wave) + lane / 8, the same for every i.
+__device__ __forceinline__ bool direct_past_k(int wave, int left) {
+  const int lane = lane_now();
+  return 8 * ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7)) >= left;
+}
+// A stage `sa` (k = 64 sa .. +64): TM loads per lane.  TAIL: K may end inside it, at a multiple of 8.
+template <int TM, int TN, bool TAIL>
 __device__ __forceinline__ void direct_load_a(const DirectCtx<TM, TN>& c, int sa, uint8_t* __restrict__ abuf) {
   const __amdgpu_buffer_rsrc_t rsrc = panel_resource(c.a_base);
+  if (TAIL && 64 * sa + 64 > c.k_end) {
+    const bool past = direct_past_k(c.wave, c.k_end - 64 * sa);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) dma16(rsrc, past ? (int)kOutside : c.a_src[i], sa * 128, abuf + (8 * i + c.wave) * 1024);
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) dma16(rsrc, c.a_src[i], sa * 128, abuf + (8 * i + c.wave) * 1024);
 }
 // B stage `sb` (k = 32 sb .. +32): TN loads per lane.  BT (B stored [N, K]): stage sb is k = 64 sb .. +64
 // of the panel's rows, 2 TN loads per lane.
-template <int TM, int TN, bool BT = false>
+template <int TM, int TN, bool BT, bool TAIL>
 __device__ __forceinline__ void direct_load_b(const DirectCtx<TM, TN>& c, int sb, uint8_t* __restrict__ bbuf) {
   const __amdgpu_buffer_rsrc_t rsrc = panel_resource(c.b_base);
   if constexpr (BT) {
+    if (TAIL && 64 * sb + 64 > c.k_end) {
+      const bool past = direct_past_k(c.wave, c.k_end - 64 * sb);
+#pragma unroll
+      for (int i = 0; i < 2 * TN; ++i) dma16(rsrc, past ? (int)kOutside : c.bt_src[i], sb * 128, bbuf + (8 * i + c.wave) * 1024);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 2 * TN; ++i) dma16(rsrc, c.bt_src[i], sb * 128, bbuf + (8 * i + c.wave) * 1024);
   } else {
+    if (TAIL && 32 * sb + 32 > c.k_end) {
+      using Cfg = DirectCfg<TM, TN>;
+      const int lane = lane_now();
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const int k = 32 * sb + (8 * i + c.wave) * Cfg::kBRowsPerLoad + lane / Cfg::kBChunks;
+        dma16(rsrc, k >= c.k_end ? (int)kOutside : c.b_src[i], sb * c.b_step, bbuf + (8 * i + c.wave) * 1024);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < TN; ++i) dma16(rsrc, c.b_src[i], sb * c.b_step, bbuf + (8 * i + c.wave) * 1024);
   }
@@ -215,7 +246,7 @@ __device__ __forceinline__ void direct_wait_barrier() {
 //   even step: [A(kt/2) B(kt+1)] [B(kt+2)] [A(kt/2+1) B(kt+3)]  -> B(kt+1) needed: TM + 2 TN may remain
 //   odd step : [B(kt+1)] [A((kt+1)/2) B(kt+2)] [B(kt+3)]        -> A needed: 2 TN may remain
 // Near the end loads are no longer issued and the waits become full waits.
-template <int DT, int TM, int TN>
+template <int DT, int TM, int TN, bool TAIL>
 __device__ __forceinline__ void direct_step_pair(const DirectCtx<TM, TN>& c, f32x4 (&acc)[2 * TN][2 * TM],
                                                  DirectFrags<TM, TN>& f, const uint8_t* __restrict__ a_cur,
                                                  const uint8_t* __restrict__ a_nxt, const uint8_t* __restrict__ b1,
@@ -228,19 +259,19 @@ __device__ __forceinline__ void direct_step_pair(const DirectCtx<TM, TN>& c, f32
   direct_phase_lo<DT>(c, acc, f, a_cur, 0);
   if (steady) direct_wait_barrier<Cfg::kWaitEven>();
   else direct_wait_barrier<0>();
-  if (kt + 4 < nk) direct_load_b(c, kt + 4, b_refill0);
+  if (kt + 4 < nk) direct_load_b<TM, TN, false, TAIL>(c, kt + 4, b_refill0);
   direct_phase_hi<DT, TM, TN, false>(c, acc, f, a_cur, b1, 1);
   // ---- odd step kt + 1
   direct_phase_lo<DT>(c, acc, f, a_cur, 1);
   if (steady) direct_wait_barrier<Cfg::kWaitOdd>();
   else direct_wait_barrier<0>();
-  if (kt + 4 < nk) direct_load_a(c, kt / 2 + 2, a_refill);
-  if (kt + 5 < nk) direct_load_b(c, kt + 5, b_refill1);
+  if (kt + 4 < nk) direct_load_a<TM, TN, TAIL>(c, kt / 2 + 2, a_refill);
+  if (kt + 5 < nk) direct_load_b<TM, TN, false, TAIL>(c, kt + 5, b_refill1);
   direct_phase_hi<DT, TM, TN, false>(c, acc, f, a_nxt, b2, 0);
 }
 
 // Source pointers of tile `id` (its position in the XCD-grouped order) and the tile's origin.
-// EDGE: M and N need not be multiples of the tile (K still of 64; an n-contiguous B has rows of a multiple of
+// EDGE: M and N need not be multiples of the tile (K of 64, or with TAIL of 8; an n-contiguous B has rows of a multiple of
 // 8 columns, padded if N is none): loads of rows / column chunks past the end are redirected to the last valid
 // row / chunk (their products land in accumulators that are never stored).  The epilogue skips what lies
 // outside the matrix and takes any alignment of output, bias and accumulator input.
@@ -301,7 +332,7 @@ __device__ __forceinline__ void direct_place(const GemmArgs& g, int id, DirectCt
 // of 64 k.  At the barrier every read of this pair's stages has returned and the next pair's
 // stages (issued at the previous barrier, 64 k ago) are awaited in full; the pair after that is
 // then requested into this pair's buffers.  BT: b1 is the pair's one 64-k stage of B^T, b2 the next.
-template <int DT, int TM, int TN, bool BT = false>
+template <int DT, int TM, int TN, bool TAIL, bool BT = false>
 __device__ __forceinline__ void direct_step_pair_1b(const DirectCtx<TM, TN>& c, f32x4 (&acc)[2 * TN][2 * TM],
                                                     DirectFrags<TM, TN>& f, const uint8_t* __restrict__ a_cur,
                                                     const uint8_t* __restrict__ a_nxt, const uint8_t* __restrict__ b1,
@@ -319,30 +350,30 @@ __device__ __forceinline__ void direct_step_pair_1b(const DirectCtx<TM, TN>& c, 
   if (TM * TN == 2 && stores_behind && kt == 0) direct_wait_barrier<Cfg::kStagedStores>();
   else direct_wait_barrier<0>();
   if (kt + 4 < nk) {
-    direct_load_a(c, kt / 2 + 2, a_refill);
+    direct_load_a<TM, TN, TAIL>(c, kt / 2 + 2, a_refill);
     if constexpr (BT) {
-      direct_load_b<TM, TN, true>(c, kt / 2 + 2, b_refill0);
+      direct_load_b<TM, TN, true, TAIL>(c, kt / 2 + 2, b_refill0);
     } else {
-      direct_load_b(c, kt + 4, b_refill0);
-      direct_load_b(c, kt + 5, b_refill1);
+      direct_load_b<TM, TN, false, TAIL>(c, kt + 4, b_refill0);
+      direct_load_b<TM, TN, false, TAIL>(c, kt + 5, b_refill1);
     }
   }
   direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_nxt, b2, 0);
 }
 
-// First loads of a tile: A stages 0, 1 and B stages 0 .. 3 (nk = K / 32 >= 2); BT: both 64-k stages of B^T.
-template <int TM, int TN, bool BT = false>
+// First loads of a tile: A stages 0, 1 and B stages 0 .. 3 (nk >= 2); BT: both 64-k stages of B^T.
+template <int TM, int TN, bool TAIL, bool BT = false>
 __device__ __forceinline__ void direct_prologue(const DirectCtx<TM, TN>& c, int nk, uint8_t* __restrict__ ring) {
   using Cfg = DirectCfg<TM, TN>;
-  direct_load_a(c, 0, ring);
-  if (nk > 2) direct_load_a(c, 1, ring + Cfg::kABytes);
+  direct_load_a<TM, TN, TAIL>(c, 0, ring);
+  if (nk > 2) direct_load_a<TM, TN, TAIL>(c, 1, ring + Cfg::kABytes);
   if constexpr (BT) {
-    direct_load_b<TM, TN, true>(c, 0, ring + Cfg::kBBase);
-    if (nk > 2) direct_load_b<TM, TN, true>(c, 1, ring + Cfg::kBBase + Cfg::kBtBytes);
+    direct_load_b<TM, TN, true, TAIL>(c, 0, ring + Cfg::kBBase);
+    if (nk > 2) direct_load_b<TM, TN, true, TAIL>(c, 1, ring + Cfg::kBBase + Cfg::kBtBytes);
   } else {
 #pragma unroll
     for (int st = 0; st < 4; ++st)
-      if (st < nk) direct_load_b(c, st, ring + Cfg::kBBase + st * Cfg::kBBytes);
+      if (st < nk) direct_load_b<TM, TN, false, TAIL>(c, st, ring + Cfg::kBBase + st * Cfg::kBBytes);
   }
 }
 
@@ -377,7 +408,7 @@ __device__ __forceinline__ void direct_load_bias(const GemmArgs& g, int n_base, 
 // those stores may stay in flight.
 // `staged`: the epilogue will want `bias` (for columns from n_base); it is loaded ahead of the
 // last two steps, whose full wait covers it.
-template <int DT, int TM, int TN, bool EDGE, bool BT = false>
+template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool BT>
 __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectCtx<TM, TN>& c,
                                                 f32x4 (&acc)[2 * TN][2 * TM], uint8_t* smem_d, int nk,
                                                 bool stores_behind, bool staged, int n_base, u32x2 (&bias)[2 * TN]) {
@@ -404,14 +435,14 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
     if constexpr (BT) {
       uint8_t* b_cur = bbuf + ((kt >> 1) & 1) * Cfg::kBtBytes;
       uint8_t* b_nxt = bbuf + (((kt >> 1) + 1) & 1) * Cfg::kBtBytes;
-      direct_step_pair_1b<DT, TM, TN, true>(c, acc, f, a_cur, a_nxt, b_cur, b_nxt, a_cur, b_cur, b_cur, kt, nk,
+      direct_step_pair_1b<DT, TM, TN, TAIL, true>(c, acc, f, a_cur, a_nxt, b_cur, b_nxt, a_cur, b_cur, b_cur, kt, nk,
                                             stores_behind);
     } else {
       uint8_t* b0 = bbuf + (kt & 3) * Cfg::kBBytes;
       uint8_t* b1 = bbuf + ((kt + 1) & 3) * Cfg::kBBytes;
       uint8_t* b2 = bbuf + ((kt + 2) & 3) * Cfg::kBBytes;
-      if constexpr (decltype(one)::value) direct_step_pair_1b<DT>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk, stores_behind);
-      else direct_step_pair<DT>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk);
+      if constexpr (decltype(one)::value) direct_step_pair_1b<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk, stores_behind);
+      else direct_step_pair<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk);
     }
   };
   if constexpr (BT || TM * TN > 2) {
@@ -562,7 +593,7 @@ __device__ __forceinline__ void direct_finish_rows(const GemmArgs& g, int wave, 
 // BLOCKS (a launch cut along K): the accumulators go out as they are, f32, to rows of whole aligned 16-byte chunks.
 // None of the epilogue variants is in that code: with the element-aligned accesses of an edge tile they took the
 // 128 x 128 tile to 136 registers, where two workgroups no longer fit a CU (M = 16, N = K = 8192 bf16: 34 -> 40 us).
-template <int DT, int TM, int TN, bool EDGE, bool HAS_NEXT, bool BT = false, bool BLOCKS = false>
+template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool HAS_NEXT, bool BT, bool BLOCKS, bool STREAM>
 __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx<TM, TN>& next, int nk,
                                               uint8_t* __restrict__ ring, uint8_t* __restrict__ stage,
                                               const f32x4 (&acc)[2 * TN][2 * TM], const u32x2 (&bias)[2 * TN], int m0,
@@ -583,7 +614,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 #pragma unroll
       for (int e = 0; e < 2; ++e) asm volatile("" ::"v"(bias[i][e]));
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with the rings
-    if constexpr (HAS_NEXT) direct_prologue<TM, TN, BT>(next, nk, ring);
+    if constexpr (HAS_NEXT) direct_prologue<TM, TN, TAIL, BT>(next, nk, ring);
     constexpr int RB = WTN * 2;                // bytes of a staged row
     constexpr int chunks = RB / 16;            // 16-byte chunks per staged row
     constexpr int rows_per_pass = 64 / chunks;
@@ -624,9 +655,11 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
           u32x4 w = *reinterpret_cast<const u32x4*>(cw + row * RB + ((ch ^ ((row >> 1) & (chunks - 1))) << 4));
           const int m = m0 + wm0 + 32 * j0 + row, n = n0 + wn0 + ch * 8;
           if constexpr (EDGE) {
-            if (m < g.M && n < g.N) store8_any(outp + (int64_t)m * g.ldc + n, w, g.N - n);
+            if (m < g.M && n < g.N) store8_any<STREAM>(outp + (int64_t)m * g.ldc + n, w, g.N - n);
           } else {
-            __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(outp + (int64_t)m * g.ldc + n));
+            u32x4* const to = reinterpret_cast<u32x4*>(outp + (int64_t)m * g.ldc + n);
+            if constexpr (STREAM) __builtin_nontemporal_store(w, to);
+            else *to = w;
           }
         }
       }
@@ -634,7 +667,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
     return;
   }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  if constexpr (HAS_NEXT) direct_prologue<TM, TN, BT>(next, nk, ring);
+  if constexpr (HAS_NEXT) direct_prologue<TM, TN, TAIL, BT>(next, nk, ring);
   if constexpr (EDGE && !BLOCKS) {
     if (g.out_dt == LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C) && !rows_of_pieces(g)) {
       direct_finish_rows<DT, TM, TN>(g, next.wave, stage, acc, m0, n0, wm0, wn0);
@@ -739,16 +772,16 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 #pragma unroll
               for (int e = 0; e < 4; ++e) v[e] += b4[e];
             }
-            // (the blocks of a launch cut along K are read again at once)
-            if constexpr (EDGE && !BLOCKS)
-              store4_any<out32 ? LH_F32 : DT, out32 && !has_c>(g.out, off, v, g.N - n);
-            else if constexpr (out32 && BLOCKS)
-              *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off) = v;
-            else if constexpr (out32)
-              __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off));
-            else
-              __builtin_nontemporal_store(u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])},
-                                          reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(g.out) + off));
+            if constexpr (EDGE && !BLOCKS) {
+              store4_any<out32 ? LH_F32 : DT, STREAM>(g.out, off, v, g.N - n);
+            } else if constexpr (out32) {
+              f32x4* const to = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.out) + off);
+              if constexpr (STREAM) __builtin_nontemporal_store(v, to);
+              else *to = v;
+            } else {
+              *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(g.out) + off) =
+                  u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
+            }
           }
         }
       }
@@ -776,8 +809,12 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 // For problems with few tiles and a long K (decode shapes), where the tile count cannot fill the CUs.
 // BT: B is stored transposed ([N, K] with row stride ldb, the layout of a torch Linear weight); its
 // panel goes through the rings like A's and no transposed copy is made.
-template <int DT, int TM, int TN, bool EDGE, bool SPLITK = false, bool BT = false>
-__global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
+// STREAM (large results, which are cut into 256 x 256 tiles): whole vectors are stored past the caches.  A kernel of its own:
+// choosing between the two stores inside one cost smaller results 1 to 3 us of instruction fetches.
+// TAIL: K is a multiple of 8 but not of 64, the last step's loads bring zeros from K on (not for the 256 x 256 tile, which
+// has no registers for it).  A kernel of its own too: asking at every load cost a lone workgroup 5 % (3 x 512 x 8000).
+template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool SPLITK, bool BT, bool STREAM>
+__device__ __forceinline__ void direct_run(const GemmArgs& g) {
   using Cfg = DirectCfg<TM, TN>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_d[];
   const int tiles1 = ((g.M + Cfg::BM - 1) / Cfg::BM) * ((g.N + Cfg::BN - 1) / Cfg::BN);
@@ -800,11 +837,11 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
   const int wm0 = (wave / WN) * Cfg::WTM, wn0 = (wave % WN) * Cfg::WTN;
   const int l16 = lane & 15, g4 = lane >> 4;
 
-  // 256 x 256 tiles, one workgroup per CU: workgroups in step store their tiles in step, and the main loops in between leave
+  // Large results, one workgroup per CU: workgroups in step store their tiles in step, and the main loops in between leave
   // the memory idle.  So some start half a tile late: those that have a tile fewer than the others where that is up to half
   // of them (they have the time), half of them where all have as many and those are enough.  M = 8192, N = 50432, K = 768
   // bf16: 559 -> 540 us, with f32 results 633 -> 605.
-  if constexpr (TM * TN == 8) {
+  if constexpr (STREAM) {
     const int grid = (int)gridDim.x;
     if (ntiles > grid) {
       const int rest = ntiles % grid;
@@ -839,14 +876,16 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
     c.bt_rd[1] = c.bt_rd[0] ^ 64;
   }
 
-  const int nk = g.K / 32;  // even: K is a multiple of 64
+  // (even: K is a multiple of 64, or the steps from K on multiply zeros)
+  const int nk = TAIL ? (g.K + 63) / 64 * 2 : g.K / 32;
+  c.k_end = g.K;
   int t = blockIdx.x;       // < ntiles: the grid is never larger than the tile list
   int m0, n0;
   {
     const int id = select(t, g_cur);
     direct_place<TM, TN, EDGE, BT>(SPLITK ? g_cur : g, xcd_remap(id, tiles1), c, m0, n0);
   }
-  direct_prologue<TM, TN, BT>(c, nk, smem_d);
+  direct_prologue<TM, TN, TAIL, BT>(c, nk, smem_d);
   // Without EDGE every lane issues all stores of a staged epilogue.
   const bool staged = !SPLITK && g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
   const bool counted_stores = !EDGE && staged;
@@ -861,7 +900,7 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
         for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.0f;
     u32x2 bias[2 * TN];
     const GemmArgs& ga = SPLITK ? g_cur : g;
-    direct_mainloop<DT, TM, TN, EDGE, BT>(ga, c, acc, smem_d, nk, counted_stores && !first, staged, n0 + wn0 + 4 * g4, bias);
+    direct_mainloop<DT, TM, TN, EDGE, TAIL, BT>(ga, c, acc, smem_d, nk, counted_stores && !first, staged, n0 + wn0 + 4 * g4, bias);
     first = false;
     const int tn = t + (int)gridDim.x;
     const bool more = tn < ntiles;
@@ -871,9 +910,9 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
     if (more) {
       const int idn = select(tn, g_nxt);
       direct_place<TM, TN, EDGE, BT>(SPLITK ? g_nxt : g, xcd_remap(idn, tiles1), cn, m1, n1);
-      direct_finish<DT, TM, TN, EDGE, true, BT, SPLITK>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
+      direct_finish<DT, TM, TN, EDGE, TAIL, true, BT, SPLITK, STREAM>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
     } else {
-      direct_finish<DT, TM, TN, EDGE, false, BT, SPLITK>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
+      direct_finish<DT, TM, TN, EDGE, TAIL, false, BT, SPLITK, STREAM>(ga, cn, nk, smem_d, stage, acc, bias, m0, n0, wm0, wn0);
     }
     if (!more) break;
     if constexpr (SPLITK) g_cur = g_nxt;
@@ -892,10 +931,20 @@ __global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
   }
 }
 
-template <int DT, int TM, int TN, bool EDGE, bool BT = false>
+template <int DT, int TM, int TN, bool EDGE, bool SPLITK = false, bool BT = false, bool STREAM = false>
+__global__ void __launch_bounds__(512) gemm16_direct(GemmArgs g) {
+  direct_run<DT, TM, TN, EDGE, false, SPLITK, BT, STREAM>(g);
+}
+template <int DT, int TM, int TN, bool BT>
+__global__ void __launch_bounds__(512) gemm16_direct_tail(GemmArgs g) {
+  direct_run<DT, TM, TN, true, true, false, BT, false>(g);
+}
+
+template <int DT, int TM, int TN, bool EDGE, bool BT = false, bool STREAM = false, bool TAIL = false>
 static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
   using Cfg = DirectCfg<TM, TN>;
-  auto kern = gemm16_direct<DT, TM, TN, EDGE, false, BT>;
+  auto kern = gemm16_direct<DT, TM, TN, EDGE, false, BT, STREAM>;
+  if constexpr (TAIL) kern = gemm16_direct_tail<DT, TM, TN, BT>;
   constexpr size_t lds = Cfg::kLdsBytes;
   static bool configured = false;
   if (!configured && !planning()) {
@@ -917,6 +966,16 @@ int launch_direct(const GemmArgs& g, hipStream_t s) {
   const bool whole = g.M % Cfg::BM == 0 && g.N % Cfg::BN == 0 && g.ldc % 8 == 0 && aligned16(g.out) &&
                      (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias)) &&
                      (!(g.flags & LH_GEMM_ACCUMULATE_C) || aligned16(g.c));
+  if constexpr (TM * TN < 8)
+    if (g.K % 64 != 0)
+      return (g.flags & LH_GEMM_TRANSPOSE_B) ? launch_direct_edge<DT, TM, TN, true, true, false, true>(g, s)
+                                             : launch_direct_edge<DT, TM, TN, true, false, false, true>(g, s);
+  if constexpr (TM * TN == 8)
+    if (large_result(g)) {
+      if (g.flags & LH_GEMM_TRANSPOSE_B)
+        return whole ? launch_direct_edge<DT, TM, TN, false, true, true>(g, s) : launch_direct_edge<DT, TM, TN, true, true, true>(g, s);
+      return whole ? launch_direct_edge<DT, TM, TN, false, false, true>(g, s) : launch_direct_edge<DT, TM, TN, true, false, true>(g, s);
+    }
   if (g.flags & LH_GEMM_TRANSPOSE_B)
     return whole ? launch_direct_edge<DT, TM, TN, false, true>(g, s) : launch_direct_edge<DT, TM, TN, true, true>(g, s);
   return whole ? launch_direct_edge<DT, TM, TN, false>(g, s) : launch_direct_edge<DT, TM, TN, true>(g, s);

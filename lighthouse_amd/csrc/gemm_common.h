@@ -119,10 +119,12 @@ __device__ __forceinline__ void store4_any(void* p, int64_t at, const f32x4& v, 
   for (int e = 0; e < 3; ++e)
     if (e < left) store_from_f32<DT>(p, at + e, v[e]);
 }
-// 8 packed 16-bit values, of which the first `left` are stored, past the caches if all are.
+// 8 packed 16-bit values, of which the first `left` are stored (STREAM: all eight past the caches).
+template <bool STREAM>
 __device__ __forceinline__ void store8_any(uint16_t* p, const u32x4& w, int left) {
   if (left >= 8) {
-    __builtin_nontemporal_store(u32x4_any(w), reinterpret_cast<u32x4_any*>(p));
+    if constexpr (STREAM) __builtin_nontemporal_store(u32x4_any(w), reinterpret_cast<u32x4_any*>(p));
+    else *reinterpret_cast<u32x4_any*>(p) = w;
     return;
   }
 #pragma unroll
@@ -494,6 +496,13 @@ __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, c
   if (g.flags & LH_GEMM_HAS_BIAS) bias = bias4<DT, true>(g, n);
   epilogue4_loaded<DT>(g, m, n, acc, bias, c);
 }
+
+// Results so large that they push the operands out of the memory-side cache (256 MB, of which reads and writes both take) leave
+// past the caches.  256 x 256 tiles, K = 768 bf16, plain and past the caches: 8192 x 50432 654 and 563 us (main loop of a tile
+// 23.6 and 17.7), f32 797 and 763; 8192 x 16392 234 and 206; 8192 x 8200 x 2048 252 either way; fp8 8192^3 407 and 401.
+// Smaller ones, which the next kernel reads, lose as often as they gain: nanoGPT blocks of 2048 rows 88 and 93 us, of 4096
+// rows 138 and 135.5.
+static inline bool large_result(const GemmArgs& g) { return (int64_t)g.M * g.ldc * (g.out_dt == LH_F32 ? 4 : 2) >= 128000000; }
 
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s);
 // Estimated time of a 16-bit product with few tiles, untransposed and aligned, not cut along K, in us.

@@ -47,3 +47,32 @@ def test_workgroups_that_start_late(M, N):
     a, b = (torch.randint(-3, 4, s, device="cuda", generator=g).float() for s in ((M, 64), (64, N)))
     got = ops.gemm(a.bfloat16(), b.bfloat16())
     assert torch.equal(got, (a @ b).bfloat16())
+
+
+@pytest.mark.parametrize("dtype,layout", [("bf16", "nn"), ("bf16", "nt"), ("f16", "tn")])
+@pytest.mark.parametrize("M,N,K", [(1000, 4096, 1000),   # 128 x 128 tiles, the step ends after 40 of 64
+                                   (1030, 4104, 72),     # one chunk of the second step
+                                   (900, 8200, 8),       # less than a step
+                                   (700, 5000, 120), (2048, 8192, 328), (2100, 6152, 184), (640, 12288, 568),
+                                   (100, 40000, 104)])
+def test_k_that_ends_inside_a_step(M, N, K, dtype, layout):
+    """Operands whose rows go on behind K, with NaN: what the last step reads past K must count as nothing."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M * K)
+    ta, tb = layout[0] == "t", layout[1] == "t"
+    av, bv = (torch.randint(-3, 4, s, device="cuda", generator=g).float() for s in ((M, K), (K, N)))
+
+    def stored(v, transposed):
+        v = v.T if transposed else v
+        buf = torch.full((v.shape[0] + 72, v.shape[1] + 72), float("nan"), device="cuda").to(DTYPES[dtype])
+        buf[:v.shape[0], :v.shape[1]] = v.to(DTYPES[dtype])
+        return buf[:v.shape[0], :v.shape[1]]
+
+    a, b = stored(av, ta), stored(bv, tb)
+    want = av @ bv
+    got = ops.gemm(a, b, out_dtype=torch.float32, transpose_a=ta, transpose_b=tb)
+    assert torch.equal(got, want)
+    bias = torch.randint(-3, 4, (N,), device="cuda", generator=g).to(DTYPES[dtype])
+    got = ops.gemm(a, b, bias, relu=True, transpose_a=ta, transpose_b=tb)
+    assert torch.equal(got, torch.relu(want + bias.float()).to(DTYPES[dtype]))
