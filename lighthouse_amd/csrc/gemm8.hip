@@ -379,7 +379,7 @@ __device__ __forceinline__ void d8_mainloop(const D8Ctx& c, f32x4 (&acc)[4][8], 
 // chunk ^ ((row / 2) % 8) against bank conflicts); the last tile of a workgroup stages its whole
 // sub-tile in the idle rings at once.  `ring` and `stage` are separate restrict parameters so
 // that the staging traffic does not wait for the asynchronous ring writes.
-template <bool HAS_NEXT>
+template <bool HAS_NEXT, bool STREAM>
 __device__ __forceinline__ void d8_finish(const GemmArgs& g, const D8Ctx& next, int nk, uint8_t* __restrict__ ring,
                                           uint8_t* __restrict__ stage, const f32x4 (&acc)[4][8], int m0, int n0, int wm0,
                                           int wn0) {
@@ -422,7 +422,9 @@ __device__ __forceinline__ void d8_finish(const GemmArgs& g, const D8Ctx& next, 
         for (int t = 0; t < JB * 32 / rows_per_pass; ++t) {
           const int row = rows_per_pass * t + lane / chunks, ch = lane % chunks;
           u32x4 w = *reinterpret_cast<const u32x4*>(cw + row * RB + ((ch ^ ((row >> 1) & (chunks - 1))) << 4));
-          *reinterpret_cast<u32x4*>(outp + (int64_t)(m0 + wm0 + 32 * j0 + row) * g.ldc + n0 + wn0 + ch * 8) = w;
+          u32x4* const to = reinterpret_cast<u32x4*>(outp + (int64_t)(m0 + wm0 + 32 * j0 + row) * g.ldc + n0 + wn0 + ch * 8);
+          if constexpr (STREAM) __builtin_nontemporal_store(w, to);
+          else *to = w;
         }
       }
     });
@@ -446,7 +448,8 @@ __device__ __forceinline__ void d8_finish(const GemmArgs& g, const D8Ctx& next, 
 // SPLITK: the tile list is g.splits copies of the problem's tiles, copy sp working on its own K
 // columns of A / rows of B and its own f32 block of the output; a second kernel adds the blocks,
 // scales and converts.  For problems with too few tiles for the CUs and a long K.
-template <bool SPLITK>
+// STREAM: a large bf16 result is stored past the caches (large_result; 8192^3 407 -> 401 us).
+template <bool SPLITK, bool STREAM = false>
 __global__ void __launch_bounds__(512) gemm8_direct(GemmArgs g) {
   constexpr int TM = 4, TN = 2, WN = 4, WTN = 64;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_8[];
@@ -519,9 +522,9 @@ __global__ void __launch_bounds__(512) gemm8_direct(GemmArgs g) {
     if (more) {
       const int idn = select(tn, g_nxt);
       d8_place(SPLITK ? g_nxt : g, xcd_remap(idn, tiles1), cn, m1, n1);
-      d8_finish<true>(ga, cn, nk, smem_8, stage, acc, m0, n0, wm0, wn0);
+      d8_finish<true, STREAM>(ga, cn, nk, smem_8, stage, acc, m0, n0, wm0, wn0);
     } else {
-      d8_finish<false>(ga, cn, nk, smem_8, stage, acc, m0, n0, wm0, wn0);
+      d8_finish<false, STREAM>(ga, cn, nk, smem_8, stage, acc, m0, n0, wm0, wn0);
     }
     if (!more) break;
     if constexpr (SPLITK) g_cur = g_nxt;
@@ -532,16 +535,21 @@ __global__ void __launch_bounds__(512) gemm8_direct(GemmArgs g) {
   }
 }
 
+template <bool STREAM>
 static int launch_direct8(const GemmArgs& g, hipStream_t s) {
+  auto kern = gemm8_direct<false, STREAM>;
   static bool configured = false;
   if (!configured && !planning()) {
-    LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm8_direct<false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, kD8LdsBytes));
+    LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     kD8LdsBytes));
     configured = true;
   }
   const int ntiles = (g.M / 256) * (g.N / 256), cus = num_cus();
-  LH_LAUNCH(gemm8_direct<false>, dim3(ntiles < cus ? ntiles : cus), dim3(512), kD8LdsBytes, s, g);
+  LH_LAUNCH(kern, dim3(ntiles < cus ? ntiles : cus), dim3(512), kD8LdsBytes, s, g);
   return check_launch("gemm8_direct");
+}
+static int launch_direct8(const GemmArgs& g, hipStream_t s) {
+  return g.out_dt != LH_F32 && large_result(g) ? launch_direct8<true>(g, s) : launch_direct8<false>(g, s);
 }
 
 // Sum of the split-K blocks ([splits][M][N] f32), scale, conversion: 4 columns per thread.
