@@ -343,19 +343,28 @@ static double direct_us(const GemmArgs& g, int sp) {
 //    128-byte lines cost a tile 1.4 times its time besides (2555 x 5480 x 3000: 103 us on copies and the 256 x 256 tile, 127 on
 //    smaller tiles as it is; 1000 x 4096 x 1000, one tile per CU: 23 and 14).
 static int direct_k_multiple(const GemmArgs& g) {
-  if (g.K % kBK == 0 || (g.flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK)) || !direct_offsets_fit(g)) return kBK;
+  if (g.K % kBK == 0 || (g.flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK))) return kBK;
   const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
   const int cus = num_cus();
   if (tiles * 2 <= cus && g.K >= 2048) return kBK;
-  GemmArgs p = g;
-  p.K = (g.K + kBK - 1) / kBK * kBK;
-  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A;
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % 8 == 0;
+  // The problem as the direct kernels would get it: an operand that is copied in any case has rows of its own.
+  const OperandCopies copied = operand_copies<2>(g, 8, 8, b_in_place);
+  GemmArgs p = g;
+  p.K = (g.K + 7) / 8 * 8;
+  if (copied.a) p.lda = p.K;
+  if (copied.b) {
+    p.ldb = (g.N + 7) / 8 * 8;
+    p.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
+  }
+  if (!direct_offsets_fit(p)) return kBK;
   const double copies = operand_copies_us<2>(g, kBK, 8, false, 0.65) - operand_copies_us<2>(g, 8, 8, b_in_place, 0.65);
   double as_is, whole;
+  const bool odd_rows = tiles > 2 * cus && p.lda % 64 != 0;
+  p.K = (g.K + kBK - 1) / kBK * kBK;
   direct_variant(p, false, &as_is);
   direct_variant(p, true, &whole);
-  if (tiles > 2 * cus && (ta ? g.K : g.lda) % 64 != 0) as_is *= 1.4;
+  if (odd_rows) as_is *= 1.4;
   return whole + copies <= as_is ? kBK : 8;
 }
 
@@ -406,8 +415,8 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // 1 x 896 x 2560: 221 -> 171; at K = 128 it loses 2 of 14).
   const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
   const bool may_copy = vec_c || (!g.ws && (g.K >= 512 || rows_fit_untransposed<2>(g))) || (int64_t)g.M * g.N * g.K >= (1 << 22);
-  // (a size query counts the copies of whole steps, the upper bound it always was; calls take no more)
-  const int kmul = planning() ? kBK : direct_k_multiple(g);
+  // (a size query counts the copies of whole steps, the upper bound it always was)
+  const int kmul = planning() ? kBK : g.k_multiple ? g.k_multiple : direct_k_multiple(g);
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kmul == 0;

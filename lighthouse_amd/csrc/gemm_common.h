@@ -27,6 +27,9 @@ struct GemmArgs {
   int one_barrier = 0;
   // B is a copy whose rows hold whole 16-byte chunks past column N (zeros): N need not be a multiple of them.
   bool b_padded = false;
+  // The operands are copies made for kernels that want K in multiples of this (0: they are the caller's).  Decided once per
+  // call: what is decided for the copies themselves may be another multiple, and a second copy would be written over the first.
+  uint8_t k_multiple = 0;
 };
 
 // Epilogue for 4 consecutive columns of one row.
@@ -318,19 +321,29 @@ inline bool rows_fit_untransposed(const GemmArgs& g) {
   return ((g.flags & LH_GEMM_TRANSPOSE_A) || fit(g.a, g.lda)) && ((g.flags & LH_GEMM_TRANSPOSE_B) || fit(g.b, g.ldb));
 }
 
-// Time of the copies that the direct kernels need in front of them, in us (0: none): what untranspose_operands and gemm_padded
-// will launch, at 3.5 us a launch and `us_per_mb` per MB of operand copied or zeroed.
+// The copies that the direct kernels need in front of them: what untranspose_operands and gemm_padded will make.
+struct OperandCopies {
+  bool a, b, odd_k, odd_n;
+};
 template <int ELEM_BYTES>
-inline double operand_copies_us(const GemmArgs& g, int k_multiple, int n_multiple, bool b_in_place, double us_per_mb) {
+inline OperandCopies operand_copies(const GemmArgs& g, int k_multiple, int n_multiple, bool b_in_place) {
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
   const bool odd_k = g.K % k_multiple != 0, odd_n = g.N % n_multiple != 0 && !g.b_padded;
   auto odd_rows = [](const void* p, int64_t ld) { return ld % (16 / ELEM_BYTES) != 0 || !aligned16(p); };
   const bool a = ta || odd_k || odd_rows(g.a, g.lda);
   const bool a_padded = a && (!ta || odd_k || odd_n);  // (by gemm_padded, which then copies a B that could stay, too)
   const bool b = tb ? !b_in_place || a_padded : odd_k || odd_n || odd_rows(g.b, g.ldb);
-  const double mb_a = a ? 1e-6 * ELEM_BYTES * g.M * g.K : 0.0, mb_b = b ? 1e-6 * ELEM_BYTES * g.K * g.N : 0.0;
-  const bool fill_a = a && ta && odd_k, fill_b = b && tb && (odd_k || odd_n);  // zeros below a transposed copy
-  const int launches = (a && ta) + (b && tb) + fill_a + fill_b + ((a && !ta) || (b && !tb));
+  return OperandCopies{a, b, odd_k, odd_n};
+}
+
+// Their time, in us (0: none): 3.5 us a launch and `us_per_mb` per MB of operand copied or zeroed.
+template <int ELEM_BYTES>
+inline double operand_copies_us(const GemmArgs& g, int k_multiple, int n_multiple, bool b_in_place, double us_per_mb) {
+  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
+  const OperandCopies c = operand_copies<ELEM_BYTES>(g, k_multiple, n_multiple, b_in_place);
+  const double mb_a = c.a ? 1e-6 * ELEM_BYTES * g.M * g.K : 0.0, mb_b = c.b ? 1e-6 * ELEM_BYTES * g.K * g.N : 0.0;
+  const bool fill_a = c.a && ta && c.odd_k, fill_b = c.b && tb && (c.odd_k || c.odd_n);  // zeros below a transposed copy
+  const int launches = (c.a && ta) + (c.b && tb) + fill_a + fill_b + ((c.a && !ta) || (c.b && !tb));
   return 3.5 * launches + us_per_mb * (mb_a * (1 + fill_a) + mb_b * (1 + fill_b));
 }
 
@@ -360,6 +373,7 @@ inline int gemm_padded(const GemmArgs& g, int k_multiple, int n_multiple, hipStr
   if (PAD_C && odd_c) bytes += round256((size_t)g.M * Np * out_bytes);
   GemmArgs p = g;
   p.K = Kp;
+  p.k_multiple = (uint8_t)k_multiple;
   if (bytes > 0) {
     void* taken = nullptr;
     if (int rc = scratch_take(g.ws, s, kScratchPad, bytes, "gemm (padded operands)", &taken)) return rc;

@@ -76,3 +76,26 @@ def test_k_that_ends_inside_a_step(M, N, K, dtype, layout):
     bias = torch.randint(-3, 4, (N,), device="cuda", generator=g).to(DTYPES[dtype])
     got = ops.gemm(a, b, bias, relu=True, transpose_a=ta, transpose_b=tb)
     assert torch.equal(got, torch.relu(want + bias.float()).to(DTYPES[dtype]))
+
+
+@pytest.mark.parametrize("dtype,transpose_b", [("bf16", False), ("f16", True)])
+@pytest.mark.parametrize("M,N,K,lda", [(4096, 8192, 1000, 1024), (2064, 5480, 1224, 1280), (2100, 6152, 72, 128)])
+def test_rows_off_16_bytes_and_a_k_inside_a_step(M, N, K, lda, dtype, transpose_b):
+    """A is copied for its alignment.  Its own rows start on 128-byte lines and the copy's do not, which the choice of what K is
+    padded to depends on; one copy is made all the same, in the library's memory (the second call finds its buffers
+    large enough) and in a workspace of the queried size."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M * K)
+    av, bv = (torch.randint(-3, 4, s, device="cuda", generator=g).float() for s in ((M, K), (K, N)))
+    buf = torch.full((M, lda), float("nan"), device="cuda").to(DTYPES[dtype])
+    a = buf[:, 1:1 + K]
+    a.copy_(av)
+    b = (bv.T if transpose_b else bv).contiguous().to(DTYPES[dtype])
+    want = av @ bv
+    for _ in range(2):
+        assert torch.equal(ops.gemm(a, b, out_dtype=torch.float32, transpose_b=transpose_b), want)
+    out = torch.empty((M, N), device="cuda")
+    need = ops.gemm_workspace_bytes(M, N, K, DTYPES[dtype], torch.float32, transpose_b=transpose_b, operands=(out, a, b, None))
+    ops.gemm(a, b, out=out, transpose_b=transpose_b, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+    assert torch.equal(out, want)

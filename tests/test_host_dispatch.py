@@ -1,0 +1,88 @@
+"""What the library's host code makes of a call, on any machine: which kernels it launches on which addresses, and what memory it
+takes.  The calls run on a recorder in the place of the HIP runtime (hip_recorder.cpp), in a process of its own."""
+
+import multiprocessing
+import random
+
+import pytest
+
+from tests import recorded_launches as rec
+
+DT = rec._lib.BF16
+OUT, A, B, BIAS, WORKSPACE = (1 << 50, 2 << 50, 3 << 50, 4 << 50, 5 << 50)  # far apart, aligned
+
+
+@pytest.fixture(scope="module")
+def recorded(tmp_path_factory):
+    """recorded(check, *args): check(recorder, *args) in a process whose library launches nothing."""
+    so = rec.build(tmp_path_factory.mktemp("recorder"))
+    with multiprocessing.get_context("spawn").Pool(1) as pool:
+        yield lambda check, *args: pool.apply(_on_recorder, (so, check, args))
+
+
+_recorder = None
+
+
+def _on_recorder(so, check, args):
+    global _recorder
+    _recorder = _recorder or rec.Recorder(so)
+    return check(_recorder, *args)
+
+
+def _product(rng, largest):
+    """A 16-bit product: any layout, row stride, alignment, K and output type."""
+    size = lambda lo, hi: int(lo * (hi / lo) ** rng.random())  # noqa: E731
+    while True:
+        M, N, K = size(1, 8192), size(1, 8192), size(1, 8192)
+        if rng.random() < 0.7:
+            K = max(K // 8 * 8, 8)
+        if rng.random() < 0.5:
+            N = max(N // 8 * 8, 8)
+        if 2 * M * N * K <= largest:
+            break
+    ta, tb = rng.random() < 0.3, rng.random() < 0.4
+    stride = lambda cols: rng.choice([cols, cols, (cols + 63) // 64 * 64, cols + 8, cols + 1, (cols + 127) // 128 * 128 + 64])  # noqa: E731
+    offset = lambda: 2 * rng.choice([0, 0, 1, 4, 8])  # noqa: E731
+    return dict(M=M, N=N, K=K, lda=stride(M if ta else K), ldb=stride(K if tb else N), ldc=stride(N), a=A + offset(), b=B + offset(),
+                out_dtype=rng.choice([DT, rec._lib.F32]), flags=(8 if ta else 0) | (16 if tb else 0) | rng.choice([0, 0, 1, 3, 33, 4]))
+
+
+def _shape(p):
+    return [p[k] for k in ("M", "N", "K", "lda", "ldb", "ldc")] + [DT, p["out_dtype"], p["flags"]]
+
+
+def _pointers(p):
+    return OUT, p["a"], p["b"], BIAS
+
+
+def _row(M, N, K, lda=None, ldb=None, offset_a=0, offset_b=0, flags=0):
+    return dict(M=M, N=N, K=K, lda=lda or (M if flags & 8 else K), ldb=ldb or (K if flags & 16 else N), ldc=N, a=A + 2 * offset_a,
+                b=B + 2 * offset_b, out_dtype=DT, flags=flags)
+
+
+# A off 16 bytes in rows that start on 128-byte lines: on a copy its rows do not, and the K that the kernels want is another.
+COPIED_A = [_row(4096, 8192, 1000, lda=1024, offset_a=1), _row(2064, 5480, 1224, lda=1280, offset_a=1),
+            _row(2560, 5120, 3000, lda=3072, offset_a=1), _row(8192, 3072, 760, lda=768, offset_a=1),
+            _row(4096, 8192, 1000, lda=1024, offset_a=1, flags=16), _row(4096, 8192, 1001, lda=1024),
+            # ... and a transposed B that would be copied into more than 32-bit offsets reach
+            _row(300, 1100000, 1000, lda=1000, offset_a=1, flags=16)]
+
+
+def _copies_once(r):
+    rng = random.Random(7)
+    problems = COPIED_A + [_product(rng, 2 * 8192 * 8192 * 2048) for _ in range(4000)]
+    for p in problems:
+        for _ in range(2):  # (the pool's buffers grow in the first call)
+            rc, launches = r.calls("lh_hip_gemm", *_pointers(p), *_shape(p), None)
+            assert rc == 0, (p, r.lib.lh_hip_last_error())
+            written = []
+            for launch in launches:
+                copies = launch.copies
+                for _, (lo, hi) in copies:
+                    assert not any(lo < end and begin < hi for begin, end in written), f"a copy of a copy: {p}"
+                written += [dst for dst, _ in copies]
+
+
+def test_an_operand_is_copied_once(recorded):
+    """A copy of a copy is wasted, and in the library's own memory it may be the same buffer."""
+    recorded(_copies_once)
