@@ -99,3 +99,22 @@ def test_rows_off_16_bytes_and_a_k_inside_a_step(M, N, K, lda, dtype, transpose_
     need = ops.gemm_workspace_bytes(M, N, K, DTYPES[dtype], torch.float32, transpose_b=transpose_b, operands=(out, a, b, None))
     ops.gemm(a, b, out=out, transpose_b=transpose_b, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("M,N,K,offset_b", [(1, 64, 1000, 0), (4, 64, 1000, 0), (7, 512, 1048, 0), (4, 64, 1000, 1)])
+def test_few_rows_of_a_transposed_a_on_a_workspace(M, N, K, offset_b):
+    """Small products whose K ends inside a step take no memory of a caller's: the queried size is 0, and enough."""
+    from lighthouse_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a, bv = (torch.randint(-3, 4, s, device="cuda", generator=g).bfloat16() for s in ((K, M), (K, N)))
+    b = torch.zeros(offset_b + N * K, device="cuda", dtype=torch.bfloat16)[offset_b:].view((N, K) if offset_b else (K, N))
+    b.copy_(bv.T if offset_b else bv)
+    out = torch.empty((M, N), device="cuda")
+    options = {"transpose_a": True, "transpose_b": bool(offset_b)}
+    need = ops.gemm_workspace_bytes(M, N, K, torch.bfloat16, torch.float32, operands=(out, a, b, None), **options)
+    assert need == 0
+    ops.gemm(a, b, out=out, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"), **options)
+    want = a.float().T @ bv.float()
+    assert torch.equal(out, want)
+    assert torch.equal(ops.gemm(a, b, out_dtype=torch.float32, **options), want)

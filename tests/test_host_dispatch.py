@@ -86,3 +86,24 @@ def _copies_once(r):
 def test_an_operand_is_copied_once(recorded):
     """A copy of a copy is wasted, and in the library's own memory it may be the same buffer."""
     recorded(_copies_once)
+
+
+# A transposed A of fewer rows than the small-tile kernels take; B transposed off 16 bytes; K inside a step.
+FEW_ROWS = [_row(M, 64, 1000, flags=8) for M in range(1, 8)] + [_row(4, 64, 1000, offset_b=1, flags=24), _row(1, 768, 3208, flags=8),
+                                                              _row(64, 8, 4, offset_b=1, flags=16)]
+
+
+def _queried_memory(r):
+    rng = random.Random(11)
+    problems = COPIED_A + FEW_ROWS + [_product(rng, rng.choice([2 << 22, 2 * 8192 * 8192 * 512])) for _ in range(8000)]
+    for p in problems:
+        need = r.lib.lh_hip_gemm_workspace_bytes_for(*_pointers(p), *_shape(p))
+        rc, launches = r.calls("lh_hip_gemm_ws", *_pointers(p), *_shape(p), WORKSPACE if need else None, need, None)
+        assert rc == 0, (p, need, r.lib.lh_hip_last_error())
+        for launch in launches:
+            for (lo, hi), _ in launch.copies:
+                assert WORKSPACE <= lo and hi <= WORKSPACE + need, p
+
+
+def test_a_workspace_of_the_queried_size_is_enough(recorded):
+    recorded(_queried_memory)
