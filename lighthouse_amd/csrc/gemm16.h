@@ -31,10 +31,10 @@ struct Mfma16<LH_F16> {
 };
 
 // The direct kernels address a tile's operand panels with 32-bit byte offsets from the panel's
-// first element: 256 rows of A, K rows of B.
+// first element: 256 rows of A, of B the rows of whole steps of 64 (those from K on are never read, but addressed).
 static inline bool direct_offsets_fit(const GemmArgs& g) {
   if (g.flags & LH_GEMM_TRANSPOSE_B) return g.lda < (1ll << 22) && g.ldb < (1ll << 22);  // 256 rows of B^T
-  return g.lda < (1ll << 22) && (int64_t)g.K * g.ldb < (1ll << 30);
+  return g.lda < (1ll << 22) && (g.K + 63ll) / 64 * 64 * g.ldb < (1ll << 30);
 }
 
 // Every row of the result starts at a multiple of 64 bytes: stores of whole row segments cover whole 64-byte pieces of memory.

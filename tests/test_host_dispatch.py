@@ -107,3 +107,28 @@ def _queried_memory(r):
 
 def test_a_workspace_of_the_queried_size_is_enough(recorded):
     recorded(_queried_memory)
+
+
+def _offsets(r):
+    """Products whose B, with K up to the end of the last step, lies on either side of 2^30 elements."""
+    in_place = set()  # (the K's whose B was read where it is, on the near side of the limit)
+    for K in (8, 40, 72, 96, 104, 200, 328, 1000, 4104):
+        steps = (K + 63) // 64 * 64
+        strides = {n + d for n in ((1 << 30) // steps // 8 * 8, (1 << 30) // K // 8 * 8, (1 << 29) // K // 8 * 8) for d in (-8, 0, 8)}
+        for ldb in sorted(strides):
+            for N in (520, ldb):
+                rc, launches = r.calls("lh_hip_gemm", OUT, A, B, BIAS, 512, N, K, K, ldb, N, DT, DT, 0, None)
+                assert rc == 0, r.lib.lh_hip_last_error()
+                for launch in launches:
+                    if "gemm16_direct" not in launch.name:
+                        continue
+                    g = launch.gemm
+                    assert (g.K + 63) // 64 * 64 * g.ldb < 1 << 30, (K, N, ldb)
+                    if "tail" in launch.name and launch.gemm.ldb == ldb:
+                        in_place.add(K)
+    assert in_place >= {200, 328, 1000}
+
+
+def test_offsets_of_the_last_step_fit_32_bits(recorded):
+    """The loads of a step that K ends in are addressed up to the end of the step, also those that touch no memory."""
+    recorded(_offsets)
