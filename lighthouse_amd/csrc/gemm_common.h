@@ -515,8 +515,9 @@ __device__ __forceinline__ void epilogue4_any(const GemmArgs& g, int m, int n, c
 // past the caches.  256 x 256 tiles, K = 768 bf16, plain and past the caches: 8192 x 50432 654 and 563 us (main loop of a tile
 // 23.6 and 17.7), f32 797 and 763; 8192 x 16392 234 and 206; 8192 x 8200 x 2048 252 either way; fp8 8192^3 407 and 401.
 // Smaller ones, which the next kernel reads, lose as often as they gain: nanoGPT blocks of 2048 rows 88 and 93 us, of 4096
-// rows 138 and 135.5.
-static inline bool large_result(const GemmArgs& g) { return (int64_t)g.M * g.ldc * (g.out_dt == LH_F32 ? 4 : 2) >= 128000000; }
+// rows 138 and 135.5.  What counts is what is written, not the rows that it lies in: 2560 columns of a buffer of 65536, M = 4096,
+// K = 1024, and a product that reads them 53 plain and 62 past the caches.
+static inline bool large_result(const GemmArgs& g) { return (int64_t)g.M * g.N * (g.out_dt == LH_F32 ? 4 : 2) >= 128000000; }
 
 int gemm16(const GemmArgs& g, int ab_dtype, hipStream_t s);
 // Estimated time of a 16-bit product with few tiles, untransposed and aligned, not cut along K, in us.

@@ -132,3 +132,25 @@ def _offsets(r):
 def test_offsets_of_the_last_step_fit_32_bits(recorded):
     """The loads of a step that K ends in are addressed up to the end of the step, also those that touch no memory."""
     recorded(_offsets)
+
+
+def _kernel(r, *args):
+    rc, launches = r.calls(*args, None)
+    assert rc == 0 and len(launches) == 1, r.lib.lh_hip_last_error()
+    return launches[0].name
+
+
+def _large_results(r):
+    f32 = rec._lib.F32
+    past_the_caches = lambda ldc, M=4096, N=4096, out=DT: _kernel(  # noqa: E731
+        r, "lh_hip_gemm", OUT, A, B, BIAS, M, N, 4096, 4096, N, ldc, DT, out, 0).endswith("ELb1EEEvNS_8GemmArgsE")
+    assert past_the_caches(50432, 8192, 50432) and past_the_caches(8192, 8192, 8192, f32)
+    assert not past_the_caches(4096) and not past_the_caches(65536) and not past_the_caches(65536, out=f32)
+    fp8 = lambda ldc, N: _kernel(r, "lh_hip_gemm_fp8", OUT, A, B, 1.0, 1.0, 8192, N, 8192, 8192, N, ldc, DT)  # noqa: E731
+    assert "gemm8_directILb0ELb1E" in fp8(8192, 8192)
+    assert "gemm8_directILb0ELb0E" in fp8(65536, 4096)
+
+
+def test_columns_of_a_wide_buffer_are_no_large_result(recorded):
+    """What counts is what is written, not the rows that it lies in."""
+    recorded(_large_results)
