@@ -344,7 +344,7 @@ static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p,
                              const void* const* bi, int64_t N, uint32_t act) -> int {
     NormedGemm n;
     GemmArgs& g = n.g;
-    g.out = out; g.c = nullptr; g.a = xs; g.b = wi[0]; g.bias = bi[0];
+    g.out = out; g.c = nullptr; g.a = xs; g.b = nullptr; g.bias = nullptr;
     g.M = (int)rows; g.N = (int)N; g.K = (int)C;
     g.lda = C; g.ldb = N; g.ldc = groups * N;
     g.flags = bias_flag(bi[0]) | act; g.out_dt = dtype; g.bias_dt = bdt; g.alpha = 1.0f;

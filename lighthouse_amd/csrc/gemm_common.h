@@ -536,7 +536,9 @@ int gemm_small(const GemmArgs& g, int dtype, int tile, hipStream_t s);
 
 // LayerNorm of x and up to three products of its result, side by side in the output, in one launch (gemm_small_norm.hip).
 struct NormedGemm {
-  GemmArgs g;  // a: x, f32; N: columns of one product; b and bias unused
+  // a: x, f32; N: columns of one product; ldc: of all of them; flags: of every product.  Its b and bias are those of no product:
+  // the kernel puts the group's bias there.
+  GemmArgs g;
   const float *gamma, *beta;
   float eps, inv_n;
   const void* b[3];

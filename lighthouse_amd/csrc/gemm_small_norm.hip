@@ -208,6 +208,7 @@ int gemm_normed_choose(const NormedGemm& n, int dtype) {
   }
   if (tile < 0) return -1;
   GemmArgs one = g;
+  one.b = n.b[0];
   one.a = n.b[0];  // (for its alignment, which the LayerNorm's own output has as well)
   one.lda = g.K;
   const double apart = 5.25 + 1.4 * n.groups * gemm16_us(one, dtype) + 1.5 * (n.groups - 1);
