@@ -1,5 +1,6 @@
-"""LayerNorm and its projections in one launch (few rows): row and column edges of the tiles, every row width class, fused
-and separate projections, against the oracle, which has the kernels' rounding points."""
+"""LayerNorm and its projections in one launch (few rows): row and column edges of the tiles, every row width, fused and
+separate projections, against the oracle, which has the kernels' rounding points.  Which of the sizes take that launch, and on
+which of its tiles, is asserted where no GPU is needed (test_host_dispatch.py)."""
 
 import numpy as np
 import pytest
@@ -15,9 +16,18 @@ pytestmark = pytest.mark.gpu
 TOLERANCE = {"bf16": 8 * 2.0**-9, "f16": 8 * 2.0**-12}
 
 
+# A row is a multiple of 128 columns there, and up to 1024; the other widths (64, 192, 320, 704, 960) and many rows run the
+# LayerNorm and the projections one after the other.
+SIZES = [(1, 64), (15, 64), (17, 128), (33, 192), (100, 256), (250, 256), (700, 256), (31, 320), (100, 512), (16, 704), (101, 768),
+         (3, 960), (65, 1024), (128, 1024)]
+# Every width on each of the tiles of 16 x 32, 16 x 64 and 32 x 64, with those above: 128 (odd) columns are 4 (odd) steps of K,
+# which eight waves share unevenly.
+SIZES += [(340, 128), (1060, 128), (340, 256), (15, 384), (130, 384), (230, 384), (3, 512), (165, 512), (31, 640), (70, 640), (130, 640),
+          (16, 768), (60, 768), (115, 768), (2, 896), (50, 896), (100, 896), (17, 1024)]
+
+
 @pytest.mark.parametrize("mode,separate", [("bf16", False), ("f16", True)])
-@pytest.mark.parametrize("T,C", [(1, 64), (15, 64), (17, 128), (33, 192), (100, 256), (250, 256), (700, 256), (31, 320), (100, 512),
-                                 (16, 704), (101, 768), (3, 960), (65, 1024), (128, 1024)])
+@pytest.mark.parametrize("T,C", SIZES)
 def test_normed_products(T, C, mode, separate):
     from lighthouse_amd import ops
 

@@ -1,8 +1,10 @@
 """What the library's host code makes of a call, on any machine: which kernels it launches on which addresses, and what memory it
 takes.  The calls run on a recorder in the place of the HIP runtime (hip_recorder.cpp), in a process of its own."""
 
+import ctypes
 import multiprocessing
 import random
+import re
 
 import pytest
 
@@ -154,3 +156,37 @@ def _large_results(r):
 def test_columns_of_a_wide_buffer_are_no_large_result(recorded):
     """What counts is what is written, not the rows that it lies in."""
     recorded(_large_results)
+
+
+def _normed(r, sizes):
+    """The tiles (rows, columns of 16) and widths (of 128) of the launches that normalise rows and multiply them, by size and type."""
+    lib, found = rec._lib, {}
+    for T, C in sizes:
+        for dtype, separate in ((lib.BF16, False), (lib.F16, True)):
+            p = lib.NanoGPTBlockParams()
+            for i, (name, _) in enumerate(p._fields_):
+                missing = ("w_qkv", "b_qkv") if separate else ("w_q", "w_k", "w_v")
+                setattr(p, name, None if name in missing else B + (i << 32))
+            opts = lib.NanoGPTBlockOpts(0 if separate else 1, lib.ACT_RELU if separate else lib.ACT_GELU_TANH,
+                                        lib.F32 if separate else dtype, 4 * C)
+            need = r.lib.lh_hip_nanogpt_block_workspace_bytes(1, T, C, dtype, ctypes.byref(opts))
+            rc, launches = r.calls("lh_hip_nanogpt_block", OUT, A, ctypes.byref(p), 1, T, C, C // 64, 1e-5, dtype, ctypes.byref(opts),
+                                   WORKSPACE, need, None)
+            assert rc == 0, r.lib.lh_hip_last_error()
+            kernels = [re.search(r"gemm_normed_kernelILi\dELi(\d)ELi(\d)ELi8ELi(\d)E", launch.name) for launch in launches]
+            found[T, C, dtype] = [tuple(int(v) for v in k.groups()) for k in kernels if k]
+    return found
+
+
+def test_sizes_of_normed_products(recorded):
+    """The sizes that the one launch is tested at take it: every width on every tile, bf16 with one weight matrix and f16 with
+    three, and the widths that are no multiple of 128 do not."""
+    from tests.test_gpu_block_normed import SIZES
+
+    found = recorded(_normed, SIZES)
+    for (T, C, dtype), kernels in found.items():
+        assert bool(kernels) == (C % 128 == 0), (T, C)
+        assert all(width == C // 128 for _, _, width in kernels)
+    for dtype in (rec._lib.BF16, rec._lib.F16):
+        reached = {k for (_, _, d), kernels in found.items() if d == dtype for k in kernels}
+        assert reached == {(*tile, width) for tile in ((1, 2), (1, 4), (2, 4)) for width in range(1, 9)}
