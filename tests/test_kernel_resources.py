@@ -41,8 +41,9 @@ def kernels(tmp_path_factory):
 
 def test_two_128x128_gemm_workgroups_fit_a_compute_unit(kernels):
     """Eight waves each: two workgroups are four waves per SIMD, which have 128 registers each."""
-    tiles = {n: k["vgpr_count"] for n, k in kernels.items() if re.search(r"gemm16_directILi[12]ELi2ELi1E", n)}
-    assert len(tiles) == 16  # bf16 / f16, whole / edge tiles, whole / cut K, B [K, N] / [N, K]
+    tiles = {n: k["vgpr_count"] for n, k in kernels.items() if re.search(r"gemm16_direct(_tail)?ILi[12]ELi2ELi1E", n)}
+    # bf16 / f16, B [K, N] / [N, K]: whole / edge tiles by whole / cut K, and a K that ends inside a step
+    assert len(tiles) == 16 + 4 and sum("tail" in n for n in tiles) == 4
     assert {n: v for n, v in tiles.items() if v > 128} == {}
 
 
