@@ -190,3 +190,21 @@ def test_sizes_of_normed_products(recorded):
     for dtype in (rec._lib.BF16, rec._lib.F16):
         reached = {k for (_, _, d), kernels in found.items() if d == dtype for k in kernels}
         assert reached == {(*tile, width) for tile in ((1, 2), (1, 4), (2, 4)) for width in range(1, 9)}
+
+
+def _copies_that_pay(r):
+    def launches(M, N, K, offset_b=0):
+        p = _row(M, N, K, offset_b=offset_b, flags=8)
+        rc, found = r.calls("lh_hip_gemm", *_pointers(p), *_shape(p), None)
+        assert rc == 0, r.lib.lh_hip_last_error()
+        return len(found)
+
+    for M, N in ((1, 64), (4, 512), (7, 4096)):
+        assert [launches(M, N, K) for K in (8, 24, 72, 136)] == [1, 1, 1, 2]
+        assert [launches(M, N, K, 1) for K in (8, 24, 72, 136)] == [1, 1, 1, 1]
+        assert launches(M, 64, 520, 1) == 2
+
+
+def test_a_few_rows_are_untransposed_where_that_pays(recorded):
+    """Fewer rows of a transposed A than the small-tile kernels take, K inside a step: a copy and the tile kernels, or one launch."""
+    recorded(_copies_that_pay)
