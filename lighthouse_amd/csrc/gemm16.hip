@@ -408,22 +408,23 @@ static int gemm16_splitk(const GemmArgs& g, uint32_t request, hipStream_t s) {
 template <int DT>
 static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   GemmArgs g = g_in;
-  // An output side of whole 16-byte chunks: what requests ask for.  Without it, or with a K that is no multiple of 64, a small
-  // problem takes no memory of a caller's workspace, here and in a size query alike, so that it never needs one.  The library's
-  // own pool it may use where the untransposed operands then fit the direct kernels, or K is long: a transposed A of fewer rows
-  // than the small tiles take, 1 x 768 x 3200 bf16, runs 34 us on a copy and 260 on the bounds-checked kernel, which gains from
-  // one as well (B unaligned, 1 x 896 x 2560: 221 -> 171; at K = 128 it loses 2 of 14).  So it is with a K that ends inside a step,
-  // which may be so short that the copy is most of the time: 4 x 512 x 24 7.3 us as it is and 10.6 on a copy, K = 72 10.3 and 10.6,
-  // K = 136 15.3 and 10.9.
-  const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
-  const bool copy_fits = rows_fit_untransposed<2>(g), copy_pays = g.K >= 512 || copy_fits;
-  const bool may_copy = (int64_t)g.M * g.N * g.K >= (1 << 22) ||
-                        (g.K % kBK == 0 ? vec_c || (!g.ws && copy_pays) : !g.ws && copy_pays && g.K >= 128);
   // (a size query counts the copies of whole steps, the upper bound it always was)
   const int kmul = planning() ? kBK : g.k_multiple ? g.k_multiple : direct_k_multiple(g);
   // A transposed B ([N, K], k contiguous) with aligned rows goes through the direct kernels as it is
   // (its panel is loaded and read like A's); a transposed A is copied into [M, K] first.
   const bool b_in_place = (g.flags & LH_GEMM_TRANSPOSE_B) && g.ldb % 8 == 0 && aligned16(g.b) && g.K % kmul == 0;
+  // An output side of whole 16-byte chunks: what requests ask for.  Without it, or with a K that is no multiple of 64, a small
+  // problem needs no memory of a caller's workspace, here and in a size query alike (the copies of such a K are made where
+  // there is room for them).  The library's own pool it may use where the untransposed operands then fit the direct kernels, or
+  // K is long: a transposed A of fewer rows than the small tiles take, 1 x 768 x 3200 bf16, runs 34 us on a copy and 260 on the
+  // bounds-checked kernel, which gains from one as well (B unaligned, 1 x 896 x 2560: 221 -> 171; at K = 128 it loses 2 of 14).
+  // So it is with a K that ends inside a step, which may be so short that the copy is most of the time: 4 x 512 x 24 7.3 us as
+  // it is and 10.6 on a copy, K = 72 10.3 and 10.6, K = 136 15.3 and 10.9.
+  const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
+  const bool copy_fits = rows_fit_untransposed<2>(g), copy_pays = g.K >= 512 || copy_fits;
+  const bool may_copy = (int64_t)g.M * g.N * g.K >= (1 << 22) ||
+                        (g.K % kBK == 0 ? vec_c || (!g.ws && copy_pays)
+                                        : copy_pays && g.K >= 128 && (!g.ws || (vec_c && untransposed_room<2>(g, b_in_place))));
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (g.flags & LH_GEMM_SPLITK_MASK) <= LH_GEMM_SPLITK_NONE &&
       !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones.  Against them stand the direct kernels, plus

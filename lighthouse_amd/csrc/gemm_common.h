@@ -287,6 +287,21 @@ __device__ __forceinline__ void epi_store4(const GemmArgs& g, int m, int n, cons
     *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(g.out) + off) = u32x2{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3])};
 }
 
+// Memory of the copies that untranspose_operands makes; `a_bytes`: those of the copy of A, in front.
+template <int ELEM_BYTES>
+inline size_t untransposed_bytes(const GemmArgs& g, size_t* a_bytes) {
+  const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
+  *a_bytes = ta ? ((size_t)g.M * g.K * ELEM_BYTES + 255) / 256 * 256 : 0;
+  return *a_bytes + (tb ? (size_t)g.K * g.N * ELEM_BYTES : 0);
+}
+// The call's workspace has room for the copies (not in a size query, which has none); `b_in_place`: a transposed B stays.
+template <int ELEM_BYTES>
+inline bool untransposed_room(GemmArgs g, bool b_in_place) {
+  if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;
+  size_t a_bytes;
+  return g.ws->base && (g.ws->used + 255) / 256 * 256 + untransposed_bytes<ELEM_BYTES>(g, &a_bytes) <= g.ws->bytes;
+}
+
 // Transposed operands (A stored [K,M], B stored [N,K]) of a problem the direct kernels would
 // otherwise take are first transposed into temporary memory (one extra pass over that
 // operand, about a tenth of a 4096^3 problem's time) instead of running the slower kernels that
@@ -295,10 +310,10 @@ template <int ELEM_BYTES>
 inline int untranspose_operands(GemmArgs& g, int k_multiple, int n_multiple, hipStream_t s) {
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
   if (!(ta || tb) || g.K % k_multiple != 0 || g.N % n_multiple != 0) return 1;
-  const size_t a_bytes = ta ? ((size_t)g.M * g.K * ELEM_BYTES + 255) / 256 * 256 : 0;
-  const size_t b_bytes = tb ? (size_t)g.K * g.N * ELEM_BYTES : 0;
+  size_t a_bytes;
+  const size_t bytes = untransposed_bytes<ELEM_BYTES>(g, &a_bytes);
   void* taken = nullptr;
-  if (int rc = scratch_take(g.ws, s, kScratchTranspose, a_bytes + b_bytes, "gemm (transposed operands)", &taken)) return rc;
+  if (int rc = scratch_take(g.ws, s, kScratchTranspose, bytes, "gemm (transposed operands)", &taken)) return rc;
   char* buf = static_cast<char*>(taken);
   if (ta) {  // stored [K, M] -> [M, K]
     if (int rc = transpose_matrix(buf, g.a, g.K, g.M, g.lda, g.K, ELEM_BYTES, s)) return rc;

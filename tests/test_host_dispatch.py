@@ -203,6 +203,11 @@ def _copies_that_pay(r):
         assert [launches(M, N, K) for K in (8, 24, 72, 136)] == [1, 1, 1, 2]
         assert [launches(M, N, K, 1) for K in (8, 24, 72, 136)] == [1, 1, 1, 1]
         assert launches(M, 64, 520, 1) == 2
+    # ... on a caller's memory where there is room
+    p = _row(4, 512, 1000, flags=8)
+    for room, expected in ((0, 1), (7936, 1), (8192, 2), (1 << 20, 2)):
+        rc, found = r.calls("lh_hip_gemm_ws", *_pointers(p), *_shape(p), WORKSPACE, room, None)
+        assert rc == 0 and len(found) == expected, (room, r.lib.lh_hip_last_error())
 
 
 def test_a_few_rows_are_untransposed_where_that_pays(recorded):
