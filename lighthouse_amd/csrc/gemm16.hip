@@ -419,12 +419,12 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
   // K is long: a transposed A of fewer rows than the small tiles take, 1 x 768 x 3200 bf16, runs 34 us on a copy and 260 on the
   // bounds-checked kernel, which gains from one as well (B unaligned, 1 x 896 x 2560: 221 -> 171; at K = 128 it loses 2 of 14).
   // So it is with a K that ends inside a step, which may be so short that the copy is most of the time: 4 x 512 x 24 7.3 us as
-  // it is and 10.6 on a copy, K = 72 10.3 and 10.6, K = 136 15.3 and 10.9.
+  // it is and 10.6 on a copy, K = 72 10.3 and 10.6, K = 136 15.3 and 10.9; 1 x 16 x 104 12.4 and 10.9.
   const bool vec_c = g.N % 8 == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias));
   const bool copy_fits = rows_fit_untransposed<2>(g), copy_pays = g.K >= 512 || copy_fits;
   const bool may_copy = (int64_t)g.M * g.N * g.K >= (1 << 22) ||
                         (g.K % kBK == 0 ? vec_c || (!g.ws && copy_pays)
-                                        : copy_pays && g.K >= 128 && (!g.ws || (vec_c && untransposed_room<2>(g, b_in_place))));
+                                        : copy_pays && g.K >= 80 && (!g.ws || (vec_c && untransposed_room<2>(g, b_in_place))));
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && (g.flags & LH_GEMM_SPLITK_MASK) <= LH_GEMM_SPLITK_NONE &&
       !planning()) {
     // Few tiles: the small-tile kernels, if they are the faster ones.  Against them stand the direct kernels, plus

@@ -200,7 +200,7 @@ def _copies_that_pay(r):
         return len(found)
 
     for M, N in ((1, 64), (4, 512), (7, 4096)):
-        assert [launches(M, N, K) for K in (8, 24, 72, 136)] == [1, 1, 1, 2]
+        assert [launches(M, N, K) for K in (8, 24, 72, 80, 136)] == [1, 1, 1, 2, 2]
         assert [launches(M, N, K, 1) for K in (8, 24, 72, 136)] == [1, 1, 1, 1]
         assert launches(M, 64, 520, 1) == 2
     # ... on a caller's memory where there is room
