@@ -24,8 +24,9 @@ HIP_SOURCES = ["runtime.hip", "gemm16.hip", "gemm16_direct.hip", "gemm32.hip", "
 # Sources compiled more than once, with different macros: {source: {suffix of the object: macros}}.
 INSTANCES = {
     "gemm16_direct.hip": {
-        f"_{dt}_{tm}{tn}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", f"-DLH_GEMM16_TM={tm}", f"-DLH_GEMM16_TN={tn}"]
-        for dt in ("bf16", "f16") for tm, tn in ((4, 2), (4, 1), (2, 2), (2, 1), (0, 0))
+        f"_{dt}_{tm}{tn}{'_large' * large}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", f"-DLH_GEMM16_TM={tm}", f"-DLH_GEMM16_TN={tn}",
+                                             f"-DLH_GEMM16_LARGE={large}"]
+        for tm, tn, large in ((4, 2, 1), (4, 2, 0), (4, 1, 0), (2, 2, 0), (2, 1, 0), (0, 0, 0)) for dt in ("bf16", "f16")
     },
 }
 

@@ -1,6 +1,6 @@
 // Direct-to-LDS GEMM kernels for 16-bit inputs.  This source is compiled once per instantiation (the objects
 // are what takes long to build): LH_GEMM16_DT the element type, LH_GEMM16_TM and LH_GEMM16_TN the workgroup tile
-// (64 TM) x (128 TN); LH_GEMM16_TM 0: the launches cut along K.
+// (64 TM) x (128 TN); LH_GEMM16_TM 0: the launches cut along K; LH_GEMM16_LARGE 1: the launches of large results (256 x 256).
 #include <type_traits>
 
 #include "gemm16.h"
@@ -971,15 +971,20 @@ int launch_direct(const GemmArgs& g, hipStream_t s) {
       return (g.flags & LH_GEMM_TRANSPOSE_B) ? launch_direct_edge<DT, TM, TN, true, true, false, true>(g, s)
                                              : launch_direct_edge<DT, TM, TN, true, false, false, true>(g, s);
   if constexpr (TM * TN == 8)
-    if (large_result(g)) {
-      if (g.flags & LH_GEMM_TRANSPOSE_B)
-        return whole ? launch_direct_edge<DT, TM, TN, false, true, true>(g, s) : launch_direct_edge<DT, TM, TN, true, true, true>(g, s);
-      return whole ? launch_direct_edge<DT, TM, TN, false, false, true>(g, s) : launch_direct_edge<DT, TM, TN, true, false, true>(g, s);
-    }
+    if (large_result(g)) return launch_direct_large<DT>(g, whole, s);
   if (g.flags & LH_GEMM_TRANSPOSE_B)
     return whole ? launch_direct_edge<DT, TM, TN, false, true>(g, s) : launch_direct_edge<DT, TM, TN, true, true>(g, s);
   return whole ? launch_direct_edge<DT, TM, TN, false>(g, s) : launch_direct_edge<DT, TM, TN, true>(g, s);
 }
+
+#if LH_GEMM16_LARGE
+template <int DT>
+int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s) {
+  if (g.flags & LH_GEMM_TRANSPOSE_B)
+    return whole ? launch_direct_edge<DT, 4, 2, false, true, true>(g, s) : launch_direct_edge<DT, 4, 2, true, true, true>(g, s);
+  return whole ? launch_direct_edge<DT, 4, 2, false, false, true>(g, s) : launch_direct_edge<DT, 4, 2, true, false, true>(g, s);
+}
+#endif
 
 // One instantiation of the kernel with its K cut (EDGE: tiles past the end of the matrix).
 template <int DT, bool EDGE, bool BT>
@@ -1009,6 +1014,8 @@ int launch_direct_splitk(const GemmArgs& g, hipStream_t s) {
 
 #if LH_GEMM16_TM == 0
 template int launch_direct_splitk<LH_GEMM16_DT>(const GemmArgs&, hipStream_t);
+#elif LH_GEMM16_LARGE
+template int launch_direct_large<LH_GEMM16_DT>(const GemmArgs&, bool, hipStream_t);
 #else
 template int launch_direct<LH_GEMM16_DT, LH_GEMM16_TM, LH_GEMM16_TN>(const GemmArgs&, hipStream_t);
 #endif
