@@ -155,9 +155,12 @@ int lh_hip_gemm(void* out, const void* a, const void* b, const void* bias, int64
  * lh_hip_gemm with its temporary memory in a caller workspace of at least
  * lh_hip_gemm_workspace_bytes(...) bytes (0 for most problems; the query assumes 16-byte aligned
  * operands and still counts a copy of a result whose N or row stride is no multiple of 16 bytes, which no
- * kernel makes any more; lh_hip_gemm_workspace_bytes_for gives what the call takes).  No allocation happens inside the call; a workspace that is too small fails with
- * LH_ERR_INVALID.  Same role as the workspace of lh_hip_nanogpt_block for callers that manage
- * device memory themselves (GPUMemoryManager, lighthouse/execution/memory_manager.py:97-151).
+ * kernel makes any more; lh_hip_gemm_workspace_bytes_for gives what the call needs).  No allocation
+ * happens inside the call; a workspace that is too small fails with LH_ERR_INVALID.  A 16-bit product of
+ * less than 2^22 multiply-adds whose K is no multiple of 64 needs none; with a transposed A of fewer than 8
+ * rows it runs faster where there is room for copies of the transposed operands.  Same role as the workspace
+ * of lh_hip_nanogpt_block for callers that manage device memory themselves (GPUMemoryManager,
+ * lighthouse/execution/memory_manager.py:97-151).
  */
 size_t lh_hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                                    int32_t ab_dtype, int32_t out_dtype, uint32_t flags);

@@ -5,10 +5,15 @@
 //
 // With few rows each of the block's launches is a chain of latencies of a few us.  Here every workgroup of the
 // small-tile GEMM (gemm_small.hip) normalises the 16 MT rows of its tile itself: its waves request the weights of their
-// whole share of K first, normalise a few rows each while those are on their way (a wave holds its rows in registers,
-// the arithmetic is layer_norm_vec's but for the order of the sums) and leave them in LDS, from where every wave reads its operand.  The rows are
-// normalised again by every workgroup beside this one: L2 traffic and a few hundred instructions, against a launch
-// and a trip of the result through memory.  Up to three weight matrices side by side (separate q, k and v) are one launch.
+// whole share of K first, normalise a few rows each while those are on their way (a wave holds its rows in registers)
+// and leave them in LDS, from where every wave reads its operand.  The rows are normalised again by every workgroup beside
+// this one: L2 traffic and a few hundred instructions, against a launch and a trip of the result through memory.  Up to
+// three weight matrices side by side (separate q, k and v) are one launch.
+//
+// The arithmetic is that of the separate kernels but for the order of the f32 sums: a row is added up over 32 lanes (layer_norm_vec:
+// 64), and K is shared by eight waves on every tile (gemm_small.hip's 32 x 64 tile: by four).  A block of 100 rows of 768 bf16
+// differs by 1.5e-5 for it, 12 of them, where 16-bit roundings fall the other way, by 3.2e-3; the error against 64 bits is the
+// same (8 seeds each: block 8.503e-4 apart and 8.500e-4 here, 12 layers and a head 2.903e-3 and 2.901e-3).
 #include "gemm_small.h"
 
 namespace lh {

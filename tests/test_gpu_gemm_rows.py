@@ -1,5 +1,5 @@
-"""f32 results of the tile GEMM kernels in rows that do not start at multiples of 64 bytes, and launches whose workgroups
-start late."""
+"""f32 results of the tile GEMM kernels in rows that do not start at multiples of 64 bytes, launches whose workgroups start
+late, and a K that ends inside a step of 64."""
 
 import pytest
 import torch
