@@ -371,6 +371,7 @@ inline double operand_copies_us(const GemmArgs& g, int k_multiple, int n_multipl
 // the 1.6 GB result back alone took 1751 us.)
 template <int ELEM_BYTES, bool PAD_C, typename Run>
 inline int gemm_padded(const GemmArgs& g, int k_multiple, int n_multiple, hipStream_t s, Run run) {
+  if (g.k_multiple) return 1;  // (copies already; the memory of the next would be theirs)
   const bool ta = g.flags & LH_GEMM_TRANSPOSE_A, tb = g.flags & LH_GEMM_TRANSPOSE_B;
   const int out_bytes = g.out_dt == LH_F32 ? 4 : 2;
   const int Kp = (g.K + k_multiple - 1) / k_multiple * k_multiple;
