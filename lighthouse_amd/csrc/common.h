@@ -168,6 +168,52 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
   return (bid % nx) * per + bid / nx;
 }
 
+// ---- weights on their way ---------------------------------------------------------------------
+// Memory that launches after this one read, up to three ranges.  A kernel of few rows leaves CUs and most of the memory's
+// bandwidth idle; workgroups of its own behind those of the work touch 4 bytes of every 128 of it, so that the launch that
+// reads it finds it in the memory-side cache.  The launch lasts until they are done: worth it only where they have CUs to
+// themselves and the work takes longer than they do.
+int num_cus();
+struct Touch {
+  const void* p[3] = {};
+  uint32_t lines[3] = {};
+  void add(const void* range, size_t bytes) {  // (a fourth is dropped)
+    for (int i = 0; i < 3 && range && bytes < 1u << 28; ++i)
+      if (!lines[i]) {
+        p[i] = range;
+        lines[i] = (uint32_t)((bytes + 127) / 128);
+        return;
+      }
+  }
+};
+// Workgroups of 512 threads for it: 4 lines a thread.
+__host__ __device__ inline unsigned touch_blocks(uint32_t lines) { return (lines + 2047) / 2048; }
+// Behind `blocks` of the work: none where not every workgroup gets a CU.
+inline unsigned touch_blocks(const Touch& t, unsigned blocks) {
+  const unsigned n = touch_blocks(t.lines[0]) + touch_blocks(t.lines[1]) + touch_blocks(t.lines[2]);
+  return n && blocks + n <= (unsigned)num_cus() ? n : 0;
+}
+__device__ __forceinline__ void touch_lines(const Touch& t, unsigned block) {
+  const void* range = t.p[0];
+  uint32_t lines = t.lines[0];
+#pragma unroll
+  for (int i = 1; i < 3; ++i)
+    if (block >= touch_blocks(lines)) {
+      block -= touch_blocks(lines);
+      range = t.p[i];
+      lines = t.lines[i];
+    }
+  const uint8_t* const p = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(range) & ~(uintptr_t)3);
+  uint32_t v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t line = min(block * 2048 + 512 * i + threadIdx.x, lines - 1);
+    v[i] = *reinterpret_cast<const uint32_t*>(p + (size_t)line * 128);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) asm volatile("" ::"v"(v[i]));
+}
+
 hipStream_t default_stream();
 // out[c][r] = in[r][c] for an R x C matrix of 2- or 4-byte elements (row strides in elements).
 int transpose_matrix(void* out, const void* in, int R, int C, int64_t ld_in, int64_t ld_out, int elem_bytes,

@@ -30,6 +30,8 @@ struct GemmArgs {
   // The operands are copies made for kernels that want K in multiples of this (0: they are the caller's).  Decided once per
   // call: what is decided for the copies themselves may be another multiple, and a second copy would be written over the first.
   uint8_t k_multiple = 0;
+  // What launches after this one read and the small-tile kernels touch for them.
+  Touch next;
 };
 
 // Epilogue for 4 consecutive columns of one row.

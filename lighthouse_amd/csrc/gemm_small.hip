@@ -123,6 +123,10 @@ __global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
   // share its cache lines.
   const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
   const int per_xcd = (tiles_m * tiles_n + 7) / 8;
+  if ((int)blockIdx.x >= 8 * per_xcd) {
+    if constexpr (NW == 8) touch_lines(g.next, blockIdx.x - 8 * per_xcd);
+    return;
+  }
   const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (tile >= tiles_m * tiles_n) return;
   const int m0 = (tile % tiles_m) * 16 * MT, n0 = (tile / tiles_m) * 16 * NT;
@@ -162,7 +166,8 @@ static int launch_small_layout(const GemmArgs& g, hipStream_t s) {
     configured = true;
   }
   const int tiles = ((g.M + 16 * MT - 1) / (16 * MT)) * ((g.N + 16 * NT - 1) / (16 * NT));
-  LH_LAUNCH(kern, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(NW * 64), Cfg::kLdsBytes, s, g);
+  const unsigned blocks = 8 * (((unsigned)tiles + 7) / 8), touching = NW == 8 ? touch_blocks(g.next, blocks) : 0;
+  LH_LAUNCH(kern, dim3(blocks + touching), dim3(NW * 64), Cfg::kLdsBytes, s, g);
   return check_launch("gemm_small");
 }
 

@@ -57,6 +57,10 @@ __global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
   // (tiles to workgroups as in gemm_small_kernel, the groups of columns one behind the other)
   const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
   const int tiles = tiles_m * tiles_n * n.groups, per_xcd = (tiles + 7) / 8;
+  if ((int)blockIdx.x >= 8 * per_xcd) {
+    touch_lines(g.next, blockIdx.x - 8 * per_xcd);
+    return;
+  }
   const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (tile >= tiles) return;
   const int panel = tile / tiles_m, group = panel / tiles_n;
@@ -157,7 +161,9 @@ static int launch_normed_rows(const NormedGemm& n, hipStream_t s) {
     configured = true;
   }
   const int tiles = ((n.g.M + 16 * MT - 1) / (16 * MT)) * ((n.g.N + 16 * NT - 1) / (16 * NT)) * n.groups;
-  LH_LAUNCH(kern, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(NW * 64), Cfg::kLdsBytes, s, n);
+  static_assert(NW == 8, "touch_lines counts on 512 threads");
+  const unsigned blocks = 8 * (((unsigned)tiles + 7) / 8);
+  LH_LAUNCH(kern, dim3(blocks + touch_blocks(n.g.next, blocks)), dim3(NW * 64), Cfg::kLdsBytes, s, n);
   return check_launch("gemm_normed");
 }
 
