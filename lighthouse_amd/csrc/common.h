@@ -194,16 +194,15 @@ inline unsigned touch_blocks(const Touch& t, unsigned blocks) {
   return n && blocks + n <= (unsigned)num_cus() ? n : 0;
 }
 __device__ __forceinline__ void touch_lines(const Touch& t, unsigned block) {
-  const void* range = t.p[0];
-  uint32_t lines = t.lines[0];
-#pragma unroll
-  for (int i = 1; i < 3; ++i)
-    if (block >= touch_blocks(lines)) {
-      block -= touch_blocks(lines);
-      range = t.p[i];
-      lines = t.lines[i];
-    }
-  const uint8_t* const p = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(range) & ~(uintptr_t)3);
+  // (Every member is read whatever the block: choosing between them where they lie puts the kernel's arguments into scratch memory.)
+  const uint64_t p0 = reinterpret_cast<uint64_t>(t.p[0]), p1 = reinterpret_cast<uint64_t>(t.p[1]), p2 = reinterpret_cast<uint64_t>(t.p[2]);
+  const uint32_t l0 = t.lines[0], l1 = t.lines[1], l2 = t.lines[2];
+  const unsigned first1 = touch_blocks(l0), first2 = first1 + touch_blocks(l1);
+  const bool in1 = block >= first1, in2 = block >= first2;
+  const uint64_t range = in2 ? p2 : in1 ? p1 : p0;
+  const uint32_t lines = in2 ? l2 : in1 ? l1 : l0;
+  block -= in2 ? first2 : in1 ? first1 : 0;
+  const uint8_t* const p = reinterpret_cast<const uint8_t*>(range & ~3ull);
   uint32_t v[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
