@@ -27,6 +27,9 @@ INSTANCES = {
         f"_{dt}_{tm}{tn}{'_large' * large}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", f"-DLH_GEMM16_TM={tm}", f"-DLH_GEMM16_TN={tn}",
                                              f"-DLH_GEMM16_LARGE={large}"]
         for tm, tn, large in ((4, 2, 1), (4, 2, 0), (4, 1, 0), (2, 2, 0), (2, 1, 0), (0, 0, 0)) for dt in ("bf16", "f16")
+    } | {
+        f"_{dt}_odd": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", "-DLH_GEMM16_TM=2", "-DLH_GEMM16_TN=1", "-DLH_GEMM16_LARGE=0", "-DLH_GEMM16_ODD=1"]
+        for dt in ("bf16", "f16")
     },
 }
 

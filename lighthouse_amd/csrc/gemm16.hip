@@ -368,6 +368,20 @@ static int direct_k_multiple(const GemmArgs& g) {
   return whole + copies <= as_is ? kBK : 8;
 }
 
+// A B that the loads into LDS cannot take (rows that are no whole aligned 16-byte chunks) is read as it is where one round of
+// workgroups of the 128 x 128 tile covers the result: the copy in a launch of its own is a good part of such a product's time.
+// Larger ones spread it over more rows of A and have the larger tiles besides; with two workgroups on a CU and a long K the tile
+// on a copy catches up (2048 x 3999 x 4096, B in memory: 84.7 us on a copy, 85.6 as it is; one workgroup, 2000 x 2001 x 4096:
+// 49.6 and 41.4).
+static bool odd_rows_stay(const GemmArgs& g) {
+  if (planning() || g.b_padded || (g.flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK | LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B)))
+    return false;
+  if (g.N % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.b)) return false;
+  const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  return g.N >= 8 && g.K % 8 == 0 && g.lda % 8 == 0 && aligned16(g.a) && (int64_t)g.M * g.N * g.K >= (1 << 22) &&
+         (tiles <= num_cus() || (tiles <= 2 * num_cus() && g.K <= 3072)) && direct_offsets_fit(g) && splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) == 1;
+}
+
 // Decode shapes: so few 128 x 128 tiles that most CUs would idle, and a K long enough to cut.
 // Returns 1 when the problem does not qualify.
 // `request`: LH_GEMM_SPLITK_* bits of the call; an explicit 2 / 4 / 8 bypasses the criteria.
@@ -434,10 +448,12 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
                       aligned16(g.a) && aligned16(g.b);
     // (a copy has whole k-steps where kmul says so)
     const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kmul - 1) / kmul * kmul) : 1;
-    const double other = direct_us(g, cuts) + operand_copies_us<2>(g, kmul, 8, b_in_place, 0.65);
+    const bool odd_rows = odd_rows_stay(g);
+    const double other = direct_us(g, cuts) + (odd_rows ? 0.0 : operand_copies_us<2>(g, kmul, 8, b_in_place, 0.65));
     int tile;
     const double us = gemm_small_choose(g, DT, &tile);
     if (tile >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, DT, tile, s);
+    if (odd_rows) return launch_odd_rows<DT>(g, s);
   }
   if ((g.flags & LH_GEMM_TILE_MASK) == LH_GEMM_TILE_AUTO && may_copy) {
     if (b_in_place) g.flags &= ~(uint32_t)LH_GEMM_TRANSPOSE_B;

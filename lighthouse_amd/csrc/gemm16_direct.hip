@@ -1,6 +1,7 @@
 // Direct-to-LDS GEMM kernels for 16-bit inputs.  This source is compiled once per instantiation (the objects
 // are what takes long to build): LH_GEMM16_DT the element type, LH_GEMM16_TM and LH_GEMM16_TN the workgroup tile
-// (64 TM) x (128 TN); LH_GEMM16_TM 0: the launches cut along K; LH_GEMM16_LARGE 1: the launches of large results (256 x 256).
+// (64 TM) x (128 TN); LH_GEMM16_TM 0: the launches cut along K; LH_GEMM16_LARGE 1: the launches of large results (256 x 256); LH_GEMM16_ODD 1:
+// the 128 x 128 tile on a B in rows of any length.
 #include <type_traits>
 
 #include "gemm16.h"
@@ -382,11 +383,11 @@ __device__ __forceinline__ void direct_prologue(const DirectCtx<TM, TN>& c, int 
 // together.  The workgroups share out the lines; more than 128 for each cost more at the start than the loop waits for later.
 // bf16, M = 8192, N = 2304, K = 768: 45.6 us with B in memory before, 36.0 now (33.7 and 34.4 with B in the caches); N = 3072
 // 56.6 and 48.2; with 256 lines for each workgroup (2048^3) 28.1 and 29.1.
+// (The launcher decides, and the code lies behind the kernel's: in its way it cost launches that touch nothing 0.1 to 0.3 us.)
 template <bool BT>
 __device__ __forceinline__ void direct_touch_b(const GemmArgs& g, int wave, uint8_t* __restrict__ stage) {
-  const int rows = BT ? g.N : g.K, per_row = ((BT ? g.K : g.N) + 63) / 64, grid = (int)gridDim.x;
-  const int64_t lines = (int64_t)rows * per_row;
-  if (lines > 128 * grid || 64 * wave * grid >= lines || rows * g.ldb >= (1ll << 30)) return;
+  const int per_row = ((BT ? g.K : g.N) + 63) / 64, lines = (BT ? g.N : g.K) * per_row, grid = (int)gridDim.x;
+  if (64 * wave * grid >= lines) return;
   const int line = (64 * wave + lane_now()) * grid + (int)blockIdx.x;
   const int at = (line / per_row * (int)g.ldb + line % per_row * 64) * 2;
   __builtin_amdgcn_raw_ptr_buffer_load_lds(panel_resource(g.b), (lds_void_t*)(stage + 256 * wave), 4,
@@ -816,6 +817,37 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
   }
 }
 
+// Where a lane's fragments are in the stages; the wave's sub-tile starts at (wm0, wn0).
+template <int TM, int TN>
+__device__ __forceinline__ void direct_lane_reads(DirectCtx<TM, TN>& c, int wave, int lane, int wm0, int wn0) {
+  using Cfg = DirectCfg<TM, TN>;
+  const int l16 = lane & 15, g4 = lane >> 4;
+  c.wave = wave;
+  // A fragment jj (second MFMA operand): row wm0 + 16 jj + l16, logical 16-byte chunk 4 kc + g4 of
+  // the row's 8 (physical chunk: ^ ((row / 2) % 8); 4 kc only flips bit 2).
+  {
+    const int r = wm0 + l16;
+    c.a_rd[0] = r * 128 + ((g4 ^ ((r >> 1) & 7)) << 4);
+    c.a_rd[1] = c.a_rd[0] ^ 64;
+  }
+  // B fragment i (first MFMA operand) through the transposing read: the 16 lanes of group g4
+  // address k rows 8 g4 + l16 / 4 (+4 for the second read), columns wn0 + 16 i + 4 (l16 % 4) .. +4,
+  // and each receives the 4 k-values of column wn0 + 16 i + l16.
+  {
+    const int krow = 8 * g4 + (l16 >> 2);
+    const int col = wn0 + 4 * (l16 & 3);
+    c.b_chunk = col >> 3;
+    c.b_swz = (4 * (krow & 3)) ^ (2 * ((krow >> 3) & 1));
+    c.b_off = krow * Cfg::kBRow + 8 * ((col >> 2) & 1);
+  }
+  // (transposed B: row wn0 + 16 i + l16 of the stage, like the A fragment)
+  {
+    const int r = wn0 + l16;
+    c.bt_rd[0] = r * 128 + ((g4 ^ ((r >> 1) & 7)) << 4);
+    c.bt_rd[1] = c.bt_rd[0] ^ 64;
+  }
+}
+
 // Persistent workgroups: one (two for the 128 x 128 tile, whose LDS is 80 KiB) per CU, each
 // walking the tile list with the grid as stride.  Tile ids congruent modulo 8 stay on one XCD,
 // which is what xcd_remap assumes.  Launching one workgroup per tile instead costs a
@@ -851,7 +883,7 @@ __device__ __forceinline__ void direct_run(const GemmArgs& g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int WN = 4;
   const int wm0 = (wave / WN) * Cfg::WTM, wn0 = (wave % WN) * Cfg::WTN;
-  const int l16 = lane & 15, g4 = lane >> 4;
+  const int g4 = lane >> 4;
 
   // Large results, one workgroup per CU: workgroups in step store their tiles in step, and the main loops in between leave
   // the memory idle.  So some start half a tile late: those that have a tile fewer than the others where that is up to half
@@ -867,30 +899,7 @@ __device__ __forceinline__ void direct_run(const GemmArgs& g) {
   }
 
   DirectCtx<TM, TN> c;
-  c.wave = wave;
-  // A fragment jj (second MFMA operand): row wm0 + 16 jj + l16, logical 16-byte chunk 4 kc + g4 of
-  // the row's 8 (physical chunk: ^ ((row / 2) % 8); 4 kc only flips bit 2).
-  {
-    const int r = wm0 + l16;
-    c.a_rd[0] = r * 128 + ((g4 ^ ((r >> 1) & 7)) << 4);
-    c.a_rd[1] = c.a_rd[0] ^ 64;
-  }
-  // B fragment i (first MFMA operand) through the transposing read: the 16 lanes of group g4
-  // address k rows 8 g4 + l16 / 4 (+4 for the second read), columns wn0 + 16 i + 4 (l16 % 4) .. +4,
-  // and each receives the 4 k-values of column wn0 + 16 i + l16.
-  {
-    const int krow = 8 * g4 + (l16 >> 2);
-    const int col = wn0 + 4 * (l16 & 3);
-    c.b_chunk = col >> 3;
-    c.b_swz = (4 * (krow & 3)) ^ (2 * ((krow >> 3) & 1));
-    c.b_off = krow * Cfg::kBRow + 8 * ((col >> 2) & 1);
-  }
-  // (transposed B: row wn0 + 16 i + l16 of the stage, like the A fragment)
-  {
-    const int r = wn0 + l16;
-    c.bt_rd[0] = r * 128 + ((g4 ^ ((r >> 1) & 7)) << 4);
-    c.bt_rd[1] = c.bt_rd[0] ^ 64;
-  }
+  direct_lane_reads(c, wave, lane, wm0, wn0);
 
   // (even: K is a multiple of 64, or the steps from K on multiply zeros)
   const int nk = TAIL ? (g.K + 63) / 64 * 2 : g.K / 32;
@@ -902,7 +911,8 @@ __device__ __forceinline__ void direct_run(const GemmArgs& g) {
     direct_place<TM, TN, EDGE, BT>(SPLITK ? g_cur : g, xcd_remap(id, tiles1), c, m0, n0);
   }
   direct_prologue<TM, TN, TAIL, BT>(c, nk, smem_d);
-  if constexpr (!SPLITK) direct_touch_b<BT>(g, wave, smem_d + Cfg::kRingBytes);
+  if constexpr (!SPLITK)
+    if (__builtin_expect(g.touch_b, 0)) direct_touch_b<BT>(g, wave, smem_d + Cfg::kRingBytes);
   // Without EDGE every lane issues all stores of a staged epilogue.
   const bool staged = !SPLITK && g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
   const bool counted_stores = !EDGE && staged;
@@ -973,7 +983,10 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
   const int resident = num_cus() * (2 * lds <= 160 * 1024 ? 2 : 1);
   GemmArgs ga = g;
   ga.one_barrier = ntiles > num_cus();
-  LH_LAUNCH(kern, dim3(ntiles < resident ? ntiles : resident), dim3(512), lds, s, ga);
+  const int grid = ntiles < resident ? ntiles : resident;
+  const int64_t rows = BT ? g.N : g.K;
+  ga.touch_b = rows * (((BT ? g.K : g.N) + 63) / 64) <= 128 * grid && rows * g.ldb < (1ll << 30);
+  LH_LAUNCH(kern, dim3(grid), dim3(512), lds, s, ga);
   return check_launch("gemm16_direct");
 }
 
@@ -1003,6 +1016,169 @@ int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s) {
 }
 #endif
 
+#if LH_GEMM16_ODD
+// ---- B in rows of any length ------------------------------------------------------------------
+// The 128 x 128 tile on an n-contiguous B whose rows are no whole aligned 16-byte chunks (N or the row stride odd, a pointer
+// off 16 bytes), which the loads into LDS cannot take.  B comes through registers instead, 16 bytes a load at element
+// alignment, and is stored into the swizzled rows that direct_read_b expects; everything else is the kernel above with one
+// barrier per 64 k.  Pair p of steps stores what pair p - 1 requested, the 64 rows of pair p + 1, into the half of the ring that
+// pair p - 1 has left, and requests the rows of pair p + 2 at once: they have a whole pair to arrive (requested behind the barrier,
+// a quarter later, 600 x 4001 x 1600 took 29.7 us instead of 22.3).  What bounds it is the latency of the operands; against it
+// stands a copy of B in a launch of its own.  bf16, on a copy and as it is: 1000 x 4097 x 1000 25.9 and 21.1 us, B in memory
+// 28.3 and 23.8; 100 x 50257 x 768, f32 result, B in memory 51.6 and 29.5.
+struct OddRows {
+  const uint8_t* base;  // the tile's first column of B (uniform)
+  int src;              // the lane's byte offset at k = 0 of the first of its two rows of 64, the other is 32 rows on
+  int row;              // its row in them
+  int col;              // its first column of the tile, past the end of B where `over` says how far
+  int over;             // elements of the chunk that lie past the end of their row (0 .. 7)
+};
+// Rows 64 p .. of B.  LAST: those that K ends in.  Rows from K on are the last one; its chunk that crosses its end, which may be
+// that of B's memory, is read from its last 8 elements.
+template <bool LAST>
+__device__ __forceinline__ void odd_request(const GemmArgs& g, const OddRows& o, int p, u32x4 (&r)[2]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (LAST) {
+      const int k = min(64 * p + 32 * i + o.row, g.K - 1);
+      const int col = k == g.K - 1 ? o.col - (o.over ? o.over : 0) : o.col;
+      r[i] = *reinterpret_cast<const u32x4_any*>(o.base + ((int64_t)k * g.ldb + col) * 2);
+    } else {
+      r[i] = *reinterpret_cast<const u32x4_any*>(o.base + (int64_t)(64 * p + 32 * i) * g.ldb * 2 + (uint32_t)o.src);
+    }
+  }
+}
+// ... into the pair's two stages at `to`.
+template <bool LAST>
+__device__ __forceinline__ void odd_store(const GemmArgs& g, const OddRows& o, int p, u32x4 (&r)[2], int wave, uint8_t* __restrict__ to) {
+  using Cfg = DirectCfg<2, 1>;
+  const int lane = lane_now();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (LAST) {
+      const int k = 64 * p + 32 * i + o.row;
+      if (k >= g.K) {
+        r[i] = u32x4{0u, 0u, 0u, 0u};
+      } else if (k == g.K - 1 && o.over) {
+        // the chunk moved down by `over` elements
+        uint64_t lo = (uint64_t)r[i][1] << 32 | r[i][0], hi = (uint64_t)r[i][3] << 32 | r[i][2];
+        if (o.over >= 4) {
+          lo = hi;
+          hi = 0;
+        }
+        const int bits = 16 * (o.over & 3);
+        if (bits) lo = lo >> bits | hi << (64 - bits);
+        hi >>= bits;
+        r[i] = u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+      }
+    }
+    *reinterpret_cast<u32x4*>(to + i * Cfg::kBBytes + wave * 1024 + lane * 16) = r[i];
+  }
+}
+// A pair of steps (direct_step_pair_1b).  REQUEST: pair p + 2 exists, LAST_REQUEST: and K ends in it; LAST_STORE: K ends in p + 1.
+template <int DT, bool TAIL, bool REQUEST, bool LAST_REQUEST, bool LAST_STORE>
+__device__ __forceinline__ void odd_step_pair(const GemmArgs& g, const DirectCtx<2, 1>& c, const OddRows& o, u32x4 (&rows)[2],
+                                              f32x4 (&acc)[2][4], DirectFrags<2, 1>& f, const uint8_t* __restrict__ a_cur,
+                                              const uint8_t* __restrict__ a_nxt, const uint8_t* __restrict__ b1,
+                                              const uint8_t* __restrict__ b2, uint8_t* __restrict__ a_refill,
+                                              uint8_t* __restrict__ b_next, int p) {
+  direct_phase_lo<DT>(c, acc, f, a_cur, 0);
+  direct_phase_hi<DT, 2, 1, false>(c, acc, f, a_cur, b1, 1);
+  odd_store<LAST_STORE>(g, o, p + 1, rows, c.wave, b_next);
+  if constexpr (REQUEST) odd_request<LAST_REQUEST>(g, o, p + 2, rows);
+  direct_phase_lo<DT>(c, acc, f, a_cur, 1);
+  direct_wait_barrier<REQUEST ? 2 : 0>();  // (the two loads of B are the latest)
+  if constexpr (REQUEST) direct_load_a<2, 1, TAIL>(c, p + 2, a_refill);
+  direct_phase_hi<DT, 2, 1, false>(c, acc, f, a_nxt, b2, 0);
+}
+
+template <int DT, bool TAIL>
+__global__ void __launch_bounds__(512, 4) gemm16_odd_rows(GemmArgs g) {
+  using Cfg = DirectCfg<2, 1>;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem_d[];
+  const int tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave / 4) * Cfg::WTM, wn0 = (wave % 4) * Cfg::WTN;
+  DirectCtx<2, 1> c;
+  direct_lane_reads(c, wave, lane, wm0, wn0);
+  c.k_end = g.K;
+  int m0, n0;
+  direct_place<2, 1, true>(g, xcd_remap(blockIdx.x, tiles), c, m0, n0);
+  OddRows o;
+  {
+    const int chunk = lane % Cfg::kBChunks;
+    o.row = wave * Cfg::kBRowsPerLoad + lane / Cfg::kBChunks;
+    // (as direct_place has it; chunks past the end of the row are its last one)
+    const int bc = chunk ^ (4 * (o.row & 3)) ^ (2 * ((o.row >> 3) & 1));
+    o.col = min(bc * 8, (g.N - 1) / 8 * 8 - n0);
+    o.over = max(n0 + o.col + 8 - g.N, 0);
+    o.base = reinterpret_cast<const uint8_t*>(reinterpret_cast<const uint16_t*>(g.b) + n0);
+    o.src = (o.row * (int)g.ldb + o.col) * 2;
+  }
+  const int pairs = (g.K + 63) / 64, nk = 2 * pairs;
+  uint8_t* const abuf = smem_d;
+  uint8_t* const bbuf = smem_d + Cfg::kBBase;
+  auto a_stage = [&](int p) { return abuf + (p & 1) * Cfg::kABytes; };
+  auto b_pair = [&](int p) { return bbuf + (p & 1) * 2 * Cfg::kBBytes; };
+
+  u32x4 rows[2];
+  if (pairs == 1) odd_request<true>(g, o, 0, rows);
+  else odd_request<false>(g, o, 0, rows);
+  direct_load_a<2, 1, TAIL>(c, 0, abuf);
+  if (pairs == 1) odd_store<true>(g, o, 0, rows, wave, bbuf);
+  else odd_store<false>(g, o, 0, rows, wave, bbuf);
+  if (pairs > 1) {
+    if (pairs == 2) odd_request<true>(g, o, 1, rows);
+    else odd_request<false>(g, o, 1, rows);
+    direct_load_a<2, 1, TAIL>(c, 1, abuf + Cfg::kABytes);
+  }
+
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  DirectFrags<2, 1> f;
+  direct_read_a<2, 1, 0>(c, abuf, 0, f.a[0]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) f.b[i] = direct_read_b<2, 1, false>(c, bbuf, 0, i);
+  int p = 0;
+  auto pair = [&](auto request, auto last_request, auto last_store) {
+    odd_step_pair<DT, TAIL, decltype(request)::value, decltype(last_request)::value, decltype(last_store)::value>(
+        g, c, o, rows, acc, f, a_stage(p), a_stage(p + 1), b_pair(p) + Cfg::kBBytes, b_pair(p + 1), a_stage(p), b_pair(p + 1), p);
+    ++p;
+  };
+  while (p + 3 < pairs) pair(std::true_type{}, std::false_type{}, std::false_type{});
+  if (p + 2 < pairs) pair(std::true_type{}, std::true_type{}, std::false_type{});
+  if (p + 1 < pairs) pair(std::false_type{}, std::false_type{}, std::true_type{});
+  const bool staged = g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
+  u32x2 bias[2];
+  if (staged) direct_load_bias<1, true>(g, n0 + wn0 + 4 * (lane >> 4), bias);
+  direct_phase_lo<DT>(c, acc, f, a_stage(p), 0);
+  direct_phase_hi<DT, 2, 1, false>(c, acc, f, a_stage(p), b_pair(p) + Cfg::kBBytes, 1);
+  direct_phase_lo<DT>(c, acc, f, a_stage(p), 1);
+  direct_phase_hi<DT, 2, 1, false, false>(c, acc, f, a_stage(p), b_pair(p), 0);
+  direct_finish<DT, 2, 1, true, TAIL, false, false, false, false>(g, c, nk, smem_d, smem_d + Cfg::kRingBytes, acc, bias, m0, n0, wm0, wn0);
+}
+
+template <int DT>
+int launch_odd_rows(const GemmArgs& g, hipStream_t s) {
+  using Cfg = DirectCfg<2, 1>;
+  auto kern = g.K % 64 != 0 ? gemm16_odd_rows<DT, true> : gemm16_odd_rows<DT, false>;
+  static bool configured = false;
+  if (!configured && !planning()) {
+    for (auto k : {gemm16_odd_rows<DT, true>, gemm16_odd_rows<DT, false>})
+      LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::kLdsBytes));
+    configured = true;
+  }
+  const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  LH_LAUNCH(kern, dim3((unsigned)tiles), dim3(512), Cfg::kLdsBytes, s, g);
+  return check_launch("gemm16_odd_rows");
+}
+template int launch_odd_rows<LH_GEMM16_DT>(const GemmArgs&, hipStream_t);
+#endif
+
 // One instantiation of the kernel with its K cut (EDGE: tiles past the end of the matrix).
 template <int DT, bool EDGE, bool BT>
 static int launch_splitk_edge(const GemmArgs& g, hipStream_t s) {
@@ -1029,7 +1205,8 @@ int launch_direct_splitk(const GemmArgs& g, hipStream_t s) {
   return edge ? launch_splitk_edge<DT, true, false>(g, s) : launch_splitk_edge<DT, false, false>(g, s);
 }
 
-#if LH_GEMM16_TM == 0
+#if LH_GEMM16_ODD
+#elif LH_GEMM16_TM == 0
 template int launch_direct_splitk<LH_GEMM16_DT>(const GemmArgs&, hipStream_t);
 #elif LH_GEMM16_LARGE
 template int launch_direct_large<LH_GEMM16_DT>(const GemmArgs&, bool, hipStream_t);
