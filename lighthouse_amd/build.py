@@ -28,8 +28,9 @@ INSTANCES = {
                                              f"-DLH_GEMM16_LARGE={large}"]
         for tm, tn, large in ((4, 2, 1), (4, 2, 0), (4, 1, 0), (2, 2, 0), (2, 1, 0), (0, 0, 0)) for dt in ("bf16", "f16")
     } | {
-        f"_{dt}_odd": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", "-DLH_GEMM16_TM=2", "-DLH_GEMM16_TN=1", "-DLH_GEMM16_LARGE=0", "-DLH_GEMM16_ODD=1"]
-        for dt in ("bf16", "f16")
+        f"_{dt}_{kind}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", "-DLH_GEMM16_TM=2", "-DLH_GEMM16_TN=1", "-DLH_GEMM16_LARGE=0",
+                          f"-DLH_GEMM16_{kind.upper()}=1"]
+        for kind in ("odd", "deep") for dt in ("bf16", "f16")
     },
 }
 

@@ -49,6 +49,9 @@ int launch_direct(const GemmArgs& g, hipStream_t s);
 // ... of its 256 x 256 tile whose results leave past the caches; `whole`: there are no edge tiles and all sides are aligned.
 template <int DT>
 int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s);
+// The 128 x 128 tile for no more tiles than CUs.
+template <int DT>
+int launch_deep(const GemmArgs& g, bool whole, hipStream_t s);
 // The 128 x 128 tile on an n-contiguous B in rows of any length and alignment.
 template <int DT>
 int launch_odd_rows(const GemmArgs& g, hipStream_t s);

@@ -1,7 +1,7 @@
 // Direct-to-LDS GEMM kernels for 16-bit inputs.  This source is compiled once per instantiation (the objects
 // are what takes long to build): LH_GEMM16_DT the element type, LH_GEMM16_TM and LH_GEMM16_TN the workgroup tile
 // (64 TM) x (128 TN); LH_GEMM16_TM 0: the launches cut along K; LH_GEMM16_LARGE 1: the launches of large results (256 x 256); LH_GEMM16_ODD 1:
-// the 128 x 128 tile on a B in rows of any length.
+// the 128 x 128 tile on a B in rows of any length; LH_GEMM16_DEEP 1: the 128 x 128 tile where no CU gets two.
 #include <type_traits>
 
 #include "gemm16.h"
@@ -996,6 +996,8 @@ int launch_direct(const GemmArgs& g, hipStream_t s) {
   const bool whole = g.M % Cfg::BM == 0 && g.N % Cfg::BN == 0 && g.ldc % 8 == 0 && aligned16(g.out) &&
                      (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias)) &&
                      (!(g.flags & LH_GEMM_ACCUMULATE_C) || aligned16(g.c));
+  if constexpr (TM * TN == 2)
+    if ((int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) <= num_cus()) return launch_deep<DT>(g, whole, s);
   if constexpr (TM * TN < 8)
     if (g.K % 64 != 0)
       return (g.flags & LH_GEMM_TRANSPOSE_B) ? launch_direct_edge<DT, TM, TN, true, true, false, true>(g, s)
@@ -1014,6 +1016,116 @@ int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s) {
     return whole ? launch_direct_edge<DT, 4, 2, false, true, true>(g, s) : launch_direct_edge<DT, 4, 2, true, true, true>(g, s);
   return whole ? launch_direct_edge<DT, 4, 2, false, false, true>(g, s) : launch_direct_edge<DT, 4, 2, true, false, true>(g, s);
 }
+#endif
+
+#if LH_GEMM16_DEEP
+// ---- one workgroup per CU ---------------------------------------------------------------------
+// The 128 x 128 tile where no CU gets a second workgroup: nobody covers the latency of its operands, but all of the CU's LDS is its
+// own.  Both rings hold four stages of 64 k (144 KiB with the staging area), so that a stage is requested three to four pairs of
+// steps before it is read, through one barrier per pair; what two of them take, 0.9 us, is less than a line's way out of memory.
+// bf16, with two stages (and two barriers) and with four, operands in the caches / in memory: 2048^3 23.5 -> 20.5 / 28.3 -> 22.4 us,
+// on a transposed B 22.8 -> 18.8 / 30.9 -> 21.7; 512 x 8192 x 2048 21.9 -> 19.3 / 28.2 -> 22.3; 2048 x 768 x 768 with a residual 11.3 -> 9.7 /
+// 16.6 -> 13.6.
+struct DeepCfg {
+  static constexpr int kStages = 4;
+  static constexpr int kBBase = kStages * DirectCfg<2, 1>::kABytes, kBBytes = 2 * DirectCfg<2, 1>::kBBytes;  // (a stage of B: 64 k)
+  static constexpr int kRingBytes = kBBase + kStages * kBBytes;
+  static constexpr int kLdsBytes = kRingBytes + DirectCfg<2, 1>::kStageBytes;
+  static constexpr int kLoads = 4;  // of a lane per stage
+};
+template <bool BT, bool TAIL>
+__device__ __forceinline__ void deep_load(const DirectCtx<2, 1>& c, int p, uint8_t* __restrict__ abuf, uint8_t* __restrict__ bbuf) {
+  direct_load_a<2, 1, TAIL>(c, p, abuf);
+  if constexpr (BT) {
+    direct_load_b<2, 1, true, TAIL>(c, p, bbuf);
+  } else {
+    direct_load_b<2, 1, false, TAIL>(c, 2 * p, bbuf);
+    direct_load_b<2, 1, false, TAIL>(c, 2 * p + 1, bbuf + DirectCfg<2, 1>::kBBytes);
+  }
+}
+// Pair p of steps (direct_step_pair_1b), of which a successor is read next: NEWER stages behind that have been requested and may
+// be on their way.  LOAD: stage p + 4 goes where p was.
+template <int DT, bool TAIL, bool BT, int NEWER, bool LOAD>
+__device__ __forceinline__ void deep_step_pair(const DirectCtx<2, 1>& c, f32x4 (&acc)[2][4], DirectFrags<2, 1>& f,
+                                               const uint8_t* __restrict__ a_cur, const uint8_t* __restrict__ a_nxt,
+                                               const uint8_t* __restrict__ b_cur, const uint8_t* __restrict__ b_nxt,
+                                               uint8_t* __restrict__ a_refill, uint8_t* __restrict__ b_refill, int p) {
+  const uint8_t* const b1 = BT ? b_cur : b_cur + DirectCfg<2, 1>::kBBytes;
+  direct_phase_lo<DT>(c, acc, f, a_cur, 0);
+  direct_phase_hi<DT, 2, 1, BT>(c, acc, f, a_cur, b1, 1);
+  direct_phase_lo<DT>(c, acc, f, a_cur, 1);
+  direct_wait_barrier<NEWER * DeepCfg::kLoads>();
+  if constexpr (LOAD) deep_load<BT, TAIL>(c, p + 4, a_refill, b_refill);
+  direct_phase_hi<DT, 2, 1, BT>(c, acc, f, a_nxt, b_nxt, 0);
+}
+
+template <int DT, bool EDGE, bool TAIL, bool BT>
+__global__ void __launch_bounds__(512) gemm16_deep(GemmArgs g) {
+  using Cfg = DirectCfg<2, 1>;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem_d[];
+  const int tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave / 4) * Cfg::WTM, wn0 = (wave % 4) * Cfg::WTN;
+  DirectCtx<2, 1> c;
+  direct_lane_reads(c, wave, lane, wm0, wn0);
+  c.k_end = g.K;
+  int m0, n0;
+  direct_place<2, 1, EDGE, BT>(g, xcd_remap(blockIdx.x, tiles), c, m0, n0);
+  const int pairs = TAIL ? (g.K + 63) / 64 : g.K / 64;
+  auto a_stage = [&](int p) { return smem_d + (p & 3) * Cfg::kABytes; };
+  auto b_stage = [&](int p) { return smem_d + DeepCfg::kBBase + (p & 3) * DeepCfg::kBBytes; };
+#pragma unroll
+  for (int p = 0; p < DeepCfg::kStages; ++p)
+    if (p < pairs) deep_load<BT, TAIL>(c, p, a_stage(p), b_stage(p));
+
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (pairs >= 4) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * DeepCfg::kLoads) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  DirectFrags<2, 1> f;
+  direct_read_a<2, 1, 0>(c, smem_d, 0, f.a[0]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) f.b[i] = direct_read_b<2, 1, BT>(c, smem_d + DeepCfg::kBBase, 0, i);
+  int p = 0;
+  auto pair = [&](auto newer, auto load) {
+    deep_step_pair<DT, TAIL, BT, decltype(newer)::value, decltype(load)::value>(c, acc, f, a_stage(p), a_stage(p + 1), b_stage(p), b_stage(p + 1),
+                                                                               a_stage(p), b_stage(p), p);
+    ++p;
+  };
+  while (p + 4 < pairs) pair(std::integral_constant<int, 2>{}, std::true_type{});
+  if (p + 3 < pairs) pair(std::integral_constant<int, 2>{}, std::false_type{});
+  if (p + 2 < pairs) pair(std::integral_constant<int, 1>{}, std::false_type{});
+  if (p + 1 < pairs) pair(std::integral_constant<int, 0>{}, std::false_type{});
+  const bool staged = g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
+  u32x2 bias[2];
+  if (staged) direct_load_bias<1, EDGE>(g, n0 + wn0 + 4 * (lane >> 4), bias);
+  direct_phase_lo<DT>(c, acc, f, a_stage(p), 0);
+  direct_phase_hi<DT, 2, 1, BT>(c, acc, f, a_stage(p), b_stage(p) + (BT ? 0 : Cfg::kBBytes), 1);
+  direct_phase_lo<DT>(c, acc, f, a_stage(p), 1);
+  direct_phase_hi<DT, 2, 1, BT, false>(c, acc, f, a_stage(p), b_stage(p), 0);
+  direct_finish<DT, 2, 1, EDGE, TAIL, false, BT, false, false>(g, c, 2 * pairs, smem_d, smem_d + DeepCfg::kRingBytes, acc, bias, m0, n0, wm0, wn0);
+}
+
+template <int DT>
+int launch_deep(const GemmArgs& g, bool whole, hipStream_t s) {
+  static constexpr decltype(&gemm16_deep<DT, true, true, false>) kernels[2][3] = {
+      {gemm16_deep<DT, false, false, false>, gemm16_deep<DT, true, false, false>, gemm16_deep<DT, true, true, false>},
+      {gemm16_deep<DT, false, false, true>, gemm16_deep<DT, true, false, true>, gemm16_deep<DT, true, true, true>}};
+  static bool configured = false;
+  if (!configured && !planning()) {
+    for (auto& layout : kernels)
+      for (auto k : layout)
+        LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, DeepCfg::kLdsBytes));
+    configured = true;
+  }
+  auto kern = kernels[(g.flags & LH_GEMM_TRANSPOSE_B) ? 1 : 0][g.K % 64 != 0 ? 2 : whole ? 0 : 1];
+  LH_LAUNCH(kern, dim3((unsigned)(((g.M + 127) / 128) * ((g.N + 127) / 128))), dim3(512), DeepCfg::kLdsBytes, s, g);
+  return check_launch("gemm16_deep");
+}
+template int launch_deep<LH_GEMM16_DT>(const GemmArgs&, bool, hipStream_t);
 #endif
 
 #if LH_GEMM16_ODD
@@ -1205,7 +1317,7 @@ int launch_direct_splitk(const GemmArgs& g, hipStream_t s) {
   return edge ? launch_splitk_edge<DT, true, false>(g, s) : launch_splitk_edge<DT, false, false>(g, s);
 }
 
-#if LH_GEMM16_ODD
+#if LH_GEMM16_ODD || LH_GEMM16_DEEP
 #elif LH_GEMM16_TM == 0
 template int launch_direct_splitk<LH_GEMM16_DT>(const GemmArgs&, hipStream_t);
 #elif LH_GEMM16_LARGE
