@@ -28,9 +28,9 @@ INSTANCES = {
                                              f"-DLH_GEMM16_LARGE={large}"]
         for tm, tn, large in ((4, 2, 1), (4, 2, 0), (4, 1, 0), (2, 2, 0), (2, 1, 0), (0, 0, 0)) for dt in ("bf16", "f16")
     } | {
-        f"_{dt}_{kind}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", "-DLH_GEMM16_TM=2", "-DLH_GEMM16_TN=1", "-DLH_GEMM16_LARGE=0",
-                          f"-DLH_GEMM16_{kind.upper()}=1"]
-        for kind in ("odd", "deep") for dt in ("bf16", "f16")
+        f"_{dt}_{kind}_{tm}{tn}": [f"-DLH_GEMM16_DT=LH_{dt.upper()}", f"-DLH_GEMM16_TM={tm}", f"-DLH_GEMM16_TN={tn}", "-DLH_GEMM16_LARGE=0",
+                                   f"-DLH_GEMM16_{kind.upper()}=1"]
+        for kind, tm, tn in (("odd", 2, 1), ("deep", 2, 1), ("deep", 2, 3), ("deep", 2, 2), ("deep", 4, 1)) for dt in ("bf16", "f16")
     },
 }
 

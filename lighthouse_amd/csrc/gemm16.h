@@ -42,6 +42,12 @@ __host__ __device__ static inline bool rows_of_pieces(const GemmArgs& g) {
   return ((reinterpret_cast<uintptr_t>(g.out) | (uintptr_t)(g.ldc * (g.out_dt == LH_F32 ? 4 : 2))) & 63) == 0;
 }
 
+// Tiles of bm x bn cover the result exactly, and all of its sides are aligned.
+static inline bool whole_tiles(const GemmArgs& g, int bm, int bn) {
+  return g.M % bm == 0 && g.N % bn == 0 && g.ldc % 8 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias)) &&
+         (!(g.flags & LH_GEMM_ACCUMULATE_C) || aligned16(g.c));
+}
+
 // Launch of the direct-to-LDS kernel with a workgroup tile of (64 TM) x (128 TN) (gemm16_direct.hip; each
 // combination is an object of its own).
 template <int DT, int TM, int TN>
@@ -49,9 +55,9 @@ int launch_direct(const GemmArgs& g, hipStream_t s);
 // ... of its 256 x 256 tile whose results leave past the caches; `whole`: there are no edge tiles and all sides are aligned.
 template <int DT>
 int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s);
-// The 128 x 128 tile for no more tiles than CUs.
-template <int DT>
-int launch_deep(const GemmArgs& g, bool whole, hipStream_t s);
+// ... with deeper rings, for no more tiles than CUs: 128 x 128, 128 x 192 (TN 3; K a multiple of 64), 128 x 256 and 256 x 128.
+template <int DT, int TM, int TN>
+int launch_deep(const GemmArgs& g, hipStream_t s);
 // The 128 x 128 tile on an n-contiguous B in rows of any length and alignment.
 template <int DT>
 int launch_odd_rows(const GemmArgs& g, hipStream_t s);

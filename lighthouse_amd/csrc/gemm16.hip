@@ -243,39 +243,57 @@ static int launch_fast(const GemmArgs& g, hipStream_t s) {
   return check_launch("gemm16_fast");
 }
 
-// Tile choice for the direct kernels: 0 = 256 x 256, 1 = 256 x 128, 2 = 128 x 256, 3 = 128 x 128.
-// Time of a launch, in us and apart from what all four share: rounds of resident workgroups (edge tiles count in full)
+// Tile choice for the direct kernels: 0 = 256 x 256, 1 = 256 x 128, 2 = 128 x 256, 3 = 128 x 128, 4 = 128 x 192.
+// Time of a launch, in us and apart from what all share: rounds of resident workgroups (edge tiles count in full)
 // times a tile's a + b K, where a is what its output costs and b K the main loop.  The 128 x 128 tile has two workgroups
-// on a CU; alone on it (no CU gets a second one) a workgroup's loop takes 0.6 of the pair's and its output 0.7.  A last
-// round that does not fill the CUs costs less than a full one: the persistent workgroups are not in step, so the
+// on a CU.  A last round that does not fill the CUs costs less than a full one: the persistent workgroups are not in step, so the
 // extra tiles run while others still finish, and fewer busy CUs hold a higher clock.  Of a round, a fraction r costs
-// part + (1 - part) r^2 (the 128 x 128 tile: r).  Least squares over 1870 problems on each of the four tiles (M 128 ... 8192,
+// part + (1 - part) r^2 (the 128 x 128 tile: r).  Least squares over 1870 problems on each of the first four tiles (M 128 ... 8192,
 // N 512 ... 50256, K 256 ... 4096); what is chosen is within 0.9 % of the best tile on average, 1.24 x at worst (the rule
 // before it, which priced a tile by its flops, 2.4 to 5.0 %, 1.67 x).
-// `whole_k`: K is a multiple of 64; else the 256 x 256 tile is left out.  `time`: the estimate.
+// Where no CU gets a second workgroup all but the 256 x 256 tile, which fills the LDS as it is, run with deeper rings
+// (gemm16_deep), and 128 x 192 for nothing else; `alone`, fitted to 4096 x 2048, 4096 x 1536, 2048 x 2048 and 8192 x 768 over K = 512 ... 4096.
+// bf16, what was chosen without and with it, operands in the caches / in memory: 8192 x 768 x 3072 with a residual 43.6 -> 40.1 /
+// 56.8 -> 49.2 us (128 x 192), K = 768 19.7 -> 18.7 / 27.2 -> 24.9, 4096 x 1536 x 2048 29.0 -> 26.5 / 34.0 -> 30.2, 4096 x 2048 x 2048 33.1 -> 32.3 /
+// 39.2 -> 35.2 (256 x 128), with f32 results 34.2 -> 33.7 / 46.8 -> 38.5 (128 x 256).
+// `whole_k`: K is a multiple of 64; else the 256 x 256 and 128 x 192 tiles are left out.  `time`: the estimate.
 struct DirectTile {
   int bm, bn;
   double b, part;
   double a[4];  // 16-bit result; f32 in rows of whole 64-byte pieces; other f32; accumulator input
 };
+static constexpr DirectTile kDirectTiles[5] = {
+    {256, 256, 0.0244, 0.69, {6.5, 9.6, 12.9, 20.5}},
+    {256, 128, 0.0141, 0.72, {4.4, 6.4, 7.5, 11.3}},
+    {128, 256, 0.0138, 0.77, {4.1, 5.9, 7.4, 10.9}},
+    {128, 128, 0.0136, 0.47, {4.1, 6.4, 6.8, 9.6}},
+    {128, 192},
+};
+static constexpr DirectTile kDirectAlone[5] = {
+    kDirectTiles[0],
+    {256, 128, 0.0131, 0.80, {4.3, 6.2, 7.3, 13.0}},
+    {128, 256, 0.0128, 0.80, {5.1, 6.4, 7.9, 10.5}},
+    {128, 128, 0.0077, 1.00, {2.9, 4.5, 4.8, 6.7}},
+    {128, 192, 0.0103, 0.80, {4.2, 5.7, 9.0, 9.3}},
+};
+static int64_t direct_tiles(const GemmArgs& g, int v) {
+  const DirectTile& t = kDirectTiles[v];
+  return (int64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
+}
 static int direct_variant(const GemmArgs& g, bool whole_k, double* time) {
-  static constexpr DirectTile tiles[4] = {
-      {256, 256, 0.0244, 0.69, {6.5, 9.6, 12.9, 20.5}},
-      {256, 128, 0.0141, 0.72, {4.4, 6.4, 7.5, 11.3}},
-      {128, 256, 0.0138, 0.77, {4.1, 5.9, 7.4, 10.9}},
-      {128, 128, 0.0136, 0.47, {4.1, 6.4, 6.8, 9.6}},
-  };
   const int out = (g.flags & LH_GEMM_ACCUMULATE_C) ? 3 : g.out_dt != LH_F32 ? 0 : rows_of_pieces(g) ? 1 : 2;
   const int cus = num_cus();
   int best = -1;
   double best_us = 0.0;
-  for (int v = whole_k ? 0 : 1; v < 4; ++v) {
-    const DirectTile& t = tiles[v];
-    const int64_t n = (int64_t)((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
-    const int slots = v < 3 ? cus : 2 * cus;
+  for (int v = whole_k ? 0 : 1; v < (whole_k ? 5 : 4); ++v) {
+    const int64_t n = direct_tiles(g, v);
+    const bool alone = n <= cus;
+    if (v == 4 && !alone) continue;
+    const DirectTile& t = alone ? kDirectAlone[v] : kDirectTiles[v];
+    const int slots = v == 3 && !alone ? 2 * cus : cus;
     const double r = (double)(n % slots) / slots;
-    const double rounds = (double)(n / slots) + (r > 0.0 ? t.part + (1.0 - t.part) * (v < 3 ? r * r : r) : 0.0);
-    const double us = v == 3 && n <= cus ? 0.7 * t.a[out] + 0.0082 * g.K : rounds * (t.a[out] + t.b * g.K);
+    const double rounds = (double)(n / slots) + (r > 0.0 ? t.part + (1.0 - t.part) * (slots == cus ? r * r : r) : 0.0);
+    const double us = rounds * (t.a[out] + t.b * g.K);
     if (best < 0 || us < best_us) {
       best = v;
       best_us = us;
@@ -411,7 +429,6 @@ static int gemm16_splitk(const GemmArgs& g, uint32_t request, hipStream_t s) {
   p.out_dt = LH_F32;
   p.bias = nullptr;
   p.flags = g.flags & LH_GEMM_TRANSPOSE_B;
-  p.one_barrier = 0;  // B is streamed from memory here: the deeper look-ahead wins (M = 16, N = K = 8192: 26.7 against 27.4 us)
   if (int rc = launch_direct_splitk<DT>(p, s)) return rc;
   const int64_t groups = (int64_t)g.M * splitk_row(g.N) / 4;
   const int rb = reduce_block(groups);
@@ -494,9 +511,11 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
     double us;
     const int v = tile != LH_GEMM_TILE_AUTO ? (int)(tile >> 8) - 1 : direct_variant(g, g.K % kBK == 0, &us);
     if (v == 0) return launch_direct<DT, 4, 2>(g, s);
-    if (v == 1) return launch_direct<DT, 4, 1>(g, s);
-    if (v == 2) return launch_direct<DT, 2, 2>(g, s);
-    if (v == 3) return launch_direct<DT, 2, 1>(g, s);
+    const bool deep = direct_tiles(g, v) <= num_cus();
+    if (v == 1) return deep ? launch_deep<DT, 4, 1>(g, s) : launch_direct<DT, 4, 1>(g, s);
+    if (v == 2) return deep ? launch_deep<DT, 2, 2>(g, s) : launch_direct<DT, 2, 2>(g, s);
+    if (v == 3) return deep ? launch_deep<DT, 2, 1>(g, s) : launch_direct<DT, 2, 1>(g, s);
+    if (v == 4) return launch_deep<DT, 2, 3>(g, s);
   }
   if (operands_ok && g.ldc % 4 == 0 && aligned16(g.out) && (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias))) {
     // (B as it is stored, also where the direct kernels would have read a transposed one in place but a row stride

@@ -31,24 +31,32 @@ constexpr int kBK = 64;
 // last MFMA that uses its predecessor), so reads always overlap MFMAs.  The barrier sits between
 // the two phases of a step and the buffers a step has finished reading are refilled right
 // behind it (B: 3 stages ahead, A: on odd steps, one 64-k stage ahead).
-// The large tiles (and the 128 x 128 tile when workgroups share a compute unit) run a second form
-// with one barrier per 64 k, the rings as two halves: direct_step_pair_1b.
+// That is the form of the launches cut along K; the others run one with a single barrier per 64 k, the rings as two
+// halves: direct_step_pair_1b.  Where no CU gets a second workgroup, rings of three or four such halves: gemm16_deep.
 //
 // A wave-wide load into LDS writes 64 x 16 contiguous LDS bytes, so rows cannot be padded;
 // bank conflicts are avoided by XOR-swizzling which 16-byte chunk of a row each lane fetches
 // (A: chunk ^ ((row / 2) % 8); B: chunk ^ 4 (k % 4) ^ 2 ((k / 8) % 2)).
+// TN 3 stands for 192 columns (gemm16_deep alone): three fragments of 16 columns for each of the four waves side by side.
+constexpr int direct_frags(int TN) { return TN == 3 ? 3 : 2 * TN; }
 template <int TM, int TN>
 struct DirectCfg {
-  static constexpr int BM = 64 * TM, BN = 128 * TN;
-  static constexpr int WTM = 32 * TM, WTN = 32 * TN;      // per-wave sub-tile
+  static constexpr int NF = direct_frags(TN);             // 16-column fragments of a wave
+  static constexpr int BM = 64 * TM, BN = 64 * NF;
+  static constexpr int WTM = 32 * TM, WTN = 16 * NF;      // per-wave sub-tile
   static constexpr int kABytes = BM * 64 * 2;             // one A stage (64 k)
   static constexpr int kBRow = BN * 2;                    // bytes of one k row of a B stage
   static constexpr int kBBytes = 32 * kBRow;              // one B stage (32 k)
   static constexpr int kBtBytes = BN * 64 * 2;            // one stage (64 k) of a transposed B: rows n, like A
+  // What the 16-byte chunks of k row `k` of an n-contiguous B are swapped with.  Rows of a multiple of 256 bytes start at the same
+  // bank; of the rows of 384 bytes every other one starts half way through the banks.
+  __device__ static constexpr int b_swizzle(int k) {
+    return TN == 3 ? (4 * ((k >> 1) & 1)) ^ (2 * ((k >> 3) & 1)) : (4 * (k & 3)) ^ (2 * ((k >> 3) & 1));
+  }
   static constexpr int kBBase = 2 * kABytes;
   static constexpr int kRingBytes = kBBase + 4 * kBBytes;
   static constexpr int kStageBytes = 8 * 32 * WTN * 2;    // output staging: 32 rows of each wave's sub-tile
-  static constexpr int kStagedStores = 2 * TM * TN;       // 16-byte stores per lane of a staged epilogue
+  static constexpr int kStagedStores = TM * NF;           // 16-byte stores per lane of a staged epilogue
   static constexpr int kLdsBytes = kRingBytes + kStageBytes;
   static constexpr int kBChunks = kBRow / 16;             // 16-byte chunks per B row
   static constexpr int kBRowsPerLoad = 1024 / kBRow;      // k rows one wave-wide load covers
@@ -98,7 +106,7 @@ struct DirectCtx {
   int wave, b_off, b_chunk, b_swz;
   int k_end;                  // (TAIL) K: loads past it bring zeros
   // B stored transposed ([N, K], k contiguous): its panel is laid out, loaded and read like A's
-  int bt_src[2 * TN];         // lane's byte offset in the B^T panel for load i at k = 0
+  int bt_src[direct_frags(TN)];         // lane's byte offset in the B^T panel for load i at k = 0
   int bt_rd[2];               // like a_rd, for row wn0 + lane % 16 of a B^T stage
 };
 
@@ -107,7 +115,7 @@ struct DirectCtx {
 template <int TM, int TN>
 struct DirectFrags {
   u32x4 a[2][TM];
-  u32x4 b[2 * TN];
+  u32x4 b[direct_frags(TN)];
 };
 
 // The lane's 16-byte chunk of a 128-byte row of a k-contiguous stage lies past the end of K (of which `left` remain at the
@@ -129,7 +137,7 @@ __device__ __forceinline__ void direct_load_a(const DirectCtx<TM, TN>& c, int sa
 #pragma unroll
   for (int i = 0; i < TM; ++i) dma16(rsrc, c.a_src[i], sa * 128, abuf + (8 * i + c.wave) * 1024);
 }
-// B stage `sb` (k = 32 sb .. +32): TN loads per lane.  BT (B stored [N, K]): stage sb is k = 64 sb .. +64
+// B stage `sb` (k = 32 sb .. +32; 192 columns: 64 sb .. +64, TAIL not): TN loads per lane.  BT (B stored [N, K]): stage sb is k = 64 sb .. +64
 // of the panel's rows, 2 TN loads per lane.
 template <int TM, int TN, bool BT, bool TAIL>
 __device__ __forceinline__ void direct_load_b(const DirectCtx<TM, TN>& c, int sb, uint8_t* __restrict__ bbuf) {
@@ -138,12 +146,13 @@ __device__ __forceinline__ void direct_load_b(const DirectCtx<TM, TN>& c, int sb
     if (TAIL && 64 * sb + 64 > c.k_end) {
       const bool past = direct_past_k(c.wave, c.k_end - 64 * sb);
 #pragma unroll
-      for (int i = 0; i < 2 * TN; ++i) dma16(rsrc, past ? (int)kOutside : c.bt_src[i], sb * 128, bbuf + (8 * i + c.wave) * 1024);
+      for (int i = 0; i < direct_frags(TN); ++i) dma16(rsrc, past ? (int)kOutside : c.bt_src[i], sb * 128, bbuf + (8 * i + c.wave) * 1024);
       return;
     }
 #pragma unroll
-    for (int i = 0; i < 2 * TN; ++i) dma16(rsrc, c.bt_src[i], sb * 128, bbuf + (8 * i + c.wave) * 1024);
+    for (int i = 0; i < direct_frags(TN); ++i) dma16(rsrc, c.bt_src[i], sb * 128, bbuf + (8 * i + c.wave) * 1024);
   } else {
+    static_assert(!TAIL || TN != 3, "whole stages");
     if (TAIL && 32 * sb + 32 > c.k_end) {
       using Cfg = DirectCfg<TM, TN>;
       const int lane = lane_now();
@@ -155,7 +164,7 @@ __device__ __forceinline__ void direct_load_b(const DirectCtx<TM, TN>& c, int sb
       return;
     }
 #pragma unroll
-    for (int i = 0; i < TN; ++i) dma16(rsrc, c.b_src[i], sb * c.b_step, bbuf + (8 * i + c.wave) * 1024);
+    for (int i = 0; i < TN; ++i) dma16(rsrc, c.b_src[i], (TN == 3 ? 2 * sb : sb) * c.b_step, bbuf + (8 * i + c.wave) * 1024);
   }
 }
 
@@ -196,35 +205,35 @@ __device__ __forceinline__ void direct_interleave_step() {
 // First phase of a step: the MFMAs of the lower row fragments (f.a[0]) against the step's B
 // fragments, under the reads of the same step's upper row fragments (32 k `kc` of stage `as`).
 template <int DT, int TM, int TN>
-__device__ __forceinline__ void direct_phase_lo(const DirectCtx<TM, TN>& c, f32x4 (&acc)[2 * TN][2 * TM],
+__device__ __forceinline__ void direct_phase_lo(const DirectCtx<TM, TN>& c, f32x4 (&acc)[direct_frags(TN)][2 * TM],
                                                 DirectFrags<TM, TN>& f, const uint8_t* __restrict__ as, int kc) {
   direct_read_a<TM, TN, 1>(c, as, kc, f.a[1]);
 #pragma unroll
-  for (int i = 0; i < 2 * TN; ++i)
+  for (int i = 0; i < direct_frags(TN); ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][j] = Mfma16<DT>::mma16(f.b[i], f.a[0][j], acc[i][j]);
-  direct_interleave_step<0, 2 * TN * TM, TM>();
+  direct_interleave_step<0, direct_frags(TN) * TM, TM>();
 }
 // Second phase: the MFMAs of the upper row fragments (f.a[1]) under the reads of the NEXT step's
 // lower row fragments (32 k `kc_n` of A stage `as_n`) and B fragments (stage `bs_n`; BT: its 32 k
 // `kc_n`), each B fragment requested behind the last MFMA that uses the one it replaces.
 // LOAD false: the tile's last step, nothing left to read.
 template <int DT, int TM, int TN, bool BT, bool LOAD = true>
-__device__ __forceinline__ void direct_phase_hi(const DirectCtx<TM, TN>& c, f32x4 (&acc)[2 * TN][2 * TM],
+__device__ __forceinline__ void direct_phase_hi(const DirectCtx<TM, TN>& c, f32x4 (&acc)[direct_frags(TN)][2 * TM],
                                                 DirectFrags<TM, TN>& f, const uint8_t* __restrict__ as_n,
                                                 const uint8_t* __restrict__ bs_n, int kc_n) {
   if constexpr (LOAD) direct_read_a<TM, TN, 0>(c, as_n, kc_n, f.a[0]);
-  u32x4 bn[2 * TN];
+  u32x4 bn[direct_frags(TN)];
 #pragma unroll
-  for (int i = 0; i < 2 * TN; ++i) {
+  for (int i = 0; i < direct_frags(TN); ++i) {
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][TM + j] = Mfma16<DT>::mma16(f.b[i], f.a[1][j], acc[i][TM + j]);
     if constexpr (LOAD) bn[i] = direct_read_b<TM, TN, BT>(c, bs_n, kc_n, i);
   }
   if constexpr (LOAD) {
 #pragma unroll
-    for (int i = 0; i < 2 * TN; ++i) f.b[i] = bn[i];
-    direct_interleave_step<0, 2 * TN * TM, TM + (BT ? 2 : 4) * TN>();
+    for (int i = 0; i < direct_frags(TN); ++i) f.b[i] = bn[i];
+    direct_interleave_step<0, direct_frags(TN) * TM, TM + (BT ? 1 : 2) * direct_frags(TN)>();
   }
 }
 // Wait until at most N of this wave's loads are still in flight and all its LDS reads have
@@ -248,7 +257,7 @@ __device__ __forceinline__ void direct_wait_barrier() {
 //   odd step : [B(kt+1)] [A((kt+1)/2) B(kt+2)] [B(kt+3)]        -> A needed: 2 TN may remain
 // Near the end loads are no longer issued and the waits become full waits.
 template <int DT, int TM, int TN, bool TAIL>
-__device__ __forceinline__ void direct_step_pair(const DirectCtx<TM, TN>& c, f32x4 (&acc)[2 * TN][2 * TM],
+__device__ __forceinline__ void direct_step_pair(const DirectCtx<TM, TN>& c, f32x4 (&acc)[direct_frags(TN)][2 * TM],
                                                  DirectFrags<TM, TN>& f, const uint8_t* __restrict__ a_cur,
                                                  const uint8_t* __restrict__ a_nxt, const uint8_t* __restrict__ b1,
                                                  const uint8_t* __restrict__ b2, uint8_t* __restrict__ a_refill,
@@ -312,7 +321,7 @@ __device__ __forceinline__ void direct_place(const GemmArgs& g, int id, DirectCt
   if constexpr (BT) {
     // B^T: exactly A's scheme on the panel's BN rows (row n of B^T = column n of B)
 #pragma unroll
-    for (int i = 0; i < 2 * TN; ++i) {
+    for (int i = 0; i < direct_frags(TN); ++i) {
       const int br = (8 * i + c.wave) * 8 + (lane >> 3);
       const int bc = (lane & 7) ^ ((br >> 1) & 7);
       const int brow = EDGE ? min(br, g.N - 1 - n0) : br;
@@ -321,8 +330,9 @@ __device__ __forceinline__ void direct_place(const GemmArgs& g, int id, DirectCt
   } else {
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
-      const int bk = (8 * i + c.wave) * Cfg::kBRowsPerLoad + lane / Cfg::kBChunks;
-      const int bc = (lane % Cfg::kBChunks) ^ (4 * (bk & 3)) ^ (2 * ((bk >> 3) & 1));
+      // (192 columns: i = 0 .. 2 are the two stages of 64 k rows, 24 chunks each, one behind the other)
+      const int chunk = (8 * i + c.wave) * 64 + lane, bk = chunk / Cfg::kBChunks;
+      const int bc = chunk % Cfg::kBChunks ^ Cfg::b_swizzle(bk);
       const int bcol = EDGE ? min(bc * 8, (g.N + 7) / 8 * 8 - 8 - n0) : bc * 8;  // column within the panel
       c.b_src[i] = (bk * ldb + bcol) * 2;
     }
@@ -334,7 +344,7 @@ __device__ __forceinline__ void direct_place(const GemmArgs& g, int id, DirectCt
 // stages (issued at the previous barrier, 64 k ago) are awaited in full; the pair after that is
 // then requested into this pair's buffers.  BT: b1 is the pair's one 64-k stage of B^T, b2 the next.
 template <int DT, int TM, int TN, bool TAIL, bool BT = false>
-__device__ __forceinline__ void direct_step_pair_1b(const DirectCtx<TM, TN>& c, f32x4 (&acc)[2 * TN][2 * TM],
+__device__ __forceinline__ void direct_step_pair_1b(const DirectCtx<TM, TN>& c, f32x4 (&acc)[direct_frags(TN)][2 * TM],
                                                     DirectFrags<TM, TN>& f, const uint8_t* __restrict__ a_cur,
                                                     const uint8_t* __restrict__ a_nxt, const uint8_t* __restrict__ b1,
                                                     const uint8_t* __restrict__ b2, uint8_t* __restrict__ a_refill,
@@ -397,12 +407,12 @@ __device__ __forceinline__ void direct_touch_b(const GemmArgs& g, int wave, uint
 // The lane's 16-bit bias values for a staged epilogue, columns n_base + 16 i .. +4, as packed
 // pairs; all loads are issued back to back.  (An f32 bias is read by the epilogue itself.)
 template <int TN, bool EDGE>
-__device__ __forceinline__ void direct_load_bias(const GemmArgs& g, int n_base, u32x2 (&bias)[2 * TN]) {
+__device__ __forceinline__ void direct_load_bias(const GemmArgs& g, int n_base, u32x2 (&bias)[direct_frags(TN)]) {
 #pragma unroll
-  for (int i = 0; i < 2 * TN; ++i) bias[i] = u32x2{0u, 0u};
+  for (int i = 0; i < direct_frags(TN); ++i) bias[i] = u32x2{0u, 0u};
   if (!(g.flags & LH_GEMM_HAS_BIAS) || g.bias_dt == LH_F32) return;
 #pragma unroll
-  for (int i = 0; i < 2 * TN; ++i) {
+  for (int i = 0; i < direct_frags(TN); ++i) {
     const int n = n_base + 16 * i;
     const uint16_t* b = reinterpret_cast<const uint16_t*>(g.bias);
     if constexpr (EDGE) {
@@ -425,18 +435,17 @@ __device__ __forceinline__ void direct_load_bias(const GemmArgs& g, int n_base, 
 // those stores may stay in flight.
 // `staged`: the epilogue will want `bias` (for columns from n_base); it is loaded ahead of the
 // last two steps, whose full wait covers it.
-template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool BT>
+template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool BT, bool SPLITK>
 __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectCtx<TM, TN>& c,
-                                                f32x4 (&acc)[2 * TN][2 * TM], uint8_t* smem_d, int nk,
-                                                bool stores_behind, bool staged, int n_base, u32x2 (&bias)[2 * TN]) {
+                                                f32x4 (&acc)[direct_frags(TN)][2 * TM], uint8_t* smem_d, int nk,
+                                                bool stores_behind, bool staged, int n_base, u32x2 (&bias)[direct_frags(TN)]) {
   using Cfg = DirectCfg<TM, TN>;
-  // One barrier per 64 k (loads one 64-k half of the rings ahead) or two (B three 32-k stages
-  // ahead).  One is 1-3 % faster for every tile with a 256 side (4096^3 109.8 -> 108.3 us) and, when
-  // two workgroups share a compute unit, 2-7 % for the 128 x 128 tile (M = 8192, N = 768, K = 3072:
-  // 46.0 -> 42.9 us); a lone 128 x 128 workgroup has nobody to cover the shorter look-ahead
-  // (2048^3 22.7 -> 24.2 us) and keeps two.
+  // One barrier per 64 k (loads one 64-k half of the rings ahead) or, where K is cut, two (B three 32-k stages
+  // ahead): there B is streamed from memory and the deeper look-ahead wins (M = 16, N = K = 8192: 26.7 against 27.4 us).
+  // One is 1-3 % faster for every tile with a 256 side (4096^3 109.8 -> 108.3 us) and 2-7 % for two 128 x 128 workgroups on a
+  // CU (M = 8192, N = 768, K = 3072: 46.0 -> 42.9 us).
   // A transposed B lives in the rings as two 64-k stages like A and always takes the one-barrier form.
-  const bool one_barrier = BT || TM * TN > 2 || g.one_barrier;
+  constexpr bool one_barrier = BT || !SPLITK;
   uint8_t* const abuf = smem_d;
   uint8_t* const bbuf = smem_d + Cfg::kBBase;
   if (stores_behind) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Cfg::kStagedStores) : "memory");
@@ -444,9 +453,9 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
   DirectFrags<TM, TN> f;
   direct_read_a<TM, TN, 0>(c, abuf, 0, f.a[0]);
 #pragma unroll
-  for (int i = 0; i < 2 * TN; ++i) f.b[i] = direct_read_b<TM, TN, BT>(c, bbuf, 0, i);
+  for (int i = 0; i < direct_frags(TN); ++i) f.b[i] = direct_read_b<TM, TN, BT>(c, bbuf, 0, i);
   int kt = 0;
-  auto pair = [&](auto one) {
+  for (; kt + 2 < nk; kt += 2) {
     uint8_t* a_cur = abuf + ((kt >> 1) & 1) * Cfg::kABytes;
     uint8_t* a_nxt = abuf + (((kt >> 1) + 1) & 1) * Cfg::kABytes;
     if constexpr (BT) {
@@ -458,16 +467,9 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
       uint8_t* b0 = bbuf + (kt & 3) * Cfg::kBBytes;
       uint8_t* b1 = bbuf + ((kt + 1) & 3) * Cfg::kBBytes;
       uint8_t* b2 = bbuf + ((kt + 2) & 3) * Cfg::kBBytes;
-      if constexpr (decltype(one)::value) direct_step_pair_1b<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk, stores_behind);
+      if constexpr (one_barrier) direct_step_pair_1b<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk, stores_behind);
       else direct_step_pair<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk);
     }
-  };
-  if constexpr (BT || TM * TN > 2) {
-    for (; kt + 2 < nk; kt += 2) pair(std::true_type{});
-  } else if (one_barrier) {
-    for (; kt + 2 < nk; kt += 2) pair(std::true_type{});
-  } else {
-    for (; kt + 2 < nk; kt += 2) pair(std::false_type{});
   }
   {
     // Last two steps: nothing left to load; stage nk - 1 of B must have landed.
@@ -475,7 +477,7 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
     const uint8_t* b1 = BT ? bbuf + ((kt >> 1) & 1) * Cfg::kBtBytes : bbuf + ((kt + 1) & 3) * Cfg::kBBytes;
     if (staged) direct_load_bias<TN, EDGE>(g, n_base, bias);
     direct_phase_lo<DT>(c, acc, f, a_cur, 0);
-    if (!one_barrier) direct_wait_barrier<0>();  // (one barrier per pair: awaited at the pair before)
+    if constexpr (!one_barrier) direct_wait_barrier<0>();  // (one barrier per pair: awaited at the pair before)
     direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_cur, b1, 1);
     direct_phase_lo<DT>(c, acc, f, a_cur, 1);
     direct_phase_hi<DT, TM, TN, BT, false>(c, acc, f, a_cur, b1, 0);
@@ -491,7 +493,7 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
 // M = 8192, N = 50257, K = 768 bf16, 256 x 256 tile: 1338 us with a segment per wave, 680 with whole rows.
 template <int DT, int TM, int TN>
 __device__ __forceinline__ void direct_finish_rows(const GemmArgs& g, int wave, uint8_t* __restrict__ stage,
-                                                   const f32x4 (&acc)[2 * TN][2 * TM], int m0, int n0, int wm0, int wn0) {
+                                                   const f32x4 (&acc)[direct_frags(TN)][2 * TM], int m0, int n0, int wm0, int wn0) {
   using Cfg = DirectCfg<TM, TN>;
   constexpr int BN = Cfg::BN, RB = BN * 4;            // bytes of a staged row, 32 of them
   static_assert(32 * RB == Cfg::kStageBytes, "16 rows of each half of the tile's rows");
@@ -547,10 +549,10 @@ __device__ __forceinline__ void direct_finish_rows(const GemmArgs& g, int wave, 
   }
   epi_dispatch_linear(g, [&](auto variant) {
     using E = decltype(variant);
-    f32x4 b4[2 * TN];
-    int put[2 * TN];
+    f32x4 b4[direct_frags(TN)];
+    int put[direct_frags(TN)];
 #pragma unroll
-    for (int i = 0; i < 2 * TN; ++i) {
+    for (int i = 0; i < direct_frags(TN); ++i) {
       b4[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       if (epi_has_bias<E>(g)) b4[i] = bias4<DT, true>(g, n0 + wn0 + 16 * i + 4 * g4);
       put[i] = at((wm0 ? 16 : 0) + l16, (wn0 >> 2) + 4 * i + g4);
@@ -558,7 +560,7 @@ __device__ __forceinline__ void direct_finish_rows(const GemmArgs& g, int wave, 
 #pragma unroll
     for (int j = 0; j < 2 * TM; ++j) {
 #pragma unroll
-      for (int i = 0; i < 2 * TN; ++i) {
+      for (int i = 0; i < direct_frags(TN); ++i) {
         float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
         epi_apply4<E>(g, b4[i], v);
         *reinterpret_cast<f32x4*>(stage + put[i]) = f32x4{v[0], v[1], v[2], v[3]};
@@ -613,7 +615,7 @@ __device__ __forceinline__ void direct_finish_rows(const GemmArgs& g, int wave, 
 template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool HAS_NEXT, bool BT, bool BLOCKS, bool STREAM>
 __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx<TM, TN>& next, int nk,
                                               uint8_t* __restrict__ ring, uint8_t* __restrict__ stage,
-                                              const f32x4 (&acc)[2 * TN][2 * TM], const u32x2 (&bias)[2 * TN], int m0,
+                                              const f32x4 (&acc)[direct_frags(TN)][2 * TM], const u32x2 (&bias)[direct_frags(TN)], int m0,
                                               int n0, int wm0, int wn0) {
   using Cfg = DirectCfg<TM, TN>;
   constexpr int WTN = Cfg::WTN;
@@ -627,14 +629,14 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
     // The bias values (loaded by the main loop, whose last wait covered them) are pinned down here:
     // a wait for them placed after the ring loads below would wait for those loads as well.
 #pragma unroll
-    for (int i = 0; i < 2 * TN; ++i)
+    for (int i = 0; i < direct_frags(TN); ++i)
 #pragma unroll
       for (int e = 0; e < 2; ++e) asm volatile("" ::"v"(bias[i][e]));
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with the rings
     if constexpr (HAS_NEXT) direct_prologue<TM, TN, TAIL, BT>(next, nk, ring);
     constexpr int RB = WTN * 2;                // bytes of a staged row
     constexpr int chunks = RB / 16;            // 16-byte chunks per staged row
-    constexpr int rows_per_pass = 64 / chunks;
+    auto at = [&](int row, int ch) { return row * RB + ((TN == 3 ? ch : ch ^ ((row >> 1) & (chunks - 1))) << 4); };
     // With a next tile loading into the rings, 32 rows at a time go through the wave's slice of
     // `stage`; the last tile of a workgroup stages its whole sub-tile in the idle rings at once.
     constexpr int JB = HAS_NEXT ? 1 : TM;
@@ -658,18 +660,18 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
 #pragma unroll
         for (int jj = 0; jj < 2 * JB; ++jj)
 #pragma unroll
-          for (int i = 0; i < 2 * TN; ++i) {
+          for (int i = 0; i < direct_frags(TN); ++i) {
             const int j = 2 * j0 + jj;           // 16-row fragment; staged row 16 jj + l16
             const u32x2 w = epi_pack4<DT, E>(g, bias_of(i), acc[i][j]);
             const int row = 16 * jj + l16;
-            *reinterpret_cast<u32x2*>(cw + row * RB + (((2 * i + (g4 >> 1)) ^ ((row >> 1) & (chunks - 1))) << 4) +
-                                      8 * (g4 & 1)) = w;
+            *reinterpret_cast<u32x2*>(cw + at(row, 2 * i + (g4 >> 1)) + 8 * (g4 & 1)) = w;
           }
         // Cfg::kStagedStores stores per lane in all; the main loop's first wait counts on it.
 #pragma unroll
-        for (int t = 0; t < JB * 32 / rows_per_pass; ++t) {
-          const int row = rows_per_pass * t + lane / chunks, ch = lane % chunks;
-          u32x4 w = *reinterpret_cast<const u32x4*>(cw + row * RB + ((ch ^ ((row >> 1) & (chunks - 1))) << 4));
+        for (int t = 0; t < JB * 32 * chunks / 64; ++t) {
+          const int row = TN == 3 ? (64 * t + lane) / chunks : 64 / chunks * t + lane / chunks;
+          const int ch = TN == 3 ? (64 * t + lane) % chunks : lane % chunks;
+          u32x4 w = *reinterpret_cast<const u32x4*>(cw + at(row, ch));
           const int m = m0 + wm0 + 32 * j0 + row, n = n0 + wn0 + ch * 8;
           if constexpr (EDGE) {
             if (m < g.M && n < g.N) store8_any<STREAM>(outp + (int64_t)m * g.ldc + n, w, g.N - n);
@@ -685,7 +687,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
   }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (HAS_NEXT) direct_prologue<TM, TN, TAIL, BT>(next, nk, ring);
-  if constexpr (EDGE && !BLOCKS) {
+  if constexpr (EDGE && !BLOCKS && TN != 3) {
     if (g.out_dt == LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C) && !rows_of_pieces(g)) {
       direct_finish_rows<DT, TM, TN>(g, next.wave, stage, acc, m0, n0, wm0, wn0);
       return;
@@ -697,7 +699,8 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
     // slice of `stage` so that the accumulator input is read and the result written as whole row
     // segments (4 elements per lane, 64 or 128 bytes per row) instead of pieces of 64 different
     // rows.  Order of operations as in epilogue4 (one rounding, after the sum).
-    constexpr int NI = TN;                     // 16-column fragments per staged block (2 blocks per wave)
+    constexpr int NI = TN == 3 ? 1 : TN;       // 16-column fragments per staged block
+    constexpr int NBLK = Cfg::NF / NI;         // blocks of a wave side by side
     constexpr int RB = NI * 64;                // bytes of a staged row
     constexpr int chunks = RB / 16;
     constexpr int rows_per_pass = 64 / chunks;
@@ -713,7 +716,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
       // in flight at once) instead of block by block between the stores of the blocks before, which the
       // loads cannot pass (input and output may be the same buffer): one exposed memory latency per
       // tile instead of eight.  The larger tiles have no registers for that.
-      constexpr bool kPreloadC = TM * TN == 2 && has_c;
+      constexpr bool kPreloadC = TM == 2 && TN != 2 && has_c;
       constexpr int NPASS = 32 / rows_per_pass;
       auto load_c = [&](int64_t off, int n) -> f32x4 {
         if constexpr (EDGE) {
@@ -725,10 +728,10 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
           return f32x4{unpack_lo<DT>(cc[0]), unpack_hi<DT>(cc[0]), unpack_lo<DT>(cc[1]), unpack_hi<DT>(cc[1])};
         }
       };
-      f32x4 cin[kPreloadC ? 2 * TM * NPASS : 1];
+      f32x4 cin[kPreloadC ? NBLK * TM * NPASS : 1];
       if constexpr (kPreloadC) {
 #pragma unroll
-        for (int ib = 0; ib < 2; ++ib)
+        for (int ib = 0; ib < NBLK; ++ib)
 #pragma unroll
           for (int j32 = 0; j32 < TM; ++j32)
 #pragma unroll
@@ -741,7 +744,7 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
             }
       }
 #pragma unroll
-      for (int ib = 0; ib < 2; ++ib) {
+      for (int ib = 0; ib < NBLK; ++ib) {
         const int n = n0 + wn0 + 16 * NI * ib + 4 * ch;  // the lane's 4 output columns
         const bool n_ok = !EDGE || n < g.N;
         f32x4 b4 = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -837,7 +840,7 @@ __device__ __forceinline__ void direct_lane_reads(DirectCtx<TM, TN>& c, int wave
     const int krow = 8 * g4 + (l16 >> 2);
     const int col = wn0 + 4 * (l16 & 3);
     c.b_chunk = col >> 3;
-    c.b_swz = (4 * (krow & 3)) ^ (2 * ((krow >> 3) & 1));
+    c.b_swz = Cfg::b_swizzle(krow);
     c.b_off = krow * Cfg::kBRow + 8 * ((col >> 2) & 1);
   }
   // (transposed B: row wn0 + 16 i + l16 of the stage, like the A fragment)
@@ -918,16 +921,16 @@ __device__ __forceinline__ void direct_run(const GemmArgs& g) {
   const bool counted_stores = !EDGE && staged;
   bool first = true;
   for (;;) {
-    f32x4 acc[2 * TN][2 * TM];
+    f32x4 acc[direct_frags(TN)][2 * TM];
 #pragma unroll
-    for (int i = 0; i < 2 * TN; ++i)
+    for (int i = 0; i < direct_frags(TN); ++i)
 #pragma unroll
       for (int j = 0; j < 2 * TM; ++j)
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.0f;
-    u32x2 bias[2 * TN];
+    u32x2 bias[direct_frags(TN)];
     const GemmArgs& ga = SPLITK ? g_cur : g;
-    direct_mainloop<DT, TM, TN, EDGE, TAIL, BT>(ga, c, acc, smem_d, nk, counted_stores && !first, staged, n0 + wn0 + 4 * g4, bias);
+    direct_mainloop<DT, TM, TN, EDGE, TAIL, BT, SPLITK>(ga, c, acc, smem_d, nk, counted_stores && !first, staged, n0 + wn0 + 4 * g4, bias);
     first = false;
     const int tn = t + (int)gridDim.x;
     const bool more = tn < ntiles;
@@ -982,7 +985,6 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
   const int ntiles = ((g.M + Cfg::BM - 1) / Cfg::BM) * ((g.N + Cfg::BN - 1) / Cfg::BN);
   const int resident = num_cus() * (2 * lds <= 160 * 1024 ? 2 : 1);
   GemmArgs ga = g;
-  ga.one_barrier = ntiles > num_cus();
   const int grid = ntiles < resident ? ntiles : resident;
   const int64_t rows = BT ? g.N : g.K;
   ga.touch_b = rows * (((BT ? g.K : g.N) + 63) / 64) <= 128 * grid && rows * g.ldb < (1ll << 30);
@@ -993,11 +995,7 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
 template <int DT, int TM, int TN>
 int launch_direct(const GemmArgs& g, hipStream_t s) {
   using Cfg = DirectCfg<TM, TN>;
-  const bool whole = g.M % Cfg::BM == 0 && g.N % Cfg::BN == 0 && g.ldc % 8 == 0 && aligned16(g.out) &&
-                     (!(g.flags & LH_GEMM_HAS_BIAS) || aligned16(g.bias)) &&
-                     (!(g.flags & LH_GEMM_ACCUMULATE_C) || aligned16(g.c));
-  if constexpr (TM * TN == 2)
-    if ((int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) <= num_cus()) return launch_deep<DT>(g, whole, s);
+  const bool whole = whole_tiles(g, Cfg::BM, Cfg::BN);
   if constexpr (TM * TN < 8)
     if (g.K % 64 != 0)
       return (g.flags & LH_GEMM_TRANSPOSE_B) ? launch_direct_edge<DT, TM, TN, true, true, false, true>(g, s)
@@ -1020,112 +1018,125 @@ int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s) {
 
 #if LH_GEMM16_DEEP
 // ---- one workgroup per CU ---------------------------------------------------------------------
-// The 128 x 128 tile where no CU gets a second workgroup: nobody covers the latency of its operands, but all of the CU's LDS is its
-// own.  Both rings hold four stages of 64 k (144 KiB with the staging area), so that a stage is requested three to four pairs of
-// steps before it is read, through one barrier per pair; what two of them take, 0.9 us, is less than a line's way out of memory.
+// Where no CU gets a second workgroup nobody covers the latency of its operands, but all of the CU's LDS is its own.  Both rings
+// hold four stages of 64 k (128 x 128 and 128 x 192 tiles; 128 x 256 and 256 x 128: three), so that a stage is requested two to four pairs of
+// steps before it is read, through one barrier per pair; what one of them takes, 0.45 us at 128 x 128, is less than a line's way out
+// of memory.  One tile per workgroup: the output is staged in the idle rings.
 // bf16, with two stages (and two barriers) and with four, operands in the caches / in memory: 2048^3 23.5 -> 20.5 / 28.3 -> 22.4 us,
 // on a transposed B 22.8 -> 18.8 / 30.9 -> 21.7; 512 x 8192 x 2048 21.9 -> 19.3 / 28.2 -> 22.3; 2048 x 768 x 768 with a residual 11.3 -> 9.7 /
 // 16.6 -> 13.6.
+template <int TM, int TN>
 struct DeepCfg {
-  static constexpr int kStages = 4;
-  static constexpr int kBBase = kStages * DirectCfg<2, 1>::kABytes, kBBytes = 2 * DirectCfg<2, 1>::kBBytes;  // (a stage of B: 64 k)
-  static constexpr int kRingBytes = kBBase + kStages * kBBytes;
-  static constexpr int kLdsBytes = kRingBytes + DirectCfg<2, 1>::kStageBytes;
-  static constexpr int kLoads = 4;  // of a lane per stage
+  using Cfg = DirectCfg<TM, TN>;
+  static constexpr int kABytes = Cfg::kABytes, kBBytes = 2 * Cfg::kBBytes;        // of a stage of 64 k
+  static constexpr int kStages = 160 * 1024 / (kABytes + kBBytes) < 4 ? 160 * 1024 / (kABytes + kBBytes) : 4;
+  static constexpr int kBBase = kStages * kABytes;
+  static constexpr int kLdsBytes = kStages * (kABytes + kBBytes);                 // (the output is staged in the rings)
+  static constexpr int kLoads = TM + Cfg::NF;                                     // of a lane per stage
 };
-template <bool BT, bool TAIL>
-__device__ __forceinline__ void deep_load(const DirectCtx<2, 1>& c, int p, uint8_t* __restrict__ abuf, uint8_t* __restrict__ bbuf) {
-  direct_load_a<2, 1, TAIL>(c, p, abuf);
-  if constexpr (BT) {
-    direct_load_b<2, 1, true, TAIL>(c, p, bbuf);
+template <int TM, int TN, bool BT, bool TAIL>
+__device__ __forceinline__ void deep_load(const DirectCtx<TM, TN>& c, int p, uint8_t* __restrict__ abuf, uint8_t* __restrict__ bbuf) {
+  direct_load_a<TM, TN, TAIL>(c, p, abuf);
+  if constexpr (BT || TN == 3) {
+    direct_load_b<TM, TN, BT, TAIL>(c, p, bbuf);
   } else {
-    direct_load_b<2, 1, false, TAIL>(c, 2 * p, bbuf);
-    direct_load_b<2, 1, false, TAIL>(c, 2 * p + 1, bbuf + DirectCfg<2, 1>::kBBytes);
+    direct_load_b<TM, TN, false, TAIL>(c, 2 * p, bbuf);
+    direct_load_b<TM, TN, false, TAIL>(c, 2 * p + 1, bbuf + DirectCfg<TM, TN>::kBBytes);
   }
 }
 // Pair p of steps (direct_step_pair_1b), of which a successor is read next: NEWER stages behind that have been requested and may
-// be on their way.  LOAD: stage p + 4 goes where p was.
-template <int DT, bool TAIL, bool BT, int NEWER, bool LOAD>
-__device__ __forceinline__ void deep_step_pair(const DirectCtx<2, 1>& c, f32x4 (&acc)[2][4], DirectFrags<2, 1>& f,
+// be on their way.  LOAD: stage p + kStages goes where p was.
+template <int DT, int TM, int TN, bool TAIL, bool BT, int NEWER, bool LOAD>
+__device__ __forceinline__ void deep_step_pair(const DirectCtx<TM, TN>& c, f32x4 (&acc)[direct_frags(TN)][2 * TM], DirectFrags<TM, TN>& f,
                                                const uint8_t* __restrict__ a_cur, const uint8_t* __restrict__ a_nxt,
                                                const uint8_t* __restrict__ b_cur, const uint8_t* __restrict__ b_nxt,
                                                uint8_t* __restrict__ a_refill, uint8_t* __restrict__ b_refill, int p) {
-  const uint8_t* const b1 = BT ? b_cur : b_cur + DirectCfg<2, 1>::kBBytes;
+  using Deep = DeepCfg<TM, TN>;
+  const uint8_t* const b1 = BT ? b_cur : b_cur + DirectCfg<TM, TN>::kBBytes;
   direct_phase_lo<DT>(c, acc, f, a_cur, 0);
-  direct_phase_hi<DT, 2, 1, BT>(c, acc, f, a_cur, b1, 1);
+  direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_cur, b1, 1);
   direct_phase_lo<DT>(c, acc, f, a_cur, 1);
-  direct_wait_barrier<NEWER * DeepCfg::kLoads>();
-  if constexpr (LOAD) deep_load<BT, TAIL>(c, p + 4, a_refill, b_refill);
-  direct_phase_hi<DT, 2, 1, BT>(c, acc, f, a_nxt, b_nxt, 0);
+  direct_wait_barrier<NEWER * Deep::kLoads>();
+  if constexpr (LOAD) deep_load<TM, TN, BT, TAIL>(c, p + Deep::kStages, a_refill, b_refill);
+  direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_nxt, b_nxt, 0);
 }
 
-template <int DT, bool EDGE, bool TAIL, bool BT>
+template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool BT>
 __global__ void __launch_bounds__(512) gemm16_deep(GemmArgs g) {
-  using Cfg = DirectCfg<2, 1>;
+  using Cfg = DirectCfg<TM, TN>;
+  using Deep = DeepCfg<TM, TN>;
+  constexpr int S = Deep::kStages;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_d[];
-  const int tiles = ((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const int tiles = ((g.M + Cfg::BM - 1) / Cfg::BM) * ((g.N + Cfg::BN - 1) / Cfg::BN);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm0 = (wave / 4) * Cfg::WTM, wn0 = (wave % 4) * Cfg::WTN;
-  DirectCtx<2, 1> c;
+  DirectCtx<TM, TN> c;
   direct_lane_reads(c, wave, lane, wm0, wn0);
   c.k_end = g.K;
   int m0, n0;
-  direct_place<2, 1, EDGE, BT>(g, xcd_remap(blockIdx.x, tiles), c, m0, n0);
+  direct_place<TM, TN, EDGE, BT>(g, xcd_remap(blockIdx.x, tiles), c, m0, n0);
   const int pairs = TAIL ? (g.K + 63) / 64 : g.K / 64;
-  auto a_stage = [&](int p) { return smem_d + (p & 3) * Cfg::kABytes; };
-  auto b_stage = [&](int p) { return smem_d + DeepCfg::kBBase + (p & 3) * DeepCfg::kBBytes; };
+  auto a_stage = [&](int slot) { return smem_d + slot * Deep::kABytes; };
+  auto b_stage = [&](int slot) { return smem_d + Deep::kBBase + slot * Deep::kBBytes; };
 #pragma unroll
-  for (int p = 0; p < DeepCfg::kStages; ++p)
-    if (p < pairs) deep_load<BT, TAIL>(c, p, a_stage(p), b_stage(p));
+  for (int p = 0; p < S; ++p)
+    if (p < pairs) deep_load<TM, TN, BT, TAIL>(c, p, a_stage(p), b_stage(p));
 
-  f32x4 acc[2][4];
+  f32x4 acc[Cfg::NF][2 * TM];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < Cfg::NF; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  if (pairs >= 4) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * DeepCfg::kLoads) : "memory");
+    for (int j = 0; j < 2 * TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  if (pairs >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * Deep::kLoads) : "memory");
   else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  DirectFrags<2, 1> f;
-  direct_read_a<2, 1, 0>(c, smem_d, 0, f.a[0]);
+  DirectFrags<TM, TN> f;
+  direct_read_a<TM, TN, 0>(c, a_stage(0), 0, f.a[0]);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) f.b[i] = direct_read_b<2, 1, BT>(c, smem_d + DeepCfg::kBBase, 0, i);
-  int p = 0;
+  for (int i = 0; i < Cfg::NF; ++i) f.b[i] = direct_read_b<TM, TN, BT>(c, b_stage(0), 0, i);
+  int p = 0, slot = 0;
   auto pair = [&](auto newer, auto load) {
-    deep_step_pair<DT, TAIL, BT, decltype(newer)::value, decltype(load)::value>(c, acc, f, a_stage(p), a_stage(p + 1), b_stage(p), b_stage(p + 1),
-                                                                               a_stage(p), b_stage(p), p);
+    const int next = slot + 1 == S ? 0 : slot + 1;
+    deep_step_pair<DT, TM, TN, TAIL, BT, decltype(newer)::value, decltype(load)::value>(
+        c, acc, f, a_stage(slot), a_stage(next), b_stage(slot), b_stage(next), a_stage(slot), b_stage(slot), p);
     ++p;
+    slot = next;
   };
-  while (p + 4 < pairs) pair(std::integral_constant<int, 2>{}, std::true_type{});
-  if (p + 3 < pairs) pair(std::integral_constant<int, 2>{}, std::false_type{});
-  if (p + 2 < pairs) pair(std::integral_constant<int, 1>{}, std::false_type{});
+  while (p + S < pairs) pair(std::integral_constant<int, S - 2>{}, std::true_type{});
+  if (p + S - 1 < pairs) pair(std::integral_constant<int, S - 2>{}, std::false_type{});
+  if (S > 3 && p + S - 2 < pairs) pair(std::integral_constant<int, S - 3>{}, std::false_type{});
   if (p + 1 < pairs) pair(std::integral_constant<int, 0>{}, std::false_type{});
   const bool staged = g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
-  u32x2 bias[2];
-  if (staged) direct_load_bias<1, EDGE>(g, n0 + wn0 + 4 * (lane >> 4), bias);
-  direct_phase_lo<DT>(c, acc, f, a_stage(p), 0);
-  direct_phase_hi<DT, 2, 1, BT>(c, acc, f, a_stage(p), b_stage(p) + (BT ? 0 : Cfg::kBBytes), 1);
-  direct_phase_lo<DT>(c, acc, f, a_stage(p), 1);
-  direct_phase_hi<DT, 2, 1, BT, false>(c, acc, f, a_stage(p), b_stage(p), 0);
-  direct_finish<DT, 2, 1, EDGE, TAIL, false, BT, false, false>(g, c, 2 * pairs, smem_d, smem_d + DeepCfg::kRingBytes, acc, bias, m0, n0, wm0, wn0);
+  u32x2 bias[Cfg::NF];
+  if (staged) direct_load_bias<TN, EDGE>(g, n0 + wn0 + 4 * (lane >> 4), bias);
+  direct_phase_lo<DT>(c, acc, f, a_stage(slot), 0);
+  direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_stage(slot), b_stage(slot) + (BT ? 0 : Cfg::kBBytes), 1);
+  direct_phase_lo<DT>(c, acc, f, a_stage(slot), 1);
+  direct_phase_hi<DT, TM, TN, BT, false>(c, acc, f, a_stage(slot), b_stage(slot), 0);
+  direct_finish<DT, TM, TN, EDGE, TAIL, false, BT, false, false>(g, c, 2 * pairs, smem_d, smem_d, acc, bias, m0, n0, wm0, wn0);
 }
 
-template <int DT>
-int launch_deep(const GemmArgs& g, bool whole, hipStream_t s) {
-  static constexpr decltype(&gemm16_deep<DT, true, true, false>) kernels[2][3] = {
-      {gemm16_deep<DT, false, false, false>, gemm16_deep<DT, true, false, false>, gemm16_deep<DT, true, true, false>},
-      {gemm16_deep<DT, false, false, true>, gemm16_deep<DT, true, false, true>, gemm16_deep<DT, true, true, true>}};
+template <int DT, int TM, int TN>
+int launch_deep(const GemmArgs& g, hipStream_t s) {
+  using Cfg = DirectCfg<TM, TN>;
+  using Deep = DeepCfg<TM, TN>;
+  static_assert(Deep::kStages == 3 || Deep::kStages == 4, "the kernel's last pairs");
+  constexpr bool tail = TN != 3;  // (192 columns take whole stages only)
+  static constexpr decltype(&gemm16_deep<DT, TM, TN, true, false, false>) kernels[2][3] = {
+      {gemm16_deep<DT, TM, TN, false, false, false>, gemm16_deep<DT, TM, TN, true, false, false>, gemm16_deep<DT, TM, TN, true, tail, false>},
+      {gemm16_deep<DT, TM, TN, false, false, true>, gemm16_deep<DT, TM, TN, true, false, true>, gemm16_deep<DT, TM, TN, true, tail, true>}};
   static bool configured = false;
   if (!configured && !planning()) {
     for (auto& layout : kernels)
       for (auto k : layout)
-        LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, DeepCfg::kLdsBytes));
+        LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, Deep::kLdsBytes));
     configured = true;
   }
+  const bool whole = whole_tiles(g, Cfg::BM, Cfg::BN);
   auto kern = kernels[(g.flags & LH_GEMM_TRANSPOSE_B) ? 1 : 0][g.K % 64 != 0 ? 2 : whole ? 0 : 1];
-  LH_LAUNCH(kern, dim3((unsigned)(((g.M + 127) / 128) * ((g.N + 127) / 128))), dim3(512), DeepCfg::kLdsBytes, s, g);
+  LH_LAUNCH(kern, dim3((unsigned)(((g.M + Cfg::BM - 1) / Cfg::BM) * ((g.N + Cfg::BN - 1) / Cfg::BN))), dim3(512), Deep::kLdsBytes, s, g);
   return check_launch("gemm16_deep");
 }
-template int launch_deep<LH_GEMM16_DT>(const GemmArgs&, bool, hipStream_t);
+template int launch_deep<LH_GEMM16_DT, LH_GEMM16_TM, LH_GEMM16_TN>(const GemmArgs&, hipStream_t);
 #endif
 
 #if LH_GEMM16_ODD

@@ -22,9 +22,6 @@ struct GemmArgs {
   int splits = 1;
   // Source of the call's temporary device memory; nullptr: the library's pool of the stream.
   Scratch* ws = nullptr;
-  // 16-bit direct kernel, 128 x 128 tile: main loop with one barrier per 64 k (set by the launcher
-  // when more than one workgroup falls on a compute unit).
-  int one_barrier = 0;
   // 16-bit direct kernel: the workgroups touch B at the start (set by the launcher).
   int touch_b = 0;
   // B is a copy whose rows hold whole 16-byte chunks past column N (zeros): N need not be a multiple of them.

@@ -1,19 +1,27 @@
-"""The 128-row tiles of problems that give no CU a second workgroup: one to six stages of K and more than the rings hold, edges of the
-tile, a K that ends inside a step, both layouts of B, every kind of output."""
+"""The tiles of problems that give no CU a second workgroup: one to six stages of K and more than the rings hold, edges of the
+tiles, a K that ends inside a step, both layouts of B, every kind of output."""
+
+import multiprocessing
+import re
 
 import pytest
 import torch
 
-pytestmark = pytest.mark.gpu
+from tests import recorded_launches as rec
 
 DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16}
 
 
+SIZES = [(2048, 2048, 64), (2048, 2048, 128), (2000, 2040, 192), (2048, 2048, 256), (1921, 1928, 320), (2048, 2048, 384),
+         (1929, 2000, 72), (1930, 2000, 200), (1000, 4096, 1000), (1999, 1992, 264), (1537, 2304, 768),
+         # more than a CU's worth of 128 x 128 tiles: 128 x 192, 256 x 128, 128 x 256
+         (8192, 768, 320), (8192, 768, 448), (8191, 760, 384), (8129, 768, 640), (4090, 1528, 512), (4096, 1536, 1024),
+         (4096, 2048, 512), (4096, 2048, 2048), (4096, 2000, 576), (4090, 2048, 768), (3900, 2000, 1000), (2048, 4096, 448), (2000, 4000, 1032), (1999, 4088, 640)]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,transpose_b", [("bf16", False), ("bf16", True), ("f16", False), ("f16", True)])
-@pytest.mark.parametrize("M,N,K", [(2048, 2048, 64), (2048, 2048, 128), (2000, 2040, 192), (2048, 2048, 256), (1921, 1928, 320), (2048, 2048, 384),
-                                   (2047, 2056, 72), (1930, 2000, 200), (1000, 4096, 1000), (1999, 1992, 264), (1537, 2304, 768),
-                                   # 192 columns: an output of that many on more rows, whole and with edges
-                                   (8192, 768, 64), (8192, 768, 448), (8191, 760, 192), (8129, 768, 128), (5461, 1144, 512)])
+@pytest.mark.parametrize("M,N,K", SIZES)
 def test_one_tile_per_cu(M, N, K, dtype, transpose_b):
     """Integer operands: the f32 sum is exact in any order, so every element has one right bit pattern."""
     from lighthouse_amd import ops
@@ -29,3 +37,25 @@ def test_one_tile_per_cu(M, N, K, dtype, transpose_b):
     assert torch.equal(ops.gemm(a, b, bias, out=out, residual=c, transpose_b=transpose_b), want + c + bias)
     out16 = torch.empty(M, N, device="cuda", dtype=dt)
     assert torch.equal(ops.gemm(a, b, out=out16, residual=c.to(dt), transpose_b=transpose_b), (want + c).to(dt))
+
+
+def _tiles(so):
+    r, found = rec.Recorder(so), set()
+    for M, N, K in SIZES:
+        for dt in (rec._lib.BF16, rec._lib.F16):
+            for out in (dt, rec._lib.F32):
+                for flags, ldb in ((0, N), (16, K)):
+                    rc, launches = r.calls("lh_hip_gemm", 1 << 50, 2 << 50, 3 << 50, 4 << 50, M, N, K, K, ldb, N, dt, out, flags, None)
+                    assert rc == 0, r.lib.lh_hip_last_error()
+                    found |= {m.groups() for m in (re.search(r"gemm16_deepILi(\d)ELi(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)E", n.name) for n in launches) if m}
+    return {tuple(int(v) for v in f) for f in found}
+
+
+def test_the_sizes_reach_every_tile(tmp_path):
+    """Type; rows / 64; columns / 128 (3: 192); edges; K ends inside a step, which 192 columns do not take; B stored [N, K]."""
+    with multiprocessing.get_context("spawn").Pool(1) as pool:
+        found = pool.apply(_tiles, (rec.build(tmp_path),))
+    for tile in ((2, 1), (2, 2), (4, 1)):
+        assert {f[3:] for f in found if f[1:3] == tile} == {(e, t, b) for e, t in ((0, 0), (1, 0), (1, 1)) for b in (0, 1)}, tile
+    assert {f[3:] for f in found if f[1:3] == (2, 3)} == {(e, 0, b) for e in (0, 1) for b in (0, 1)}
+    assert {f[0] for f in found} == {rec._lib.BF16, rec._lib.F16}
