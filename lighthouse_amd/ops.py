@@ -15,9 +15,9 @@ from .utils.numpy import lh_dtype
 
 
 def _stream() -> int:
-    """Raw handle of torch's current stream on the current device (the accessor torch's own
-    extensions use: no Stream object is built per launch)."""
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    """Raw handle of torch's current stream on the current device (the accessors torch's own
+    extensions use: no Stream object is built per launch; torch is up, the call's tensors are on the GPU)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need_cuda(*tensors) -> None:
@@ -145,7 +145,7 @@ def gemm(a, b, bias=None, *, out=None, out_dtype=None, relu=False, gelu=False, a
              | (_lib.GEMM_TRANSPOSE_A if transpose_a else 0) | (_lib.GEMM_TRANSPOSE_B if transpose_b else 0))
     if tile is None and split_k is None and not transpose_a:  # (a transposed B runs on the same kernels in place)
         db = _tuned_db()  # tuned parameters for this shape, if the database has any
-        if db is not None:
+        if db is not None and db.entries:
             tile, split_k = db.lookup_gemm(_DTYPE_NAMES[a.dtype], M, N, K)
             # (a request needs aligned rows; tuned entries assume them)
             if (tile is not None or split_k is not None) and not _rows_aligned16(a, b, out, bias):
@@ -253,6 +253,22 @@ def _strides3(t) -> _lib.Strides3:
     return _lib.Strides3(t.stride(0), t.stride(1), t.stride(2))
 
 
+def _strides3_of(*tensors):
+    """Those of each tensor; tensors laid out alike share one (each costs 0.5 us to make)."""
+    first = tensors[0].stride()
+    shared = _lib.Strides3(*first[:3])
+    return [shared if t.stride() == first else _strides3(t) for t in tensors]
+
+
+def _attention_request(rows_per_wave, stages, kv_split, scale_in_f32) -> int:
+    """The bits of the causal word that ask for a kernel variant."""
+    if not ((rows_per_wave or 0) in _lib.ATTN_ROWS and (stages or 0) in _lib.ATTN_STAGES and (kv_split or 0) in _lib.ATTN_KSPLIT):
+        raise ValueError(f"rows_per_wave must be one of {sorted(_lib.ATTN_ROWS)[1:]}, stages one of {sorted(_lib.ATTN_STAGES)[1:]}, "
+                         f"kv_split one of {sorted(_lib.ATTN_KSPLIT)[1:]}")
+    return (_lib.ATTN_ROWS[rows_per_wave or 0] | _lib.ATTN_STAGES[stages or 0] | _lib.ATTN_KSPLIT[kv_split or 0]
+            | (_lib.ATTN_SCALE_F32 if scale_in_f32 else 0))
+
+
 def attention(q, k, v, *, causal=False, scale=None, out=None, rows_per_wave=None, stages=None, kv_split=None,
               workspace=None, scale_in_f32=False):
     """Fused attention forward on [Z,H,T,d] tensors (any strides with unit stride along d).
@@ -272,23 +288,21 @@ def attention(q, k, v, *, causal=False, scale=None, out=None, rows_per_wave=None
              "attention expects Q, K, V of one dtype (float32, bfloat16 or float16)")
     if out is None:
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    _require(tuple(out.shape) == tuple(q.shape) and out.dtype == q.dtype, "out must have the shape and dtype of Q")
-    for t in (q, k, v, out):
-        if t.stride(3) != 1:
-            raise ValueError("innermost stride must be 1")
+    elif out.shape != q.shape or out.dtype != q.dtype:
+        raise ValueError("out must have the shape and dtype of Q")
+    if q.stride(3) != 1 or k.stride(3) != 1 or v.stride(3) != 1 or out.stride(3) != 1:
+        raise ValueError("innermost stride must be 1")
     _need_cuda(q, k, v, out)
     Z, H, T, d = q.shape
     if rows_per_wave is None and stages is None and kv_split is None and d == 64 and q.dtype != torch.float32:
         db = _tuned_db()
-        if db is not None:
+        if db is not None and db.entries:
             rows_per_wave, stages, kv_split = db.lookup_attention("bf16" if q.dtype == torch.bfloat16 else "f16", Z * H, T, d, causal)
             if (rows_per_wave or stages or kv_split) and not _rows_aligned16(q, k, v, out):
                 rows_per_wave = stages = kv_split = None
-    if not ((rows_per_wave or 0) in _lib.ATTN_ROWS and (stages or 0) in _lib.ATTN_STAGES and (kv_split or 0) in _lib.ATTN_KSPLIT):
-        raise ValueError(f"rows_per_wave must be one of {sorted(_lib.ATTN_ROWS)[1:]}, stages one of {sorted(_lib.ATTN_STAGES)[1:]}, "
-                         f"kv_split one of {sorted(_lib.ATTN_KSPLIT)[1:]}")
-    word = ((_lib.ATTN_CAUSAL if causal else 0) | _lib.ATTN_ROWS[rows_per_wave or 0] | _lib.ATTN_STAGES[stages or 0]
-            | _lib.ATTN_KSPLIT[kv_split or 0] | (_lib.ATTN_SCALE_F32 if scale_in_f32 else 0))
+    word = _lib.ATTN_CAUSAL if causal else 0
+    if rows_per_wave or stages or kv_split or scale_in_f32:
+        word |= _attention_request(rows_per_wave, stages, kv_split, scale_in_f32)
     if workspace is not None:
         _require(workspace.dtype == torch.uint8 and workspace.dim() == 1 and workspace.is_contiguous(),
                  "workspace must be a contiguous uint8 vector")
@@ -301,7 +315,7 @@ def attention(q, k, v, *, causal=False, scale=None, out=None, rows_per_wave=None
         return out
     _lib.check(_lib.load().lh_hip_attention(
         out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), Z, H, T, d,
-        _strides3(out), _strides3(q), _strides3(k), _strides3(v),
+        *_strides3_of(out, q, k, v),
         float(scale) if scale is not None else 1.0 / math.sqrt(d), word, lh_dtype(q.dtype), _stream()),
         "attention")
     return out
