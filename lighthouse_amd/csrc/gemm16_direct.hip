@@ -1016,7 +1016,7 @@ int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s) {
 }
 #endif
 
-#if LH_GEMM16_DEEP
+#if LH_GEMM16_DEEP || LH_GEMM16_TM == 0
 // ---- one workgroup per CU ---------------------------------------------------------------------
 // Where no CU gets a second workgroup nobody covers the latency of its operands, but all of the CU's LDS is its own.  Both rings
 // hold four stages of 64 k (128 x 128 and 128 x 192 tiles; 128 x 256 and 256 x 128: three), so that a stage is requested two to four pairs of
@@ -1061,7 +1061,8 @@ __device__ __forceinline__ void deep_step_pair(const DirectCtx<TM, TN>& c, f32x4
   direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_nxt, b_nxt, 0);
 }
 
-template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool BT>
+// SPLITK: the grid is g.splits copies of the tiles, each on its own piece of K and f32 block of the output (direct_run).
+template <int DT, int TM, int TN, bool EDGE, bool TAIL, bool BT, bool SPLITK = false>
 __global__ void __launch_bounds__(512) gemm16_deep(GemmArgs g) {
   using Cfg = DirectCfg<TM, TN>;
   using Deep = DeepCfg<TM, TN>;
@@ -1074,7 +1075,15 @@ __global__ void __launch_bounds__(512) gemm16_deep(GemmArgs g) {
   direct_lane_reads(c, wave, lane, wm0, wn0);
   c.k_end = g.K;
   int m0, n0;
-  direct_place<TM, TN, EDGE, BT>(g, xcd_remap(blockIdx.x, tiles), c, m0, n0);
+  int id = blockIdx.x;
+  if constexpr (SPLITK) {
+    const int sp = __builtin_amdgcn_readfirstlane(id / tiles);
+    id -= sp * tiles;
+    g.a = reinterpret_cast<const uint16_t*>(g.a) + (int64_t)sp * g.K;
+    g.b = reinterpret_cast<const uint16_t*>(g.b) + (int64_t)sp * g.K * (BT ? 1 : g.ldb);
+    g.out = reinterpret_cast<float*>(g.out) + (int64_t)sp * g.M * g.ldc;
+  }
+  direct_place<TM, TN, EDGE, BT>(g, xcd_remap(id, tiles), c, m0, n0);
   const int pairs = TAIL ? (g.K + 63) / 64 : g.K / 64;
   auto a_stage = [&](int slot) { return smem_d + slot * Deep::kABytes; };
   auto b_stage = [&](int slot) { return smem_d + Deep::kBBase + slot * Deep::kBBytes; };
@@ -1105,16 +1114,17 @@ __global__ void __launch_bounds__(512) gemm16_deep(GemmArgs g) {
   if (p + S - 1 < pairs) pair(std::integral_constant<int, S - 2>{}, std::false_type{});
   if (S > 3 && p + S - 2 < pairs) pair(std::integral_constant<int, S - 3>{}, std::false_type{});
   if (p + 1 < pairs) pair(std::integral_constant<int, 0>{}, std::false_type{});
-  const bool staged = g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
+  const bool staged = !SPLITK && g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);
   u32x2 bias[Cfg::NF];
   if (staged) direct_load_bias<TN, EDGE>(g, n0 + wn0 + 4 * (lane >> 4), bias);
   direct_phase_lo<DT>(c, acc, f, a_stage(slot), 0);
   direct_phase_hi<DT, TM, TN, BT>(c, acc, f, a_stage(slot), b_stage(slot) + (BT ? 0 : Cfg::kBBytes), 1);
   direct_phase_lo<DT>(c, acc, f, a_stage(slot), 1);
   direct_phase_hi<DT, TM, TN, BT, false>(c, acc, f, a_stage(slot), b_stage(slot), 0);
-  direct_finish<DT, TM, TN, EDGE, TAIL, false, BT, false, false>(g, c, 2 * pairs, smem_d, smem_d, acc, bias, m0, n0, wm0, wn0);
+  direct_finish<DT, TM, TN, EDGE, TAIL, false, BT, SPLITK, false>(g, c, 2 * pairs, smem_d, smem_d, acc, bias, m0, n0, wm0, wn0);
 }
 
+#if LH_GEMM16_DEEP
 template <int DT, int TM, int TN>
 int launch_deep(const GemmArgs& g, hipStream_t s) {
   using Cfg = DirectCfg<TM, TN>;
@@ -1137,6 +1147,7 @@ int launch_deep(const GemmArgs& g, hipStream_t s) {
   return check_launch("gemm16_deep");
 }
 template int launch_deep<LH_GEMM16_DT, LH_GEMM16_TM, LH_GEMM16_TN>(const GemmArgs&, hipStream_t);
+#endif
 #endif
 
 #if LH_GEMM16_ODD
@@ -1308,6 +1319,14 @@ static int launch_splitk_edge(const GemmArgs& g, hipStream_t s) {
   using Cfg = DirectCfg<2, 1>;
   auto kern = gemm16_direct<DT, 2, 1, EDGE, true, BT>;
   static bool configured = false;
+#if LH_GEMM16_TM == 0
+  // No CU gets a second workgroup: deeper rings.  bf16, operands in the caches / in memory: 1024 x 1024 x 8192 29.3 -> 27.5 / 35.3 -> 29.0 us,
+  // 128 x 4096 x 4096 18.5 -> 15.9 / 21.3 -> 18.6, 2048 x 768 x 3072 with a residual 24.3 -> 22.0 / 30.3 -> 25.3.
+  using Deep = DeepCfg<2, 1>;
+  auto deep = gemm16_deep<DT, 2, 1, EDGE, false, BT, true>;
+  if (!configured && !planning())
+    LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(deep), hipFuncAttributeMaxDynamicSharedMemorySize, Deep::kLdsBytes));
+#endif
   if (!configured && !planning()) {
     LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)Cfg::kLdsBytes));
@@ -1315,6 +1334,12 @@ static int launch_splitk_edge(const GemmArgs& g, hipStream_t s) {
   }
   const int64_t total = (int64_t)((g.M + Cfg::BM - 1) / Cfg::BM) * ((g.N + Cfg::BN - 1) / Cfg::BN) * g.splits;
   const int64_t resident = 2 * (int64_t)num_cus();
+#if LH_GEMM16_TM == 0
+  if (2 * total <= resident) {
+    LH_LAUNCH(deep, dim3((unsigned)total), dim3(512), Deep::kLdsBytes, s, g);
+    return check_launch("gemm16_deep (split K)");
+  }
+#endif
   LH_LAUNCH(kern, dim3((unsigned)(total < resident ? total : resident)), dim3(512), Cfg::kLdsBytes, s, g);
   return check_launch("gemm16_direct (split K)");
 }
