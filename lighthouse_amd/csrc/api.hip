@@ -35,9 +35,8 @@ static int gemm_common_checks(const char* who, const void* out, const void* a, c
 // Internal form with a separate accumulator input, bias type and source of temporary memory.
 int gemm_run(void* out, const void* c, const void* a, const void* b, const void* bias, int64_t M, int64_t N, int64_t K,
              int64_t lda, int64_t ldb, int64_t ldc, int ab_dtype, int out_dtype, int bias_dtype, uint32_t flags,
-             hipStream_t s, Scratch* ws = nullptr, const Touch& next = Touch{}) {
+             hipStream_t s, Scratch* ws = nullptr) {
   GemmArgs g;
-  g.next = next;
   g.out = out; g.c = c; g.a = a; g.b = b; g.bias = bias;
   g.M = (int)M; g.N = (int)N; g.K = (int)K;
   g.lda = lda; g.ldb = ldb; g.ldc = ldc;
@@ -351,7 +350,7 @@ static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p,
                              const void* const* bi, int64_t N, uint32_t act, const Touch& next) -> int {
     NormedGemm n;
     GemmArgs& g = n.g;
-    g.next = next;
+    n.next = next;
     g.out = out; g.c = nullptr; g.a = xs; g.b = nullptr; g.bias = nullptr;
     g.M = (int)rows; g.N = (int)N; g.K = (int)C;
     g.lda = C; g.ldb = N; g.ldc = groups * N;
@@ -408,8 +407,9 @@ static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p,
                             cfg.activation == LH_ACT_RELU ? LH_GEMM_HAS_RELU : LH_GEMM_HAS_GELU, next_w)))
     return rc;
   // y = a + h W2 + b2
+  ws.next = next_block;
   return gemm_run(y, a, hid, p->w_proj, p->b_proj, rows, C, hidden, hidden, C, C, dtype, LH_F32, bdt,
-                  bias_flag(p->b_proj) | LH_GEMM_ACCUMULATE_C, s, &ws, next_block);
+                  bias_flag(p->b_proj) | LH_GEMM_ACCUMULATE_C, s, &ws);
 }
 
 int lh_hip_nanogpt_block(float* y, const float* x, const lh_nanogpt_block_params* p, int64_t B, int64_t T, int64_t C,

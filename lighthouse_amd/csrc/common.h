@@ -249,6 +249,9 @@ struct Scratch {
   size_t bytes = 0;
   size_t used = 0;
   size_t need = 0;
+  // What launches after the call read; the small-tile GEMM kernels touch it.  (Here and not in the kernels' arguments, which cost a
+  // dispatch of any of them 0.1 us more if they were longer.)
+  Touch next;
 };
 int scratch_take(Scratch* ws, hipStream_t s, int slot, size_t bytes, const char* what, void** out);
 bool planning();

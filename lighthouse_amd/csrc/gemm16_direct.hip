@@ -393,7 +393,8 @@ __device__ __forceinline__ void direct_prologue(const DirectCtx<TM, TN>& c, int 
 // together.  The workgroups share out the lines; more than 128 for each cost more at the start than the loop waits for later.
 // bf16, M = 8192, N = 2304, K = 768: 45.6 us with B in memory before, 36.0 now (33.7 and 34.4 with B in the caches); N = 3072
 // 56.6 and 48.2; with 256 lines for each workgroup (2048^3) 28.1 and 29.1.
-// (The launcher decides, and the code lies behind the kernel's: in its way it cost launches that touch nothing 0.1 to 0.3 us.)
+// (The launcher decides, and the code lies behind the kernel's: in its way it cost launches that touch nothing 0.1 to 0.3 us.
+// The 256 x 256 tile has none of it: there a B of so few lines is a short K or a narrow result, and 4096^3 took 0.7 us longer.)
 template <bool BT>
 __device__ __forceinline__ void direct_touch_b(const GemmArgs& g, int wave, uint8_t* __restrict__ stage) {
   const int per_row = ((BT ? g.K : g.N) + 63) / 64, lines = (BT ? g.N : g.K) * per_row, grid = (int)gridDim.x;
@@ -914,7 +915,7 @@ __device__ __forceinline__ void direct_run(const GemmArgs& g) {
     direct_place<TM, TN, EDGE, BT>(SPLITK ? g_cur : g, xcd_remap(id, tiles1), c, m0, n0);
   }
   direct_prologue<TM, TN, TAIL, BT>(c, nk, smem_d);
-  if constexpr (!SPLITK)
+  if constexpr (!SPLITK && TM * TN < 8)
     if (__builtin_expect(g.touch_b, 0)) direct_touch_b<BT>(g, wave, smem_d + Cfg::kRingBytes);
   // Without EDGE every lane issues all stores of a staged epilogue.
   const bool staged = !SPLITK && g.out_dt != LH_F32 && !(g.flags & LH_GEMM_ACCUMULATE_C);

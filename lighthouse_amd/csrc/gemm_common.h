@@ -29,8 +29,6 @@ struct GemmArgs {
   // The operands are copies made for kernels that want K in multiples of this (0: they are the caller's).  Decided once per
   // call: what is decided for the copies themselves may be another multiple, and a second copy would be written over the first.
   uint8_t k_multiple = 0;
-  // What launches after this one read and the small-tile kernels touch for them.
-  Touch next;
 };
 
 // Epilogue for 4 consecutive columns of one row.
@@ -561,6 +559,7 @@ struct NormedGemm {
   const void* b[3];
   const void* bias[3];
   int groups;
+  Touch next;  // what launches after this one read
 };
 // The tile it would run on; -1: the LayerNorm and the products on their own are the faster way, or it does not take them.
 int gemm_normed_choose(const NormedGemm& n, int dtype);

@@ -112,7 +112,7 @@ __device__ __forceinline__ void small_multiply(const typename Cfg::PA& pa, const
 }
 
 template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
-__global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
+__global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g, Touch next) {
   typedef SmallCfg<DT, MT, NT, NW, AKC, BKC> Cfg;
   constexpr int EDT = DT == LH_F8E4M3 ? LH_BF16 : DT;  // the type a 16-bit output, bias or accumulator input has
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_small[];
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
   const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
   const int per_xcd = (tiles_m * tiles_n + 7) / 8;
   if ((int)blockIdx.x >= 8 * per_xcd) {
-    if constexpr (NW == 8) touch_lines(g.next, blockIdx.x - 8 * per_xcd);
+    if constexpr (NW == 8) touch_lines(next, blockIdx.x - 8 * per_xcd);
     return;
   }
   const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
@@ -166,8 +166,8 @@ static int launch_small_layout(const GemmArgs& g, hipStream_t s) {
     configured = true;
   }
   const int tiles = ((g.M + 16 * MT - 1) / (16 * MT)) * ((g.N + 16 * NT - 1) / (16 * NT));
-  const unsigned blocks = 8 * (((unsigned)tiles + 7) / 8), touching = NW == 8 ? touch_blocks(g.next, blocks) : 0;
-  LH_LAUNCH(kern, dim3(blocks + touching), dim3(NW * 64), Cfg::kLdsBytes, s, g);
+  const unsigned blocks = 8 * (((unsigned)tiles + 7) / 8), touching = NW == 8 && g.ws ? touch_blocks(g.ws->next, blocks) : 0;
+  LH_LAUNCH(kern, dim3(blocks + touching), dim3(NW * 64), Cfg::kLdsBytes, s, g, touching ? g.ws->next : Touch{});
   return check_launch("gemm_small");
 }
 

@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
   const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
   const int tiles = tiles_m * tiles_n * n.groups, per_xcd = (tiles + 7) / 8;
   if ((int)blockIdx.x >= 8 * per_xcd) {
-    touch_lines(g.next, blockIdx.x - 8 * per_xcd);
+    touch_lines(n.next, blockIdx.x - 8 * per_xcd);
     return;
   }
   const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
@@ -163,7 +163,7 @@ static int launch_normed_rows(const NormedGemm& n, hipStream_t s) {
   const int tiles = ((n.g.M + 16 * MT - 1) / (16 * MT)) * ((n.g.N + 16 * NT - 1) / (16 * NT)) * n.groups;
   static_assert(NW == 8, "touch_lines counts on 512 threads");
   const unsigned blocks = 8 * (((unsigned)tiles + 7) / 8);
-  LH_LAUNCH(kern, dim3(blocks + touch_blocks(n.g.next, blocks)), dim3(NW * 64), Cfg::kLdsBytes, s, n);
+  LH_LAUNCH(kern, dim3(blocks + touch_blocks(n.next, blocks)), dim3(NW * 64), Cfg::kLdsBytes, s, n);
   return check_launch("gemm_normed");
 }
 
