@@ -456,7 +456,7 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
 #pragma unroll
   for (int i = 0; i < direct_frags(TN); ++i) f.b[i] = direct_read_b<TM, TN, BT>(c, bbuf, 0, i);
   int kt = 0;
-  for (; kt + 2 < nk; kt += 2) {
+  auto pair = [&] {
     uint8_t* a_cur = abuf + ((kt >> 1) & 1) * Cfg::kABytes;
     uint8_t* a_nxt = abuf + (((kt >> 1) + 1) & 1) * Cfg::kABytes;
     if constexpr (BT) {
@@ -471,7 +471,8 @@ __device__ __forceinline__ void direct_mainloop(const GemmArgs& g, const DirectC
       if constexpr (one_barrier) direct_step_pair_1b<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk, stores_behind);
       else direct_step_pair<DT, TM, TN, TAIL>(c, acc, f, a_cur, a_nxt, b1, b2, a_cur, b0, b1, kt, nk);
     }
-  }
+  };
+  for (; kt + 2 < nk; kt += 2) pair();
   {
     // Last two steps: nothing left to load; stage nk - 1 of B must have landed.
     const uint8_t* a_cur = abuf + ((kt >> 1) & 1) * Cfg::kABytes;
