@@ -61,6 +61,17 @@ def test_small_tile_gemms_are_built_for_the_layouts_that_exist(kernels):
     assert {t: of_type.count(t) for t in set(of_type)} == {_lib.F32: 24, _lib.BF16: 24, _lib.F16: 24, _lib.F8E4M3: 6}
 
 
+def test_what_to_touch_is_an_argument_of_the_touching_kernels_alone(kernels):
+    """Arguments cost every dispatch of a kernel, whether a call of it touches the weights of later launches or not."""
+    touching = {n for n in kernels if "5Touch" in n}
+    assert touching and all(re.search(r"gemm_small_touchingILi\dE|gemm_normed_kernelI.*NormedGemmENS_5TouchEj$", n) for n in touching)
+    assert not any(f"touchingILi{_lib.F8E4M3}E" in n for n in touching)
+    for n in touching:  # (each has a twin that takes none)
+        twin = n.replace("NS_5TouchEj", "").replace("small_touching", "small_kernel").replace("_ZN2lh19", "_ZN2lh17")
+        twin = twin.replace("EEEvNS_8Gemm", "ELb1ELb0EEEvNS_8Gemm") if "small" in twin else twin
+        assert kernels[twin]["kernarg_segment_size"] + 44 == kernels[n]["kernarg_segment_size"], n
+
+
 def test_cut_gemms_load_without_loops_over_resources(kernels):
     """The panels of a workgroup are the same for its lanes: a load whose resource the compiler holds in vector registers sits
     in a loop over the lanes' resources (exec is narrowed right before it), which the kernels cut along K once had in
