@@ -350,6 +350,7 @@ static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p,
                              const void* const* bi, int64_t N, uint32_t act, const Touch& next) -> int {
     NormedGemm n;
     GemmArgs& g = n.g;
+    n.next = next;
     g.out = out; g.c = nullptr; g.a = xs; g.b = nullptr; g.bias = nullptr;
     g.M = (int)rows; g.N = (int)N; g.K = (int)C;
     g.lda = C; g.ldb = N; g.ldc = groups * N;
@@ -361,7 +362,7 @@ static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p,
     }
     n.groups = groups;
     const int tile = gemm_normed_choose(n, dtype);
-    if (tile >= 0) return gemm_normed(n, next, dtype, tile, s);
+    if (tile >= 0) return gemm_normed(n, dtype, tile, s);
     if (int e = layer_norm(ln, xs, gamma, beta, rows, C, eps, LH_F32, dtype, false, s)) return e;
     for (int i = 0; i < groups; ++i)
       if (int e2 = gemm_run(static_cast<char*>(out) + (size_t)i * N * e, nullptr, ln, wi[i], bi[i], rows, N, C, C, N, groups * N, dtype,

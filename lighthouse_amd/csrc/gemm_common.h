@@ -559,10 +559,10 @@ struct NormedGemm {
   const void* b[3];
   const void* bias[3];
   int groups;
+  Touch next;  // what launches after this one read
 };
 // The tile it would run on; -1: the LayerNorm and the products on their own are the faster way, or it does not take them.
 int gemm_normed_choose(const NormedGemm& n, int dtype);
-// `next`: what launches after this one read.
-int gemm_normed(const NormedGemm& n, const Touch& next, int dtype, int tile, hipStream_t s);
+int gemm_normed(const NormedGemm& n, int dtype, int tile, hipStream_t s);
 
 }  // namespace lh

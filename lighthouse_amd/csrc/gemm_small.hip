@@ -111,8 +111,9 @@ __device__ __forceinline__ void small_multiply(const typename Cfg::PA& pa, const
   else if (P == 3) run(std::integral_constant<int, P == 3 ? 5 : 1>{});
 }
 
-template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
-__device__ __forceinline__ void small_run(const GemmArgs& g) {
+// `next`: nothing, or the Touch of the launches after this one.
+template <int DT, int MT, int NT, int NW, bool AKC, bool BKC, typename... Next>
+__device__ __forceinline__ void small_run(const GemmArgs& g, const Next&... next) {
   typedef SmallCfg<DT, MT, NT, NW, AKC, BKC> Cfg;
   constexpr int EDT = DT == LH_F8E4M3 ? LH_BF16 : DT;  // the type a 16-bit output, bias or accumulator input has
   extern __shared__ __attribute__((aligned(16))) uint8_t smem_small[];
@@ -123,6 +124,10 @@ __device__ __forceinline__ void small_run(const GemmArgs& g) {
   // share its cache lines.
   const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
   const int per_xcd = (tiles_m * tiles_n + 7) / 8;
+  if constexpr (sizeof...(Next) > 0) {
+    // (their number as an argument, asked for first, cost 0.2 us: the other arguments were loaded behind it)
+    if ((int)blockIdx.x >= 8 * per_xcd) return touch_lines(next..., blockIdx.x - 8 * per_xcd);
+  }
   const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (tile >= tiles_m * tiles_n) return;
   const int m0 = (tile % tiles_m) * 16 * MT, n0 = (tile / tiles_m) * 16 * NT;
@@ -155,12 +160,11 @@ template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
 __global__ void __launch_bounds__(NW * 64) gemm_small_kernel(GemmArgs g) {
   small_run<DT, MT, NT, NW, AKC, BKC>(g);
 }
-// ... of which the workgroups from `blocks` on touch what later launches read.  (A kernel of its own: as an argument of the one above
+// ... of which the workgroups behind those of the work touch what later launches read.  (A kernel of its own: as an argument of the one above
 // what to touch cost every product on small tiles 0.03 to 0.1 us, 1 % of 3.6 us, f32 and fp8 ones that never touch anything too.)
 template <int DT, int MT, int NT, int NW>
-__global__ void __launch_bounds__(NW * 64) gemm_small_touching(GemmArgs g, Touch next, unsigned blocks) {
-  if (blockIdx.x >= blocks) touch_lines(next, blockIdx.x - blocks);
-  else small_run<DT, MT, NT, NW, true, false>(g);
+__global__ void __launch_bounds__(NW * 64) gemm_small_touching(GemmArgs g, Touch next) {
+  small_run<DT, MT, NT, NW, true, false>(g, next);
 }
 
 template <int DT, int MT, int NT, int NW, bool AKC, bool BKC>
@@ -181,7 +185,7 @@ static int launch_small_layout(const GemmArgs& g, hipStream_t s) {
   // (what touches is the nanoGPT block, whose operands are untransposed and not fp8)
   if constexpr (NW == 8 && AKC && !BKC && DT != LH_F8E4M3) {
     if (const unsigned touching = g.ws ? touch_blocks(g.ws->next, blocks) : 0)
-      return launch(gemm_small_touching<DT, MT, NT, NW>, blocks + touching, g.ws->next, blocks);
+      return launch(gemm_small_touching<DT, MT, NT, NW>, blocks + touching, g.ws->next);
   }
   return launch(gemm_small_kernel<DT, MT, NT, NW, AKC, BKC>, blocks);
 }

@@ -45,7 +45,7 @@ struct NormCfg {
 };
 
 template <int DT, int MT, int NT, int NW, int V>
-__device__ __forceinline__ void normed_run(const NormedGemm& n) {
+__global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
   typedef NormCfg<DT, MT, NT, NW, V> Cfg;
   constexpr int K = Cfg::K, KSTEP = Cfg::KSTEP, P = Cfg::P, ES = Cfg::ES;
   constexpr int R = 8 * MT / NW;  // pairs of rows a wave normalises
@@ -57,6 +57,10 @@ __device__ __forceinline__ void normed_run(const NormedGemm& n) {
   // (tiles to workgroups as in gemm_small_kernel, the groups of columns one behind the other)
   const int tiles_m = (g.M + 16 * MT - 1) / (16 * MT), tiles_n = (g.N + 16 * NT - 1) / (16 * NT);
   const int tiles = tiles_m * tiles_n * n.groups, per_xcd = (tiles + 7) / 8;
+  if ((int)blockIdx.x >= 8 * per_xcd) {
+    touch_lines(n.next, blockIdx.x - 8 * per_xcd);
+    return;
+  }
   const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (tile >= tiles) return;
   const int panel = tile / tiles_m, group = panel / tiles_n;
@@ -147,50 +151,33 @@ __device__ __forceinline__ void normed_run(const NormedGemm& n) {
 }
 
 template <int DT, int MT, int NT, int NW, int V>
-__global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n) {
-  normed_run<DT, MT, NT, NW, V>(n);
-}
-// ... of which the workgroups from `blocks` on touch what later launches read (as in gemm_small.hip).
-template <int DT, int MT, int NT, int NW, int V>
-__global__ void __launch_bounds__(NW * 64) gemm_normed_kernel(NormedGemm n, Touch next, unsigned blocks) {
-  static_assert(NW == 8, "touch_lines counts on 512 threads");
-  if (blockIdx.x >= blocks) touch_lines(next, blockIdx.x - blocks);
-  else normed_run<DT, MT, NT, NW, V>(n);
-}
-
-template <int DT, int MT, int NT, int NW, int V>
-static int launch_normed_rows(const NormedGemm& n, const Touch& next, hipStream_t s) {
+static int launch_normed_rows(const NormedGemm& n, hipStream_t s) {
   typedef NormCfg<DT, MT, NT, NW, V> Cfg;
+  auto kern = gemm_normed_kernel<DT, MT, NT, NW, V>;
+  static bool configured = false;
+  if (Cfg::kLdsBytes > 64 * 1024 && !configured && !planning()) {
+    LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     Cfg::kLdsBytes));
+    configured = true;
+  }
   const int tiles = ((n.g.M + 16 * MT - 1) / (16 * MT)) * ((n.g.N + 16 * NT - 1) / (16 * NT)) * n.groups;
+  static_assert(NW == 8, "touch_lines counts on 512 threads");
   const unsigned blocks = 8 * (((unsigned)tiles + 7) / 8);
-  using Plain = void (*)(NormedGemm);
-  using Touching = void (*)(NormedGemm, Touch, unsigned);
-  const auto launch = [&](auto kern, unsigned grid, auto... more) -> int {
-    static bool configured = false;
-    if (Cfg::kLdsBytes > 64 * 1024 && !configured && !planning()) {
-      LH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       Cfg::kLdsBytes));
-      configured = true;
-    }
-    LH_LAUNCH(kern, dim3(grid), dim3(NW * 64), Cfg::kLdsBytes, s, n, more...);
-    return check_launch("gemm_normed");
-  };
-  if (const unsigned touching = touch_blocks(next, blocks))
-    return launch(Touching(gemm_normed_kernel<DT, MT, NT, NW, V>), blocks + touching, next, blocks);
-  return launch(Plain(gemm_normed_kernel<DT, MT, NT, NW, V>), blocks);
+  LH_LAUNCH(kern, dim3(blocks + touch_blocks(n.next, blocks)), dim3(NW * 64), Cfg::kLdsBytes, s, n);
+  return check_launch("gemm_normed");
 }
 
 template <int DT, int MT, int NT, int NW>
-static int launch_normed(const NormedGemm& n, const Touch& next, hipStream_t s) {
+static int launch_normed(const NormedGemm& n, hipStream_t s) {
   switch (n.g.K / 128) {
-    case 1: return launch_normed_rows<DT, MT, NT, NW, 1>(n, next, s);
-    case 2: return launch_normed_rows<DT, MT, NT, NW, 2>(n, next, s);
-    case 3: return launch_normed_rows<DT, MT, NT, NW, 3>(n, next, s);
-    case 4: return launch_normed_rows<DT, MT, NT, NW, 4>(n, next, s);
-    case 5: return launch_normed_rows<DT, MT, NT, NW, 5>(n, next, s);
-    case 6: return launch_normed_rows<DT, MT, NT, NW, 6>(n, next, s);
-    case 7: return launch_normed_rows<DT, MT, NT, NW, 7>(n, next, s);
-    default: return launch_normed_rows<DT, MT, NT, NW, 8>(n, next, s);
+    case 1: return launch_normed_rows<DT, MT, NT, NW, 1>(n, s);
+    case 2: return launch_normed_rows<DT, MT, NT, NW, 2>(n, s);
+    case 3: return launch_normed_rows<DT, MT, NT, NW, 3>(n, s);
+    case 4: return launch_normed_rows<DT, MT, NT, NW, 4>(n, s);
+    case 5: return launch_normed_rows<DT, MT, NT, NW, 5>(n, s);
+    case 6: return launch_normed_rows<DT, MT, NT, NW, 6>(n, s);
+    case 7: return launch_normed_rows<DT, MT, NT, NW, 7>(n, s);
+    default: return launch_normed_rows<DT, MT, NT, NW, 8>(n, s);
   }
 }
 
@@ -239,10 +226,10 @@ int gemm_normed_choose(const NormedGemm& n, int dtype) {
   return best < apart ? tile : -1;
 }
 
-int gemm_normed(const NormedGemm& n, const Touch& next, int dtype, int tile, hipStream_t s) {
+int gemm_normed(const NormedGemm& n, int dtype, int tile, hipStream_t s) {
   if (dtype == LH_BF16)
-    return tile == 0 ? launch_normed<LH_BF16, 1, 2, 8>(n, next, s) : tile == 1 ? launch_normed<LH_BF16, 1, 4, 8>(n, next, s) : launch_normed<LH_BF16, 2, 4, 8>(n, next, s);
-  return tile == 0 ? launch_normed<LH_F16, 1, 2, 8>(n, next, s) : tile == 1 ? launch_normed<LH_F16, 1, 4, 8>(n, next, s) : launch_normed<LH_F16, 2, 4, 8>(n, next, s);
+    return tile == 0 ? launch_normed<LH_BF16, 1, 2, 8>(n, s) : tile == 1 ? launch_normed<LH_BF16, 1, 4, 8>(n, s) : launch_normed<LH_BF16, 2, 4, 8>(n, s);
+  return tile == 0 ? launch_normed<LH_F16, 1, 2, 8>(n, s) : tile == 1 ? launch_normed<LH_F16, 1, 4, 8>(n, s) : launch_normed<LH_F16, 2, 4, 8>(n, s);
 }
 
 }  // namespace lh
