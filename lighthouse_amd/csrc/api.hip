@@ -318,10 +318,17 @@ size_t lh_hip_nanogpt_block_workspace_bytes(int64_t B, int64_t T, int64_t C, int
 
 // The block's launches; `workspace` is large enough (a size query is not free: the forward asks once for all its blocks).
 // With few rows a launch waits for its weights, which a network of more weights than the memory-side cache holds gets from memory
-// in every pass.  So the MLP's first product touches its second one's, and that those of the block `after` this one.  Forward of one
-// prompt of 100 tokens, 12 blocks of 768 and a head of 50257 words, bf16: 511 -> 463 us (464 -> 389 with the same weights in
-// every block).  The first launch, which takes a whole round of CUs, and the two short ones behind it touch nothing: they
+// in every pass.  So the MLP's first product touches its second one's, and that those of the block `after` this one, where each is
+// one launch that leaves CUs for it (touch_blocks); the down-projection on 16 x 16 tiles of 16 waves, which it takes at 768 up to 64 rows,
+// touches nothing.  Forward of one prompt of 100 tokens, 12 blocks of 768 and a head of 50257 words, bf16: 511 -> 463 us (464 -> 389 with the
+// same weights in every block).  The first launch, which takes a whole round of CUs, and the two short ones behind it touch nothing: they
 // would last longer for it (543 us with the attention and the projection touching, 516 with the first).
+// The first product touches from C = 384 on: below, its launch is over before the weights are there.  Forwards of 12 blocks over
+// 8 ... 200 rows, without and with it, us, weights out of memory / in the caches: C = 256 257 -> 268 to 287 -> 297 / 0 to 2 % more; C = 384
+// 323 -> 318 (16 rows), 355 -> 347 (220), others the same / 1 % more; C = 512 359 -> 331 (8 rows), 368 -> 348 (100), 385 -> 356 (150), 64 rows the same / 0 to 1 % more; C = 768 451 -> 414 (16),
+// 469 -> 420 (100) / 0 to 1 % more; 160 rows, where no CUs are left, the same.  A block on its own: 16 x 768 35.5 -> 32.6 / 27.1 -> 27.7,
+// 100 x 768 37.2 -> 35.2 / 31.4 -> 31.8, 16 x 1024 43.3 -> 38.4 / 30.9 -> 33.2 (the most it costs: so few rows wait for the
+// memory's bandwidth already).
 static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p, int64_t B, int64_t T, int64_t C, int64_t n_head,
                      float eps, int32_t dtype, const BlockConfig& cfg, void* workspace, size_t workspace_bytes, void* stream,
                      const lh_nanogpt_block_params* after = nullptr) {
@@ -394,13 +401,13 @@ static int block_run(float* y, const float* x, const lh_nanogpt_block_params* p,
                      bias_flag(p->b_o) | LH_GEMM_ACCUMULATE_C, s, &ws)))
     return rc;
   Touch next_w, next_block;
-  next_w.add(p->w_proj, (size_t)hidden * C * e);
-  if (after) {
-    if (after->w_qkv) next_block.add(after->w_qkv, (size_t)C * 3 * C * e);
-    else
-      for (const void* w1 : {after->w_q, after->w_k, after->w_v}) next_block.add(w1, (size_t)C * C * e);
+  if (C >= 384) next_w.add(p->w_proj, (size_t)hidden * C * e);
+  if (after && after->w_qkv) {
+    next_block.add(after->w_qkv, (size_t)C * 3 * C * e);
     next_block.add(after->w_o, (size_t)C * C * e);
     next_block.add(after->w_fc, (size_t)C * hidden * e);
+  } else if (after) {  // (three ranges are all there is room for)
+    for (const void* w1 : {after->w_q, after->w_k, after->w_v}) next_block.add(w1, (size_t)C * C * e);
   }
   // h = act(LN(a) W1 + b1)
   if ((rc = normed_products(hid, a, p->ln2_g, p->ln2_b, 1, &p->w_fc, &p->b_fc, hidden,

@@ -169,15 +169,15 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
 }
 
 // ---- weights on their way ---------------------------------------------------------------------
-// Memory that launches after this one read, up to three ranges.  A kernel of few rows leaves CUs and most of the memory's
-// bandwidth idle; workgroups of its own behind those of the work touch 4 bytes of every 128 of it, so that the launch that
-// reads it finds it in the memory-side cache.  The launch lasts until they are done: worth it only where they have CUs to
-// themselves and the work takes longer than they do.
+// Memory that launches after this one read, up to three ranges.  A kernel of few rows leaves CUs and memory bandwidth idle;
+// workgroups of its own behind those of the work touch 2 bytes of every 128 of it, so that the launch that reads it finds
+// it in the memory-side cache.  The launch lasts until they are done.  So they are launched only where they and the work all get
+// CUs to themselves, all of them or none (touch_blocks); that the work takes longer than they do is for the caller to know.
 int num_cus();
 struct Touch {
   const void* p[3] = {};
   uint32_t lines[3] = {};
-  void add(const void* range, size_t bytes) {  // (a fourth is dropped)
+  void add(const void* range, size_t bytes) {  // (of elements of 2 or 4 bytes; three times at most)
     for (int i = 0; i < 3 && range && bytes < 1u << 28; ++i)
       if (!lines[i]) {
         p[i] = range;
@@ -202,12 +202,12 @@ __device__ __forceinline__ void touch_lines(const Touch& t, unsigned block) {
   const uint64_t range = in2 ? p2 : in1 ? p1 : p0;
   const uint32_t lines = in2 ? l2 : in1 ? l1 : l0;
   block -= in2 ? first2 : in1 ? first1 : 0;
-  const uint8_t* const p = reinterpret_cast<const uint8_t*>(range & ~3ull);
+  const uint8_t* const p = reinterpret_cast<const uint8_t*>(range);
   uint32_t v[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const uint32_t line = min(block * 2048 + 512 * i + threadIdx.x, lines - 1);
-    v[i] = *reinterpret_cast<const uint32_t*>(p + (size_t)line * 128);
+    v[i] = *reinterpret_cast<const uint16_t*>(p + (size_t)line * 128);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) asm volatile("" ::"v"(v[i]));
@@ -249,8 +249,8 @@ struct Scratch {
   size_t bytes = 0;
   size_t used = 0;
   size_t need = 0;
-  // What launches after the call read; the small-tile GEMM kernels touch it.  (Here and not in the kernels' arguments, which cost a
-  // dispatch of any of them 0.1 us more if they were longer.)
+  // What launches after the call read; small-tile GEMM kernels with 8 waves touch it.  (Here and not in GemmArgs, which cost a
+  // dispatch of every GEMM kernel 0.1 us more if they were longer.)
   Touch next;
 };
 int scratch_take(Scratch* ws, hipStream_t s, int slot, size_t bytes, const char* what, void** out);

@@ -15,7 +15,7 @@ struct Launch {
   const char* name;       // mangled name of the kernel
   uint32_t grid, block;   // along x
   unsigned char arg0[80]; // the first argument (GemmArgs up to its strides, or PadCopy)
-  unsigned char arg1[48]; // the second (PadCopy)
+  unsigned char arg1[48]; // the second (PadCopy, or Touch, which ends a NormedGemm)
 };
 
 static std::map<const void*, std::string> names;
@@ -61,6 +61,8 @@ int hipLaunchKernel(const void* host, dim3 grid, dim3 block, void** args, size_t
     std::memcpy(l.arg1, args[1], 48);
   } else if (std::strstr(l.name, "gemm") != nullptr && std::strstr(l.name, "reduce") == nullptr) {
     std::memcpy(l.arg0, args[0], sizeof(l.arg0));
+    if (std::strstr(l.name, "5Touch") != nullptr) std::memcpy(l.arg1, args[1], 40);
+    if (std::strstr(l.name, "gemm_normed") != nullptr) std::memcpy(l.arg1, static_cast<unsigned char*>(args[0]) + 200, 40);
   }
   launches.push_back(l);
   return 0;

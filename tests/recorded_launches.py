@@ -22,6 +22,10 @@ class GemmArgs(ctypes.Structure):
                [(n, ctypes.c_int32) for n in ("M", "N", "K")] + [(n, ctypes.c_int64) for n in ("lda", "ldb", "ldc")]
 
 
+class Touch(ctypes.Structure):
+    _fields_ = [("p", ctypes.c_uint64 * 3), ("lines", ctypes.c_uint32 * 3)]
+
+
 class Launch(ctypes.Structure):
     _fields_ = [("mangled", ctypes.c_char_p), ("grid", ctypes.c_uint32), ("block", ctypes.c_uint32),
                 ("arg0", ctypes.c_ubyte * 80), ("arg1", ctypes.c_ubyte * 48)]
@@ -33,6 +37,12 @@ class Launch(ctypes.Structure):
     @property
     def gemm(self):
         return GemmArgs.from_buffer_copy(self.arg0)
+
+    @property
+    def touched(self):
+        """(first byte, lines of 128 bytes) of each range that the launch touches for later ones."""
+        t = Touch.from_buffer_copy(self.arg1) if "5Touch" in self.name or "gemm_normed" in self.name else Touch()
+        return [(p, n) for p, n in zip(t.p, t.lines) if n]
 
     @property
     def copies(self):
