@@ -1098,7 +1098,10 @@ __global__ void __launch_bounds__(512) gemm16_deep(GemmArgs g) {
   for (int i = 0; i < Cfg::NF; ++i)
 #pragma unroll
     for (int j = 0; j < 2 * TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // (the first stage; those behind it may be on their way)
   if (pairs >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * Deep::kLoads) : "memory");
+  else if (S > 3 && pairs == 3) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * Deep::kLoads) : "memory");
+  else if (pairs == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Deep::kLoads) : "memory");
   else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   DirectFrags<TM, TN> f;
   direct_read_a<TM, TN, 0>(c, a_stage(0), 0, f.a[0]);
