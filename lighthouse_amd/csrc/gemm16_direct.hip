@@ -393,8 +393,12 @@ __device__ __forceinline__ void direct_prologue(const DirectCtx<TM, TN>& c, int 
 // together.  The workgroups share out the lines; more than 128 for each cost more at the start than the loop waits for later.
 // bf16, M = 8192, N = 2304, K = 768: 45.6 us with B in memory before, 36.0 now (33.7 and 34.4 with B in the caches); N = 3072
 // 56.6 and 48.2; with 256 lines for each workgroup (2048^3) 28.1 and 29.1.
+// From K = 512 on.  Over 1700 products of 257 to 2048 tiles of 128 x 128, on it / without it, operands in the caches, B in memory, all in
+// memory: K <= 448 1.010, 1.004, 1.000; 512 and 576 1.008, 1.000, 0.992; 640 ... 896 1.008, 0.992, 0.988; above 1.002, 0.970, 0.991 (B stored [N, K] gains
+// a little earlier, at 512 0.98 with B in memory, and [K, N] later).
 // (The launcher decides, and the code lies behind the kernel's: in its way it cost launches that touch nothing 0.1 to 0.3 us.
 // The 256 x 256 tile has none of it: there a B of so few lines is a short K or a narrow result, and 4096^3 took 0.7 us longer.)
+constexpr int kTouchFrom = 512;
 template <bool BT>
 __device__ __forceinline__ void direct_touch_b(const GemmArgs& g, int wave, uint8_t* __restrict__ stage) {
   const int per_row = ((BT ? g.K : g.N) + 63) / 64, lines = (BT ? g.N : g.K) * per_row, grid = (int)gridDim.x;
@@ -989,7 +993,7 @@ static int launch_direct_edge(const GemmArgs& g, hipStream_t s) {
   GemmArgs ga = g;
   const int grid = ntiles < resident ? ntiles : resident;
   const int64_t rows = BT ? g.N : g.K;
-  ga.touch_b = rows * (((BT ? g.K : g.N) + 63) / 64) <= 128 * grid && rows * g.ldb < (1ll << 30);
+  ga.touch_b = g.K >= kTouchFrom && rows * (((BT ? g.K : g.N) + 63) / 64) <= 128 * grid && rows * g.ldb < (1ll << 30);
   LH_LAUNCH(kern, dim3(grid), dim3(512), lds, s, ga);
   return check_launch("gemm16_direct");
 }

@@ -14,7 +14,7 @@ struct dim3 {
 struct Launch {
   const char* name;       // mangled name of the kernel
   uint32_t grid, block;   // along x
-  unsigned char arg0[80]; // the first argument (GemmArgs up to its strides, or PadCopy)
+  unsigned char arg0[120]; // the first argument (GemmArgs, or PadCopy)
   unsigned char arg1[48]; // the second (PadCopy, or Touch, which ends a NormedGemm)
 };
 

@@ -19,7 +19,9 @@ class PadCopy(ctypes.Structure):
 
 class GemmArgs(ctypes.Structure):
     _fields_ = [(n, ctypes.c_uint64) for n in ("out", "c", "a", "b", "bias")] + \
-               [(n, ctypes.c_int32) for n in ("M", "N", "K")] + [(n, ctypes.c_int64) for n in ("lda", "ldb", "ldc")]
+               [(n, ctypes.c_int32) for n in ("M", "N", "K")] + [(n, ctypes.c_int64) for n in ("lda", "ldb", "ldc")] + \
+               [(n, ctypes.c_int32) for n in ("flags", "out_dt", "bias_dt")] + [("alpha", ctypes.c_float), ("splits", ctypes.c_int32)] + \
+               [("ws", ctypes.c_uint64), ("touch_b", ctypes.c_int32)]
 
 
 class Touch(ctypes.Structure):
@@ -28,7 +30,7 @@ class Touch(ctypes.Structure):
 
 class Launch(ctypes.Structure):
     _fields_ = [("mangled", ctypes.c_char_p), ("grid", ctypes.c_uint32), ("block", ctypes.c_uint32),
-                ("arg0", ctypes.c_ubyte * 80), ("arg1", ctypes.c_ubyte * 48)]
+                ("arg0", ctypes.c_ubyte * 120), ("arg1", ctypes.c_ubyte * 48)]
 
     @property
     def name(self):

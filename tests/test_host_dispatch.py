@@ -158,6 +158,22 @@ def test_columns_of_a_wide_buffer_are_no_large_result(recorded):
     recorded(_large_results)
 
 
+def _touching(r):
+    def touches(M, N, K, flags=0):
+        rc, launches = r.calls("lh_hip_gemm", OUT, A, B, BIAS, M, N, K, K, K if flags & 16 else N, N, DT, DT, flags, None)
+        assert rc == 0 and len(launches) == 1 and "gemm16_direct" in launches[0].name, r.lib.lh_hip_last_error()
+        return bool(launches[0].gemm.touch_b)
+
+    for flags in (0, 16):  # (1152 tiles of 128 x 128 on 512 workgroups, 288 on as many)
+        assert [touches(8192, 2304, K, flags) for K in (128, 448, 512, 768, 1792, 2048)] == [False, False, True, True, True, False]
+        assert [touches(3072, 1536, K, flags) for K in (448, 504, 512, 520)] == [False, False, True, True]
+
+
+def test_a_long_enough_b_of_few_lines_is_touched(recorded):
+    """What the direct kernels touch at the start: from K = 512 on, up to 128 lines of B for every workgroup."""
+    recorded(_touching)
+
+
 def _normed(r, sizes):
     """The tiles (rows, columns of 16) and widths (of 128) of the launches that normalise rows and multiply them, by size and type."""
     lib, found = rec._lib, {}
