@@ -12,6 +12,8 @@
 //
 // Generic kernel: any shape, stride and transpose combination, 64 x 64 x 32 tiles with
 // bounds-checked scalar loads.
+#include <algorithm>
+
 #include "gemm16.h"
 
 namespace lh {
@@ -389,15 +391,15 @@ static int direct_k_multiple(const GemmArgs& g) {
 // A B that the loads into LDS cannot take (rows that are no whole aligned 16-byte chunks) is read as it is where one round of
 // workgroups of the 128 x 128 tile covers the result: the copy in a launch of its own is a good part of such a product's time.
 // Larger ones spread it over more rows of A and have the larger tiles besides; with two workgroups on a CU and a long K the tile
-// on a copy catches up (2048 x 3999 x 4096, B in memory: 84.7 us on a copy, 85.6 as it is; one workgroup, 2000 x 2001 x 4096:
-// 49.6 and 41.4).
+// on a copy catches up: 84 such products, as it is against on a copy, 0.69 of the time for K <= 512, 0.84 up to 1536, 0.87 up to 2560 and
+// 1.10 up to 3072 (3146 x 1547 x 2784 49.0 us on a copy, 55.4 as it is; one workgroup, 2000 x 2001 x 4096: 49.6 and 41.4).
 static bool odd_rows_stay(const GemmArgs& g) {
   if (planning() || g.b_padded || (g.flags & (LH_GEMM_TILE_MASK | LH_GEMM_SPLITK_MASK | LH_GEMM_TRANSPOSE_A | LH_GEMM_TRANSPOSE_B)))
     return false;
   if (g.N % 8 == 0 && g.ldb % 8 == 0 && aligned16(g.b)) return false;
   const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
   return g.N >= 8 && g.K % 8 == 0 && g.lda % 8 == 0 && aligned16(g.a) && (int64_t)g.M * g.N * g.K >= (1 << 22) &&
-         (tiles <= num_cus() || (tiles <= 2 * num_cus() && g.K <= 3072)) && direct_offsets_fit(g) && splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) == 1;
+         (tiles <= num_cus() || (tiles <= 2 * num_cus() && g.K <= 2560)) && direct_offsets_fit(g) && splitk_count(g.M, g.N, (g.K + kBK - 1) / kBK * kBK) == 1;
 }
 
 // Decode shapes: so few 128 x 128 tiles that most CUs would idle, and a K long enough to cut.
@@ -465,8 +467,13 @@ static int gemm16_dispatch(const GemmArgs& g_in, hipStream_t s) {
                       aligned16(g.a) && aligned16(g.b);
     // (a copy has whole k-steps where kmul says so)
     const int cuts = may_copy && !(g.flags & LH_GEMM_SPLITK_MASK) ? splitk_count(g.M, g.N, (g.K + kmul - 1) / kmul * kmul) : 1;
+    // B in odd rows takes 1.25 of the direct kernels' time (median 1.28 on 1000 products) and no copy.  855 of them, M 1 ... 8192,
+    // N 65 ... 16384, K 64 ... 8192: chosen so 0.3 % slower than the better of the two on average, one of them slower than with the copy
+    // counted alone, by 1.23 (priced at 1.0 37 were, 8 x 14521 x 1552 10.5 -> 21.7 us).  An f32 result counts the copy: the small tiles
+    // add up eight shares of K, and one chain of sums instead would be 1.2 (K = 128) to 3 times (K = 7000) as far from 64 bits.
     const bool odd_rows = odd_rows_stay(g);
-    const double other = direct_us(g, cuts) + (odd_rows ? 0.0 : operand_copies_us<2>(g, kmul, 8, b_in_place, 0.65));
+    double other = direct_us(g, cuts) + operand_copies_us<2>(g, kmul, 8, b_in_place, 0.65);
+    if (odd_rows && g.out_dt != LH_F32) other = std::min(other, 1.25 * direct_us(g, 1));
     int tile;
     const double us = gemm_small_choose(g, DT, &tile);
     if (tile >= 0 && (us * kSmallMargin < other || (!fits && (int64_t)g.M * g.N * g.K < (1 << 22)))) return gemm_small(g, DT, tile, s);

@@ -37,12 +37,13 @@ def test_odd_rows(M, N, K, pad, offset, dtype):
     assert torch.equal(got, torch.relu(want + bias).to(DTYPES[dtype]))
 
 
-def _names(so, sizes):
+def _names(so, sizes, f32=False):
     r = rec.Recorder(so)
     found = {}
     for M, N, K, pad, offset in sizes:
         for dt in (rec._lib.BF16, rec._lib.F16):
-            rc, launches = r.calls("lh_hip_gemm", 1 << 50, 2 << 50, (3 << 50) + 2 * offset, 4 << 50, M, N, K, K, N + pad, N, dt, dt, 1, None)
+            rc, launches = r.calls("lh_hip_gemm", 1 << 50, 2 << 50, (3 << 50) + 2 * offset, 4 << 50, M, N, K, K, N + pad, N, dt,
+                                   rec._lib.F32 if f32 else dt, 1, None)
             assert rc == 0, r.lib.lh_hip_last_error()
             found[M, N, K, pad, offset, dt] = [launch.name for launch in launches]
     return found
@@ -59,3 +60,19 @@ def test_who_takes_odd_rows(tmp_path):
             assert not any("gemm16_odd_rows" in n for n in names), (M, N, K, names)
         else:
             assert len(names) == 1 and f"gemm16_odd_rowsILi{1 if dt == rec._lib.BF16 else 2}ELb{int(K % 64 != 0)}E" in names[0], (M, N, K, names)
+
+
+def test_few_rows_stay_on_the_small_tiles(tmp_path):
+    """Where they are the faster kernels, and for every f32 result that they take: their sums over eight shares of K are nearer to
+    64 bits than one chain.  A long K with two workgroups on a CU is faster on a copy."""
+    small = [(8, 14521, 1552, 0, 0), (32, 13636, 2344, 0, 0), (1, 15466, 792, 0, 0), (2319, 267, 368, 0, 0)]
+    odd = [(256, 12202, 536, 0, 0), (196, 5130, 264, 0, 0), (2747, 442, 472, 0, 0)]  # (f32 results: the small tiles)
+    both = [(3353, 541, 3528, 0, 0), (1000, 4097, 1000, 0, 0), (100, 50257, 768, 0, 0), (3146, 1547, 2560, 0, 0)]
+    copied = [(3146, 1547, 2784, 0, 0), (4928, 903, 2944, 0, 0)]
+    kind = lambda names: "small" if "gemm_small" in names[0] else "odd" if "gemm16_odd_rows" in names[0] else "copied"  # noqa: E731
+    with multiprocessing.get_context("spawn").Pool(1) as pool:
+        so = rec.build(tmp_path)
+        for f32, expected in ((False, {"small": small, "odd": odd + both, "copied": copied}), (True, {"small": small + odd, "odd": both, "copied": copied})):
+            for want, sizes in expected.items():
+                for size, names in pool.apply(_names, (so, sizes, f32)).items():
+                    assert kind(names) == want and (len(names) > 1) == (want == "copied"), (size, f32, names)
