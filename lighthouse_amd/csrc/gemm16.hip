@@ -251,10 +251,14 @@ static int launch_fast(const GemmArgs& g, hipStream_t s) {
 // on a CU.  A last round that does not fill the CUs costs less than a full one: the persistent workgroups are not in step, so the
 // extra tiles run while others still finish, and fewer busy CUs hold a higher clock.  Of a round, a fraction r costs
 // part + (1 - part) r^2 (the 128 x 128 tile: r).  Least squares over 1870 problems on each of the first four tiles (M 128 ... 8192,
-// N 512 ... 50256, K 256 ... 4096); what is chosen is within 0.9 % of the best tile on average, 1.24 x at worst (the rule
-// before it, which priced a tile by its flops, 2.4 to 5.0 %, 1.67 x).
+// N 512 ... 50256, K 256 ... 4096), on rings of two stages: what was chosen was within 0.9 % of the best tile on average, 1.24 x at worst (the
+// rule before it, which priced a tile by its flops, 2.4 to 5.0 %, 1.67 x).
 // Where no CU gets a second workgroup all but the 256 x 256 tile, which fills the LDS as it is, run with deeper rings
 // (gemm16_deep), and 128 x 192 for nothing else; `alone`, fitted to 4096 x 2048, 4096 x 1536, 2048 x 2048 and 8192 x 768 over K = 512 ... 4096.
+// Both tables together, over 3950 problems of 60 to 1024 tiles of 128 x 128 of which some tile gives no CU two workgroups (M 129 ... 8192, N 64 ... 8192,
+// K 64 ... 5000, either B, every kind of output, edges and partial rounds among them) on every tile: within 0.9 % of the best one on average with
+// operands in the caches, 1.33 x at worst, 0.5 % and 1.24 x from memory.  Against the table without `alone` and rings of two stages 0.91 and 0.88 of
+// the time; 0.6 % of them take 3 % longer or more (3840 x 2048 x 128 into f32: 9.7 -> 10.9 us on 256 x 128).
 // bf16, what was chosen without and with it, operands in the caches / in memory: 8192 x 768 x 3072 with a residual 43.6 -> 40.1 /
 // 56.8 -> 49.2 us (128 x 192), K = 768 19.7 -> 18.7 / 27.2 -> 24.9, 4096 x 1536 x 2048 29.0 -> 26.5 / 34.0 -> 30.2, 4096 x 2048 x 2048 33.1 -> 32.3 /
 // 39.2 -> 35.2 (256 x 128), with f32 results 34.2 -> 33.7 / 46.8 -> 38.5 (128 x 256).

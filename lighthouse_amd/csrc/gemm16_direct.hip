@@ -1,7 +1,8 @@
 // Direct-to-LDS GEMM kernels for 16-bit inputs.  This source is compiled once per instantiation (the objects
 // are what takes long to build): LH_GEMM16_DT the element type, LH_GEMM16_TM and LH_GEMM16_TN the workgroup tile
 // (64 TM) x (128 TN); LH_GEMM16_TM 0: the launches cut along K; LH_GEMM16_LARGE 1: the launches of large results (256 x 256); LH_GEMM16_ODD 1:
-// the 128 x 128 tile on a B in rows of any length; LH_GEMM16_DEEP 1: the 128 x 128 tile where no CU gets two.
+// the 128 x 128 tile on a B in rows of any length; LH_GEMM16_DEEP 1: the tile (128 x 128, 128 x 192, 128 x 256, 256 x 128) where no CU gets
+// two workgroups.
 #include <type_traits>
 
 #include "gemm16.h"
@@ -718,10 +719,10 @@ __device__ __forceinline__ void direct_finish(const GemmArgs& g, const DirectCtx
     auto body = [&](auto variant, auto out32_c, auto has_c_c) {
       using E = decltype(variant);
       constexpr bool out32 = decltype(out32_c)::value, has_c = decltype(has_c_c)::value;
-      // The 128 x 128 tile requests its whole accumulator input up front (8 row segments per lane, all
-      // in flight at once) instead of block by block between the stores of the blocks before, which the
-      // loads cannot pass (input and output may be the same buffer): one exposed memory latency per
-      // tile instead of eight.  The larger tiles have no registers for that.
+      // The 128 x 128 and 128 x 192 tiles request their whole accumulator input up front (8 and 12 row
+      // segments per lane, all in flight at once) instead of block by block between the stores of the
+      // blocks before, which the loads cannot pass (input and output may be the same buffer): one exposed
+      // memory latency per tile instead of eight or twelve.  The larger tiles have no registers for that.
       constexpr bool kPreloadC = TM == 2 && TN != 2 && has_c;
       constexpr int NPASS = 32 / rows_per_pass;
       auto load_c = [&](int64_t off, int n) -> f32x4 {
@@ -1025,9 +1026,13 @@ int launch_direct_large(const GemmArgs& g, bool whole, hipStream_t s) {
 #if LH_GEMM16_DEEP || LH_GEMM16_TM == 0
 // ---- one workgroup per CU ---------------------------------------------------------------------
 // Where no CU gets a second workgroup nobody covers the latency of its operands, but all of the CU's LDS is its own.  Both rings
-// hold four stages of 64 k (128 x 128 and 128 x 192 tiles; 128 x 256 and 256 x 128: three), so that a stage is requested two to four pairs of
+// hold four stages of 64 k (128 x 128 and 128 x 192 tiles; 128 x 256 and 256 x 128: three), so that a stage is requested three (two) pairs of
 // steps before it is read, through one barrier per pair; what one of them takes, 0.45 us at 128 x 128, is less than a line's way out
 // of memory.  One tile per workgroup: the output is staged in the idle rings.
+// The price: 128 KiB of a CU's LDS at 128 x 128 (two stages: 80), 144 to 160 at the others, so that products on two streams no longer share
+// CUs.  Two of one size, each on a stream of its own, us per pair with two stages and with four: 2048^3 32.5 -> 35.8, 8192 x 768 x 768
+// 19.9 -> 23.0, 1000 x 4096 x 1000 19.8 -> 22.7 (tiles for more than half of the CUs); 1536 x 1536 x 1024 15.0 -> 13.8, 2048 x 1024 x 1024
+// 14.2 -> 11.6 (for less).
 // bf16, with two stages (and two barriers) and with four, operands in the caches / in memory: 2048^3 23.5 -> 20.5 / 28.3 -> 22.4 us,
 // on a transposed B 22.8 -> 18.8 / 30.9 -> 21.7; 512 x 8192 x 2048 21.9 -> 19.3 / 28.2 -> 22.3; 2048 x 768 x 768 with a residual 11.3 -> 9.7 /
 // 16.6 -> 13.6.
@@ -1184,7 +1189,7 @@ __device__ __forceinline__ void odd_request(const GemmArgs& g, const OddRows& o,
   for (int i = 0; i < 2; ++i) {
     if constexpr (LAST) {
       const int k = min(64 * p + 32 * i + o.row, g.K - 1);
-      const int col = k == g.K - 1 ? o.col - (o.over ? o.over : 0) : o.col;
+      const int col = k == g.K - 1 ? o.col - o.over : o.col;
       r[i] = *reinterpret_cast<const u32x4_any*>(o.base + ((int64_t)k * g.ldb + col) * 2);
     } else {
       r[i] = *reinterpret_cast<const u32x4_any*>(o.base + (int64_t)(64 * p + 32 * i) * g.ldb * 2 + (uint32_t)o.src);
